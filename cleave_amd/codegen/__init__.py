@@ -49,6 +49,20 @@ def tail_requested(tile) -> bool:
     return bool(int(tile.get("TAIL", 0)))
 
 
+def phased_matmul(plan: KernelPlan, tile) -> bool:
+    """Which 256 x 256 products run on ``gemm_phased.hip`` (two wave groups alternating between memory and
+    matrix work) instead of the lock-step ``gemm_dma.hip``: all that it has a form for.  It needs eight waves
+    (two per SIMD, one multiplying while the other reads), at least the two K steps its pipeline holds, and rows
+    of C that leave as 16-byte pieces; the fused norm, the row-sum walk and the load and matrix-op knobs are the
+    lock-step kernel's.  us, lock-step / phased: 8192^3 bf16 (N, K) weight 806 / 695, 4096 x 14336 x 4096 f16 393 / 352
+    (with the last half round split), SwiGLU of that size 743 / 670, 3000 x 5000 x 2048 56 / 52; at the small end
+    2999 x 1000 x 192 9.8 / 8.2."""
+    p = plan.problem
+    return (tile["BM"] == tile["BN"] == 256 and tile["WM"] * tile["WN"] == 8 and tile["WN"] in (2, 4)
+            and plan.family in ("matmul", "swiglu") and p["K"] // (plan.split_factor or 1) >= 128 and p["N"] % 8 == 0
+            and int(tile.get("STAGES", 2)) == 2 and not {"ASM_LOADS", "ASM_MFMA", "SPREAD_LOADS"} & set(tile))
+
+
 def _c_param(p: ParamSpec) -> str:
     if p.role == "scalar":
         return f"{_C_TYPES[p.dtype]} {p.name}"
@@ -296,7 +310,7 @@ class HipCodeGen:
         if swiglu and (tile["BN"] // tile["WN"] // 16) % 2:
             raise CodegenError("a SwiGLU wave owns an even number of column fragments")
         batch = max(p["batch_A"], p["batch_B"])
-        unit.templates.append("gemm_dma.hip")
+        unit.templates += ["gemm_tile.hip", "gemm_phased.hip" if phased_matmul(plan, tile) else "gemm_dma.hip"]
         if partial:
             if tile["BK"] != 64 or p["K"] % (splits * 64):
                 raise CodegenError(f"K={p['K']} is not a multiple of splits*64={splits * 64}")
