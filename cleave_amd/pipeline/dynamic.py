@@ -335,6 +335,9 @@ class PagedKernel(Kernel):
                          input_shapes=[], **kernel_kw)
         self._compiled, self._argument_order = compiled, None
         self._by_role = {}               # "split" / "single" -> (compiled kernel, argument order), built on first use
+        self._plans = {}                 # role (None: the main kernel) -> native call plan, or False
+        kept = attention.inputs
+        self._n_kept, self._query_at = len(kept), next(i for i, p in enumerate(kept) if p.name == attention.query.name)
 
     # ---- persistence
     def save(self, path):
@@ -445,7 +448,42 @@ class PagedKernel(Kernel):
                 raise ValueError(f"{self.name}: page_size=1 reads no {p.name}; pass None")
         return bound
 
+    def _native_plan(self, role):
+        """The native call plan of the kernel that ``role`` names: arguments in the order of the inputs it reads."""
+        from ..runtime.dispatch import chain_plan
+
+        if role is None:
+            self.compile()
+            compiled, order = self._compiled, self._order()
+        else:
+            compiled, order = self._dispatched(0, role=role)
+        kept = list(self.attention.inputs)
+        declared = [p for p in compiled.params if p.role in ("input", "scalar")]
+        if compiled.out_idx is not None or len(declared) != len(order):
+            return False
+        position = {id(p): i for i, p in enumerate(kept)}
+        sources = {d.name: ("arg", position[id(p)]) for d, p in zip(declared, order)}
+        by_position = {position[id(p)]: d for d, p in zip(declared, order)}
+        return chain_plan([(compiled, sources)], arguments=[(by_position[i], None) for i in range(len(kept))], as_tuple=True) or False
+
     def __call__(self, *positional, longest=None, **named):
+        role, plan = None, False
+        if not named and len(positional) == self._n_kept:
+            # (a token rule, where one was made, decides before `longest` does)
+            role = self.token_role(positional[self._query_at].shape[0])
+            if role is None and longest is not None:
+                role = self.dispatch_role(longest)
+            plan = self._plans.get(role)
+            if plan:
+                done = plan(*positional)
+                if done is not NotImplemented:
+                    return done
+        done = self._checked_call(positional, longest, named)
+        if plan is None:                 # a first call of this kernel went through: later ones take the native plan
+            self._plans[role] = self._native_plan(role)
+        return done
+
+    def _checked_call(self, positional, longest, named):
         import torch
 
         bound = self._bind(positional, named)

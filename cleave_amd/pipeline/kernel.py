@@ -96,6 +96,7 @@ class Kernel:
         self.unrunnable = unrunnable
         self.meta = dict(meta or {})
         self._callables = None
+        self._plan = None                # the native call plan over all stages, made on the first call
 
     def __repr__(self):
         timing = f"{self.latency_us:.2f} us" if self.latency_us is not None else "?"
@@ -146,7 +147,52 @@ class Kernel:
                 raise ValueError(f"{self.name}: input {name!r} has shape {tuple(tensor.shape)}, expected {shape}")
         return list(positional)
 
+    def _native_plan(self):
+        """One native plan for the whole chain (the partials between stages are scratch of a call), or
+        False where a stage's shapes are not all known or do not line up."""
+        from types import SimpleNamespace
+
+        from ..runtime.dispatch import chain_plan
+
+        self.compile()
+        dtype_of: dict = {}
+        stages = []
+        for stage, kernel in zip(self.stages, self._callables):
+            shape_of = {p.name: tuple(p.shape) for p in kernel.params}
+            sources = {}
+            for p in stage.params:
+                origin_shape = None
+                if p.source == FROM_PROGRAM:
+                    if not 0 <= p.index < len(self.input_shapes):
+                        return False
+                    origin_shape = self.input_shapes[p.index]
+                    dtype_of.setdefault(p.index, next(q.dtype for q in kernel.params if q.name == p.name))
+                elif not stages or p.index >= sum(q.role == "output" for q in stages[-1][0].params):
+                    return False
+                declared = shape_of.get(p.name)
+                if declared is None or not all(isinstance(e, int) for e in declared) or (
+                        origin_shape is not None and math.prod(origin_shape) != math.prod(declared)):
+                    return False
+                sources[p.name] = ("arg" if p.source == FROM_PROGRAM else "stage", p.index)
+            if kernel.dyn_dims or any(p.role in ("input", "scalar") and p.name not in sources for p in kernel.params):
+                return False
+            stages.append((kernel, sources))
+        if set(dtype_of) != set(range(len(self.input_shapes))):
+            return False
+        arguments = [(SimpleNamespace(role="input", dtype=dtype_of[i]), shape) for i, shape in enumerate(self.input_shapes)]
+        return chain_plan(stages, arguments=arguments, output_shapes=self.output_shapes, as_tuple=True) or False
+
     def __call__(self, *positional, **named):
+        if self._plan and not named:
+            done = self._plan(*positional)
+            if done is not NotImplemented:
+                return done
+        done = self._checked_call(positional, named)
+        if self._plan is None:           # a first call went through: later ones take the native plan
+            self._plan = self._native_plan()
+        return done
+
+    def _checked_call(self, positional, named):
         from ..runtime.reference import order_inputs_for_kernel
 
         program_inputs = self._arguments(positional, named)

@@ -13,6 +13,7 @@ replaces the TVM adapter objects the reference's helpers poke at.
 from __future__ import annotations
 
 import ast
+import functools
 import hashlib
 import threading
 from dataclasses import dataclass
@@ -61,19 +62,24 @@ def _ceildiv(a, b):
     return -(-int(a) // int(b))
 
 
-def eval_extent(expr, dims: dict) -> int:
-    """Evaluate a grid extent: integers, dim names, ``+ - * // %`` and ``ceildiv/min/max``."""
-    if isinstance(expr, int):
-        return expr
-    tree = ast.parse(str(expr), mode="eval")
+@functools.lru_cache(maxsize=4096)
+def _compiled_extent(expr: str):
+    tree = ast.parse(expr, mode="eval")
     for node in ast.walk(tree):
         if not isinstance(node, _ALLOWED_NODES):
             raise CompileError(f"grid expression {expr!r} uses {type(node).__name__}")
         if isinstance(node, ast.Call) and not (isinstance(node.func, ast.Name) and node.func.id in ("ceildiv", "min", "max")):
             raise CompileError(f"grid expression {expr!r} calls something other than ceildiv/min/max")
+    return compile(tree, "<grid>", "eval")
+
+
+def eval_extent(expr, dims: dict) -> int:
+    """Evaluate a grid extent: integers, dim names, ``+ - * // %`` and ``ceildiv/min/max``."""
+    if isinstance(expr, int):
+        return expr
     env = {"ceildiv": _ceildiv, "min": min, "max": max, **dims}
     try:
-        return int(eval(compile(tree, "<grid>", "eval"), {"__builtins__": {}}, env))  # noqa: S307 - AST checked above
+        return int(eval(_compiled_extent(str(expr)), {"__builtins__": {}}, env))  # noqa: S307 - AST checked there
     except NameError as e:
         raise CompileError(f"grid expression {expr!r}: {e}") from e
 
@@ -136,7 +142,7 @@ class CompiledKernel:
         self.out_idx = None if out_idx is None else [int(i) for i in out_idx]
         self._code = code
         self._module = None
-        self._scratch = {}
+        self._plan = None                # the native call plan, made on the first call
         self._caller_params = [p for p in self.params if p.role != "scratch"]
         self._n_out = sum(p.role == "output" for p in self.params)
         if self.out_idx is not None:
@@ -249,11 +255,9 @@ class CompiledKernel:
             if p.role != "scratch":
                 continue
             owner = p.alias or p.name
-            shape = self._shape(p, dims)
-            key = (owner, shape, str(device))
-            if key not in self._scratch:
-                self._scratch[key] = fresh(shape, getattr(torch, p.dtype))
-            bound[p.name] = self._scratch[key]
+            if owner not in bound:
+                bound[owner] = fresh(self._shape(p, dims), getattr(torch, p.dtype))
+            bound[p.name] = bound[owner]
         return outs
 
     def _descs(self, bound, dims, fixed=None, refs=None):
@@ -290,6 +294,22 @@ class CompiledKernel:
 
     # ------------------------------------------------------------------ run
     def __call__(self, *args):
+        plan = self._plan
+        if plan:
+            done = plan(*args)
+            if done is not NotImplemented:
+                return done
+        done = self._checked_call(*args)
+        if plan is None:             # a first call went through: later ones take the native plan
+            from .dispatch import chain_plan
+
+            self._plan = chain_plan([(self, None)]) or False
+        return done
+
+    def _checked_call(self, *args):
+        """The call in Python, step by step: what a native plan does not take comes here, and leaves with the
+        reason if it is an error.  Scratch lives for the call only (torch's allocator gives it out again in
+        stream order), so calls on several streams or threads do not share it."""
         import torch
 
         bound, dims, device = self._bind(args)
@@ -349,11 +369,12 @@ class CompiledKernel:
         import torch
 
         sets = [args] + list(rotate or [])
-        all_descs, all_keep, held = [], [], []
+        all_descs, all_keep, held, buffers = [], [], [], []
         device = None
         for a in sets:
             bound, dims, device = self._bind(a)
             held.append(self._materialise(bound, dims, device))
+            buffers.append(bound)      # scratch included: the launches below hold its addresses
             if self.out_idx is not None:
                 for t in held[-1]:
                     t.zero_()      # the outputs are this call's own: whatever they hold afterwards, the timed launches wrote

@@ -1,0 +1,97 @@
+"""The native call path (``csrc/dispatch.cpp``) against the checked Python path it stands in for: same
+results bit for bit for fused pairs, chains of stages, caller-owned outputs and paged operators with
+run-time extents; the same errors where arguments do not fit; scratch of calls on different streams
+and threads kept apart."""
+
+import threading
+
+import pytest
+import torch
+
+import cleave_amd.lang as cl
+from cleave_amd import examples as C
+from cleave_amd import pipeline as P
+from cleave_amd.dynamic import reference as dref
+from cleave_amd.dynamic.paging import PAGED_DECODE_SLAB, CombineTiling, DenseAttention, PagingSpec, build_split_decode
+from cleave_amd.codegen import HipCodeGen
+from cleave_amd.pipeline.direct import kernel_for
+from cleave_amd.runtime.compile import _compile, _load_main_kernel_from_code
+
+pytestmark = pytest.mark.gpu
+SHAPES = dict(M=16, K=512, N=384)
+
+
+def _split_kernel():
+    kernel = kernel_for(C.rmsnorm_matmul.trace(cl.f16, **SHAPES), template="skinny", tiling=dict(WAVES_N=1, WAVES_K=2), split=4)
+    args = [t.cuda() for t in C.inputs_c2(SHAPES)]
+    want = kernel(*args)                       # (the first call goes the checked way and leaves a plan)
+    assert kernel._plan
+    return kernel, args, want
+
+
+def test_fused_pair_and_its_errors():
+    kernel, args, want = _split_kernel()
+    assert torch.equal(kernel(*args), want) and torch.equal(kernel._checked_call(*args), want)
+    with pytest.raises(TypeError, match="expects 3 arguments"):
+        kernel(*args[:2])
+    with pytest.raises(TypeError, match="dtype"):
+        kernel(args[0].float(), *args[1:])
+    with pytest.raises(ValueError, match="contiguous"):
+        kernel(args[0].t().contiguous().t(), *args[1:])
+    with pytest.raises(ValueError, match="shape"):
+        kernel(args[0][:8], *args[1:])
+    with pytest.raises(ValueError, match="only run on the GPU"):
+        kernel(args[0].cpu(), *args[1:])
+    with pytest.raises(TypeError, match="torch tensor"):
+        kernel(None, *args[1:])
+
+
+def test_chain_of_stages_is_one_plan(cache_root):
+    kernel = P.compile(C.rmsnorm_matmul, shapes=SHAPES, dtype=cl.f16, split=cl.Split("K", (4,)), cache_kernels=False,
+                       schedule=P.ScheduleConfig(topk=2, split_k=(4,)), eval=P.EvalConfig(warmup=1, iters=3, max_parallel=0))
+    chain = next(k for k in (kernel, *kernel.report.contenders(top=8, within=100.0)) if len(k.stages) == 2)
+    args = [t.cuda() for t in C.inputs_c2(SHAPES)]
+    want = chain(*args)
+    assert chain._plan and torch.equal(chain(*args), want) and torch.equal(chain(x=args[0], gamma=args[1], w=args[2]), want)
+    with pytest.raises(ValueError, match="expected"):
+        chain(args[0][:8], *args[1:])
+
+
+def test_paged_pair_with_caller_owned_outputs_and_run_time_extents():
+    spec = PagingSpec(num_qo_heads=32, num_kv_heads=8, kind=PAGED_DECODE_SLAB, page_size=64)
+    dense = DenseAttention(16, 32, 128, 512, "float16", "float16", waves=8, chunk_pages=-1, lockstep=True)
+    source = HipCodeGen().gen(build_split_decode(spec, dense, 8, CombineTiling(split=8)))
+    kernel = _compile(_load_main_kernel_from_code(source), None)
+    for lens in ([1], [70, 500, 64], [3000, 1, 200, 65, 64, 1000, 129]):
+        pages = sum(-(-n // 64) for n in lens)
+        args = dref.gqa_paged_decode_inputs((len(lens), 32, 8, 128, pages + 3, pages), lens, page_size=64, dtype=torch.float16)
+        got, checked = ([torch.full((len(lens), 32, 128), float("nan"), dtype=torch.float16, device="cuda"),
+                         torch.full((len(lens), 32), float("nan"), device="cuda")] for _ in range(2))
+        assert kernel._checked_call(*args, *checked) is None and kernel(*args, *got) is None
+        assert torch.equal(got[0], checked[0]) and torch.equal(got[1], checked[1]) and bool(torch.isfinite(got[1]).all())
+    assert kernel._plan
+    with pytest.raises(ValueError, match="conflicts"):
+        kernel(*args, got[0][:2], got[1])
+
+
+def test_threads_on_their_own_streams_do_not_share_scratch():
+    kernel, args, _ = _split_kernel()
+    inputs = [[t + 0 for t in args] for _ in range(4)]
+    for i, ins in enumerate(inputs):
+        ins[0] = ins[0] * (i + 1) + i
+    wants = [kernel(*ins) for ins in inputs]
+    torch.cuda.synchronize()
+    wrong = []
+
+    def work(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            outs = [kernel(*inputs[i]) for _ in range(50)]
+            torch.cuda.current_stream().synchronize()
+        wrong.extend(i for o in outs if not torch.equal(o, wants[i]))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
