@@ -617,7 +617,9 @@ class HipCodeGen:
         vsplit = int(t.get("VSPLIT", 1))
         if waves not in (1, 2, 4, 8):
             raise CodegenError("the MLA template runs 1, 2, 4 or 8 waves per workgroup")
-        if waves % vsplit or p["heads"] % (16 * hg * waves // vsplit) or (p["ckv"] // 16) % (4 * vsplit):
+        # (a combine on its own has no wave grid: held to the default four waves of 16 heads, operators of 16 or 32
+        # heads had no split form at all)
+        if partial and (waves % vsplit or p["heads"] % (16 * hg * waves // vsplit) or (p["ckv"] // 16) % (4 * vsplit)):
             raise CodegenError(f"{p['heads']} heads / {p['ckv']} features do not divide into {waves} waves of "
                                f"{16 * hg} heads sharing a head set by {vsplit}")
         if p["ckv"] % 64 or p["kpe"] % 64:
