@@ -154,49 +154,117 @@ def resolve_workloads(attention, workloads=None, tolerance=None):
     raise TypeError(f"workloads must be a cl.workloads spec or a factory, got {workloads!r}")
 
 
+def crossing(low: int, low_ratio: float, high: int, high_ratio: float) -> int:
+    """The first tile count in (``low``, ``high``] at which the split pair is the faster one, with its time over the
+    single kernel's given at both ends and taken as a power of the tile count between them.  (Workloads of 16
+    and 384 tiles used to put the threshold at 384: seven requests of up to 96 tiles ran the single kernel in
+    31 us where the pair takes 17.)"""
+    if low_ratio <= 1.0 or high_ratio >= 1.0:          # no change of sides between them: the middle
+        at = math.sqrt(low * high)
+    else:
+        at = low * (high / low) ** (math.log(low_ratio) / (math.log(low_ratio) - math.log(high_ratio)))
+    return min(high, max(low + 1, math.ceil(at)))
+
+
+def split_threshold(tiles: dict, split_us: dict, single_us: dict) -> int:
+    """The tile count from which the split pair runs, with the smallest geometric-mean time over the workloads
+    timed (the lower one on a tie).  All thresholds between two neighbouring workloads share that mean; the one
+    taken is where the two kernels' times cross between them."""
+    from ..runtime.autotune import geomean
+
+    keys = [k for k in tiles if k in split_us and k in single_us]
+    seen = sorted({tiles[k] for k in keys})
+
+    def cost(threshold):
+        return geomean([(split_us if tiles[k] >= threshold else single_us)[k] for k in keys])
+
+    def ratio(at):
+        return geomean([split_us[k] / single_us[k] for k in keys if tiles[k] == at])
+
+    best = min(sorted({*seen, 1, max(seen) + 1}), key=lambda t: (cost(t), t))
+    if best in seen[1:]:
+        below = seen[seen.index(best) - 1]
+        best = crossing(below, ratio(below), best, ratio(best))
+    return int(best)
+
+
+def lone_request(kernel, inputs, expected, indptr_at):
+    """A workload cut down to its longest request: the extents of every input are known by their names in
+    the kernel's parameters (the batch, its row pointers, its slice of the page table; caches stay whole)."""
+    bounds = inputs[indptr_at].tolist()
+    b = max(range(len(bounds) - 1), key=lambda r: bounds[r + 1] - bounds[r])
+    declared = [p for p in kernel.params if p.role in ("input", "scalar")]
+    named = {declared[indptr_at].shape[0]: len(bounds)}
+    batch, lo, hi = len(bounds) - 1, bounds[b], bounds[b + 1]
+    cut = []
+    for p, value in zip(declared, inputs):
+        if p.role == "scalar":
+            cut.append(value)
+        elif p.shape[0] in named:
+            cut.append(value[b:b + 2] - value[b])
+        elif len(p.shape) == 1 and not isinstance(p.shape[0], int) and value.shape[0] >= hi and value.shape[0] != batch:
+            cut.append(value[lo:hi].contiguous())
+        elif value.shape[0] == batch:
+            cut.append(value[b:b + 1].contiguous())
+        else:
+            cut.append(value)
+    return cut, [t[b:b + 1].contiguous() for t in expected]
+
+
 def calibrate_dispatch(pair, solo, factory, spec) -> dict:
     """When should a call run the split pair rather than the single kernel?
 
-    Both are timed on every workload.  A workload is described by one number, the kv tiles of its
-    longest request (``indptr`` units x page size / kv tile, rounded up); the rule is "split from
-    ``min_tiles`` tiles on", and ``min_tiles`` is the threshold with the smallest geometric-mean
-    time over the workloads (the smaller threshold on a tie)."""
+    Both are timed on every workload.  A workload is described by the kv tiles of its longest request
+    (``indptr`` units x page size / kv tile, rounded up), and the rule is "split from ``min_tiles`` tiles on".
+    The single kernel has one workgroup per request and kv head, so what a split is worth also depends on
+    whether those fill the chip: for batches of fewer than ``few_requests`` requests (workgroups for less than
+    a quarter of the compute units; 18 requests of up to 1056 tokens, 144 workgroups, still run 16 us unsplit and
+    22 split) the threshold is ``lone_tiles``, calibrated on each workload's longest request
+    alone.  (With one threshold, taken from batches of 64 requests, three requests of up to 2882 tokens ran the
+    single kernel in 26 us where the pair takes 11.)"""
     import dataclasses
 
+    from ..core.target import current_target
     from ..runtime.autotune import benchmark_over_workloads, geomean, param_index
 
     pair, solo = dataclasses.replace(pair, latency_us={}), dataclasses.replace(solo, latency_us={})
     indptr_at = param_index(solo.kernel, f"PlaceHolder_{spec.indptr_input}")
     tokens_per_unit, kv_tile = int(getattr(spec, "page_size", 1)), int(pair.tiling.kv_tile)
-    longest = {}
+    longest, requests = {}, {}
 
     def observed():
         for key, inputs, expected in factory(0)():
             bounds = inputs[indptr_at].tolist()
             units = max(hi - lo for lo, hi in zip(bounds, bounds[1:]))
-            longest[key] = math.ceil(units * tokens_per_unit / kv_tile)
+            longest[key], requests[key] = math.ceil(units * tokens_per_unit / kv_tile), len(bounds) - 1
             yield key, inputs, expected
 
+    def alone():
+        for key, inputs, expected in factory(0)():
+            yield (key, *lone_request(solo.kernel, inputs, expected, indptr_at))
+
     benchmark_over_workloads([pair, solo], observed, ramp_seconds=0.2)
+    min_tiles = split_threshold(longest, pair.latency_us, solo.latency_us)
+    few_requests = current_target().arch.compute_units // (4 * int(getattr(spec, "num_kv_heads", 1))) + 1
+    lone_pair, lone_solo = dataclasses.replace(pair, latency_us={}), dataclasses.replace(solo, latency_us={})
+    benchmark_over_workloads([lone_pair, lone_solo], alone, ramp_seconds=0.0)
+    lone_tiles = split_threshold(longest, lone_pair.latency_us, lone_solo.latency_us)
     keys = [k for k in longest if k in pair.latency_us and k in solo.latency_us]
 
-    def chosen(key, threshold):
-        return pair if longest[key] >= threshold else solo
+    def splits(key):
+        return longest[key] >= (lone_tiles if requests[key] < few_requests else min_tiles)
 
-    def cost(threshold):
-        return geomean([chosen(k, threshold).latency_us[k] for k in keys])
-
-    thresholds = sorted({longest[k] for k in keys} | {1, max(longest.values()) + 1})
-    min_tiles = min(thresholds, key=lambda t: (cost(t), t))
+    per_workload = {k: (pair if splits(k) else solo).latency_us[k] for k in keys}
     return {
-        "rule": "run the split pair when the longest request has at least min_tiles KV tiles "
-                "(indptr units x page_size tokens / kv_tile), else the single kernel",
-        "min_tiles": int(min_tiles), "kv_tile": kv_tile, "page_size": tokens_per_unit, "indptr_index": indptr_at,
+        "rule": "run the split pair when the longest request has at least min_tiles KV tiles (lone_tiles for batches of fewer "
+                "than few_requests requests; indptr units x page_size tokens / kv_tile), else the single kernel",
+        "min_tiles": min_tiles, "lone_tiles": lone_tiles, "few_requests": few_requests, "kv_tile": kv_tile,
+        "page_size": tokens_per_unit, "indptr_index": indptr_at,
         "split_label": pair.label, "single_label": solo.label,
-        "n_workloads": len(keys), "split_runs": sum(longest[k] >= min_tiles for k in keys),
-        "geomean_us": {"hybrid": cost(min_tiles), "split": geomean([pair.latency_us[k] for k in keys]),
+        "n_workloads": len(keys), "split_runs": sum(map(splits, keys)),
+        "geomean_us": {"hybrid": geomean(list(per_workload.values())), "split": geomean([pair.latency_us[k] for k in keys]),
                        "single": geomean([solo.latency_us[k] for k in keys])},
-        "per_workload_us": {k: chosen(k, min_tiles).latency_us[k] for k in keys},
+        "per_workload_us": per_workload,
     }
 
 
@@ -398,13 +466,15 @@ class PagedKernel(Kernel):
             self._argument_order = self._order_for(self._compiled)
         return self._argument_order
 
-    def dispatch_role(self, longest: int) -> str:
-        """``"split"`` or ``"single"`` for a batch whose longest request spans ``longest`` page-table
-        units, by the calibrated rule (kv tiles of the longest request against ``min_tiles``)."""
+    def dispatch_role(self, longest: int, requests: int | None = None) -> str:
+        """``"split"`` or ``"single"`` for a batch of ``requests`` requests whose longest spans ``longest``
+        page-table units, by the calibrated rule (kv tiles of the longest request against ``min_tiles``, or
+        ``lone_tiles`` where the requests are too few to fill the chip)."""
         if not self.dispatch or set(self.dispatch_sources) < {"split", "single"}:
             raise CleaveError(f"{self.name}: no split / single calibration was made (or saved) for this operator")
         tiles = math.ceil(int(longest) * int(self.dispatch["page_size"]) / int(self.dispatch["kv_tile"]))
-        return "split" if tiles >= int(self.dispatch["min_tiles"]) else "single"
+        few = requests is not None and requests < int(self.dispatch.get("few_requests", 0))
+        return "split" if tiles >= int(self.dispatch["lone_tiles" if few else "min_tiles"]) else "single"
 
     def token_role(self, tokens: int):
         """``"few"`` or ``"many"`` for a call with ``tokens`` packed query tokens, by the rule
@@ -472,7 +542,7 @@ class PagedKernel(Kernel):
             # (a token rule, where one was made, decides before `longest` does)
             role = self.token_role(positional[self._query_at].shape[0])
             if role is None and longest is not None:
-                role = self.dispatch_role(longest)
+                role = self.dispatch_role(longest, positional[self._query_at].shape[0])
             plan = self._plans.get(role)
             if plan:
                 done = plan(*positional)
@@ -494,7 +564,7 @@ class PagedKernel(Kernel):
             self.compile()
             compiled, order = self._compiled, self._order()
         else:
-            compiled, order = self._dispatched(longest)
+            compiled, order = self._dispatched(longest, role=self.dispatch_role(longest, bound[self.attention.query.name].shape[0]))
         sizes = {}
         for p in self.attention.inputs:
             if not p.is_scalar:

@@ -356,3 +356,30 @@ def test_token_threshold_of_the_prefill_dispatch():
     t, _ = pick_token_threshold(winner, {"a": 3.0, "b": 9.0, "c": 14.0, "d": 600.0}, tokens)
     assert t == 1
     assert pick_token_threshold(winner, {"x": 1.0}, tokens) == (None, float("inf"))
+
+
+def test_split_threshold_lies_where_the_times_cross():
+    """The dispatch threshold between two neighbouring workloads is put where the two kernels' times cross, not on
+    the longer of the two; without a change of sides it stays at the ends."""
+    from cleave_amd.pipeline.dynamic import crossing, split_threshold
+
+    tiles = {"a": 4, "b": 16, "c": 256}
+    single = {"a": 5.0, "b": 6.0, "c": 60.0}
+    assert split_threshold(tiles, {"a": 7.0, "b": 8.0, "c": 15.0}, single) == crossing(16, 8 / 6, 256, 15 / 60) in range(17, 64)
+    assert split_threshold(tiles, {k: 1.5 * v for k, v in single.items()}, single) == 257      # never
+    assert split_threshold(tiles, {k: 0.5 * v for k, v in single.items()}, single) == 1         # always
+    assert crossing(16, 1.3, 17, 0.9) == 17 and crossing(4, 2.0, 16, 0.5) == 8
+
+
+def test_lone_request_keeps_one_requests_rows_and_table():
+    from cleave_amd.pipeline.dynamic import lone_request
+    from cleave_amd.runtime.compile import _load_main_kernel_from_code
+    from cleave_amd.dynamic import OPERATORS
+
+    loaded = _load_main_kernel_from_code(OPERATORS["gqa_paged_decode_h32_kv8_d128_ps64"].kernel_source())
+    q, cache = torch.arange(3.0)[:, None, None].expand(3, 32, 128), torch.zeros(9, 64, 8, 128)
+    inputs = [q, cache, cache, torch.tensor([0, 2, 6, 7]), torch.arange(7), torch.tensor([5, 6, 7]), 0.1]
+    cut, expected = lone_request(loaded, inputs, [q], 3)
+    assert cut[0].shape[0] == 1 and float(cut[0][0, 0, 0]) == 1.0 and cut[1] is cache and cut[6] == 0.1
+    assert cut[3].tolist() == [0, 4] and cut[4].tolist() == [2, 3, 4, 5] and cut[5].tolist() == [6]
+    assert float(expected[0][0, 0, 0]) == 1.0
