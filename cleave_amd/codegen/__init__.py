@@ -49,20 +49,6 @@ def tail_requested(tile) -> bool:
     return bool(int(tile.get("TAIL", 0)))
 
 
-def phased_matmul(plan: KernelPlan, tile) -> bool:
-    """Which 256 x 256 products run on ``gemm_phased.hip`` (two wave groups alternating between memory and
-    matrix work) instead of the lock-step ``gemm_dma.hip``: all that it has a form for.  It needs eight waves
-    (two per SIMD, one multiplying while the other reads), at least the two K steps its pipeline holds, and rows
-    of C that leave as 16-byte pieces; the fused norm, the row-sum walk and the load and matrix-op knobs are the
-    lock-step kernel's.  us, lock-step / phased: 8192^3 bf16 (N, K) weight 806 / 695, 4096 x 14336 x 4096 f16 393 / 352
-    (with the last half round split), SwiGLU of that size 743 / 670, 3000 x 5000 x 2048 56 / 52; at the small end
-    2999 x 1000 x 192 9.8 / 8.2."""
-    p = plan.problem
-    return (tile["BM"] == tile["BN"] == 256 and tile["WM"] * tile["WN"] == 8 and tile["WN"] in (2, 4)
-            and plan.family in ("matmul", "swiglu") and p["K"] // (plan.split_factor or 1) >= 128 and p["N"] % 8 == 0
-            and int(tile.get("STAGES", 2)) == 2 and not {"ASM_LOADS", "ASM_MFMA", "SPREAD_LOADS"} & set(tile))
-
-
 def _c_param(p: ParamSpec) -> str:
     if p.role == "scalar":
         return f"{_C_TYPES[p.dtype]} {p.name}"
@@ -263,6 +249,9 @@ class HipCodeGen:
 
     def _emit_gemm(self, unit, plan, params, partial, combine, fused):
         p, t = plan.problem, plan.tiling
+        if int(t.get("DMA", 0)):
+            # the direct-to-LDS form for a contraction whose last 64-wide step is partly filled
+            return self._emit_gemm_dma(unit, plan, params, partial, combine, fused)
         self._matmul_common(unit, plan, params, partial, combine, fused)
         tile = dict(BM=64, BN=64, BK=64, WM=1, WN=1)
         tile.update(t)
@@ -295,7 +284,7 @@ class HipCodeGen:
             raise CodegenError(f"the direct-to-LDS matmul template has no {plan.family} form")
         self._matmul_common(unit, plan, params, partial, combine, fused)
         tile = dict(BM=128, BN=128, BK=64, WM=2, WN=2)
-        tile.update(t)
+        tile.update({k: v for k, v in t.items() if k != "DMA"})
         for k, v in tile.items():
             unit.define(f"CL_{k}", v)
         splits = plan.split_factor or 1
@@ -310,10 +299,12 @@ class HipCodeGen:
         if swiglu and (tile["BN"] // tile["WN"] // 16) % 2:
             raise CodegenError("a SwiGLU wave owns an even number of column fragments")
         batch = max(p["batch_A"], p["batch_B"])
-        unit.templates += ["gemm_tile.hip", "gemm_phased.hip" if phased_matmul(plan, tile) else "gemm_dma.hip"]
+        from ..schedule.policy import phased_matmul
+
+        unit.templates += ["gemm_tile.hip", "gemm_phased.hip" if phased_matmul(plan.family, p, splits, tile) else "gemm_dma.hip"]
         if partial:
-            if tile["BK"] != 64 or p["K"] % (splits * 64):
-                raise CodegenError(f"K={p['K']} is not a multiple of splits*64={splits * 64}")
+            if tile["BK"] != 64 or (p["K"] % (splits * 64) and (splits > 1 or p["K"] % 8 or plan.family not in ("matmul", "rmsnorm_matmul"))):
+                raise CodegenError(f"K={p['K']} is neither a multiple of splits*64={splits * 64} nor, for an unsplit product, of 8")
             if (not p["trans_B"] and p["N"] % 8) or (p["trans_A"] and p["M"] % 8) or p["K"] % 8:
                 raise CodegenError("16-byte global chunks need the minor extent of each operand to be a multiple of 8")
             grid = (1 if rowsum else -(-p["N"] // out_bn), -(-p["M"] // tile["BM"]), batch * splits)

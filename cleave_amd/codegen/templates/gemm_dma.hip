@@ -134,7 +134,7 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
   const int batch = blockIdx.z / CL_SPLITS, split = blockIdx.z % CL_SPLITS;
   constexpr int k_per_split = CL_K / CL_SPLITS;
   const int k_begin = split * k_per_split;
-  constexpr int KT_K = k_per_split / GD_BK;                     // steps along K
+  constexpr int KT_K = (k_per_split + GD_BK - 1) / GD_BK;       // steps along K (the last one partly filled: GD_K_LEFT)
   constexpr int KT = KT_K * (CL_ROWSUM ? CL_N / CL_BN : 1);     // ... times the column tiles one workgroup walks
 #if CL_ROWSUM
   static_assert(CL_N % CL_BN == 0 && CL_SPLITS == 1 && GD_BATCH == 1, "row sums walk whole column tiles, unsplit");
@@ -277,17 +277,24 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
 #define GD_A_AT(kt) (a_base + (i64)(kt) * a_step)
 #define GD_B_AT(kt) (b_base + (i64)(kt) * b_step)
 #endif
-#define GD_ISSUE(kt, a_lds, b_lds)                              \
-  opa.issue(GD_A_AT(kt), GD_LDS_BYTE(a_lds), wave_byte);        \
-  opb.issue(GD_B_AT(kt), GD_LDS_BYTE(b_lds), wave_byte);        \
+#define GD_LEFT_AT(kt) (GD_K_LEFT > 0 && (kt) % KT_K == KT_K - 1)
+#define GD_ISSUE(kt, a_lds, b_lds)                                  \
+  if (GD_LEFT_AT(kt)) {                                             \
+    opa.issue_left(GD_A_AT(kt), GD_LDS_BYTE(a_lds), wave_byte);     \
+    opb.issue_left(GD_B_AT(kt), GD_LDS_BYTE(b_lds), wave_byte);     \
+  } else {                                                          \
+    opa.issue(GD_A_AT(kt), GD_LDS_BYTE(a_lds), wave_byte);          \
+    opb.issue(GD_B_AT(kt), GD_LDS_BYTE(b_lds), wave_byte);          \
+  }                                                                 \
   __builtin_amdgcn_sched_barrier(0);
 #define GD_ISSUE_SLICE(r, kt, a_lds, b_lds)                                                         \
   {                                                                                                 \
     constexpr int ua_ = decltype(opa)::PER, ub_ = decltype(opb)::PER;                               \
     constexpr int per_row_ = (ua_ + ub_ + 2 * TM - 1) / (2 * TM);                             \
     _Pragma("unroll") for (int q_ = (r) * per_row_; q_ < ((r) + 1) * per_row_; ++q_) {             \
-      if (q_ < ua_) opa.issue_unit(q_, GD_A_AT(kt), GD_LDS_BYTE(a_lds), wave_byte);                 \
-      else if (q_ < ua_ + ub_) opb.issue_unit(q_ - ua_, GD_B_AT(kt), GD_LDS_BYTE(b_lds), wave_byte); \
+      if (q_ < ua_) opa.issue_unit_of(q_, GD_A_AT(kt), GD_LDS_BYTE(a_lds), wave_byte, GD_LEFT_AT(kt)); \
+      else if (q_ < ua_ + ub_)                                                                      \
+        opb.issue_unit_of(q_ - ua_, GD_B_AT(kt), GD_LDS_BYTE(b_lds), wave_byte, GD_LEFT_AT(kt));    \
     }                                                                                               \
   }
 #define GD_NO_NEXT(r)

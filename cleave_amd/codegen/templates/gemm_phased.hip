@@ -1,15 +1,15 @@
 // ---- MFMA matmul in two wave groups that alternate between memory and matrix work ----------------
 //
-// C[M, N] = A[M, K] * B[K, N] on 256 x 256 tiles, eight waves (two per SIMD), K in steps of 64,
-// tiles global -> LDS directly.  The lock-step kernel (gemm_dma.hip) lets all eight waves load,
-// read and multiply at the same time: after every barrier both waves of a SIMD stand in their tile
-// loads and operand reads with the matrix unit idle (2870 clocks a step for 2048 of matrix work).
-// Here a step is four phases, each one memory part and one matrix part, and waves 4-7 run one part
+// C[M, N] = A[M, K] * B[K, N] on 256 x 256, 128 x 256 or 256 x 128 tiles, eight waves (two per SIMD), K in
+// steps of 64, tiles global -> LDS directly.  The lock-step kernel (gemm_dma.hip) lets all eight waves
+// load, read and multiply at the same time: after every barrier both waves of a SIMD stand in their tile
+// loads and operand reads with the matrix unit idle (2870 clocks a 256 x 256 step for 2048 of matrix work).
+// Here a step is cut into phases, each one memory part and one matrix part, and waves 4-7 run one part
 // behind waves 0-3: on every SIMD one wave reads its next operands and asks for tiles while the
 // other's sixteen matrix ops (256 clocks) own the matrix unit, then they trade.
 //
-// The 64 KiB of a step are four half tiles (A rows 0-127 and 128-255, B columns likewise); a wave's
-// 128 x 64 outputs are 64 x 32 quadrants of every pair of halves, one per phase:
+// A step's tiles are four halves (upper and lower rows of A, left and right columns of B), and a wave owns
+// the same part of every pair of halves.  256 x 256 (GP_QUADS), one pair of halves per phase:
 //
 //   phase   multiplies   reads for it (memory part)   asks for (two steps ahead)
 //     1      A0 B0        A0                           B0
@@ -17,30 +17,37 @@
 //     3      A1 B1        A1                           B1
 //     4      A1 B0        B0 of the next step          A1
 //
+// The smaller tiles have half the matrix ops, so a phase takes both B halves:
+//
+//     1      A0 B0, A0 B1   A0, B1                     A1 of the next step, B0 of the one after
+//     2      A1 B0, A1 B1   A1, B0 of the next step    A0, B1 of the one after
+//
 // A half is read exactly once per step, by both groups before the barrier that closes the later
 // group's memory part; one phase on its LDS slot is free and its successor two steps on is asked
-// for.  So two stages hold loads that are seven phases (1.75 steps) ahead of their use, two loads
-// per wave and phase, never a burst; the wait in front of a half's phase counts the six halves
-// asked for after it (gp_wait).
+// for.  So two stages hold loads that are 1.75 (1.5) steps ahead of their use, a few per wave and phase,
+// never a burst; the wait in front of a half's phase counts the loads asked for after it (gp_wait).
 //
-// Measured, 8192^3 bf16 with a (N, K) weight: 695 us (1.58 PFLOP/s) against 806 lock-step; the matrix unit is
+// Measured, 8192^3 bf16 with a (N, K) weight: 701 us (1.57 PFLOP/s) against 806 lock-step; the matrix unit is
 // busy 86 % of the clocks (70 % lock-step) at 1.76 GHz (1.96): what bounds it is the power the matrix ops
 // draw on random operands.  A (K, N) weight runs at the same speed: its transposing reads hide in the memory
-// parts.  4096 x 14336 x 4096: 352 us (393), SwiGLU of that size 670 (743).
+// parts.  4096 x 14336 x 4096: 352 us (393), SwiGLU of that size 676 (752); with two phases a step instead of four
+// these take 1 % longer.  128 x 256 tiles on 2048 x 4096 x 4096: 56.3 us (60.1 lock-step with three stages), 256 x 128 on
+// 724 x 6272 x 640: 10.7 us (13.3).
 //
-//   CL_BM = CL_BN = 256, CL_WM x CL_WN = 8 waves; CL_TRANS_A / CL_TRANS_B, CL_BATCH_A/B, CL_SPLITS,
-//   CL_TAIL, CL_SWIGLU (B half 1 = the gate weight's columns) as in gemm_dma.hip.
+//   CL_BM, CL_BN, CL_WM x CL_WN = 8 waves; CL_TRANS_A / CL_TRANS_B, CL_BATCH_A/B, CL_SPLITS, CL_TAIL (256 x 256
+//   only), CL_SWIGLU (B half 1 = the gate weight's columns) as in gemm_dma.hip.
 
-static_assert(GD_WAVES == 8 && CL_BM == 256 && CL_BN == 256, "the phased matmul: 256 x 256 tiles on eight waves");
+#define GP_QUADS (CL_BM == 256 && CL_BN == 256)
+static_assert(GD_WAVES == 8 && CL_BM % 128 == 0 && CL_BN % 128 == 0, "the phased matmul: eight waves, halves of whole 64-row pieces");
 static_assert(CL_N % 8 == 0, "rows of C leave as 16-byte pieces");
 #if CL_NORM || CL_ROWSUM
 #error "the phased matmul has no fused norm and no row-sum walk"
 #endif
 
-#define GP_HN 128                                      // columns of a B half
+#define GP_HN (CL_BN / 2)                              // columns of a B half
 #define GP_TNH (GP_HN / CL_WN / 16)                    // column fragments per wave and half
 static_assert(GP_TNH % 2 == 0, "the epilogue pairs column fragments");
-#define GP_SLOT (128 * GD_BK)                          // elements of a half tile's image
+#define GP_SLOT ((CL_BM > CL_BN ? CL_BM : CL_BN) / 2 * GD_BK)   // elements of a half tile's image
 __shared__ __attribute__((aligned(1024))) elem_t gp_lds[8 * GP_SLOT];
 // (B's four images below A's: what one lane pattern reads of an operand lies within the 64 KiB that
 // the offset field of an LDS instruction reaches)
@@ -88,7 +95,7 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
   const int batch = blockIdx.z / CL_SPLITS, split = blockIdx.z % CL_SPLITS;
   constexpr int k_per_split = CL_K / CL_SPLITS;
   const int k_begin = split * k_per_split;
-  constexpr int KT = k_per_split / GD_BK;
+  constexpr int KT = (k_per_split + GD_BK - 1) / GD_BK;   // (the last one partly filled: GD_K_LEFT)
   static_assert(KT >= 2, "two stages are asked for ahead of the loop");
 
   const elem_t* A = CL_ARG_A + (i64)(batch / (GD_BATCH / CL_BATCH_A)) * CL_M * CL_K;
@@ -181,16 +188,18 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
       for (int v = 0; v < 2; ++v)
 #pragma unroll
         for (int j = 0; j < GP_TNH; ++j) acc[h][i][v][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  elem8 fa[2][TMH], fx[2][GP_TNH], fy[2][GP_TNH];   // fx / fy: B0 and B1 of a step, trading names every step
+  elem8 fa[2][TMH], fb1[2][GP_TNH], fx[2][GP_TNH], fy[2][GP_TNH];   // fx / fy: B0 of a step and of the next, trading names
 
-#define GP_READ_A(stage, item)                                                 \
-  _Pragma("unroll") for (int s = 0; s < 2; ++s)                                \
+#define GP_READ_A(stage, item)                                                                      \
+  _Pragma("unroll") for (int s = 0; s < 2; ++s)                                                     \
   _Pragma("unroll") for (int i = 0; i < TMH; ++i) fa[s][i] = GP_AFRAG((stage) * 2 + ((item) & 1), i, s);
-#define GP_READ_B(f, stage, item)                                              \
-  _Pragma("unroll") for (int s = 0; s < 2; ++s)                                \
+#define GP_READ_B(f, stage, item)                                                                   \
+  _Pragma("unroll") for (int s = 0; s < 2; ++s)                                                     \
   _Pragma("unroll") for (int j = 0; j < GP_TNH; ++j) f[s][j] = GP_BFRAG((stage) * 2 + ((item) & 1), j, s);
 #define GP_LOAD(op, base, stage, item) op.issue(base, GD_LDS_BYTE(GP_IMG(stage, item)), wave_byte);
+#define GP_LOAD_LEFT(op, base, stage, item) op.issue_left(base, GD_LDS_BYTE(GP_IMG(stage, item)), wave_byte);
 #define GP_NONE
+#if GP_QUADS
   // One phase: the memory part (operand reads, loads, the wait for both the reads and the half the
   // next phase reads), and behind a barrier the matrix part.
 #define GP_PHASE(READS, LOADS, left, ha, hb, f)                                                     \
@@ -210,49 +219,109 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
   // A step on stage S with loads two steps ahead (six halves stay in flight at every wait).  B0 is in
   // `p` already; B1 goes into `q`, and after its last use (phase 3) so does B0 of the next step.
 #define GP_STEP_(S, p, q, L1, L2, L3, L4, w1, w2, w3, w4, NEXT)                                     \
-  GP_PHASE(GP_READ_A(S, GP_A0), L1, w1, 0, 0, p)                                            \
-  GP_PHASE(GP_READ_B(q, S, GP_B1), L2, w2, 0, 1, q)                                         \
-  GP_PHASE(GP_READ_A(S, GP_A1), L3, w3, 1, 1, q)                                            \
+  GP_PHASE(GP_READ_A(S, GP_A0), L1, w1, 0, 0, p)                                                    \
+  GP_PHASE(GP_READ_B(q, S, GP_B1), L2, w2, 0, 1, q)                                                 \
+  GP_PHASE(GP_READ_A(S, GP_A1), L3, w3, 1, 1, q)                                                    \
   GP_PHASE(NEXT, L4, w4, 1, 0, p)
 #define GP_NEXT(S, q) GP_READ_B(q, 1 - (S), GP_B0)
-#define GP_STEP(S, p, q)                                                                            \
-  GP_STEP_(S, p, q, GP_LOAD(opb0, pb0, S, GP_B0), GP_LOAD(opa0, pa, S, GP_A0), GP_LOAD(opb1, pb1, S, GP_B1), \
-           GP_LOAD(opa1, pa, S, GP_A1), 3 * (la + lb), 3 * (la + lb), 3 * (la + lb), 3 * (la + lb), GP_NEXT(S, q)) \
+#define GP_STEP(S, p, q, NEXT_STEP, LATER_, LATER)                                                  \
+  GP_STEP_(S, p, q, LATER(opb0, pb0, S, GP_B0), LATER(opa0, pa, S, GP_A0), LATER(opb1, pb1, S, GP_B1), LATER(opa1, pa, S, GP_A1), \
+           3 * (la + lb), 3 * (la + lb), 3 * (la + lb), 3 * (la + lb), GP_NEXT(S, q))               \
   pa += a_step; pb0 += b_step; pb1 += b_step;
   // The last two steps ask for nothing more: the waits count down what is still on its way.
 #define GP_STEP_LAST2(S, p, q)                                                                      \
   GP_STEP_(S, p, q, GP_NONE, GP_NONE, GP_NONE, GP_NONE, 3 * la + 2 * lb, 2 * la + 2 * lb, 2 * la + lb, la + lb, GP_NEXT(S, q))
-#define GP_STEP_LAST(S, p, q) GP_STEP_(S, p, q, GP_NONE, GP_NONE, GP_NONE, GP_NONE, la, 0, 0, 0, GP_NONE)
+#define GP_STEP_LAST(S, p, q)                                                                       \
+  GP_STEP_(S, p, q, GP_NONE, GP_NONE, GP_NONE, GP_NONE, la, 0, 0, 0, GP_NONE)
 
-#pragma unroll
-  for (int st = 0; st < 2; ++st) {
-    GP_LOAD(opb0, pb0, st, GP_B0)
-    GP_LOAD(opa0, pa, st, GP_A0)
-    GP_LOAD(opb1, pb1, st, GP_B1)
-    GP_LOAD(opa1, pa, st, GP_A1)
-    pa += a_step; pb0 += b_step; pb1 += b_step;
+#define GP_END(S, p, q) GP_STEP_LAST2(S, p, q) GP_STEP_LAST(1 - (S), q, p)
+
+#define GP_ASK(stage, LOAD)                                                                         \
+  LOAD(opb0, pb0, stage, GP_B0) LOAD(opa0, pa, stage, GP_A0) LOAD(opb1, pb1, stage, GP_B1) LOAD(opa1, pa, stage, GP_A1) \
+  pa += a_step; pb0 += b_step; pb1 += b_step;
+  GP_ASK(0, GP_LOAD)
+  if constexpr (GD_K_LEFT > 0 && KT == 2) { GP_ASK(1, GP_LOAD_LEFT) } else { GP_ASK(1, GP_LOAD) }
+  constexpr int ahead = 3 * (la + lb);                 // loads still out when a phase's operands have landed
+#else
+  // One phase: the memory part (operand reads, loads, the wait for both the reads and what the next
+  // phase reads), and behind a barrier the matrix part: A half h times both B halves.
+#define GP_PHASE(READS, LOADS, left, h, b0)                                                         \
+  READS                                                                                             \
+  __builtin_amdgcn_sched_barrier(0);                                                                \
+  LOADS                                                                                             \
+  __builtin_amdgcn_sched_barrier(0);                                                                \
+  __builtin_amdgcn_s_waitcnt(gp_wait(left));                                                        \
+  gp_barrier();                                                                                     \
+  __builtin_amdgcn_s_setprio(1);                                                                    \
+  _Pragma("unroll") for (int s = 0; s < 2; ++s)                                                     \
+  _Pragma("unroll") for (int i = 0; i < TMH; ++i) {                                                 \
+    _Pragma("unroll") for (int j = 0; j < GP_TNH; ++j) acc[h][i][0][j] = mfma16(b0[s][j], fa[s][i], acc[h][i][0][j]);  \
+    _Pragma("unroll") for (int j = 0; j < GP_TNH; ++j) acc[h][i][1][j] = mfma16(fb1[s][j], fa[s][i], acc[h][i][1][j]); \
+  }                                                                                                 \
+  __builtin_amdgcn_s_setprio(0);                                                                    \
+  gp_barrier();
+  // Step k on stage S: `pa`, `pb0`, `pb1` stand at step k + 2.
+#define GP_STEP(S, p, q, A1, B0, LATER)                                                             \
+  GP_PHASE(GP_READ_A(S, GP_A0) GP_READ_B(fb1, S, GP_B1),                                            \
+           A1(opa1, pa - a_step, 1 - (S), GP_A1) B0(opb0, pb0, S, GP_B0), 2 * (la + lb), 0, p)      \
+  GP_PHASE(GP_READ_A(S, GP_A1) GP_READ_B(q, 1 - (S), GP_B0),                                        \
+           LATER(opa0, pa, S, GP_A0) LATER(opb1, pb1, S, GP_B1), 2 * (la + lb), 1, p)               \
+  pa += a_step; pb0 += b_step; pb1 += b_step;
+  // The last two steps: only the last A half is still to be asked for; the waits count down.
+#define GP_STEP_LAST2(S, p, q, A1)                                                                  \
+  GP_PHASE(GP_READ_A(S, GP_A0) GP_READ_B(fb1, S, GP_B1), A1(opa1, pa - a_step, 1 - (S), GP_A1), 2 * la + lb, 0, p) \
+  GP_PHASE(GP_READ_A(S, GP_A1) GP_READ_B(q, 1 - (S), GP_B0), GP_NONE, la, 1, p)
+#define GP_STEP_LAST(S, p)                                                                          \
+  GP_PHASE(GP_READ_A(S, GP_A0) GP_READ_B(fb1, S, GP_B1), GP_NONE, 0, 0, p)                          \
+  GP_PHASE(GP_READ_A(S, GP_A1), GP_NONE, 0, 1, p)
+
+#define GP_END(S, p, q)                                                                             \
+  if constexpr (GD_K_LEFT > 0) { GP_STEP_LAST2(S, p, q, GP_LOAD_LEFT) } else { GP_STEP_LAST2(S, p, q, GP_LOAD) } \
+  GP_STEP_LAST(1 - (S), q)
+
+  // Ahead of the loop, in the order the steps ask: everything of step 0, and B0, A0, B1 of step 1.
+  {
+    const elem_t *pa1 = pa + a_step, *pb01 = pb0 + b_step, *pb11 = pb1 + b_step;
+    GP_LOAD(opb0, pb0, 0, GP_B0)
+    GP_LOAD(opa0, pa, 0, GP_A0) GP_LOAD(opb1, pb1, 0, GP_B1)
+    GP_LOAD(opa1, pa, 0, GP_A1)
+    if constexpr (GD_K_LEFT > 0 && KT == 2) {
+      GP_LOAD_LEFT(opb0, pb01, 1, GP_B0) GP_LOAD_LEFT(opa0, pa1, 1, GP_A0) GP_LOAD_LEFT(opb1, pb11, 1, GP_B1)
+    } else {
+      GP_LOAD(opb0, pb01, 1, GP_B0) GP_LOAD(opa0, pa1, 1, GP_A0) GP_LOAD(opb1, pb11, 1, GP_B1)
+    }
+    pa += 2 * a_step; pb0 += 2 * b_step; pb1 += 2 * b_step;
   }
-  __builtin_amdgcn_s_waitcnt(gp_wait(3 * (la + lb)));
+  constexpr int ahead = 2 * (la + lb);
+#endif
+  __builtin_amdgcn_s_waitcnt(gp_wait(ahead));
   gp_barrier();
   GP_READ_B(fx, 0, GP_B0)
   __builtin_amdgcn_sched_barrier(0);
-  __builtin_amdgcn_s_waitcnt(gp_wait(3 * (la + lb)));
+  __builtin_amdgcn_s_waitcnt(gp_wait(ahead));
   gp_barrier();                                        // (B0's slot may be asked for from here on)
   if (late) gp_barrier();
 
-  for (int pair = 0; pair < (KT - 2) / 2; ++pair) {
+  // (F steps ask for whole steps; with a partly filled last step, one more asks for that one)
+  constexpr int F = KT - 2 - (GD_K_LEFT > 0 && KT > 2);
+  for (int pair = 0; pair < F / 2; ++pair) {
     keep_addresses();
-    GP_STEP(0, fx, fy)
-    GP_STEP(1, fy, fx)
+    GP_STEP(0, fx, fy, GP_LOAD, GP_LOAD, GP_LOAD)
+    GP_STEP(1, fy, fx, GP_LOAD, GP_LOAD, GP_LOAD)
   }
   keep_addresses();
-  if constexpr (KT % 2 == 0) {
-    GP_STEP_LAST2(0, fx, fy)
-    GP_STEP_LAST(1, fy, fx)
+  if constexpr (F % 2 == 1 && F == KT - 2) {
+    GP_STEP(0, fx, fy, GP_LOAD, GP_LOAD, GP_LOAD)
+    GP_END(1, fy, fx)
+  } else if constexpr (F % 2 == 1) {
+    GP_STEP(0, fx, fy, GP_LOAD, GP_LOAD, GP_LOAD)
+    GP_STEP(1, fy, fx, GP_LOAD, GP_LOAD_LEFT, GP_LOAD_LEFT)
+    GP_END(0, fx, fy)
+  } else if constexpr (F < KT - 2) {
+    GP_STEP(0, fx, fy, GP_LOAD, GP_LOAD_LEFT, GP_LOAD_LEFT)
+    GP_END(1, fy, fx)
   } else {
-    GP_STEP(0, fx, fy)
-    GP_STEP_LAST2(1, fy, fx)
-    GP_STEP_LAST(0, fx, fy)
+    GP_END(0, fx, fy)
   }
   if (!late) gp_barrier();
 
@@ -262,7 +331,7 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
   asm volatile("" : "+v"(tid));
   const int ec = tid & 15, eg = (tid >> 4) & 3;
   const int erow = (tid >> 6) / CL_WN * (HM / CL_WM) + ec, ecol = (tid >> 6) % CL_WN * (GP_HN / CL_WN);
-  // ---- epilogue: acc[h][i][v][j][r] = C[m0 + h HM + am + 16 i + c][n0 + 128 v + bn + 16 j + 4 g + r]
+  // ---- epilogue: acc[h][i][v][j][r] = C[m0 + h HM + am + 16 i + c][n0 + HN v + bn + 16 j + 4 g + r]
 #pragma unroll
   for (int h = 0; h < 2; ++h)
 #pragma unroll

@@ -113,7 +113,23 @@ def gemm_candidates(low, role, factor, arch: Arch):
     return out
 
 
-def gemm_dma_candidates(low, role, factor, arch: Arch):
+def phased_matmul(family, problem, splits, tile) -> bool:
+    """Which products run on ``gemm_phased.hip`` (two wave groups alternating between memory and matrix work)
+    instead of the lock-step ``gemm_dma.hip``: all that it has a form for.  It needs eight waves (two per SIMD,
+    one multiplying while the other reads) with 16 matrix ops each per phase, at least the two K steps its
+    pipeline holds, and rows of C that leave as 16-byte pieces; the fused norm, the row-sum walk and the load
+    and matrix-op knobs are the lock-step kernel's.  us, lock-step / phased: 8192^3 bf16 (N, K) weight 806 / 701,
+    4096 x 14336 x 4096 f16 393 / 352 (with the last half round split), SwiGLU of that size 752 / 676, 3000 x 5000 x 2048
+    56 / 52; 128 x 256 tiles (three stages lock-step) 2048 x 4096 x 4096 60.1 / 56.3, 724 x 6272 x 640 13.3 / 10.7; at the
+    small end 2999 x 1000 x 192 9.8 / 8.2."""
+    bm, bn, wm, wn = (int(tile[k]) for k in ("BM", "BN", "WM", "WN"))
+    sizes = (bm, bn) == (256, 256) or ((bm, bn) in ((128, 256), (256, 128)) and not int(tile.get("TAIL", 0)))
+    return (sizes and wm * wn == 8 and bn // 2 // wn % 32 == 0 and bm // 2 // wm % 16 == 0 and family in ("matmul", "swiglu")
+            and problem["K"] // splits > 64 and problem["N"] % 8 == 0 and int(tile.get("STAGES", 2)) == 2
+            and not {"ASM_LOADS", "ASM_MFMA", "SPREAD_LOADS"} & set(tile))
+
+
+def gemm_dma_candidates(low, role, factor, arch: Arch, twin_of=None):
     """Tilings of the direct-to-LDS matmul: the plain matmul, and the RMSNorm -> matmul without a
     learned weight, unsplit (the norm then scales the product's rows; with a weight the operand
     would have to pass through registers on its way to LDS).  No staging registers, so the budget is accumulators plus two
@@ -126,9 +142,10 @@ def gemm_dma_candidates(low, role, factor, arch: Arch):
     if low.family != "matmul" and not post_norm:
         return []
     M, N, K = p["M"], p["N"], p["K"]
-    if K % (splits * 64) or (not p["trans_B"] and N % 8) or (p["trans_A"] and M % 8):
+    # (unsplit, the last K step may be partly filled: its chunks past K are fetched as zeros)
+    if K % (splits * 64 if splits > 1 else 8) or (not p["trans_B"] and N % 8) or (p["trans_A"] and M % 8):
         return []
-    kps = K // splits
+    kps = _ceil(K // splits, 64) * 64
     batch = max(p["batch_A"], p["batch_B"])
     out = []
     shapes = (16, 32, 64, 128, 256)
@@ -170,15 +187,21 @@ def gemm_dma_candidates(low, role, factor, arch: Arch):
         # (equal tiles: the wave grids with more waves have measured a few per cent faster -- more loads in flight)
         score = passes * pass_clk * (1.0 + 0.03 / (wm * wn))
         tiling = dict(BM=bm, BN=bn, BK=64, WM=wm, WN=wn)
+        # (128 x 256 and 256 x 128 tiles whose wave groups alternate between memory and matrix work: 6 to 25 % ahead of
+        # the three-stage lock-step form of the same tile, which itself ranks at 0.85; SwiGLU keeps both, the
+        # lock-step form ahead)
+        phased = bm * bn == 128 * 256 and not post_norm and twin_of != "matmul_rowsum" and phased_matmul("matmul", p, splits, tiling)
+        if phased:
+            score *= 0.8502 if twin_of else 0.8
         out.append(TileDict("gemm_dma", role, tiling, output_tile=[bm, bn], rstep_map={"k": 64}, n_threads=threads,
                             split_factor=factor, score=score, lds_bytes=lds, est_vgprs=vgprs))
         # Three LDS stages where three images fit beside as many workgroups per compute unit as two
         # allow: the loads of a step asked for two steps ahead and spread over the whole step
         # (256 x 128 tiles on 4096 x 14336 x 4096: 426 us against 526).
-        if (3 * (bm + bn) * 128 * per_cu <= arch.lds_bytes and units_a % (wm * wn) == 0 and units_b % (wm * wn) == 0
+        if ((twin_of or not phased) and 3 * (bm + bn) * 128 * per_cu <= arch.lds_bytes and units_a % (wm * wn) == 0 and units_b % (wm * wn) == 0
                 and not post_norm):
             out.append(TileDict("gemm_dma", role, dict(tiling, STAGES=3), output_tile=[bm, bn], rstep_map={"k": 64},
-                                n_threads=threads, split_factor=factor, score=0.85 * score, lds_bytes=3 * lds // 2,
+                                n_threads=threads, split_factor=factor, score=0.85 * (score / 0.8502 if phased else score), lds_bytes=3 * lds // 2,
                                 est_vgprs=vgprs))
         # A last round that fills at most half of the machine: its tiles as two half-height
         # workgroups each (row-major A, one workgroup per compute unit, unsplit, unbatched).
@@ -188,6 +211,10 @@ def gemm_dma_candidates(low, role, factor, arch: Arch):
             out.append(TileDict("gemm_dma", role, dict(tiling, TAIL=tail), output_tile=[bm, bn], rstep_map={"k": 64},
                                 n_threads=threads, split_factor=factor, score=(passes - 0.45) * pass_clk,
                                 lds_bytes=lds, est_vgprs=vgprs))
+    if K % 64:
+        # (under the name of the template that takes such lengths; DMA picks its direct-to-LDS form)
+        for c in out:
+            c.template, c.tiling = "gemm", dict(c.tiling, DMA=1)
     return out
 
 
@@ -197,12 +224,12 @@ def swiglu_candidates(low, role, factor, arch: Arch):
     which every wave owns an even number of column fragments (half of them per weight)."""
     import copy
 
-    if factor and factor > 1:
+    if (factor and factor > 1) or low.problem["K"] % 64:
         return []
     twin = copy.copy(low)
     twin.family, twin.problem = "matmul", dict(low.problem, N=2 * low.problem["N"])
     out = []
-    for c in gemm_dma_candidates(twin, role, None, arch):
+    for c in gemm_dma_candidates(twin, role, None, arch, twin_of="swiglu"):
         t = c.tiling
         tn = t["BN"] // t["WN"] // 16
         if tn % 2 or low.problem["N"] % (t["BN"] // 2):
@@ -219,13 +246,13 @@ def rowsum_candidates(low, role, factor, arch: Arch):
     step sequences of ``(N / BN) * (K / 64)`` steps the machine runs one after another."""
     import copy
 
-    if factor and factor > 1:
+    if (factor and factor > 1) or low.problem["K"] % 64:
         return []
     p = low.problem
     twin = copy.copy(low)
     twin.family = "matmul"
     out = []
-    for c in gemm_dma_candidates(twin, role, None, arch):
+    for c in gemm_dma_candidates(twin, role, None, arch, twin_of="matmul_rowsum"):
         t = c.tiling
         if p["N"] % t["BN"]:
             continue

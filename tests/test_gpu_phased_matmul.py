@@ -1,6 +1,6 @@
-"""GPU parity of the 256 x 256 matmul whose two wave groups alternate between memory and matrix work, against
-the numpy oracle at the sizes where its walk can go wrong: two to five K steps (the loop, the two steps without
-loads behind it, both stage parities), whole halves of a tile past the edge, edges of one row and of one
+"""GPU parity of the matmul whose two wave groups alternate between memory and matrix work, against
+the numpy oracle at the sizes where its walk can go wrong: two to seven K steps (the loop, the two steps without
+loads behind it, both stage parities), a last step that K fills only partly, whole halves of a tile past the edge, edges of one row and of one
 8-column piece, all operand layouts, split ranges, batches, half-height tail tiles and the SwiGLU form.
 Tolerance 1e-2 / 1e-2 as for every f16 / bf16 kernel here (outputs are of order one or below, and one
 rounding to bf16 is 2^-9)."""
@@ -23,41 +23,66 @@ def matmul_tn(x: cl.Tensor["K", "M"], w: cl.Tensor["K", "N"]):
     return x.mT @ w
 
 
-def _check(fn, dtype, shapes, grid=(2, 4), split=None, **knobs):
+TILES = {"256x256_2x4": (256, 256, 2, 4), "256x256_4x2": (256, 256, 4, 2), "128x256_2x4": (128, 256, 2, 4),
+         "128x256_4x2": (128, 256, 4, 2), "256x128_4x2": (256, 128, 4, 2)}
+
+
+def _check(fn, dtype, shapes, tile=TILES["256x256_2x4"], split=None, **knobs):
     prog = fn.trace(dtype, **shapes)
     x, *weights = prog.random_inputs(seed=7)
     args = [x] + [(w.float() / shapes["K"] ** 0.5).to(w.dtype) for w in weights]
-    tiling = dict(BM=256, BN=256, BK=64, WM=grid[0], WN=grid[1], **knobs)
+    tiling = dict(zip(("BM", "BN", "WM", "WN"), tile), BK=64, **knobs)
     print(f"case {prog.name} {dtype} {shapes} {tiling} split={split}", flush=True)
     kernel = kernel_for(prog, template="gemm_dma", tiling=tiling, split=split)
-    assert "gp_barrier" in kernel.get_kernel_source()
+    phased = tile in TILES.values() and shapes["K"] // (split or 1) > 64
+    assert phased == ("gp_barrier" in kernel.get_kernel_source())
     got = kernel(*args)
     torch.cuda.synchronize()
     want = program_oracle.evaluate(prog, [t.cpu() for t in args])[0]
     np.testing.assert_allclose(got.float().cpu().numpy().reshape(want.shape), want, rtol=1e-2, atol=1e-2)
 
 
-@pytest.mark.parametrize("grid", [(2, 4), (4, 2)], ids=["2x4", "4x2"])
+@pytest.mark.parametrize("tile", TILES.values(), ids=TILES)
 @pytest.mark.parametrize("m,n,k", [(256, 256, 128), (257, 264, 192), (100, 72, 256), (600, 776, 320), (129, 392, 448)])
 @pytest.mark.parametrize("fn,dtype", [(C.matmul, cl.f16), (C.matmul_nt, cl.bf16), (matmul_tn, cl.f16)], ids=["nn", "nt", "tn"])
-def test_layouts_edges_and_step_counts(fn, dtype, m, n, k, grid):
+def test_layouts_edges_and_step_counts(fn, dtype, m, n, k, tile):
     if fn is matmul_tn:
         m = -(-m // 8) * 8                      # its A rows are read as 16-byte pieces along M
-    _check(fn, dtype, dict(M=m, N=n, K=k), grid)
+    _check(fn, dtype, dict(M=m, N=n, K=k), tile)
+
+
+@pytest.mark.parametrize("tile", [*TILES.values(), (64, 128, 2, 4), (128, 128, 2, 2)], ids=[*TILES, "64x128_lockstep", "128x128_lockstep"])
+@pytest.mark.parametrize("k", [72, 136, 184, 248, 328, 440])
+def test_partly_filled_last_step(tile, k):
+    """Chunks past K come as zeros for both operands (every layout; batches, whose rows continue past K in memory), in the
+    lock-step kernel too."""
+    for fn, dtype in ((C.matmul, cl.f16), (C.matmul_nt, cl.bf16), (matmul_tn, cl.f16)):
+        _check(fn, dtype, dict(M=304, N=264, K=k), tile)
+    _check(C.batched_matmul, cl.f16, dict(BX=2, BW=2, M=130, N=136, K=k), tile)
+
+
+@pytest.mark.parametrize("k", [8, 40, 136, 200, 328])
+def test_partly_filled_last_step_of_three_stages_and_small_tiles(k):
+    for tile, knobs in (((64, 64, 2, 2), dict(STAGES=3)), ((16, 32, 1, 2), {}), ((16, 64, 1, 4), {})):
+        _check(C.matmul, cl.f16, dict(M=100, N=136, K=k), tile, **knobs)
+        _check(C.matmul_nt, cl.bf16, dict(M=100, N=136, K=k), tile, **knobs)
 
 
 @pytest.mark.parametrize("tail", [1, 4, 8])
 def test_half_height_tail_tiles(tail):
     _check(C.matmul, cl.f16, dict(M=512, N=1032, K=320), TAIL=tail)
-    _check(C.matmul_nt, cl.bf16, dict(M=512, N=1032, K=256), grid=(4, 2), TAIL=tail)
+    _check(C.matmul_nt, cl.bf16, dict(M=512, N=1032, K=256), tile=TILES["256x256_4x2"], TAIL=tail)
 
 
 def test_split_ranges_and_batches():
-    _check(C.matmul, cl.f16, dict(M=300, N=264, K=768), split=3)
-    _check(C.batched_matmul, cl.bf16, dict(BX=4, BW=2, M=264, N=136, K=192))
+    for tile in (TILES["256x256_2x4"], TILES["128x256_2x4"]):
+        _check(C.matmul, cl.f16, dict(M=300, N=264, K=768), tile, split=3)
+        _check(C.batched_matmul, cl.bf16, dict(BX=4, BW=2, M=264, N=136, K=192), tile)
 
 
 @pytest.mark.parametrize("m,n,k", [(256, 128, 128), (300, 384, 320)])
 def test_swiglu(m, n, k):
+    _check(C.swiglu, cl.f16, dict(M=m, N=n, K=k), tile=TILES["128x256_2x4"], SWIGLU=1)
+    _check(C.swiglu, cl.f16, dict(M=m, N=n, K=k), tile=TILES["256x128_4x2"], SWIGLU=1)
     _check(C.swiglu, cl.f16, dict(M=m, N=n, K=k), SWIGLU=1)
-    _check(C.swiglu, cl.bf16, dict(M=m, N=n, K=k), grid=(4, 2), SWIGLU=1)
+    _check(C.swiglu, cl.bf16, dict(M=m, N=n, K=k), tile=TILES["256x256_4x2"], SWIGLU=1)
