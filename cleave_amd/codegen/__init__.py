@@ -299,9 +299,10 @@ class HipCodeGen:
         if swiglu and (tile["BN"] // tile["WN"] // 16) % 2:
             raise CodegenError("a SwiGLU wave owns an even number of column fragments")
         batch = max(p["batch_A"], p["batch_B"])
-        from ..schedule.policy import phased_matmul
+        from ..schedule.policy import kwaves_lds_bytes, phased_matmul
 
-        unit.templates += ["gemm_tile.hip", "gemm_phased.hip" if phased_matmul(plan.family, p, splits, tile) else "gemm_dma.hip"]
+        kw = int(tile.get("KW", 0))
+        unit.templates += ["gemm_tile.hip", "gemm_kwaves.hip" if kw else "gemm_phased.hip" if phased_matmul(plan.family, p, splits, tile) else "gemm_dma.hip"]
         if partial:
             if tile["BK"] != 64 or (p["K"] % (splits * 64) and (splits > 1 or p["K"] % 8 or plan.family not in ("matmul", "rmsnorm_matmul"))):
                 raise CodegenError(f"K={p['K']} is neither a multiple of splits*64={splits * 64} nor, for an unsplit product, of 8")
@@ -309,6 +310,14 @@ class HipCodeGen:
                 raise CodegenError("16-byte global chunks need the minor extent of each operand to be a multiple of 8")
             grid = (1 if rowsum else -(-p["N"] // out_bn), -(-p["M"] // tile["BM"]), batch * splits)
             stages = int(tile.get("STAGES", 2))
+            if kw:
+                if (plan.family != "matmul" or splits > 1 or combine or tile["WM"] * tile["WN"] != 1 or kw not in (2, 4, 8, 16)
+                        or "STAGES" in tile or p["N"] % 4 or tile["BM"] % 16 or tile["BN"] % 16 or tail_requested(tile)
+                        or kwaves_lds_bytes(tile["BM"], tile["BN"], kw) > 160 * 1024):
+                    raise CodegenError("waves that share K: a plain unsplit product, 2 to 16 waves that each own the whole tile, "
+                                       "two images per wave within 160 KiB, N a multiple of 4")
+                unit.launch(ENTRY, grid, kw * 64, 0, self._partial_args)
+                return
             if stages != 2:
                 waves = tile["WM"] * tile["WN"]
                 if (stages != 3 or rowsum or not int(tile.get("ASM_LOADS", 1)) or 3 * (tile["BM"] + tile["BN"]) * 128 > 160 * 1024

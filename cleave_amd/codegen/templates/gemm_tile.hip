@@ -19,6 +19,11 @@
 #define CL_GROUP_M 8
 #endif
 #define GD_XCDS 8
+#ifndef CL_KW
+#define GD_LOAD_WAVE ((int)(threadIdx.x >> 6))    // the wave's place among those that share a tile's loads
+#else
+#define GD_LOAD_WAVE 0                             // (waves that share K load tiles of their own)
+#endif
 #ifndef CL_SPREAD_LOADS
 #define CL_SPREAD_LOADS 0
 #endif
@@ -95,7 +100,7 @@ struct GdOperand {
   // ext0: first row/column of the tile, lim: tensor extent along that axis, pitch: elements;
   // first: where this operand's rows / columns start inside the tile (its offsets stay relative to ext0)
   CL_METHOD void init(int ext0, int lim, int pitch, i64 twin = 0, int first = 0) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = GD_LOAD_WAVE;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       const int u = wave + i * GD_WAVES;

@@ -211,11 +211,56 @@ def gemm_dma_candidates(low, role, factor, arch: Arch, twin_of=None):
             out.append(TileDict("gemm_dma", role, dict(tiling, TAIL=tail), output_tile=[bm, bn], rstep_map={"k": 64},
                                 n_threads=threads, split_factor=factor, score=(passes - 0.45) * pass_clk,
                                 lds_bytes=lds, est_vgprs=vgprs))
+    if not twin_of and not post_norm:
+        # the two best plain tilings stay ahead of them: measured, not modelled, is how they get past
+        ranked = sorted(c.score for c in out)
+        for c in kwaves_candidates(low, role, factor, arch):
+            c.score = max([c.score] + [1.0001 * s for s in ranked[1:2]])
+            out.append(c)
     if K % 64:
         # (under the name of the template that takes such lengths; DMA picks its direct-to-LDS form)
         for c in out:
             c.template, c.tiling = "gemm", dict(c.tiling, DMA=1)
     return out
+
+
+def kwaves_lds_bytes(bm, bn, kw):
+    """LDS of the matmul whose waves share K: two images of both tiles per wave, reused for the final sums."""
+    return max(kw * 2 * (bm + bn) * 128, kw * bm * bn * 4)
+
+
+def kwaves_candidates(low, role, factor, arch: Arch):
+    """Tilings of the matmul whose waves share K, for products of few tiles and a long contraction (at least eight
+    64-wide steps, at most 1024 tiles of 32 x 32): the two the model likes best.  What a step costs a compute unit is
+    the 64-byte requests its waves make, one a clock at best (measured alike with two, three and four images per
+    wave: 47 bytes a clock): two per K-minor row (three where rows are not whole 128-byte lines), one per 32 columns of
+    a K-major row."""
+    p = low.problem
+    M, N, K = p["M"], p["N"], p["K"]
+    batch = max(p["batch_A"], p["batch_B"])
+    steps = _ceil(K, 64)
+    if (low.family != "matmul" or role != "main" or (factor or 1) > 1 or K % 8 or N % 8 or (p["trans_A"] and M % 8)
+            or steps < 8 or _ceil(M, 32) * _ceil(N, 32) * batch > 1024):
+        return []
+
+    def requests(extent, k_major):
+        return 64 * _ceil(extent, 32) if k_major else extent * (2 if K % 64 == 0 else 3)
+
+    out = []
+    for (bm, bn), kw in itertools.product(((16, 16), (16, 32), (32, 16), (32, 32), (32, 64), (64, 32), (64, 64)), (4, 8)):
+        lds = kwaves_lds_bytes(bm, bn, kw)
+        if lds > arch.lds_bytes or kw > steps or (bm > 16 and bm >= 2 * M) or (bn > 16 and bn >= 2 * N):
+            continue
+        blocks = _ceil(M, bm) * _ceil(N, bn) * batch
+        per_cu = max(1, min(arch.lds_bytes // lds, 32 // kw))
+        live = min(per_cu, _ceil(blocks, arch.compute_units))
+        step_clk = max(1000.0, live * kw * (requests(bm, p["trans_A"]) + requests(bn, not p["trans_B"])) * 1.3)
+        score = _waves_time(blocks, per_cu, arch) * (_ceil(steps, kw) * step_clk + 4000 + 60 * kw)
+        out.append(TileDict("gemm_dma", role, dict(BM=bm, BN=bn, BK=64, WM=1, WN=1, KW=kw), output_tile=[bm, bn],
+                            rstep_map={"k": 64}, n_threads=kw * 64, split_factor=factor, score=score, lds_bytes=lds,
+                            est_vgprs=bm * bn // 64 + 60))
+    out.sort(key=lambda c: (c.score, c.key()))
+    return out[:2]
 
 
 def swiglu_candidates(low, role, factor, arch: Arch):

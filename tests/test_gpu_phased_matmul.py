@@ -74,6 +74,16 @@ def test_half_height_tail_tiles(tail):
     _check(C.matmul_nt, cl.bf16, dict(M=512, N=1032, K=256), tile=TILES["256x256_4x2"], TAIL=tail)
 
 
+@pytest.mark.parametrize("tile,kw", [((16, 16), 8), ((16, 32), 4), ((32, 16), 2), ((32, 32), 8), ((32, 64), 4), ((64, 64), 4), ((16, 16), 16)],
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else f"kw{v}")
+@pytest.mark.parametrize("k", [8, 64, 200, 512, 1096])
+def test_waves_that_share_the_contraction(tile, kw, k):
+    """Fewer steps than waves (some own none), one to many steps per wave, a partly filled last step, ragged edges."""
+    for fn, dtype in ((C.matmul, cl.f16), (C.matmul_nt, cl.bf16), (matmul_tn, cl.f16)):
+        _check(fn, dtype, dict(M=72, N=104, K=k), (*tile, 1, 1), KW=kw)
+    _check(C.batched_matmul, cl.f16, dict(BX=4, BW=2, M=50, N=72, K=k), (*tile, 1, 1), KW=kw)
+
+
 def test_split_ranges_and_batches():
     for tile in (TILES["256x256_2x4"], TILES["128x256_2x4"]):
         _check(C.matmul, cl.f16, dict(M=300, N=264, K=768), tile, split=3)
