@@ -83,7 +83,9 @@ bool read_expr(PyObject* o, Expr* e) {
       if (++i >= PySequence_Fast_GET_SIZE(seq)) { ok = false; break; }
       e->push_back(PyLong_AsLongLong(PySequence_Fast_GET_ITEM(seq, i)));
       if (++depth > 32) ok = false;
-    } else if (v != NEG) {
+    } else if (v == NEG) {
+      if (depth < 1) ok = false;
+    } else {
       if (--depth < 1 || v < 0 || v > MAX_) ok = false;
     }
   }
@@ -96,6 +98,7 @@ enum ArgKind { TENSOR, F32, I32 };
 struct Arg {
   int kind;
   at::ScalarType dtype;
+  uintptr_t misaligned;          // TENSOR: address bits that have to be zero (the kernel's loads need them so)
   std::vector<int64_t> dim;      // TENSOR, per axis: >= 0 an extent; -1 - d binds run-time dim d; INT64_MIN an expression
   std::vector<Expr> expr;        // the expressions, in axis order
 };
@@ -141,7 +144,17 @@ at::ScalarType scalar_type(const char* name) {
 
 #define MISS() do { Py_RETURN_NOTIMPLEMENTED; } while (0)
 
-PyObject* call(PyObject* self_, PyObject* const* argv, size_t nargsf, PyObject* kwnames) {
+// A tensor whose sizes and memory are what they seem: not fake or traced (Python key), batched or wrapped by a
+// transform (vmap, grad), a zero without memory, or a lazy negation.  The others go through torch's own accessors in
+// the Python path, which raise what they always raised.
+bool plain(const at::Tensor& t) {
+  constexpr c10::DispatchKeySet others({c10::DispatchKey::Python, c10::DispatchKey::PythonTLSSnapshot, c10::DispatchKey::FuncTorchBatched,
+                                        c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Functionalize, c10::DispatchKey::ZeroTensor,
+                                        c10::DispatchKey::Negative, c10::DispatchKey::Conjugate});
+  return t.defined() && !t.key_set().has_any(others) && t.has_storage();
+}
+
+PyObject* call_plain(PyObject* self_, PyObject* const* argv, size_t nargsf, PyObject* kwnames) {
   Plan* self = reinterpret_cast<Plan*>(self_);
   const size_t n = PyVectorcall_NARGS(nargsf);
   const std::vector<Arg>& spec = *self->args;
@@ -168,6 +181,7 @@ PyObject* call(PyObject* self_, PyObject* const* argv, size_t nargsf, PyObject* 
     }
     if (!THPVariable_Check(o)) MISS();
     const at::Tensor& t = THPVariable_Unpack(o);
+    if (!plain(t)) MISS();
     if (t.layout() != at::kStrided || t.device().type() != at::kCUDA || t.scalar_type() != a.dtype || !t.is_contiguous()) MISS();
     if (device < 0) device = t.device().index();
     else if (device != t.device().index()) MISS();
@@ -183,7 +197,8 @@ PyObject* call(PyObject* self_, PyObject* const* argv, size_t nargsf, PyObject* 
         else if (d != sizes[k]) MISS();
       }
     }
-    arg_value[i].p = t.data_ptr();
+    arg_value[i].p = t.mutable_data_ptr();
+    if (reinterpret_cast<uintptr_t>(arg_value[i].p) & a.misaligned) MISS();
   }
   if (device < 0) MISS();
   for (int i = 0; i < self->n_dims; ++i) if (dims[i] < 0) MISS();
@@ -221,66 +236,76 @@ PyObject* call(PyObject* self_, PyObject* const* argv, size_t nargsf, PyObject* 
       else grids[l][k] = (uint32_t)v;
     }
 
+  if (c10::impl::VirtualGuardImpl(c10::DeviceType::CUDA).getDevice().index() != device) MISS();
+  const auto on_device = at::TensorOptions().device(at::kCUDA, device);
+  at::Tensor outs[kMaxOuts];
+  void* out_ptr[kMaxOuts];
+  for (size_t i = 0; i < self->outs->size(); ++i) {
+    const Out& o = (*self->outs)[i];
+    int64_t shape[8];
+    for (size_t k = 0; k < o.shape.size(); ++k)
+      if (!evaluate(o.shape[k], dims, &shape[k]) || shape[k] < 0) MISS();
+    outs[i] = at::empty(at::IntArrayRef(shape, o.shape.size()), on_device.dtype(o.dtype));
+    out_ptr[i] = outs[i].data_ptr();
+  }
+  at::Tensor scratch;
+  void* temp_ptr[kMaxTemps];
+  if (!self->temps->empty() && !empty) {
+    int64_t at_byte[kMaxTemps], total = 0;
+    for (size_t i = 0; i < self->temps->size(); ++i) {
+      int64_t v;
+      if (!evaluate((*self->temps)[i], dims, &v) || v < 0) MISS();
+      at_byte[i] = total;
+      total += (v + 255) / 256 * 256;
+    }
+    scratch = at::empty({total}, on_device.dtype(at::kByte));
+    for (size_t i = 0; i < self->temps->size(); ++i) temp_ptr[i] = static_cast<char*>(scratch.data_ptr()) + at_byte[i];
+  }
+  if (!empty) {
+    PyObject* index = PyLong_FromLong(device);
+    if (!index) return nullptr;
+    PyObject* handle = PyObject_CallOneArg(self->raw_stream, index);
+    Py_DECREF(index);
+    if (!handle) return nullptr;
+    void* stream = PyLong_AsVoidPtr(handle);
+    Py_DECREF(handle);
+    if (PyErr_Occurred()) return nullptr;
+    // (a launch waits where the stream's queue is full: other threads run meanwhile)
+    PyThreadState* released = PyEval_SaveThread();
+    int failed = 0;
+    for (size_t l = 0; l < self->launches->size() && !failed; ++l) {
+      const Launch& q = (*self->launches)[l];
+      void* values[kMaxValues];
+      int nv = 0;
+      for (const Value& v : q.values)
+        values[nv++] = v.kind == V_ARG ? (void*)&arg_value[v.index] : v.kind == V_OUT ? (void*)&out_ptr[v.index]
+                       : v.kind == V_TEMP ? (void*)&temp_ptr[v.index] : (void*)&dim_value[v.index];
+      failed = self->launch(q.fn, grids[l], q.block, q.lds, stream, values, nv);
+    }
+    PyEval_RestoreThread(released);
+    if (failed) {
+      PyErr_Format(PyExc_RuntimeError, "chip_launch: %s", self->last_error());
+      return nullptr;
+    }
+  }
+  if (self->result == 0) Py_RETURN_NONE;
+  const size_t n_out = self->outs->size();
+  if (n_out == 1) return THPVariable_Wrap(std::move(outs[0]));
+  PyObject* many = self->result == 1 ? PyList_New(n_out) : PyTuple_New(n_out);
+  if (!many) return nullptr;
+  for (size_t i = 0; i < n_out; ++i) {
+    PyObject* t = THPVariable_Wrap(std::move(outs[i]));
+    if (!t) { Py_DECREF(many); return nullptr; }
+    if (self->result == 1) PyList_SET_ITEM(many, i, t);
+    else PyTuple_SET_ITEM(many, i, t);
+  }
+  return many;
+}
+
+// (no C++ exception may leave a C entry)
+PyObject* call(PyObject* self, PyObject* const* argv, size_t nargsf, PyObject* kwnames) {
   try {
-    if (c10::impl::VirtualGuardImpl(c10::DeviceType::CUDA).getDevice().index() != device) MISS();
-    const auto on_device = at::TensorOptions().device(at::kCUDA, device);
-    at::Tensor outs[kMaxOuts];
-    void* out_ptr[kMaxOuts];
-    for (size_t i = 0; i < self->outs->size(); ++i) {
-      const Out& o = (*self->outs)[i];
-      int64_t shape[8];
-      for (size_t k = 0; k < o.shape.size(); ++k)
-        if (!evaluate(o.shape[k], dims, &shape[k]) || shape[k] < 0) MISS();
-      outs[i] = at::empty(at::IntArrayRef(shape, o.shape.size()), on_device.dtype(o.dtype));
-      out_ptr[i] = outs[i].data_ptr();
-    }
-    at::Tensor scratch;
-    void* temp_ptr[kMaxTemps];
-    if (!self->temps->empty() && !empty) {
-      int64_t at_byte[kMaxTemps], total = 0;
-      for (size_t i = 0; i < self->temps->size(); ++i) {
-        int64_t v;
-        if (!evaluate((*self->temps)[i], dims, &v) || v < 0) MISS();
-        at_byte[i] = total;
-        total += (v + 255) / 256 * 256;
-      }
-      scratch = at::empty({total}, on_device.dtype(at::kByte));
-      for (size_t i = 0; i < self->temps->size(); ++i) temp_ptr[i] = static_cast<char*>(scratch.data_ptr()) + at_byte[i];
-    }
-    if (!empty) {
-      PyObject* index = PyLong_FromLong(device);
-      if (!index) return nullptr;
-      PyObject* handle = PyObject_CallOneArg(self->raw_stream, index);
-      Py_DECREF(index);
-      if (!handle) return nullptr;
-      void* stream = PyLong_AsVoidPtr(handle);
-      Py_DECREF(handle);
-      if (PyErr_Occurred()) return nullptr;
-      for (size_t l = 0; l < self->launches->size(); ++l) {
-        const Launch& q = (*self->launches)[l];
-        void* values[kMaxValues];
-        int nv = 0;
-        for (const Value& v : q.values)
-          values[nv++] = v.kind == V_ARG ? (void*)&arg_value[v.index] : v.kind == V_OUT ? (void*)&out_ptr[v.index]
-                         : v.kind == V_TEMP ? (void*)&temp_ptr[v.index] : (void*)&dim_value[v.index];
-        if (self->launch(q.fn, grids[l], q.block, q.lds, stream, values, nv)) {
-          PyErr_Format(PyExc_RuntimeError, "chip_launch: %s", self->last_error());
-          return nullptr;
-        }
-      }
-    }
-    if (self->result == 0) Py_RETURN_NONE;
-    const size_t n_out = self->outs->size();
-    if (n_out == 1) return THPVariable_Wrap(std::move(outs[0]));
-    PyObject* many = self->result == 1 ? PyList_New(n_out) : PyTuple_New(n_out);
-    if (!many) return nullptr;
-    for (size_t i = 0; i < n_out; ++i) {
-      PyObject* t = THPVariable_Wrap(std::move(outs[i]));
-      if (!t) { Py_DECREF(many); return nullptr; }
-      if (self->result == 1) PyList_SET_ITEM(many, i, t);
-      else PyTuple_SET_ITEM(many, i, t);
-    }
-    return many;
+    return call_plain(self, argv, nargsf, kwnames);
   } catch (const std::exception& e) {
     // an allocation that failed, say: torch's own error type is raised by the Python path's allocation
     PyErr_Clear();
@@ -306,7 +331,10 @@ bool read_plan(Plan* p, PyObject* args, PyObject* derived, PyObject* outs, PyObj
         Arg a;
         const char* dtype;
         PyObject* dims;
-        if (!PyArg_ParseTuple(o, "isO", &a.kind, &dtype, &dims)) return false;
+        unsigned align;
+        if (!PyArg_ParseTuple(o, "isOI", &a.kind, &dtype, &dims, &align)) return false;
+        if (align == 0 || (align & (align - 1))) return bad("an alignment is a power of two");
+        a.misaligned = align - 1;
         a.dtype = scalar_type(dtype);
         if (a.kind == TENSOR && a.dtype == at::ScalarType::Undefined) return bad("unknown element type");
         if (!for_each(dims, [&](PyObject* d) {

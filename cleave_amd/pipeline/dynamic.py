@@ -538,7 +538,7 @@ class PagedKernel(Kernel):
 
     def __call__(self, *positional, longest=None, **named):
         role, plan = None, False
-        if not named and len(positional) == self._n_kept:
+        if not named and len(positional) == self._n_kept and positional[self._query_at] is not None:
             # (a token rule, where one was made, decides before `longest` does)
             role = self.token_role(positional[self._query_at].shape[0])
             if role is None and longest is not None:

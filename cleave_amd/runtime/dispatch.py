@@ -76,10 +76,10 @@ def postfix(expr, dims: dict) -> list:
     return walk(ast.parse(str(expr), mode="eval").body)
 
 
-def _argument(p, dims: dict, shape=None):
-    """``(kind, dtype, dims)`` of one argument; plain names found on the way get an index in ``dims``."""
+def _argument(p, dims: dict, shape=None, align=1):
+    """``(kind, dtype, dims, alignment)`` of one argument; plain names found on the way get an index in ``dims``."""
     if p.role == "scalar":
-        return (F32 if p.dtype.startswith("float") else I32, "", ())
+        return (F32 if p.dtype.startswith("float") else I32, "", (), 1)
     axes = []
     for extent in p.shape if shape is None else shape:
         if isinstance(extent, int):
@@ -88,7 +88,7 @@ def _argument(p, dims: dict, shape=None):
             axes.append(-1 - dims.setdefault(str(extent), len(dims)))
         else:
             axes.append(str(extent))          # resolved once every plain name is known
-    return (TENSOR, p.dtype, axes)
+    return (TENSOR, p.dtype, axes, align)
 
 
 def chain_plan(stages, *, arguments=None, output_shapes=None, as_tuple=False):
@@ -108,7 +108,8 @@ def chain_plan(stages, *, arguments=None, output_shapes=None, as_tuple=False):
         caller = [p for p in last.params if p.role != "scratch" and (p.role != "output" or last.out_idx is None)]
         arguments = [(p, None) for p in caller]
         stages = [(last, {p.name: ("arg", i) for i, p in enumerate(caller)})]
-    args = [_argument(p, dims, shape) for p, shape in arguments]
+    align = max(kernel.input_align for kernel, _ in stages)
+    args = [_argument(p, dims, shape, align if p.role == "input" else 1) for p, shape in arguments]
     n_dims = len(dims)
     derived = []
     for kernel, _ in stages:
@@ -119,7 +120,7 @@ def chain_plan(stages, *, arguments=None, output_shapes=None, as_tuple=False):
                 derived.append(program)
     if any(d not in dims for kernel, _ in stages for d in kernel.dyn_dims):
         return None
-    args = [(kind, dtype, [a if isinstance(a, int) else postfix(a, dims) for a in axes]) for kind, dtype, axes in args]
+    args = [(kind, dtype, [a if isinstance(a, int) else postfix(a, dims) for a in axes], al) for kind, dtype, axes, al in args]
 
     outs, temps, launches, before = [], [], [], []
     for kernel, sources in stages:

@@ -95,3 +95,17 @@ def test_threads_on_their_own_streams_do_not_share_scratch():
     for t in threads:
         t.join()
     assert not wrong
+
+
+def test_operands_between_two_16_byte_pieces_are_copied_for_the_direct_to_lds_kernels():
+    """A view one element into a buffer: the checked path and the native one give what the aligned operand gives."""
+    shapes = dict(M=66, N=136, K=200)
+    kernel = kernel_for(C.matmul.trace(cl.f16, **shapes), template="gemm", tiling=dict(BM=64, BN=64, BK=64, WM=2, WN=2, DMA=1))
+    a, b = (torch.randn(*s, dtype=torch.float16, device="cuda") for s in ((66, 200), (200, 136)))
+    want = kernel(a, b)
+    moved = []
+    for t in (a, b):
+        buffer = torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")
+        moved.append(buffer[1:].view(t.shape).copy_(t))
+    assert kernel._plan and kernel._plan(*moved) is NotImplemented
+    assert torch.equal(kernel(*moved), want) and torch.equal(kernel._checked_call(*moved), want)
