@@ -657,9 +657,9 @@ class HipCodeGen:
         if p["heads"] % 64 or p["ckv"] % 128 or p["kpe"] % 64:
             raise CodegenError("the score-wave / value-wave MLA kernel needs heads % 64 == 0, a latent width in "
                                "multiples of 128 and a rope width in multiples of 64")
-        from ..schedule.policy import mla_lds_bytes
+        from ..schedule.policy import mla_duo_lds_bytes
 
-        if mla_lds_bytes(p["ckv"], p["kpe"], 4) + 9 * 1024 > 160 * 1024:
+        if mla_duo_lds_bytes(p["ckv"], p["kpe"]) > 160 * 1024:
             raise CodegenError("four images of the paired-wave MLA kernel do not fit LDS at these widths")
         for k, v in (("CL_HEADS", p["heads"]), ("CL_CKV", p["ckv"]), ("CL_KPE", p["kpe"]), ("CL_SKV", p["skv"]),
                      ("CL_BATCH", p["batch"]), ("CL_PO_ELEM", 1)):
@@ -731,6 +731,15 @@ class HipCodeGen:
         for role, macro in (("Q", "CL_ARG_Q"), ("QPE", "CL_ARG_QPE"), ("KV", "CL_ARG_KV"), ("KPE", "CL_ARG_KPE"),
                             ("INDPTR", "CL_ARG_INDPTR"), ("INDICES", "CL_ARG_INDICES")):
             unit.define(macro, op[role])
+        if int(t.get("DUO", 0)):
+            from ..schedule.policy import mla_duo_lds_bytes
+
+            if not prefill or tok != 4 or stages != 2 or ksplit != 1 or p["ckv"] % 128 or mla_duo_lds_bytes(p["ckv"], p["kpe"], True) > 160 * 1024:
+                raise CodegenError("score waves and value waves on a token table: causal prefill with four query tokens per item, a "
+                                   "latent width in multiples of 128 and four images within 160 KiB of LDS")
+            unit.templates += ["mla_decode_duo.hip", "attn_combine.hip"]
+            unit.launch(ENTRY, (f"ceildiv({p['dim_names']['total_q']}, 4) + batch", p["heads"] // 16, 1), 512, 0, self._partial_args)
+            return
         unit.templates += ["mla_paged_decode.hip", "attn_combine.hip"]
         if partial:
             items = f"ceildiv({p['dim_names']['n_idx']}, chunk_pages) + {batch_name}" if chunked else batch_name

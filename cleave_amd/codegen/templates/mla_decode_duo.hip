@@ -56,7 +56,22 @@
 //
 //   CL_HEADS (multiple of 64)  CL_CKV (multiple of 128)  CL_KPE (multiple of 64)  CL_SKV  CL_BATCH
 //   CL_SPLITS  CL_SCALE_LOG2E  CL_PO_ELEM (must be 1: split partials normalised, in the element type)
+//
+// CL_PREFILL: paged causal prefill over ragged query rows.  The 64 rows of a workgroup are four consecutive
+// query tokens of one request (a new item at every multiple of four packed tokens and at every request boundary) x
+// 16 heads, so a 16-row tile is one token and its causal limit is uniform over a wave; the key rows are looked up
+// in the token table (every value wave keeps the entries of its own rows in LDS, fetched on its load counter a step
+// ahead of the rows).  The first step's reference point is the maximum of both token halves (one more barrier), and the
+// score waves sum the unrounded weights for the lse.  The one-wave-per-token kernel reads 68 KB out of LDS per token
+// and step at one head group's 69 matrix ops; here it is 36.  us, the best of its forms / this one, 16 heads of 512 + 64:
+// 5376 tokens over 24 requests with prefixes 121 / 94, 9164 over 32 197 / 162, 1424 over 16 31 / 27, 350 tokens of one
+// request 21.5 / 17.3; behind for short keys on few items (37 tokens of 4 requests 6.2 / 8.2).  What bounds it now: an
+// item's query rows come and its output rows leave (136 KB) while its compute unit multiplies nothing.
+//   CL_HEADS (multiple of 16); run-time: total_q, num_pages, n_idx, batch; scalar sm_scale (any sign)
 
+#ifndef CL_PREFILL
+#define CL_PREFILL 0
+#endif
 #if CL_SPLITS > 1 && !CL_PO_ELEM
 #error "the score-wave / value-wave kernel writes its split partials in the element type"
 #endif
@@ -89,11 +104,22 @@
 #define MD_V_UNITS (MD_PANELS - CL_S_PANELS)    // loads per value wave and step once the score waves share them
 static_assert(CL_S_PANELS >= 0 && CL_S_PANELS < MD_PANELS, "the value waves keep at least one panel");
 static_assert(CL_CKV % 128 == 0 && CL_KPE % 64 == 0, "whole 64-feature panels, the latent ones halved between two value waves");
+#if CL_PREFILL
+#define MD_TOKENS 4                              // query tokens of a workgroup, 16 heads each
+#define MD_SCALE 1.0f                            // (scores are scaled as they come: the run-time scale may have any sign)
+static_assert(CL_HEADS % 16 == 0 && CL_SPLITS == 1, "16 heads of four tokens per workgroup, unsplit");
+#else
+#define MD_SCALE CL_SCALE_LOG2E
 static_assert(CL_HEADS % MD_HEADS_PER_BLOCK == 0, "64 heads per workgroup");
 static_assert(CL_SCALE_LOG2E > 0.f, "the largest raw score must be the largest scaled one");
+#endif
 static_assert(MD_UNITS_PER < 32, "load counter range");
 static_assert(MD_FBW % 2 == 0, "a value wave's feature blocks leave in pairs");
+#if CL_PREFILL
+constexpr bool MD_RAGGED = false;
+#else
 constexpr bool MD_RAGGED = CL_SKV % MD_STEP != 0;
+#endif
 
 __shared__ __attribute__((aligned(1024))) elem_t md_tiles[MD_STAGES * MD_TILE];
 // [step parity][head set][head tile][token half][lane]: the lane's four weights of each token half.  A
@@ -103,6 +129,12 @@ __shared__ __attribute__((aligned(1024))) elem_t md_tiles[MD_STAGES * MD_TILE];
 __shared__ __attribute__((aligned(16))) u32x2 md_weights[2][2][2][2][64];
 // [step parity][head set][head tile][head][token half]: the reference point those weights stand against
 __shared__ __attribute__((aligned(8))) float md_ref[2][2][2][16][2];
+#if CL_PREFILL
+// [value wave][step % 4][lane]: the table entry of the key row this lane fetches; [head set][tile][head][token half]: the
+// reference point and the sum of the unrounded weights a score wave ends with
+__shared__ __attribute__((aligned(256))) int md_ids[4][4][64];
+__shared__ __attribute__((aligned(8))) f32x2 md_sums[2][2][16][2];
+#endif
 
 typedef short md_s16x4 __attribute__((ext_vector_type(4)));
 typedef short md_s16x8 __attribute__((ext_vector_type(8)));
@@ -134,9 +166,29 @@ CL_DEVICE void md_dma16_loose(const void* gptr, unsigned lds_byte) {
                :: "v"(gptr), "s"(__builtin_amdgcn_readfirstlane(lds_byte)) : "m0");
 }
 
+#if CL_PREFILL
+// 4 bytes per lane, the same way
+CL_DEVICE void md_dma4(const void* gptr, unsigned lds_byte) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off"
+               :: "v"(gptr), "s"(__builtin_amdgcn_readfirstlane(lds_byte)) : "memory", "m0");
+}
+
+// value wave `lw`: panels P.. of the step whose rows this lane's pointers name
+template <int P>
+CL_DEVICE void md_issue_rows(const char* lat_src, const char* pe_src, unsigned stage_byte, int lw) {
+  if constexpr (P < MD_PANELS) {
+    constexpr int OFF = 128 * (P < MD_LAT_PANELS ? P : P - MD_LAT_PANELS);
+    md_dma16<OFF>(P < MD_LAT_PANELS ? lat_src : pe_src, stage_byte + (unsigned)(P * MD_PANEL * 2 + lw * 1024) - OFF);
+    md_issue_rows<P + 1>(lat_src, pe_src, stage_byte, lw);
+  }
+}
+CL_DEVICE int md_clamp(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
+#endif
+
 // every LDS access of this wave has completed, then the workgroup barrier
 CL_DEVICE void md_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
+#if !CL_PREFILL
 // value wave `lw` (0..3): its loads of one step, panel P onwards -- token rows 8 lw + lane / 8 of
 // every panel, the chunk that belongs in slot lane % 8
 template <int P>
@@ -183,6 +235,7 @@ CL_DEVICE void md_issue_panel(int p, u32 lat_off, u32 pe_off, const elem_t* lat_
                        : reinterpret_cast<const char*>(pe_rows + col) + pe_off, lds_byte);
   }
 }
+#endif
 #if CL_EMIT_PARTIAL
 extern "C" __global__ void __launch_bounds__(MD_THREADS)
 CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
@@ -195,6 +248,48 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
   const int set = wave & 1;
   const int fhalf = (wave >> 1) & 1;                      // score waves: the token half
   const int loader = 2 * (wave & 1) + fhalf;              // value waves: which 8-token group of every panel they load
+#if CL_PREFILL
+  // the request whose items include `item`: the last b with b + qo_indptr[b] / MD_TOKENS <= item; token t of it sees
+  // the keys kv_pos <= kv_len - q_len + (t - q0)
+  const int item = blockIdx.x, head0 = 16 * blockIdx.y;
+  const ClRequest found = cl_find_request(CL_ARG_QINDPTR, batch, total_q, MD_TOKENS, 1, item, lane, CL_ARG_INDPTR, n_idx);
+  const int q0 = found.p0, q1 = found.p1, chunk = item - found.req;
+  const int t_lo = q0 > chunk * MD_TOKENS ? q0 : chunk * MD_TOKENS;
+  const int t_hi = q1 < (chunk + 1) * MD_TOKENS ? q1 : (chunk + 1) * MD_TOKENS;
+  if (t_hi <= t_lo) return;                           // an index no (chunk, request) pair maps to
+  const int lo = found.s0, kv_len = found.s1 > lo ? found.s1 - lo : 0;
+  const int first_seen = kv_len - (q1 - q0) + (t_lo - q0) + 1;         // keys the item's first token sees (before clamping)
+  const int hi = lo + md_clamp(first_seen + (t_hi - 1 - t_lo), 0, kv_len);
+  const int n_own = __builtin_amdgcn_readfirstlane((hi - lo + MD_STEP - 1) / MD_STEP);
+  const unsigned tiles_byte = (unsigned)(size_t)(__attribute__((address_space(3))) elem_t*)md_tiles;
+  // This lane fetches key row 8 loader + lane / 8 of every step, the chunk that belongs in slot lane % 8.  Its table
+  // entries (positions past the item's end repeat the last one; ids are clamped into the pool) travel through LDS on
+  // the same load counter as the rows: those of step s + 1 are asked for ahead of the rows of step s.
+  const int row_in_step = 8 * loader + (lane >> 3);
+  const int row_chunk = (lane & 7) ^ md_swz(row_in_step);
+  const unsigned ids_byte = (unsigned)(size_t)(__attribute__((address_space(3))) int*)&md_ids[loader][0][0];
+  auto ask_ids = [&](int s) __attribute__((always_inline)) {
+    const int pos = lo + s * MD_STEP + row_in_step;
+    md_dma4(CL_ARG_INDICES + (pos < hi - 1 ? pos : hi - 1), ids_byte + (unsigned)((s & 3) * 256));
+  };
+  if (n_own > 0) {
+    if (!scores) {
+      ask_ids(0);
+      ask_ids(1);
+      ask_ids(2);
+    }
+    for (int k = wave; k < MD_QCHUNKS; k += MD_THREADS / 64) {         // (the rows in LDS: as below)
+      const int n = 64 * k + lane;
+      const int row = n / MD_QCHUNKS, pos = n % MD_QCHUNKS;
+      const int h = md_trade03(row);
+      const int q = (pos & ~7) | ((pos ^ h) & 7);
+      const int token = t_lo + (h >> 4) < t_hi ? t_lo + (h >> 4) : t_hi - 1;
+      const i64 qrow = (i64)token * CL_HEADS + head0 + (h & 15);
+      md_dma16<0>(q < CL_CKV / 8 ? CL_ARG_Q + qrow * CL_CKV + 8 * q : CL_ARG_QPE + qrow * CL_KPE + 8 * (q - CL_CKV / 8),
+                  tiles_byte + (unsigned)(2 * MD_TILE * 2 + 1024 * k));
+    }
+  }
+#else
   // Workgroups go to the eight XCDs (one L2 each) round-robin in launch order.  Every workgroup
   // of a batch entry is given to one XCD (batch entry b to XCD b % 8): the head blocks of a split
   // read the same kv rows and the splits of a head block the same Q rows, so each row comes out of
@@ -257,6 +352,7 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
     lat_off = (u32)((r * CL_CKV + 8 * chunk) * 2);
     pe_off = (u32)((r * CL_KPE + 8 * chunk) * 2);
   }
+#endif
   if (scores) {
     // =========================================================================== score wave
     // Q fragments (B operand): lane (c, g) holds q[head 16 t + c][32 j + 8 g .. + 8] for head tile t
@@ -279,12 +375,30 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
     }
     float m_run[2] = {CL_NEG_BIG, CL_NEG_BIG};      // reference point of head c of each tile (log2 domain), uniform over g
     const int half = fhalf;
+#if CL_PREFILL
+    const float scale_log2e = sm_scale * 1.4426950408889634f;
+    float l_exact[2] = {0.f, 0.f};                  // this lane's share of the sum of the unrounded weights
+    int n_tok[2];                                   // keys the token of each tile sees
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+      n_tok[t] = t_lo + 2 * set + t < t_hi ? md_clamp(first_seen + 2 * set + t, 0, kv_len) : 0;
+#endif
     const int a_lo = (16 * half + c) * 64 + ((g ^ md_swz(c)) << 3);
 
     for (int it = 0; it <= n_own; ++it) {
 #if CL_S_PANELS
       // this wave's panels of image `it` have landed: at most those of image it + 1 are on their way
       __builtin_amdgcn_s_waitcnt(0x0F70 | (CL_S_PANELS & 15));
+#endif
+#if CL_PREFILL
+      if (it == n_own) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          l_exact[t] += lane_xor(l_exact[t], lane, 16);
+          l_exact[t] += lane_xor(l_exact[t], lane, 32);
+          if (g == 0) md_sums[set][t][c][half] = (f32x2){m_run[t], l_exact[t]};
+        }
+      }
 #endif
       md_barrier();                                 // image `it` has landed (the value waves waited for it)
       if (it == n_own) break;
@@ -336,6 +450,19 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
 #pragma unroll
       for (int t = 0; t < 2; ++t) st[t] = sp[t][0] + sp[t][1];
 
+#if CL_PREFILL
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        st[t] *= scale_log2e;
+        if ((it + 1) * MD_STEP > n_tok[t]) {        // keys past the token's limit: weight exp2(-huge) = 0
+          const int t0 = it * MD_STEP + 16 * half + 4 * g;
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (t0 + r >= n_tok[t]) st[t][r] = CL_NEG_BIG;
+        }
+      }
+      const float m_before[2] = {m_run[0], m_run[1]};
+#else
       if (MD_RAGGED) {
         const int t0 = (step_begin + it) * MD_STEP + 16 * half + 4 * g;
 #pragma unroll
@@ -344,10 +471,11 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
           for (int r = 0; r < 4; ++r)
             if (t0 + r >= CL_SKV) st[t][r] = CL_NEG_BIG;      // weight exp2(-huge) = 0
       }
+#endif
       float mx[2];
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
-        mx[t] = fmaxf(fmaxf(st[t][0], st[t][1]), fmaxf(st[t][2], st[t][3])) * CL_SCALE_LOG2E;
+        mx[t] = fmaxf(fmaxf(st[t][0], st[t][1]), fmaxf(st[t][2], st[t][3])) * MD_SCALE;
         m_run[t] = fmaxf(m_run[t], other[t]);         // adopted where higher
       }
       if (it == 0 || __builtin_amdgcn_ballot_w64(mx[0] > m_run[0] + MD_RESCALE_STEP || mx[1] > m_run[1] + MD_RESCALE_STEP)) {
@@ -361,13 +489,37 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
             m_run[t] = fmaxf(v, MD_REF_FLOOR);      // nothing behind it yet: the step's own maximum
           else if (v > m_run[t] + MD_RESCALE_STEP)
             m_run[t] = v;
+#if CL_PREFILL
+          if (it == 0 && g == 0) md_ref[1][set][t][c][half] = m_run[t];
+#endif
         }
+#if CL_PREFILL
+        if (it == 0) {
+          // both token halves start from the larger of their maxima: no weight of the first step is scaled (and
+          // rounded) a second time.  (This slot is written again behind the next iteration's barrier.)
+          md_barrier();
+#pragma unroll
+          for (int t = 0; t < 2; ++t) m_run[t] = fmaxf(m_run[t], md_ref[1][set][t][c][half ^ 1]);
+        }
+#endif
       }
+#if CL_PREFILL
+      if (__builtin_amdgcn_ballot_w64(m_run[0] != m_before[0] || m_run[1] != m_before[1])) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t) l_exact[t] *= fast_exp2(m_before[t] - m_run[t]);
+      }
+#endif
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         elem4 pf;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) pf[r] = to_elem(fast_exp2(__builtin_fmaf(st[t][r], CL_SCALE_LOG2E, -m_run[t])));
+        for (int r = 0; r < 4; ++r) {
+          const float p = fast_exp2(__builtin_fmaf(st[t][r], MD_SCALE, -m_run[t]));
+#if CL_PREFILL
+          l_exact[t] += p;
+#endif
+          pf[r] = to_elem(p);
+        }
         md_weights[it & 1][set][t][half][lane] = __builtin_bit_cast(u32x2, pf);
         if (g == 0) md_ref[it & 1][set][t][c][half] = m_run[t];
       }
@@ -379,6 +531,19 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
   }
 
   // ============================================================================= value wave
+#if CL_PREFILL
+  auto row_of = [&](int s) __attribute__((always_inline)) { return md_clamp(md_ids[loader][s & 3][lane], 0, num_pages - 1); };
+  auto lat_of = [&](int id) __attribute__((always_inline)) {
+    return reinterpret_cast<const char*>(CL_ARG_KV) + ((i64)id * CL_CKV + 8 * row_chunk) * 2;
+  };
+  auto pe_of = [&](int id) __attribute__((always_inline)) {
+    return reinterpret_cast<const char*>(CL_ARG_KPE) + ((i64)id * CL_KPE + 8 * row_chunk) * 2;
+  };
+  auto issue = [&](int s) __attribute__((always_inline)) {
+    const int id = row_of(s);
+    md_issue_rows<0>(lat_of(id), pe_of(id), tiles_byte + (unsigned)((s % MD_STAGES) * MD_TILE * 2), loader);
+  };
+#else
   // loads of step index s (relative to the split), clamped onto the split's last step so that the
   // load counter holds the same number of steps at every wait
   auto issue = [&](int s) __attribute__((always_inline)) {
@@ -388,6 +553,7 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
     md_issue_from<0>(lat_off, pe_off, kv + (i64)t0 * CL_CKV, kpe + (i64)t0 * CL_KPE, t0,
                      tiles_byte + (unsigned)((s % MD_STAGES) * MD_TILE * 2), loader);
   };
+#endif
   f32x4 acc[2][MD_FBW];                             // acc[t][fb][r] = O[head 16 t + c][16 (FBW fhalf + fb) + 4 g + r]
 #pragma unroll
   for (int t = 0; t < 2; ++t)
@@ -403,6 +569,11 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
   const int v_lo = fhalf * (MD_FBW / 4) * MD_PANEL + vtok * 64 + (((((c & 3) >> 1)) ^ md_swz(vtok)) << 3) + 4 * (c & 1);
 
   if (n_own > 0) {
+#if CL_PREFILL
+    // the entries of the first three steps, asked for ahead of this wave's Q runs
+    __builtin_amdgcn_s_waitcnt(0x0F70 | ((MD_QCHUNKS / 8) & 15) | (((MD_QCHUNKS / 8) >> 4) << 14));
+    asm volatile("" ::: "memory");
+#endif
     issue(0);
     issue(1);
     // this wave's Q runs (asked for before the two images) have landed, then everybody else's
@@ -429,8 +600,14 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
     if (n_own > 0) __builtin_amdgcn_s_waitcnt(0x0F70 | (MD_V_UNITS & 15) | ((MD_V_UNITS >> 4) << 14));
     md_barrier();
     const elem_t* next_tile = md_tiles + (it % MD_STAGES) * MD_TILE;           // image `it`: there from here on
+#if CL_PREFILL
+    if (n_own > 0) ask_ids(it + 3);                 // (ahead of the rows of it + 2: the next wait covers it)
+#endif
     if (it == 0) {
       if (it < n_own) issue(it + 2);
+#if CL_PREFILL
+      if (n_own > 0) md_barrier();                  // (the score waves exchange their first maxima)
+#endif
 #pragma unroll
       for (int fb = 0; fb < MD_PRE; ++fb) operand(next_tile, fb, pre_lo[fb], pre_hi[fb]);
       continue;
@@ -467,10 +644,15 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
     // last image is asked for again, into the slot of image n_own + 1 (which holds or awaits the
     // same rows): the load counter then holds the same number of loads at every wait.
     const int ahead = it + 2 < n_own + 1 ? it + 2 : n_own + 1;
+#if CL_PREFILL
+    const int id = row_of(ahead);                   // (past the item's end: its last row)
+    const char *lat_src = lat_of(id), *pe_src = pe_of(id);
+#else
     const int rel = ahead < n_own - 1 ? ahead : n_own - 1;
     const int t0 = (step_begin + rel) * MD_STEP;
     const elem_t* lat_rows = kv + (i64)t0 * CL_CKV;
     const elem_t* pe_rows = kpe + (i64)t0 * CL_KPE;
+#endif
     const unsigned stage_byte = tiles_byte + (unsigned)((ahead % MD_STAGES) * MD_TILE * 2);
     // out^T block fb: rows = features 16 fb + (0..15), slots = tokens 4 g + (0..3), 16 + 4 g + (0..3)
 #pragma unroll
@@ -486,7 +668,14 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
         operand(next_tile, fb + MD_PRE - MD_FBW, pre_lo[fb % MD_PRE], pre_hi[fb % MD_PRE]);
 #pragma unroll
       for (int pn = CL_S_PANELS; pn < MD_PANELS; ++pn)
-        if (((pn - CL_S_PANELS) * MD_FBW) / MD_V_UNITS == fb) md_issue_panel(pn, lat_off, pe_off, lat_rows, pe_rows, t0, stage_byte, loader);
+        if (((pn - CL_S_PANELS) * MD_FBW) / MD_V_UNITS == fb) {
+#if CL_PREFILL
+          md_dma16_loose(pn < MD_LAT_PANELS ? lat_src + 128 * pn : pe_src + 128 * (pn - MD_LAT_PANELS),
+                         stage_byte + (unsigned)(pn * MD_PANEL * 2 + loader * 1024));
+#else
+          md_issue_panel(pn, lat_off, pe_off, lat_rows, pe_rows, t0, stage_byte, loader);
+#endif
+        }
     }
 #pragma unroll
     for (int n = 0; n < MD_FBW; ++n) {
@@ -508,7 +697,13 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
     const float m = m_acc[t], l = l_acc[t][0];
+#if CL_PREFILL
+    if (t_lo + 2 * set + t >= t_hi) continue;                      // (a tile past the item's tokens)
+    const i64 orow = (i64)(t_lo + 2 * set + t) * CL_HEADS + head0;
+    (void)m;
+#else
     const i64 orow = row0 + 16 * t;                                // first head row of this tile
+#endif
     const float inv = 1.0f / fmaxf(l, 1.0e-30f);
 #if CL_SPLITS > 1
     const i64 prow = (i64)split * CL_TOTAL_ROWS + orow;
@@ -519,7 +714,14 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
     }
 #else
     elem_t* dst = CL_ARG_OUT + (orow + c) * CL_CKV + 16 * MD_FBW * fhalf + 16 * (g & 1) + 4 * (g & 2);
-#if CL_EMIT_LSE
+#if CL_EMIT_LSE && CL_PREFILL
+    if (g == 0 && fhalf == 0) {
+      const f32x2 a = md_sums[set][t][c][0], b = md_sums[set][t][c][1];
+      const float m_both = fmaxf(a[0], b[0]);
+      const float l_both = a[1] * fast_exp2(a[0] - m_both) + b[1] * fast_exp2(b[0] - m_both);
+      CL_ARG_LSE[orow + c] = l_both > 0.f ? m_both + fast_log2(l_both) : CL_NEG_INF;
+    }
+#elif CL_EMIT_LSE
     if (g == 0 && fhalf == 0) CL_ARG_LSE[orow + c] = l > 0.f ? m + fast_log2(l) : CL_NEG_INF;
 #endif
 #endif

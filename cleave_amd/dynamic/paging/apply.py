@@ -337,7 +337,7 @@ def mla_chunk_pages_expr(spec: MLASpec, chunk_pages: int) -> str:
     return f"max(32, min(512, ceildiv({spec.index_dim}, max(1, {2 * cus} - {spec.batch_dim}))))"
 
 
-def _mla_plan(spec: MLASpec, dense: DenseMLA, role, params, operands, split=None, tok: int = 1) -> KernelPlan:
+def _mla_plan(spec: MLASpec, dense: DenseMLA, role, params, operands, split=None, tok: int = 1, duo: bool = False) -> KernelPlan:
     prefill = spec.kind == MLA_PAGED_PREFILL_CAUSAL
     dim_names = {"total_q": spec.tokens_dim, "num_pages": spec.pages_dim, "n_idx": spec.index_dim} if prefill else \
         {"batch": spec.batch_dim, "num_pages": spec.pages_dim, "n_idx": spec.index_dim}
@@ -357,11 +357,15 @@ def _mla_plan(spec: MLASpec, dense: DenseMLA, role, params, operands, split=None
     if dense.ksplit != 1 and not split:
         tiling["KSPLIT"] = int(dense.ksplit)
     threads = dense.n_threads * max(int(tok) if prefill else 1, int(tiling.get("KSPLIT", 1)))
+    if duo:
+        tiling["DUO"], threads = 1, 512
     label = f"kv={dense.kv_tile} q={dense.heads * (int(tok) if prefill else 1)} thr={threads}"
     if dense.stages != 2:
         label += f" stages={dense.stages}"
     if tiling.get("KSPLIT"):
         label += f" ksplit={dense.ksplit}"
+    if duo:
+        label += " duo"
     return KernelPlan(template="mla_decode", role=role, family="mla", dtype=dense.dtype, extra=extra, problem=problem,
                       tiling=tiling, params=params, operands=operands, split_factor=split, dyn_dims=dyn,
                       n_threads=threads, label=label)
@@ -391,9 +395,16 @@ def mla_prefill_variants(plan: KernelPlan, spec) -> list:
     two to four images of a step in LDS (the search times each: an item's waves share its key
     images, which divides the traffic into the CU and raises the number of waves a CU holds, but
     they also share the LDS bandwidth that bounds this kernel's matrix work; more images keep the
-    rows of more steps in flight, which a lone item needs and many resident items do not)."""
-    return [apply_paging(plan, spec, tok=t, stages=s, ksplit=k)
-            for t, s, k in ((2, 2, 1), (2, 3, 1), (2, 4, 1), (4, 2, 1), (4, 4, 1), (1, 2, 1), (1, 3, 1), (1, 2, 2))]
+    rows of more steps in flight, which a lone item needs and many resident items do not); and, where
+    its images fit, four tokens per item with score waves and value waves."""
+    from ...schedule.policy import mla_duo_lds_bytes
+
+    out = [apply_paging(plan, spec, tok=t, stages=s, ksplit=k)
+           for t, s, k in ((2, 2, 1), (2, 3, 1), (2, 4, 1), (4, 2, 1), (4, 4, 1), (1, 2, 1), (1, 3, 1), (1, 2, 2))]
+    dense = read_dense_mla(plan)
+    if dense.ckv % 128 == 0 and mla_duo_lds_bytes(dense.ckv, dense.kpe, True) <= 160 * 1024:
+        out.append(apply_paging(plan, spec, tok=4, duo=True))
+    return out
 
 
 def mla_decode_variants(plan: KernelPlan, spec) -> list:
@@ -402,10 +413,10 @@ def mla_decode_variants(plan: KernelPlan, spec) -> list:
     return [apply_paging(plan, spec, stages=s, ksplit=k) for s, k in ((2, 1), (3, 1), (2, 2))]
 
 
-def apply_paging(plan: KernelPlan, spec, tok: int = 2, stages: int = 2, ksplit: int = 1) -> KernelPlan:
+def apply_paging(plan: KernelPlan, spec, tok: int = 2, stages: int = 2, ksplit: int = 1, duo: bool = False) -> KernelPlan:
     """A single paged kernel at ``plan``'s tiling (``tok``: query tokens per work item of the
     paged MLA causal prefill layer; ``stages``: images of a step the paged MLA kernels keep in LDS;
-    ``ksplit``: waves that deal an item's steps out between them)."""
+    ``ksplit``: waves that deal an item's steps out between them; ``duo``: score waves and value waves)."""
     spec.validate()
     if isinstance(spec, MLASpec):
         dense = dataclasses.replace(read_dense_mla(plan), stages=int(stages), ksplit=int(ksplit))
@@ -414,7 +425,7 @@ def apply_paging(plan: KernelPlan, spec, tok: int = 2, stages: int = 2, ksplit: 
         _check_tiling(spec, dense)
         params, operands = _mla_params(spec, dense)
         outs, out_ops = _mla_outputs(spec, dense)
-        return _mla_plan(spec, dense, "main", params + outs, {**operands, **out_ops}, tok=tok)
+        return _mla_plan(spec, dense, "main", params + outs, {**operands, **out_ops}, tok=tok, duo=duo)
     dense = read_dense_attention(plan)
     _check_tiling(spec, dense)
     if spec.kind in CAUSAL_KINDS:

@@ -515,6 +515,12 @@ def mla_lds_bytes(ckv, kpe, stages=3):
     return stages * ((ckv + kpe) // 64) * 32 * 64 * 2
 
 
+def mla_duo_lds_bytes(ckv, kpe, prefill=False):
+    """LDS of the score-wave / value-wave kernel: four images, weights and reference points in flight, and for prefill the
+    table entries of four steps and the final sums."""
+    return mla_lds_bytes(ckv, kpe, 4) + (14 if prefill else 9) * 1024
+
+
 def mla_ok(low) -> bool:
     p = low.problem
     return p["heads"] % 16 == 0 and p["ckv"] % 64 == 0 and p["kpe"] % 64 == 0
@@ -573,7 +579,7 @@ def mla_candidates(low, role, factor, arch: Arch):
     # The score-wave / value-wave form: eight waves own 64 heads, every LDS operand feeds two matrix
     # ops.  Measured 25-30 % ahead of the best form above wherever both run, so it is ranked first
     # (with the shorter read-ahead of its value operands as a second candidate).
-    duo_lds = mla_lds_bytes(p["ckv"], p["kpe"], 4) + 9 * 1024
+    duo_lds = mla_duo_lds_bytes(p["ckv"], p["kpe"])
     if out and p["heads"] % 64 == 0 and p["ckv"] % 128 == 0 and duo_lds <= arch.lds_bytes:
         best = min(c.score for c in out)
         # (third: the score waves ask for about half of every image's panels -- a wave that waits for the

@@ -172,3 +172,35 @@ def test_paged_mla_causal_prefill(q_lens, kv_lens, tok, stages, ksplit):
     live = np.isfinite(want_l)
     np.testing.assert_allclose(got_l[live], want_l[live], rtol=1e-3, atol=1e-3)
     assert np.all(np.isneginf(got_l[~live])) and np.all(got_o[~live.any(axis=1)] == 0)
+
+
+def mla_duo_prefill_kernel(heads, ckv, dtype):
+    spec = MLASpec(num_qo_heads=heads, kind=MLA_PAGED_PREFILL_CAUSAL, causal=True)
+    dense = DenseMLA(heads, ckv, 64, dtype, dtype)
+    params, ops = _mla_params(spec, dense)
+    outs, out_ops = _mla_outputs(spec, dense)
+    loaded = _load_main_kernel_from_code(HipCodeGen().gen(_mla_plan(spec, dense, "main", params + outs, {**ops, **out_ops}, tok=4, duo=True)))
+    return _compile(loaded, loaded.manifest["out_idx"])
+
+
+@pytest.mark.parametrize("heads,ckv,dtype,scale", [(16, 512, "bfloat16", 0.05), (32, 256, "bfloat16", -0.05), (16, 512, "float16", 0.3)])
+@pytest.mark.parametrize("q_lens,kv_lens", [([1, 4, 5, 33, 0, 40, 7], [1, 4, 40, 33, 9, 300, 3]), ([6, 0, 3], [0, 5, 3]), ([90], [700]), ([3, 9], [2, 5]),
+                                            ([1] * 70, [1 + 3 * i for i in range(70)]), ([2, 2, 2], [16, 17, 65])])
+def test_paged_mla_prefill_with_score_and_value_waves(q_lens, kv_lens, heads, ckv, dtype, scale):
+    """Four tokens per item in tiles of one token: items cut by request boundaries, tokens that see no key beside live
+    ones, one to more steps than images, limits inside either token half, more than 64 requests; two head groups, a
+    narrower latent row, a negative scale, scores large enough to raise the reference point.  The oracle in float64
+    on the same inputs: the output is rounded once (2^-9 relative in bf16, 2^-12 in f16) and the weights once."""
+    tq, tk = sum(q_lens), sum(kv_lens)
+    kind = getattr(torch, dtype)
+    args = dref.mla_paged_prefill_inputs((heads, ckv, 64, 4 * tk + 64, tk + 3, tq), q_lens, kv_lens, device="cpu", dtype=kind, scale=scale)
+    args[6][tk:] = 2 ** 30
+    print(f"paged mla duo prefill q_lens={q_lens[:8]} kv_lens={kv_lens[:8]} heads={heads} ckv={ckv} {dtype}", flush=True)
+    out, lse = mla_duo_prefill_kernel(heads, ckv, dtype)(*[a.cuda() if isinstance(a, torch.Tensor) else a for a in args])
+    torch.cuda.synchronize()
+    got_o, got_l = out.float().cpu().numpy(), lse.cpu().numpy()
+    want_o, want_l = paged_oracle.mla_prefill(*args[:7], q_lens, kv_lens, args[7])
+    np.testing.assert_allclose(got_o, want_o, rtol=1e-2, atol=2e-2)
+    live = np.isfinite(want_l)
+    np.testing.assert_allclose(got_l[live], want_l[live], rtol=1e-5, atol=2e-4)
+    assert np.all(np.isneginf(got_l[~live])) and np.all(got_o[~live.any(axis=1)] == 0)
