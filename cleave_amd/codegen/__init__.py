@@ -28,7 +28,13 @@ ENTRY = "main_kernel"
 COMBINE_ENTRY = "main_kernel_combine"
 MANIFEST_BEGIN = "// CLEAVE-HIP-MANIFEST-BEGIN"
 MANIFEST_END = "// CLEAVE-HIP-MANIFEST-END"
+ALIGN16 = "// CLEAVE-HIP-ALIGN16:"          # the line after the manifest that names the inputs of DIRECT_TO_LDS
 LOG2E = 1.4426950408889634
+
+# The operands that a template moves from global memory straight into LDS in 16-byte pieces.  Such a load needs its pieces
+# at multiples of 16 bytes; everything else is read through registers, which takes any element's address.
+DIRECT_TO_LDS = {"gemm_tile.hip": ("A", "B", "C"), "mla_decode.hip": ("KV", "KPE"), "mla_paged_decode.hip": ("KV", "KPE"),
+                 "mla_decode_duo.hip": ("Q", "QPE", "KV", "KPE"), "attn_prefill_lds.hip": ("K", "V")}
 
 _C_TYPES = {"float16": "elem_t", "bfloat16": "elem_t", "float32": "float", "int32": "int"}
 
@@ -64,6 +70,7 @@ class _Unit:
         self.defines: list = []
         self.launches: list = []
         self.templates: list = ["common.hip"]
+        self.direct: dict = {}          # operand role -> the parameter it is read from, where that is not the plan's own
 
     def define(self, name, value):
         if isinstance(value, bool):
@@ -156,6 +163,8 @@ class HipCodeGen:
             "out_idx": list(range(-n_out, 0)), "launches": unit.launches,
         }
         head = [MANIFEST_BEGIN] + ["// " + line for line in json.dumps(manifest, indent=1).splitlines()] + [MANIFEST_END]
+        direct = {unit.direct.get(role, plan.operands.get(role)) for name in unit.templates for role in DIRECT_TO_LDS.get(name, ())}
+        head.append(" ".join([ALIGN16] + [p.name for p in params if p.role == "input" and p.name in direct]))
         body = [f"// ---- template: {plan.template}  role: {plan.role}  {plan.label}"]
         body += unit.defines
         for name in unit.templates:
@@ -526,6 +535,7 @@ class HipCodeGen:
             key = self._by_name(params)[op["K"]]
             at = next(i for i, q in enumerate(params) if q.role in ("scratch", "output"))
             params.insert(at, ParamSpec("Scratch_kn", key.dtype, key.shape, "scratch"))
+            unit.direct["K"] = "Scratch_kn"
         self._attn_common(unit, plan, params, partial, combine, False, p["vdim"], p["units"] * rows, False)
         for k, v in (("CL_DENSE", 1), ("CL_RAGGED", 1), ("CL_HEAD_DIM", d), ("CL_KV_HEADS", 1), ("CL_Q_HEADS", 1),
                      ("CL_ROWS", rows), ("CL_SKV", p["skv"])):
@@ -751,6 +761,19 @@ class HipCodeGen:
             unit.launch(entry, (f"ceildiv(({batch_name} * {p['heads']}) * {p['ckv'] // 4}, 256)", 1, 1), 256, 0, args)
 
 
+def aligned_inputs(source: str, params) -> frozenset:
+    """The inputs that a generated source reads in 16-byte pieces past the registers: what its ``ALIGN16`` line names, or,
+    in a source written before that line was, every 16-bit input of a source that has such loads."""
+    for line in source.splitlines():
+        if line.startswith(ALIGN16):
+            return frozenset(line[len(ALIGN16):].split())
+        if line.startswith("// ---- template:"):
+            break
+    if "global_load_lds" not in source:
+        return frozenset()
+    return frozenset(p.name for p in params if p.role == "input" and p.dtype in ("float16", "bfloat16"))
+
+
 def parse_manifest(source: str) -> dict:
     """The manifest a generated source carries (raises ``CodegenError`` when it has none)."""
     try:
@@ -765,4 +788,4 @@ def parse_manifest(source: str) -> dict:
         raise CodegenError(f"kernel manifest is not valid JSON: {e}") from e
 
 
-__all__ = ["HipCodeGen", "parse_manifest", "ENTRY", "COMBINE_ENTRY", "TEMPLATE_DIR"]
+__all__ = ["HipCodeGen", "parse_manifest", "aligned_inputs", "ENTRY", "COMBINE_ENTRY", "TEMPLATE_DIR"]

@@ -18,7 +18,7 @@ import hashlib
 import threading
 from dataclasses import dataclass
 
-from ..codegen import HipCodeGen, parse_manifest
+from ..codegen import HipCodeGen, aligned_inputs, parse_manifest
 from ..core.errors import BackendUnavailable, CompileError
 from ..schedule.plan import ParamSpec
 from . import shim
@@ -143,10 +143,9 @@ class CompiledKernel:
         self._code = code
         self._module = None
         self._plan = None                # the native call plan, made on the first call
-        # The direct-to-LDS matmuls move 16-byte pieces of their operands past the registers: an operand that
-        # starts between two of them (a view one element into a buffer) is copied for the call.
-        manifest = self.manifest
-        self.input_align = 16 if manifest.get("template") == "gemm_dma" or (manifest.get("tiling") or {}).get("DMA") else 1
+        # Inputs whose 16-byte pieces the kernel moves past the registers: one that starts between two of them (a
+        # view one element into a buffer) is copied for the call.
+        self.aligned_inputs = aligned_inputs(loaded.source, self.params)
         self._caller_params = [p for p in self.params if p.role != "scratch"]
         self._n_out = sum(p.role == "output" for p in self.params)
         if self.out_idx is not None:
@@ -317,9 +316,9 @@ class CompiledKernel:
         import torch
 
         bound, dims, device = self._bind(args)
-        for p in self.params:
-            if p.role == "input" and bound[p.name].data_ptr() % self.input_align:
-                bound[p.name] = bound[p.name].clone()
+        for name in self.aligned_inputs:
+            if bound[name].data_ptr() % 16:
+                bound[name] = bound[name].clone()
         outs = self._materialise(bound, dims, device)
         with torch.cuda.device(device):
             descs, keep = self._descs(bound, dims)

@@ -108,8 +108,8 @@ def chain_plan(stages, *, arguments=None, output_shapes=None, as_tuple=False):
         caller = [p for p in last.params if p.role != "scratch" and (p.role != "output" or last.out_idx is None)]
         arguments = [(p, None) for p in caller]
         stages = [(last, {p.name: ("arg", i) for i, p in enumerate(caller)})]
-    align = max(kernel.input_align for kernel, _ in stages)
-    args = [_argument(p, dims, shape, align if p.role == "input" else 1) for p, shape in arguments]
+    aligned = {sources[name] for kernel, sources in stages for name in kernel.aligned_inputs}
+    args = [_argument(p, dims, shape, 16 if ("arg", i) in aligned else 1) for i, (p, shape) in enumerate(arguments)]
     n_dims = len(dims)
     derived = []
     for kernel, _ in stages:

@@ -109,3 +109,46 @@ def test_operands_between_two_16_byte_pieces_are_copied_for_the_direct_to_lds_ke
         moved.append(buffer[1:].view(t.shape).copy_(t))
     assert kernel._plan and kernel._plan(*moved) is NotImplemented
     assert torch.equal(kernel(*moved), want) and torch.equal(kernel._checked_call(*moved), want)
+
+
+def _direct_to_lds_cases():
+    from cleave_amd.dynamic.paging import MLA_PAGED_PREFILL_CAUSAL, DenseMLA, MLASpec
+    from cleave_amd.dynamic.paging.apply import _mla_outputs, _mla_params, _mla_plan
+
+    def mla_prefill(duo):
+        spec, dense = MLASpec(num_qo_heads=16, kind=MLA_PAGED_PREFILL_CAUSAL, causal=True), DenseMLA(16, 512, 64, "bfloat16", "bfloat16")
+        (params, ops), (outs, out_ops) = _mla_params(spec, dense), _mla_outputs(spec, dense)
+        loaded = _load_main_kernel_from_code(HipCodeGen().gen(
+            _mla_plan(spec, dense, "main", params + outs, {**ops, **out_ops}, tok=4, duo=duo)))
+        q_lens, kv_lens = [3, 9], [40, 9]
+        return _compile(loaded, loaded.manifest["out_idx"]), dref.mla_paged_prefill_inputs((16, 512, 64, 96, 49, 12), q_lens, kv_lens)
+
+    def mla(tiling):
+        shapes = dict(B=1, H=64, D=512, PE=64, SKV=70)
+        return kernel_for(C.mla_decode.trace(cl.bf16, **shapes), template="mla_decode", tiling=tiling), C.inputs_c4(shapes)
+
+    def attention():
+        shapes = dict(HQ=8, HKV=8, SQ=130, SKV=70, D=128)
+        return kernel_for(C.gqa_decode_exact.trace(cl.f16, **shapes), template="attn_prefill", tiling=dict(SHARED=1)), C.inputs_c3(shapes)
+
+    return {"mla_prefill_duo": lambda: mla_prefill(True), "mla_prefill": lambda: mla_prefill(False), "mla_duo": lambda: mla(dict(DUO=1)),
+            "mla": lambda: mla(dict(WAVES=4)), "attention": attention}
+
+
+@pytest.mark.parametrize("case", _direct_to_lds_cases())
+def test_operands_between_two_16_byte_pieces(case):
+    """Every 16-bit operand in turn as a view one element into a buffer: the same bits as from the aligned one."""
+    kernel, args = _direct_to_lds_cases()[case]()
+    args = [a.cuda() if isinstance(a, torch.Tensor) else a for a in args]
+
+    def run(ins):
+        got = kernel(*ins)
+        return list(got) if isinstance(got, (list, tuple)) else [got]
+
+    want = run(args)
+    for i, t in enumerate(args):
+        if isinstance(t, torch.Tensor) and t.element_size() == 2:
+            buffer = torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")
+            ins = [*args[:i], buffer[1:].view(t.shape).copy_(t), *args[i + 1:]]
+            print(f"{case}: operand {i} {tuple(t.shape)} one element into its buffer", flush=True)
+            assert all(torch.equal(a, b) for a, b in zip(run(ins), want)), i
