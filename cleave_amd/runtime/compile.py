@@ -227,6 +227,12 @@ class CompiledKernel:
             raise ValueError(f"run-time dims {missing} could not be inferred from the arguments")
         return bound, dims, device
 
+    def _align(self, bound):
+        """Copies, for the launches that read ``bound``, of the ``aligned_inputs`` that start between two 16-byte pieces."""
+        for name in self.aligned_inputs:
+            if bound[name].data_ptr() % 16:
+                bound[name] = bound[name].clone()
+
     def _shape(self, p: ParamSpec, dims) -> tuple:
         return tuple(s if isinstance(s, int) else eval_extent(s, dims) for s in p.shape)
 
@@ -316,9 +322,7 @@ class CompiledKernel:
         import torch
 
         bound, dims, device = self._bind(args)
-        for name in self.aligned_inputs:
-            if bound[name].data_ptr() % 16:
-                bound[name] = bound[name].clone()
+        self._align(bound)
         outs = self._materialise(bound, dims, device)
         with torch.cuda.device(device):
             descs, keep = self._descs(bound, dims)
@@ -351,12 +355,14 @@ class CompiledKernel:
         (split partials) live in the native library's fixed per-GPU array instead of tensors.  The
         kernel must have been made with ``out_idx=None``; ``args`` are the inputs, scalars and
         outputs in parameter order.  A layout beyond the array's size is refused by the library.
-        Calls that overlap on one GPU share the array and race."""
+        Calls that overlap on one GPU share the array and race.  (One of the ``aligned_inputs`` that starts
+        between two 16-byte pieces is copied for the call: the one allocation there can be.)"""
         import torch
 
         if self.out_idx is not None:
             raise TypeError("call_fixed_scratch needs caller-owned outputs: compile with out_idx=None")
         bound, dims, device = self._bind(args)
+        self._align(bound)
         fixed, nbytes = self.fixed_scratch_layout(dims)
         refs = []
         with torch.cuda.device(device):
@@ -379,6 +385,7 @@ class CompiledKernel:
         device = None
         for a in sets:
             bound, dims, device = self._bind(a)
+            self._align(bound)
             held.append(self._materialise(bound, dims, device))
             buffers.append(bound)      # scratch included: the launches below hold its addresses
             if self.out_idx is not None:

@@ -152,3 +152,23 @@ def test_operands_between_two_16_byte_pieces(case):
             ins = [*args[:i], buffer[1:].view(t.shape).copy_(t), *args[i + 1:]]
             print(f"{case}: operand {i} {tuple(t.shape)} one element into its buffer", flush=True)
             assert all(torch.equal(a, b) for a, b in zip(run(ins), want)), i
+
+
+@pytest.mark.parametrize("k", [128, 200], ids=["whole_steps", "partly_filled"])
+def test_timed_and_allocation_free_calls_take_such_operands_too(k):
+    shapes = dict(M=66, N=136, K=k)
+    tile = dict(BM=64, BN=64, BK=64, WM=2, WN=2)
+    kernel = kernel_for(C.matmul.trace(cl.f16, **shapes), **(dict(template="gemm", tiling=dict(tile, DMA=1)) if k % 64 else
+                                                            dict(template="gemm_dma", tiling=tile)))
+    owned = _compile(kernel.loaded, None)
+    a, b = (torch.randn(*s, dtype=torch.float16, device="cuda") for s in ((66, k), (k, 136)))
+    want = kernel(a, b)
+    moved = [torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")[1:].view(t.shape).copy_(t) for t in (a, b)]
+    out = torch.zeros_like(want)
+    owned.call_fixed_scratch(*moved, out)
+    assert torch.equal(out, want)
+    out.zero_()
+    owned.time(*moved, out, warmup=1, iters=2, rotate=[(*moved, out)])
+    assert torch.equal(out, want)
+    kernel.time(*moved, warmup=1, iters=2)
+    assert torch.equal(kernel.last_timed_outputs[0], want)
