@@ -189,23 +189,21 @@ def split_threshold(tiles: dict, split_us: dict, single_us: dict) -> int:
 
 
 def lone_request(kernel, inputs, expected, indptr_at):
-    """A workload cut down to its longest request: the extents of every input are known by their names in
-    the kernel's parameters (the batch, its row pointers, its slice of the page table; caches stay whole)."""
+    """A workload cut down to its longest request.  What an input's leading extent is called in the kernel's parameters
+    says how: the batch (the outputs' leading extent), its row pointers, or, of the other vectors, the page table's
+    length; caches stay whole, also where their pages are as many as the requests."""
     bounds = inputs[indptr_at].tolist()
     b = max(range(len(bounds) - 1), key=lambda r: bounds[r + 1] - bounds[r])
     declared = [p for p in kernel.params if p.role in ("input", "scalar")]
-    named = {declared[indptr_at].shape[0]: len(bounds)}
-    batch, lo, hi = len(bounds) - 1, bounds[b], bounds[b + 1]
+    batch = next(p for p in kernel.params if p.role == "output").shape[0]
     cut = []
-    for p, value in zip(declared, inputs):
-        if p.role == "scalar":
-            cut.append(value)
-        elif p.shape[0] in named:
+    for i, (p, value) in enumerate(zip(declared, inputs)):
+        if i == indptr_at:
             cut.append(value[b:b + 2] - value[b])
-        elif len(p.shape) == 1 and not isinstance(p.shape[0], int) and value.shape[0] >= hi and value.shape[0] != batch:
-            cut.append(value[lo:hi].contiguous())
-        elif value.shape[0] == batch:
+        elif p.role == "input" and p.shape[0] == batch:
             cut.append(value[b:b + 1].contiguous())
+        elif p.role == "input" and len(p.shape) == 1:
+            cut.append(value[bounds[b]:bounds[b + 1]].contiguous())
         else:
             cut.append(value)
     return cut, [t[b:b + 1].contiguous() for t in expected]

@@ -383,3 +383,37 @@ def test_lone_request_keeps_one_requests_rows_and_table():
     assert cut[0].shape[0] == 1 and float(cut[0][0, 0, 0]) == 1.0 and cut[1] is cache and cut[6] == 0.1
     assert cut[3].tolist() == [0, 4] and cut[4].tolist() == [2, 3, 4, 5] and cut[5].tolist() == [6]
     assert float(expected[0][0, 0, 0]) == 1.0
+
+
+@pytest.mark.parametrize("name", ["gqa_paged_decode_h32_kv8_d128_ps64", "gqa_paged_decode_h32_kv8_d128_ps1", "mla_paged_decode_h16_ckv512_kpe64_ps1"])
+@pytest.mark.parametrize("bounds,pages", [([0, 1, 2, 3], 3), ([0, 0, 2, 3], 9), ([0, 0, 2, 3], 3), ([0, 2, 2, 4, 5], 5)])
+def test_lone_request_goes_by_the_extents_names(name, bounds, pages):
+    """As many pages, or as many table entries, as there are requests: the caches stay whole, the table is the request's."""
+    from cleave_amd.dynamic import OPERATORS
+    from cleave_amd.pipeline.dynamic import lone_request
+    from cleave_amd.runtime.autotune import param_index
+    from cleave_amd.runtime.compile import _load_main_kernel_from_code
+
+    loaded = _load_main_kernel_from_code(OPERATORS[name].kernel_source())
+    batch, table = len(bounds) - 1, bounds[-1]
+    extents = {"batch": batch, "num_pages": pages, "len_indptr": batch + 1, "n_idx": table}
+    inputs = []
+    for p in loaded.params:
+        if p.role == "scalar":
+            inputs.append(0.1)
+        elif p.role == "input":
+            shape = [extents.get(e, e) for e in p.shape]
+            inputs.append(torch.arange(shape[0], dtype=torch.int32) if len(shape) == 1 else torch.zeros(shape))
+    at = param_index(loaded, "PlaceHolder_KV_INDPTR")
+    inputs[at] = torch.tensor(bounds, dtype=torch.int32)
+    cut, _ = lone_request(loaded, inputs, [], at)
+    b = max(range(batch), key=lambda r: bounds[r + 1] - bounds[r])
+    for p, value, whole in zip((p for p in loaded.params if p.role != "output"), cut, inputs):
+        if p.role == "scalar" or p.shape[0] == "num_pages":
+            assert value is whole
+        elif p.shape[0] == "n_idx":
+            assert value.tolist() == list(range(bounds[b], bounds[b + 1]))
+        elif p.shape[0] == "batch":
+            assert value.shape[0] == 1 and (len(p.shape) > 1 or value.tolist() == [b])
+        else:
+            assert value.tolist() == [0, bounds[b + 1] - bounds[b]]
