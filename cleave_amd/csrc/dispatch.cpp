@@ -29,7 +29,6 @@ namespace {
 
 typedef int (*launch_fn)(void* fn, const uint32_t grid[3], const uint32_t block[3], uint32_t lds, void* stream,
                          void** args, int nargs);
-typedef const char* (*error_fn)();
 
 // ---- extents: integers, or expressions over the run-time dims in postfix form ----------------------
 enum Op : int64_t { CONST_, DIM, ADD, SUB, MUL, FLOORDIV, MOD, NEG, CEILDIV, MIN_, MAX_ };
@@ -127,8 +126,8 @@ struct Plan {
   int result;                    // 0: None, 1: a tensor or a list of tensors, 2: a tensor or a tuple
   PyObject* keep;                // what the function handles belong to
   PyObject* raw_stream;          // device index -> the current stream's handle
+  PyObject* fail;                // status of a launch that failed -> raises
   launch_fn launch;
-  error_fn last_error;
 };
 
 constexpr int kMaxDims = 32, kMaxValues = 64, kMaxOuts = 8, kMaxTemps = 16;
@@ -284,7 +283,10 @@ PyObject* call_plain(PyObject* self_, PyObject* const* argv, size_t nargsf, PyOb
     }
     PyEval_RestoreThread(released);
     if (failed) {
-      PyErr_Format(PyExc_RuntimeError, "chip_launch: %s", self->last_error());
+      // (the error types of the library's Python binding; its error text is this thread's own)
+      PyObject* none = PyObject_CallFunction(self->fail, "i", failed);
+      Py_XDECREF(none);
+      if (!PyErr_Occurred()) PyErr_Format(PyExc_RuntimeError, "a launch failed with status %d", failed);
       return nullptr;
     }
   }
@@ -421,17 +423,18 @@ void plan_dealloc(PyObject* o) {
   delete p->args; delete p->derived; delete p->outs; delete p->temps; delete p->launches;
   Py_XDECREF(p->keep);
   Py_XDECREF(p->raw_stream);
+  Py_XDECREF(p->fail);
   Py_TYPE(o)->tp_free(o);
 }
 
 PyTypeObject PlanType = {PyVarObject_HEAD_INIT(nullptr, 0) "cleave_amd._dispatch.Plan"};
 
-// make_plan(args, n_dims, derived, outs, temps, launches, result, keep, raw_stream, launch address, last-error address)
+// make_plan(args, n_dims, derived, outs, temps, launches, result, keep, raw_stream, fail, launch address)
 PyObject* make_plan(PyObject*, PyObject* a) {
-  PyObject *args, *derived, *outs, *temps, *launches, *keep, *raw;
+  PyObject *args, *derived, *outs, *temps, *launches, *keep, *raw, *fail;
   int n_dims, result;
-  unsigned long long launch, err;
-  if (!PyArg_ParseTuple(a, "OiOOOOiOOKK", &args, &n_dims, &derived, &outs, &temps, &launches, &result, &keep, &raw, &launch, &err)) return nullptr;
+  unsigned long long launch;
+  if (!PyArg_ParseTuple(a, "OiOOOOiOOOK", &args, &n_dims, &derived, &outs, &temps, &launches, &result, &keep, &raw, &fail, &launch)) return nullptr;
   Plan* p = PyObject_New(Plan, &PlanType);
   if (!p) return nullptr;
   p->vectorcall = call;
@@ -441,8 +444,8 @@ PyObject* make_plan(PyObject*, PyObject* a) {
   p->result = result;
   Py_INCREF(keep); p->keep = keep;
   Py_INCREF(raw); p->raw_stream = raw;
+  Py_INCREF(fail); p->fail = fail;
   p->launch = reinterpret_cast<launch_fn>(launch);
-  p->last_error = reinterpret_cast<error_fn>(err);
   if (!read_plan(p, args, derived, outs, temps, launches)) { Py_DECREF(p); return nullptr; }
   return reinterpret_cast<PyObject*>(p);
 }

@@ -164,13 +164,14 @@ def chain_plan(stages, *, arguments=None, output_shapes=None, as_tuple=False):
                              tuple(int(b) for b in block), int(launch["lds"]), values))
         before = produced
     lib = shim.load()
-
-    def address(function):
-        return ctypes.cast(function, ctypes.c_void_p).value
-
     return module.make_plan(args, n_dims, derived, outs, temps, launches, 2 if as_tuple else 1 if outs else 0,
                             tuple(kernel.module for kernel, _ in stages), torch._C._cuda_getCurrentRawStream,
-                            address(lib.chip_launch), address(lib.chip_last_error))
+                            _launch_failed, ctypes.cast(lib.chip_launch, ctypes.c_void_p).value)
+
+
+def _launch_failed(status):
+    """What a failed launch raises: the errors of the checked path (its text is the calling thread's own)."""
+    shim._check(status, "chip_launch_seq")
 
 
 def _number(text):

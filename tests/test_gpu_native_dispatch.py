@@ -172,3 +172,19 @@ def test_timed_and_allocation_free_calls_take_such_operands_too(k):
     assert torch.equal(out, want)
     kernel.time(*moved, warmup=1, iters=2)
     assert torch.equal(kernel.last_timed_outputs[0], want)
+
+
+@pytest.mark.parametrize("change,error,text", [(dict(lds=1 << 20), "LdsExceeded", "LDS limit exceeded"), (dict(block=[2048, 1, 1]), "HipError", "1024 threads")])
+def test_a_launch_the_library_refuses_raises_what_the_checked_path_raises(change, error, text):
+    """Refused by the library's own checks, ahead of any launch."""
+    from cleave_amd.runtime.dispatch import chain_plan
+
+    kernel, args, _ = _split_kernel()
+    kernel.manifest["launches"][0].update(change)
+    plan = chain_plan([(kernel, None)])
+    raised = []
+    for call in (kernel._checked_call, plan):
+        with pytest.raises(Exception, match=text) as e:
+            call(*args)
+        raised.append((type(e.value), str(e.value), getattr(e.value, "status", None)))
+    assert raised[0] == raised[1] and raised[0][0].__name__ == error
