@@ -548,7 +548,9 @@ class PagedKernel(Kernel):
                     return done
         done = self._checked_call(positional, longest, named)
         if plan is None:                 # a first call of this kernel went through: later ones take the native plan
-            self._plans[role] = self._native_plan(role)
+            from ..runtime.dispatch import plan_or_false
+
+            self._plans[role] = plan_or_false(lambda: self._native_plan(role))
         return done
 
     def _checked_call(self, positional, longest, named):

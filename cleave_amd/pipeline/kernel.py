@@ -161,7 +161,9 @@ class Kernel:
             shape_of = {p.name: tuple(p.shape) for p in kernel.params}
             sources = {}
             for p in stage.params:
-                origin_shape = None
+                declared, origin_shape = shape_of.get(p.name), None
+                if declared is None or not all(isinstance(e, int) for e in declared):
+                    return False
                 if p.source == FROM_PROGRAM:
                     if not 0 <= p.index < len(self.input_shapes):
                         return False
@@ -169,9 +171,7 @@ class Kernel:
                     dtype_of.setdefault(p.index, next(q.dtype for q in kernel.params if q.name == p.name))
                 elif not stages or p.index >= sum(q.role == "output" for q in stages[-1][0].params):
                     return False
-                declared = shape_of.get(p.name)
-                if declared is None or not all(isinstance(e, int) for e in declared) or (
-                        origin_shape is not None and math.prod(origin_shape) != math.prod(declared)):
+                if origin_shape is not None and math.prod(origin_shape) != math.prod(declared):
                     return False
                 sources[p.name] = ("arg" if p.source == FROM_PROGRAM else "stage", p.index)
             if kernel.dyn_dims or any(p.role in ("input", "scalar") and p.name not in sources for p in kernel.params):
@@ -189,7 +189,9 @@ class Kernel:
                 return done
         done = self._checked_call(positional, named)
         if self._plan is None:           # a first call went through: later ones take the native plan
-            self._plan = self._native_plan()
+            from ..runtime.dispatch import plan_or_false
+
+            self._plan = plan_or_false(self._native_plan)
         return done
 
     def _checked_call(self, positional, named):

@@ -310,9 +310,9 @@ class CompiledKernel:
                 return done
         done = self._checked_call(*args)
         if plan is None:             # a first call went through: later ones take the native plan
-            from .dispatch import chain_plan
+            from .dispatch import chain_plan, plan_or_false
 
-            self._plan = chain_plan([(self, None)]) or False
+            self._plan = plan_or_false(lambda: chain_plan([(self, None)]))
         return done
 
     def _checked_call(self, *args):

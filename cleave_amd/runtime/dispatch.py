@@ -14,6 +14,7 @@ import importlib.util
 import math
 import sys
 import threading
+import warnings
 
 from ..core.errors import BackendUnavailable, CompileError
 from . import shim
@@ -41,7 +42,7 @@ def native():
             path = shim.CSRC_DIR / MODULE_NAME
             if not path.is_file():
                 raise BackendUnavailable(f"{path} is missing: build it with `python -c 'import __graft_entry__ as g; "
-                                         "g.build()'` or `make -C cleave_amd/csrc`; there is no fallback path")
+                                         "g.build()'` or `make -C cleave_amd/csrc`; until then calls go step by step in Python")
             name = "cleave_amd.csrc._dispatch"
             spec = importlib.util.spec_from_file_location(name, path)
             module = importlib.util.module_from_spec(spec)
@@ -91,8 +92,24 @@ def _argument(p, dims: dict, shape=None, align=1):
     return (TENSOR, p.dtype, axes, align)
 
 
+def plan_or_false(make):
+    """``make()``, a native call plan; False where there is none, and calls stay on the checked Python path: the extension
+    module is not built or does not load (said once), or the kernels are beyond what a plan holds (its numbers of
+    dims, arguments, scratch buffers, output axes and launches, and its operators in extents)."""
+    try:
+        native()
+    except (BackendUnavailable, ImportError, OSError) as e:
+        warnings.warn(f"calls of compiled kernels go step by step in Python: {e}", RuntimeWarning, stacklevel=3)
+        return False
+    try:
+        return make() or False
+    except (CompileError, ValueError, OverflowError):
+        return False
+
+
 def chain_plan(stages, *, arguments=None, output_shapes=None, as_tuple=False):
-    """A native call plan, or None where the kernels do not fit one.
+    """A native call plan, or None where a kernel has a run-time extent that no argument names.  Kernels beyond the
+    limits of a plan raise ``ValueError`` or ``CompileError`` (``plan_or_false`` answers False for them).
 
     ``stages``: ``[(compiled kernel, sources)]`` in order; ``sources[name]`` is ``("arg", i)`` or
     ``("stage", j)`` (output j of the stage before) for every input and scalar of the kernel, or
