@@ -61,7 +61,9 @@
 // query tokens of one request (a new item at every multiple of four packed tokens and at every request boundary) x
 // 16 heads, so a 16-row tile is one token and its causal limit is uniform over a wave; the key rows are looked up
 // in the token table (every value wave keeps the entries of its own rows in LDS, fetched on its load counter a step
-// ahead of the rows).  The first step's reference point is the maximum of both token halves (one more barrier), and the
+// ahead of the rows).  The first step's reference point is the maximum of both token halves (one more barrier), reference
+// points are whole numbers, so that moving a token half's weights to a higher point is exact and they are rounded once
+// (f16 weights that end below 2^-14 of the point excepted: there the move rounds to the subnormal spacing, 2^-24), and the
 // score waves sum the unrounded weights for the lse.  The one-wave-per-token kernel reads 68 KB out of LDS per token
 // and step at one head group's 69 matrix ops; here it is 36.  us, the best of its forms / this one, 16 heads of 512 + 64:
 // 5376 tokens over 24 requests with prefixes 121 / 91, 9164 over 32 197 / 162, 1424 over 16 31 / 27, 350 tokens of one
@@ -107,9 +109,11 @@ static_assert(CL_CKV % 128 == 0 && CL_KPE % 64 == 0, "whole 64-feature panels, t
 #if CL_PREFILL
 #define MD_TOKENS 4                              // query tokens of a workgroup, 16 heads each
 #define MD_SCALE 1.0f                            // (scores are scaled as they come: the run-time scale may have any sign)
+#define MD_POINT(v) floorf(v)                     // whole reference points
 static_assert(CL_HEADS % 16 == 0 && CL_SPLITS == 1, "16 heads of four tokens per workgroup, unsplit");
 #else
 #define MD_SCALE CL_SCALE_LOG2E
+#define MD_POINT(v) (v)
 static_assert(CL_HEADS % MD_HEADS_PER_BLOCK == 0, "64 heads per workgroup");
 static_assert(CL_SCALE_LOG2E > 0.f, "the largest raw score must be the largest scaled one");
 #endif
@@ -489,9 +493,9 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
           v = fmaxf(v, lane_xor(v, lane, 16));
           v = fmaxf(v, lane_xor(v, lane, 32));
           if (it == 0)
-            m_run[t] = fmaxf(v, MD_REF_FLOOR);      // nothing behind it yet: the step's own maximum
+            m_run[t] = fmaxf(MD_POINT(v), MD_REF_FLOOR);      // nothing behind it yet: the step's own maximum
           else if (v > m_run[t] + MD_RESCALE_STEP)
-            m_run[t] = v;
+            m_run[t] = MD_POINT(v);
 #if CL_PREFILL
           if (it == 0 && g == 0) md_ref[1][set][t][c][half] = m_run[t];
 #endif
@@ -633,13 +637,20 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
       for (int t = 0; t < 2; ++t) {
         const float m_new = fmaxf(ref[t][0], ref[t][1]);          // never below m_acc
         const float alpha = fast_exp2(m_acc[t] - m_new);
-        const float f_lo = fast_exp2(ref[t][0] - m_new), f_hi = fast_exp2(ref[t][1] - m_new);
         m_acc[t] = m_new;
 #pragma unroll
         for (int fb = 0; fb < MD_FBW; ++fb) acc[t][fb] *= alpha;
         l_acc[t] *= alpha;
+#if CL_PREFILL
+        // (exact: the points are whole numbers.  Far below the new one, any exponent that leaves zero will do)
+        const int f_lo = (int)fmaxf(ref[t][0] - m_new, -1000.f), f_hi = (int)fmaxf(ref[t][1] - m_new, -1000.f);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) pf[t][i] = to_elem(__builtin_amdgcn_ldexpf(to_f32(pf[t][i]), i < 4 ? f_lo : f_hi));
+#else
+        const float f_lo = fast_exp2(ref[t][0] - m_new), f_hi = fast_exp2(ref[t][1] - m_new);
 #pragma unroll
         for (int i = 0; i < 8; ++i) pf[t][i] = to_elem(to_f32(pf[t][i]) * (i < 4 ? f_lo : f_hi));
+#endif
       }
     }
     // The loads of image it + 2 (into the slot image it - 2 has left) are asked for between the
