@@ -664,13 +664,11 @@ class HipCodeGen:
         scores of 32 heads x half of each step's tokens, four the value products of 32 heads x half
         the latent features."""
         p, t, op = plan.problem, plan.tiling, plan.operands
-        if p["heads"] % 64 or p["ckv"] % 128 or p["kpe"] % 64:
-            raise CodegenError("the score-wave / value-wave MLA kernel needs heads % 64 == 0, a latent width in "
-                               "multiples of 128 and a rope width in multiples of 64")
-        from ..schedule.policy import mla_duo_lds_bytes
+        from ..schedule.policy import mla_duo_fits
 
-        if mla_duo_lds_bytes(p["ckv"], p["kpe"]) > 160 * 1024:
-            raise CodegenError("four images of the paired-wave MLA kernel do not fit LDS at these widths")
+        if p["heads"] % 64 or not mla_duo_fits(p["ckv"], p["kpe"]):
+            raise CodegenError("the score-wave / value-wave MLA kernel needs heads % 64 == 0, a latent width in multiples of 128, "
+                               "a rope width of an odd number of 64s, and four images within 160 KiB of LDS")
         for k, v in (("CL_HEADS", p["heads"]), ("CL_CKV", p["ckv"]), ("CL_KPE", p["kpe"]), ("CL_SKV", p["skv"]),
                      ("CL_BATCH", p["batch"]), ("CL_PO_ELEM", 1)):
             unit.define(k, v)
@@ -742,11 +740,12 @@ class HipCodeGen:
                             ("INDPTR", "CL_ARG_INDPTR"), ("INDICES", "CL_ARG_INDICES")):
             unit.define(macro, op[role])
         if int(t.get("DUO", 0)):
-            from ..schedule.policy import mla_duo_lds_bytes
+            from ..schedule.policy import mla_duo_fits
 
-            if not prefill or tok != 4 or stages != 2 or ksplit != 1 or p["ckv"] % 128 or mla_duo_lds_bytes(p["ckv"], p["kpe"], True) > 160 * 1024:
+            if not prefill or tok != 4 or stages != 2 or ksplit != 1 or not mla_duo_fits(p["ckv"], p["kpe"], True):
                 raise CodegenError("score waves and value waves on a token table: causal prefill with four query tokens per item, a "
-                                   "latent width in multiples of 128 and four images within 160 KiB of LDS")
+                                   "latent width in multiples of 128, a rope width of an odd number of 64s, and four images "
+                                   "within 160 KiB of LDS")
             unit.templates += ["mla_decode_duo.hip", "attn_combine.hip"]
             unit.launch(ENTRY, (f"ceildiv({p['dim_names']['total_q']}, 4) + batch", p["heads"] // 16, 1), 512, 0, self._partial_args)
             return

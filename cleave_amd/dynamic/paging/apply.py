@@ -397,12 +397,12 @@ def mla_prefill_variants(plan: KernelPlan, spec) -> list:
     they also share the LDS bandwidth that bounds this kernel's matrix work; more images keep the
     rows of more steps in flight, which a lone item needs and many resident items do not); and, where
     its images fit, four tokens per item with score waves and value waves."""
-    from ...schedule.policy import mla_duo_lds_bytes
+    from ...schedule.policy import mla_duo_fits
 
     out = [apply_paging(plan, spec, tok=t, stages=s, ksplit=k)
            for t, s, k in ((2, 2, 1), (2, 3, 1), (2, 4, 1), (4, 2, 1), (4, 4, 1), (1, 2, 1), (1, 3, 1), (1, 2, 2))]
     dense = read_dense_mla(plan)
-    if dense.ckv % 128 == 0 and mla_duo_lds_bytes(dense.ckv, dense.kpe, True) <= 160 * 1024:
+    if mla_duo_fits(dense.ckv, dense.kpe, prefill=True):
         out.append(apply_paging(plan, spec, tok=4, duo=True))
     return out
 

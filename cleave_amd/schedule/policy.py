@@ -521,6 +521,13 @@ def mla_duo_lds_bytes(ckv, kpe, prefill=False):
     return mla_lds_bytes(ckv, kpe, 4) + (14 if prefill else 9) * 1024
 
 
+def mla_duo_fits(ckv, kpe, prefill=False) -> bool:
+    """Widths the score-wave / value-wave kernel is written for: two value waves halve the latent row's 64-feature panels,
+    and the Q rows in LDS are an odd number of 64-feature runs long (128 bytes off between neighbours: no bank conflicts),
+    with four images in a workgroup's LDS.  (A rope width of 128 passed here and failed in the compiler.)"""
+    return ckv % 128 == 0 and kpe % 128 == 64 and mla_duo_lds_bytes(ckv, kpe, prefill) <= 160 * 1024
+
+
 def mla_ok(low) -> bool:
     p = low.problem
     return p["heads"] % 16 == 0 and p["ckv"] % 64 == 0 and p["kpe"] % 64 == 0
@@ -580,7 +587,7 @@ def mla_candidates(low, role, factor, arch: Arch):
     # ops.  Measured 25-30 % ahead of the best form above wherever both run, so it is ranked first
     # (with the shorter read-ahead of its value operands as a second candidate).
     duo_lds = mla_duo_lds_bytes(p["ckv"], p["kpe"])
-    if out and p["heads"] % 64 == 0 and p["ckv"] % 128 == 0 and duo_lds <= arch.lds_bytes:
+    if out and p["heads"] % 64 == 0 and mla_duo_fits(p["ckv"], p["kpe"]) and duo_lds <= arch.lds_bytes:
         best = min(c.score for c in out)
         # (third: the score waves ask for about half of every image's panels -- a wave that waits for the
         # path into the compute unit does not hold up the other wave of its SIMD, and the value

@@ -448,3 +448,26 @@ def test_shipped_registry_kernels_keep_their_values_in_registers():
             assert entry["spilled_vgprs"] == 0 and entry["scratch_bytes"] == 0, (name, entry)
             if name.startswith("gqa_paged_decode"):
                 assert entry["vgprs"] <= 256, (name, entry)
+
+
+@pytest.mark.parametrize("ckv,kpe,fits", [(256, 64, True), (128, 192, True), (128, 128, False), (384, 128, False), (512, 192, False)])
+def test_score_wave_mla_kernels_are_offered_where_they_compile(ckv, kpe, fits):
+    """Decode and paged prefill: an even rope width makes the Q rows in LDS collide, which the kernel asserts against: the
+    emitter refuses it and the search does not offer it.  What is offered compiles."""
+    from cleave_amd.dynamic.paging import MLA_PAGED_PREFILL_CAUSAL, DenseMLA, MLASpec, apply_paging
+    from cleave_amd.dynamic.paging.apply import mla_prefill_variants
+    from cleave_amd.runtime import shim
+
+    dense = stage_graph(C.mla_decode.trace(cl.bf16, B=1, H=64, D=ckv, PE=kpe, SKV=256))
+    spec = MLASpec(num_qo_heads=64, kind=MLA_PAGED_PREFILL_CAUSAL, causal=True)
+    plan = apply_tiling(TileDict("mla_decode", "main", dict(WAVES=4), flat_graph=dense))
+    offered = [c for c in search_tiling(dense) if c.tiling.get("DUO")], [v for v in mla_prefill_variants(plan, spec) if v.tiling.get("DUO")]
+    assert all(bool(o) == fits for o in offered)
+    makers = (lambda: HipCodeGen().gen(apply_tiling(TileDict("mla_decode", "main", dict(DUO=1), flat_graph=dense))),
+              lambda: HipCodeGen().gen(apply_paging(plan, spec, tok=4, duo=True)))
+    for make in makers:
+        if fits:
+            assert shim.compile_source(make())[0]
+        else:
+            with pytest.raises(CodegenError, match="latent width"):
+                make()
