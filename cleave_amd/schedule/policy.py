@@ -187,21 +187,20 @@ def gemm_dma_candidates(low, role, factor, arch: Arch, twin_of=None):
         # (equal tiles: the wave grids with more waves have measured a few per cent faster -- more loads in flight)
         score = passes * pass_clk * (1.0 + 0.03 / (wm * wn))
         tiling = dict(BM=bm, BN=bn, BK=64, WM=wm, WN=wn)
-        # (128 x 256 and 256 x 128 tiles whose wave groups alternate between memory and matrix work: 6 to 25 % ahead of
-        # the three-stage lock-step form of the same tile, which itself ranks at 0.85; SwiGLU keeps both, the
-        # lock-step form ahead)
+        # 128 x 256 and 256 x 128 tiles whose wave groups alternate between memory and matrix work: 6 to 25 % ahead of
+        # the three-stage lock-step form of the same tile (which ranks at 0.85), so a plain product has no use for that
+        # one.  SwiGLU's two weights keep both, this one right behind: the search times them.
         phased = bm * bn == 128 * 256 and not post_norm and twin_of != "matmul_rowsum" and phased_matmul("matmul", p, splits, tiling)
-        if phased:
-            score *= 0.8502 if twin_of else 0.8
+        place = score if not phased else math.nextafter(0.85 * score, math.inf) if twin_of else 0.8 * score
         out.append(TileDict("gemm_dma", role, tiling, output_tile=[bm, bn], rstep_map={"k": 64}, n_threads=threads,
-                            split_factor=factor, score=score, lds_bytes=lds, est_vgprs=vgprs))
+                            split_factor=factor, score=place, lds_bytes=lds, est_vgprs=vgprs))
         # Three LDS stages where three images fit beside as many workgroups per compute unit as two
         # allow: the loads of a step asked for two steps ahead and spread over the whole step
         # (256 x 128 tiles on 4096 x 14336 x 4096: 426 us against 526).
         if ((twin_of or not phased) and 3 * (bm + bn) * 128 * per_cu <= arch.lds_bytes and units_a % (wm * wn) == 0 and units_b % (wm * wn) == 0
                 and not post_norm):
             out.append(TileDict("gemm_dma", role, dict(tiling, STAGES=3), output_tile=[bm, bn], rstep_map={"k": 64},
-                                n_threads=threads, split_factor=factor, score=0.85 * (score / 0.8502 if phased else score), lds_bytes=3 * lds // 2,
+                                n_threads=threads, split_factor=factor, score=0.85 * score, lds_bytes=3 * lds // 2,
                                 est_vgprs=vgprs))
         # A last round that fills at most half of the machine: its tiles as two half-height
         # workgroups each (row-major A, one workgroup per compute unit, unsplit, unbatched).
@@ -212,10 +211,11 @@ def gemm_dma_candidates(low, role, factor, arch: Arch, twin_of=None):
                                 n_threads=threads, split_factor=factor, score=(passes - 0.45) * pass_clk,
                                 lds_bytes=lds, est_vgprs=vgprs))
     if not twin_of and not post_norm:
-        # the two best plain tilings stay ahead of them: measured, not modelled, is how they get past
-        ranked = sorted(c.score for c in out)
+        # Third and fourth at best, behind the two best tilings of one wave grid per tile: the request model below ranks the
+        # K-sharing tilings among themselves, and timing, not the model, puts one of them first.
+        second = sorted(c.score for c in out)[1:2]
         for c in kwaves_candidates(low, role, factor, arch):
-            c.score = max([c.score] + [1.0001 * s for s in ranked[1:2]])
+            c.score = max([c.score] + [math.nextafter(s, math.inf) for s in second])
             out.append(c)
     if K % 64:
         # (under the name of the template that takes such lengths; DMA picks its direct-to-LDS form)
