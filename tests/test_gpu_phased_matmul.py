@@ -74,6 +74,44 @@ def test_half_height_tail_tiles(tail):
     _check(C.matmul_nt, cl.bf16, dict(M=512, N=1032, K=256), tile=TILES["256x256_4x2"], TAIL=tail)
 
 
+@pytest.mark.parametrize("tail", [1, 4])
+@pytest.mark.parametrize("k", [136, 200, 328, 392])
+def test_half_height_tail_tiles_with_a_partly_filled_last_step(tail, k):
+    """The phased and the lock-step kernel, whole tiles and halves (two to seven steps, both stage parities)."""
+    _check(C.matmul, cl.f16, dict(M=512, N=1032, K=k), TAIL=tail)
+    _check(C.matmul_nt, cl.bf16, dict(M=512, N=1032, K=k), tile=TILES["256x256_4x2"], TAIL=tail)
+    _check(C.matmul, cl.f16, dict(M=256, N=264, K=k), tile=(128, 128, 2, 2), TAIL=tail)
+
+
+@pytest.mark.parametrize("tile", [(128, 128, 2, 2), (256, 64, 4, 2), (64, 256, 2, 4)], ids=lambda t: f"{t[0]}x{t[1]}")
+@pytest.mark.parametrize("k", [40, 136, 200, 328])
+def test_partly_filled_last_step_of_three_stages_on_larger_tiles(tile, k):
+    for fn, dtype in ((C.matmul, cl.f16), (C.matmul_nt, cl.bf16), (matmul_tn, cl.f16)):
+        _check(fn, dtype, dict(M=304, N=264, K=k), tile, STAGES=3)
+
+
+@pytest.mark.parametrize("dtype", [cl.f16, cl.bf16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("fn", [C.rmsnorm_matmul_plain, C.rmsnorm_matmul_eps], ids=["plain", "eps"])
+@pytest.mark.parametrize("k", [72, 200, 328])
+def test_fused_norm_with_a_partly_filled_last_step(fn, dtype, k):
+    """The rows' squares are summed over the images, zeros past K among them, and divided by K itself; as the search names
+    such tilings (``gemm`` with DMA).  Every output is one rounding of a value of order one and the row scale's: 2e-2 as
+    for whole steps in bf16 (8 bits), 1e-2 in f16."""
+    for tile, m, knobs in (((16, 32, 1, 2), 100, {}), ((64, 64, 2, 2), 200, {}), ((256, 128, 4, 2), 304, {}), ((256, 256, 4, 2), 512, dict(TAIL=2))):
+        shapes = dict(M=m, N=264, K=k)
+        prog = fn.trace(dtype, **shapes)
+        ins = [t.to(dtype.torch) for t in C.inputs_plain_norm(shapes)]
+        tiling = dict(zip(("BM", "BN", "WM", "WN"), tile), BK=64, DMA=1, **knobs)
+        print(f"case {prog.name} {dtype} {shapes} {tiling}", flush=True)
+        kernel = kernel_for(prog, template="gemm", tiling=tiling)
+        assert "gd_sumsq" in kernel.get_kernel_source()
+        got = kernel(*[t.cuda() for t in ins])
+        torch.cuda.synchronize()
+        want = program_oracle.evaluate(prog, ins)[0]
+        tol = 2e-2 if dtype is cl.bf16 else 1e-2
+        np.testing.assert_allclose(got.float().cpu().numpy(), want, rtol=tol, atol=tol)
+
+
 @pytest.mark.parametrize("tile,kw", [((16, 16), 8), ((16, 32), 4), ((32, 16), 2), ((32, 32), 8), ((32, 64), 4), ((64, 64), 4), ((16, 16), 16)],
                          ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else f"kw{v}")
 @pytest.mark.parametrize("k", [8, 64, 200, 512, 1096])
