@@ -209,17 +209,23 @@ def lone_request(kernel, inputs, expected, indptr_at):
     return cut, [t[b:b + 1].contiguous() for t in expected]
 
 
+def few_requests(spec, compute_units: int) -> int:
+    """The number of requests from which the single kernel has workgroups for a quarter of the compute units: one per
+    request and kv head, or, for latent attention, per request and 16 query heads."""
+    per_request = int(spec.num_kv_heads) if hasattr(spec, "num_kv_heads") else -(-int(spec.num_qo_heads) // 16)
+    return compute_units // (4 * per_request) + 1
+
+
 def calibrate_dispatch(pair, solo, factory, spec) -> dict:
     """When should a call run the split pair rather than the single kernel?
 
     Both are timed on every workload.  A workload is described by the kv tiles of its longest request
     (``indptr`` units x page size / kv tile, rounded up), and the rule is "split from ``min_tiles`` tiles on".
-    The single kernel has one workgroup per request and kv head, so what a split is worth also depends on
-    whether those fill the chip: for batches of fewer than ``few_requests`` requests (workgroups for less than
-    a quarter of the compute units; 18 requests of up to 1056 tokens, 144 workgroups, still run 16 us unsplit and
-    22 split) the threshold is ``lone_tiles``, calibrated on each workload's longest request
-    alone.  (With one threshold, taken from batches of 64 requests, three requests of up to 2882 tokens ran the
-    single kernel in 26 us where the pair takes 11.)"""
+    What a split is worth also depends on whether the single kernel's workgroups fill the chip: for batches of
+    fewer than ``few_requests`` requests (workgroups for less than a quarter of the compute units; 18 requests of
+    up to 1056 tokens, 144 workgroups, still run 16 us unsplit and 22 split) the threshold is ``lone_tiles``,
+    calibrated on each workload's longest request alone.  (With one threshold, taken from batches of 64 requests,
+    three requests of up to 2882 tokens ran the single kernel in 26 us where the pair takes 11.)"""
     import dataclasses
 
     from ..core.target import current_target
@@ -243,20 +249,20 @@ def calibrate_dispatch(pair, solo, factory, spec) -> dict:
 
     benchmark_over_workloads([pair, solo], observed, ramp_seconds=0.2)
     min_tiles = split_threshold(longest, pair.latency_us, solo.latency_us)
-    few_requests = current_target().arch.compute_units // (4 * int(getattr(spec, "num_kv_heads", 1))) + 1
+    few = few_requests(spec, current_target().arch.compute_units)
     lone_pair, lone_solo = dataclasses.replace(pair, latency_us={}), dataclasses.replace(solo, latency_us={})
     benchmark_over_workloads([lone_pair, lone_solo], alone, ramp_seconds=0.0)
     lone_tiles = split_threshold(longest, lone_pair.latency_us, lone_solo.latency_us)
     keys = [k for k in longest if k in pair.latency_us and k in solo.latency_us]
 
     def splits(key):
-        return longest[key] >= (lone_tiles if requests[key] < few_requests else min_tiles)
+        return longest[key] >= (lone_tiles if requests[key] < few else min_tiles)
 
     per_workload = {k: (pair if splits(k) else solo).latency_us[k] for k in keys}
     return {
         "rule": "run the split pair when the longest request has at least min_tiles KV tiles (lone_tiles for batches of fewer "
                 "than few_requests requests; indptr units x page_size tokens / kv_tile), else the single kernel",
-        "min_tiles": min_tiles, "lone_tiles": lone_tiles, "few_requests": few_requests, "kv_tile": kv_tile,
+        "min_tiles": min_tiles, "lone_tiles": lone_tiles, "few_requests": few, "kv_tile": kv_tile,
         "page_size": tokens_per_unit, "indptr_index": indptr_at,
         "split_label": pair.label, "single_label": solo.label,
         "n_workloads": len(keys), "split_runs": sum(map(splits, keys)),

@@ -417,3 +417,18 @@ def test_lone_request_goes_by_the_extents_names(name, bounds, pages):
             assert value.shape[0] == 1 and (len(p.shape) > 1 or value.tolist() == [b])
         else:
             assert value.tolist() == [0, bounds[b + 1] - bounds[b]]
+
+
+def test_requests_that_fill_a_quarter_of_the_chip():
+    """The single kernel's workgroups per request are its second grid extent: kv heads, or groups of 16 heads of a latent row."""
+    from cleave_amd.codegen import HipCodeGen, parse_manifest
+    from cleave_amd.dynamic.paging import PAGED_DECODE_SLAB, DenseMLA, MLASpec, PagingSpec
+    from cleave_amd.dynamic.paging.apply import _mla_outputs, _mla_params, _mla_plan
+    from cleave_amd.pipeline.dynamic import few_requests
+
+    for heads, want in ((16, 65), (128, 9)):
+        spec, dense = MLASpec(num_qo_heads=heads), DenseMLA(heads, 512, 64, "bfloat16", "bfloat16")
+        (params, ops), (outs, out_ops) = _mla_params(spec, dense), _mla_outputs(spec, dense)
+        grid = parse_manifest(HipCodeGen().gen(_mla_plan(spec, dense, "main", params + outs, {**ops, **out_ops})))["launches"][0]["grid"]
+        assert few_requests(spec, 256) == want == 256 // (4 * int(grid[1])) + 1
+    assert few_requests(PagingSpec(num_qo_heads=32, num_kv_heads=8, kind=PAGED_DECODE_SLAB, page_size=64), 256) == 9
