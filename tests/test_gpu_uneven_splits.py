@@ -39,6 +39,28 @@ def test_mla_decode(heads, tiling, skv):
     _check(C.mla_decode.trace(cl.bf16, **shapes), C.inputs_c4(shapes), template="mla_decode", tiling=tiling, split=8)
 
 
+@pytest.mark.parametrize("skv", [1, 33, 289, 613])
+def test_many_row_attention(skv):
+    """The kernel whose waves share the keys: softmax, keys wider than values, QK-norm, and plain sums (their scale as in the
+    chained tests: outputs follow the number of keys)."""
+    shared = dict(template="attn_prefill", tiling=dict(SHARED=1), split=8)
+    for fn, dtype, shapes in ((C.gqa_decode_exact, cl.f16, dict(HQ=8, HKV=2, SQ=70, SKV=skv, D=64)),
+                              (C.mla_prefill, cl.bf16, dict(H=2, SQ=100, SKV=skv, DK=192, DV=128)),
+                              (C.qknorm, cl.f16, dict(HQ=4, HKV=2, SQ=70, SKV=skv, D=128))):
+        prog = fn.trace(dtype, **shapes)
+        _check(prog, prog.random_inputs(seed=skv, device="cpu"), **shared)
+    prog = C.matmul_matmul.trace(cl.f16, H=2, SQ=70, SKV=skv, D=64)
+    first, *rest = prog.random_inputs(seed=skv, device="cpu")
+    _check(prog, [(first.float() / (8 * skv)).to(first.dtype), *rest], **shared)
+
+
+@pytest.mark.parametrize("skv", [33, 289])
+def test_gqa_decode_of_narrow_heads_in_groups(skv):
+    shapes = dict(HQ=64, HKV=8, SQ=1, SKV=skv, D=64)
+    for waves in (1, 4):
+        _check(C.gqa_decode_exact.trace(cl.f16, **shapes), C.inputs_c3(shapes), template="attn_decode", tiling=dict(WAVES=waves), split=16)
+
+
 def test_factors_that_are_neither_divisors_nor_powers_of_two_are_still_refused():
     g = stage_graph(C.gqa_decode_exact.trace(cl.f16, HQ=8, HKV=8, SQ=1, SKV=289, D=128))
     for factor in (3, 6, 12):
