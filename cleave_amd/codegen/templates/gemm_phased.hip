@@ -27,12 +27,12 @@
 // for.  So two stages hold loads that are 1.75 (1.5) steps ahead of their use, a few per wave and phase,
 // never a burst; the wait in front of a half's phase counts the loads asked for after it (gp_wait).
 //
-// Measured, 8192^3 bf16 with a (N, K) weight: 701 us (1.57 PFLOP/s) against 806 lock-step; the matrix unit is
-// busy 86 % of the clocks (70 % lock-step) at 1.76 GHz (1.96): what bounds it is the power the matrix ops
-// draw on random operands.  A (K, N) weight runs at the same speed: its transposing reads hide in the memory
-// parts.  4096 x 14336 x 4096: 352 us (393), SwiGLU of that size 676 (752); with two phases a step instead of four
-// these take 1 % longer.  128 x 256 tiles on 2048 x 4096 x 4096: 56.3 us (60.1 lock-step with three stages), 256 x 128 on
-// 724 x 6272 x 640: 10.7 us (13.3).
+// Measured, 8192^3 bf16 with a (N, K) weight: 701 us (1.57 PFLOP/s) against 806 lock-step; by its counters the
+// matrix unit is busy 89 % of the clocks (64 % lock-step) at 1.65 GHz (2.02): what bounds it is the power the
+// matrix ops draw on random operands.  A (K, N) weight runs at the same speed: its transposing reads hide in
+// the memory parts.  4096 x 14336 x 4096: 352 us (393), busy 82 % at 1.58 GHz (62 %, 1.84); SwiGLU of that size
+// 676 (752); with two phases a step instead of four these take 1 % longer.  128 x 256 tiles on 2048 x 4096 x 4096:
+// 56.3 us (60.1 lock-step with three stages), 256 x 128 on 724 x 6272 x 640: 10.7 us (13.3).
 //
 //   CL_BM, CL_BN, CL_WM x CL_WN = 8 waves; CL_TRANS_A / CL_TRANS_B, CL_BATCH_A/B, CL_SPLITS, CL_TAIL (256 x 256
 //   only), CL_SWIGLU (B half 1 = the gate weight's columns) as in gemm_dma.hip.
