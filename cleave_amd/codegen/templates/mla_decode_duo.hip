@@ -61,12 +61,11 @@
 // query tokens of one request (a new item at every multiple of four packed tokens and at every request boundary) x
 // 16 heads, so a 16-row tile is one token and its causal limit is uniform over a wave; the key rows are looked up
 // in the token table (every value wave keeps the entries of its own rows in LDS, fetched on its load counter a step
-// ahead of the rows).  The first step's reference point is the maximum of both token halves (one more barrier), reference
-// points are whole numbers, so that moving a token half's weights to a higher point is exact and they are rounded once
-// (f16 weights that end below 2^-14 of the point excepted: there the move rounds to the subnormal spacing, 2^-24), and the
-// score waves sum the unrounded weights for the lse.  The one-wave-per-token kernel reads 68 KB out of LDS per token
-// and step at one head group's 69 matrix ops; here it is 36.  us, the best of its forms / this one, 16 heads of 512 + 64:
-// 5376 tokens over 24 requests with prefixes 121 / 91, 9164 over 32 197 / 162, 1424 over 16 31 / 27, 350 tokens of one
+// ahead of the rows).  The first step's reference point is the maximum of both token halves (one more barrier); where
+// one half raises its point later, the other's weights are not scaled and rounded again: their product is taken by itself
+// and moved (cold).  The score waves sum the unrounded weights for the lse.  The one-wave-per-token kernel reads 68 KB
+// out of LDS per token and step at one head group's 69 matrix ops; here it is 36.  us, the best of its forms / this one,
+// 16 heads of 512 + 64: 5376 tokens over 24 requests with prefixes 121 / 91, 9164 over 32 197 / 162, 1424 over 16 31 / 27, 350 tokens of one
 // request 21.5 / 17.3; behind for short keys on few items (37 tokens of 4 requests 6.2 / 8.2).  What bounds it now: an
 // item's query rows come and its output rows leave (136 KB) while its compute unit multiplies nothing.
 //   CL_HEADS (multiple of 16); run-time: total_q, num_pages, n_idx, batch; scalar sm_scale (any sign)
@@ -109,11 +108,9 @@ static_assert(CL_CKV % 128 == 0 && CL_KPE % 64 == 0, "whole 64-feature panels, t
 #if CL_PREFILL
 #define MD_TOKENS 4                              // query tokens of a workgroup, 16 heads each
 #define MD_SCALE 1.0f                            // (scores are scaled as they come: the run-time scale may have any sign)
-#define MD_POINT(v) floorf(v)                     // whole reference points
 static_assert(CL_HEADS % 16 == 0 && CL_SPLITS == 1, "16 heads of four tokens per workgroup, unsplit");
 #else
 #define MD_SCALE CL_SCALE_LOG2E
-#define MD_POINT(v) (v)
 static_assert(CL_HEADS % MD_HEADS_PER_BLOCK == 0, "64 heads per workgroup");
 static_assert(CL_SCALE_LOG2E > 0.f, "the largest raw score must be the largest scaled one");
 #endif
@@ -185,6 +182,14 @@ CL_DEVICE void md_issue_rows(const char* lat_src, const char* pe_src, unsigned s
     md_dma16<OFF>(P < MD_LAT_PANELS ? lat_src : pe_src, stage_byte + (unsigned)(P * MD_PANEL * 2 + lw * 1024) - OFF);
     md_issue_rows<P + 1>(lat_src, pe_src, stage_byte, lw);
   }
+}
+// a lane's eight weights with the token halves that are not wanted set to zero.  (Hidden from the optimiser: seeing a
+// selection it copied the whole value product for weights taken as they are, and spilled the second set of accumulators.)
+CL_DEVICE elem8 md_halves(elem8 p, bool want_lo, bool want_hi) {
+  const u32x4 w = __builtin_bit_cast(u32x4, p);
+  u32x4 y = {want_lo ? w[0] : 0u, want_lo ? w[1] : 0u, want_hi ? w[2] : 0u, want_hi ? w[3] : 0u};
+  asm volatile("" : "+v"(y));
+  return as_elem8(y);
 }
 CL_DEVICE int md_clamp(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
 #endif
@@ -493,9 +498,9 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
           v = fmaxf(v, lane_xor(v, lane, 16));
           v = fmaxf(v, lane_xor(v, lane, 32));
           if (it == 0)
-            m_run[t] = fmaxf(MD_POINT(v), MD_REF_FLOOR);      // nothing behind it yet: the step's own maximum
+            m_run[t] = fmaxf(v, MD_REF_FLOOR);      // nothing behind it yet: the step's own maximum
           else if (v > m_run[t] + MD_RESCALE_STEP)
-            m_run[t] = MD_POINT(v);
+            m_run[t] = v;
 #if CL_PREFILL
           if (it == 0 && g == 0) md_ref[1][set][t][c][half] = m_run[t];
 #endif
@@ -613,7 +618,14 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
     if (it == 0) {
       if (it < n_own) issue(it + 2);
 #if CL_PREFILL
-      if (n_own > 0) md_barrier();                  // (the score waves exchange their first maxima)
+      if (n_own > 0) {
+        md_barrier();                               // (the score waves exchange their first maxima: the points of step 0)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          const f32x2 first = *reinterpret_cast<const f32x2*>(&md_ref[1][set][t][c][0]);
+          m_acc[t] = fmaxf(first[0], first[1]);
+        }
+      }
 #endif
 #pragma unroll
       for (int fb = 0; fb < MD_PRE; ++fb) operand(next_tile, fb, pre_lo[fb], pre_hi[fb]);
@@ -630,6 +642,37 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
       }
       ref[t] = *reinterpret_cast<const f32x2*>(&md_ref[(it - 1) & 1][set][t][c][0]);
     }
+#if CL_PREFILL
+    if (__builtin_amdgcn_ballot_w64(ref[0][0] != m_acc[0] || ref[0][1] != m_acc[0] || ref[1][0] != m_acc[1] ||
+                                    ref[1][1] != m_acc[1])) {
+      // cold: a score wave raised a reference point at this step.  The half that stands against the lower point is multiplied
+      // here, by itself, and its product moves to the higher point: its weights are 16 bits already, scaled they would be
+      // rounded a second time.
+      elem8 p_low[2];
+      float alpha[2], f_low[2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const float m_new = fmaxf(ref[t][0], ref[t][1]);          // never below m_acc
+        alpha[t] = fast_exp2(m_acc[t] - m_new);
+        f_low[t] = fast_exp2(fminf(ref[t][0], ref[t][1]) - m_new);
+        m_acc[t] = m_new;
+        p_low[t] = md_halves(pf[t], ref[t][0] < ref[t][1], ref[t][1] < ref[t][0]);
+        pf[t] = md_halves(pf[t], ref[t][0] >= ref[t][1], ref[t][1] >= ref[t][0]);
+        l_acc[t] = l_acc[t] * alpha[t] + mfma16(ones, p_low[t], (f32x4){0.f, 0.f, 0.f, 0.f}) * f_low[t];
+      }
+#pragma unroll
+      for (int fb = 0; fb < MD_FBW; ++fb) {
+        __builtin_amdgcn_sched_barrier(0);
+        md_s16x4 lo, hi;
+        operand(tile, fb, lo, hi);
+        const elem8 a = __builtin_bit_cast(elem8, (md_s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+          acc[t][fb] = acc[t][fb] * alpha[t] + mfma16(a, p_low[t], (f32x4){0.f, 0.f, 0.f, 0.f}) * f_low[t];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#else
     if (__builtin_amdgcn_ballot_w64(ref[0][0] != m_acc[0] || ref[0][1] != m_acc[0] || ref[1][0] != m_acc[1] ||
                                     ref[1][1] != m_acc[1])) {
       // cold: a score wave raised a reference point at this step (or this is the first step)
@@ -637,22 +680,16 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
       for (int t = 0; t < 2; ++t) {
         const float m_new = fmaxf(ref[t][0], ref[t][1]);          // never below m_acc
         const float alpha = fast_exp2(m_acc[t] - m_new);
+        const float f_lo = fast_exp2(ref[t][0] - m_new), f_hi = fast_exp2(ref[t][1] - m_new);
         m_acc[t] = m_new;
 #pragma unroll
         for (int fb = 0; fb < MD_FBW; ++fb) acc[t][fb] *= alpha;
         l_acc[t] *= alpha;
-#if CL_PREFILL
-        // (exact: the points are whole numbers.  Far below the new one, any exponent that leaves zero will do)
-        const int f_lo = (int)fmaxf(ref[t][0] - m_new, -1000.f), f_hi = (int)fmaxf(ref[t][1] - m_new, -1000.f);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) pf[t][i] = to_elem(__builtin_amdgcn_ldexpf(to_f32(pf[t][i]), i < 4 ? f_lo : f_hi));
-#else
-        const float f_lo = fast_exp2(ref[t][0] - m_new), f_hi = fast_exp2(ref[t][1] - m_new);
 #pragma unroll
         for (int i = 0; i < 8; ++i) pf[t][i] = to_elem(to_f32(pf[t][i]) * (i < 4 ? f_lo : f_hi));
-#endif
       }
     }
+#endif
     // The loads of image it + 2 (into the slot image it - 2 has left) are asked for between the
     // matrix ops, panel p after feature block p * MD_FBW / MD_PANELS.  Past the split's end the
     // last image is asked for again, into the slot of image n_own + 1 (which holds or awaits the
