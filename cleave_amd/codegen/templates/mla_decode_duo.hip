@@ -107,6 +107,7 @@ static_assert(CL_S_PANELS >= 0 && CL_S_PANELS < MD_PANELS, "the value waves keep
 static_assert(CL_CKV % 128 == 0 && CL_KPE % 64 == 0, "whole 64-feature panels, the latent ones halved between two value waves");
 #if CL_PREFILL
 #define MD_TOKENS 4                              // query tokens of a workgroup, 16 heads each
+#define MD_COLD (MD_FBW % 8 == 0 ? 8 : 4)        // feature blocks read together where a reference point was raised
 #define MD_SCALE 1.0f                            // (scores are scaled as they come: the run-time scale may have any sign)
 static_assert(CL_HEADS % 16 == 0 && CL_SPLITS == 1, "16 heads of four tokens per workgroup, unsplit");
 #else
@@ -646,29 +647,51 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
     if (__builtin_amdgcn_ballot_w64(ref[0][0] != m_acc[0] || ref[0][1] != m_acc[0] || ref[1][0] != m_acc[1] ||
                                     ref[1][1] != m_acc[1])) {
       // cold: a score wave raised a reference point at this step.  The half that stands against the lower point is multiplied
-      // here, by itself, and its product moves to the higher point: its weights are 16 bits already, scaled they would be
-      // rounded a second time.
+      // here, by itself, and the sums with it move to the higher point: its weights are 16 bits already, scaled they would
+      // be rounded a second time.  Per head tile, as mostly one of the two has a raised head: 8987 tokens at a scale that
+      // raises a point on every sixth step 160 us, both tiles together 163, weights rounded twice 157.
       elem8 p_low[2];
-      float alpha[2], f_low[2];
+      float alpha[2];
+      if (__builtin_amdgcn_ballot_w64(fminf(ref[0][0], ref[0][1]) > m_acc[0] || fminf(ref[1][0], ref[1][1]) > m_acc[1])) {
+        // (both halves raised theirs: the sums move to the lower one first)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          const float low = fminf(ref[t][0], ref[t][1]), a = fast_exp2(m_acc[t] - low);
+          m_acc[t] = low;
+#pragma unroll
+          for (int fb = 0; fb < MD_FBW; ++fb) acc[t][fb] *= a;
+          l_acc[t] *= a;
+        }
+      }
+      bool raised[2];
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         const float m_new = fmaxf(ref[t][0], ref[t][1]);          // never below m_acc
         alpha[t] = fast_exp2(m_acc[t] - m_new);
-        f_low[t] = fast_exp2(fminf(ref[t][0], ref[t][1]) - m_new);
+        raised[t] = __builtin_amdgcn_ballot_w64(ref[t][0] != m_acc[t] || ref[t][1] != m_acc[t]) != 0;
         m_acc[t] = m_new;
         p_low[t] = md_halves(pf[t], ref[t][0] < ref[t][1], ref[t][1] < ref[t][0]);
         pf[t] = md_halves(pf[t], ref[t][0] >= ref[t][1], ref[t][1] >= ref[t][0]);
-        l_acc[t] = l_acc[t] * alpha[t] + mfma16(ones, p_low[t], (f32x4){0.f, 0.f, 0.f, 0.f}) * f_low[t];
+        l_acc[t] = mfma16(ones, p_low[t], l_acc[t]) * alpha[t];
       }
 #pragma unroll
-      for (int fb = 0; fb < MD_FBW; ++fb) {
-        __builtin_amdgcn_sched_barrier(0);
-        md_s16x4 lo, hi;
-        operand(tile, fb, lo, hi);
-        const elem8 a = __builtin_bit_cast(elem8, (md_s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+      for (int t = 0; t < 2; ++t) {
+        if (!raised[t]) continue;
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
-          acc[t][fb] = acc[t][fb] * alpha[t] + mfma16(a, p_low[t], (f32x4){0.f, 0.f, 0.f, 0.f}) * f_low[t];
+        for (int fb0 = 0; fb0 < MD_FBW; fb0 += MD_COLD) {
+          __builtin_amdgcn_sched_barrier(0);
+          elem8 a[MD_COLD];
+#pragma unroll
+          for (int q = 0; q < MD_COLD; ++q) {
+            md_s16x4 lo, hi;
+            operand(tile, fb0 + q, lo, hi);
+            a[q] = __builtin_bit_cast(elem8, (md_s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+          }
+#pragma unroll
+          for (int q = 0; q < MD_COLD; ++q) acc[t][fb0 + q] = mfma16(a[q], p_low[t], acc[t][fb0 + q]);
+#pragma unroll
+          for (int q = 0; q < MD_COLD; ++q) acc[t][fb0 + q] *= alpha[t];
+        }
       }
       __builtin_amdgcn_sched_barrier(0);
     }

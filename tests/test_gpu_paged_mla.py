@@ -206,10 +206,11 @@ def test_paged_mla_prefill_with_score_and_value_waves(q_lens, kv_lens, heads, ck
     assert np.all(np.isneginf(got_l[~live])) and np.all(got_o[~live.any(axis=1)] == 0)
 
 
-@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
-def test_weights_are_rounded_once_where_one_token_half_raises_the_reference_point(dtype):
-    """Step 2 holds scores just under the raising limit (2^8 over step 1) in its first token half and one past it in the
-    second, whose point both then take.  The latent rows are +1 and -1 on the first half's keys and 0 elsewhere: the output is
+@pytest.mark.parametrize("first", [7.75, 8.5], ids=["one_raises", "both_raise"])
+@pytest.mark.parametrize("dtype,ckv", [("bfloat16", 512), ("float16", 512), ("bfloat16", 128), ("float16", 384)])
+def test_weights_are_rounded_once_where_one_token_half_raises_the_reference_point(dtype, ckv, first):
+    """Step 2 holds scores just under the raising limit (2^8 over step 1), or just past it, in its first token half and higher
+    ones in the second, whose point both then take.  The latent rows are +1 and -1 on the first half's keys and 0 elsewhere: the output is
     the difference of rounded weights.  Against float64, the one-wave-per-token form, which rounds a weight once, sets the
     error: rounding twice, the score-wave form measured 1.27 (bf16) and 1.22 (f16) times it, rounding once 0.74 of it.  (1024
     independent pairs of weights: the ratio is known to 4 %.)"""
@@ -218,9 +219,9 @@ def test_weights_are_rounded_once_where_one_token_half_raises_the_reference_poin
     gen = torch.Generator().manual_seed(3)
     score = torch.full((live + tail,), -30.0)
     score[:32] = 0.0
-    score[32:48] = torch.where(torch.arange(16) % 2 == 0, 7.75, 7.5)
-    score[48] = 8.5
-    latent = torch.zeros(live + tail, 512)
+    score[32:48] = torch.where(torch.arange(16) % 2 == 0, first, first - 0.25)
+    score[48] = first + 0.75
+    latent = torch.zeros(live + tail, ckv)
     latent[32:48] = torch.where(torch.arange(16) % 2 == 0, 1.0, -1.0)[:, None]
     k_pe = torch.zeros(live + tail, 64)
     k_pe[:, 0] = score
@@ -230,7 +231,7 @@ def test_weights_are_rounded_once_where_one_token_half_raises_the_reference_poin
     q_pe[:, :, 1] = torch.rand(tq, heads, generator=gen) * 0.25           # (a shift of the keys that carry a 1 there)
     k_pe[32:48, 1] = torch.where(torch.arange(16) % 2 == 0, 1.0, 0.5)
     ptr = [torch.tensor([0, n], dtype=torch.int32) for n in (tq, live + tail)]
-    args = [torch.zeros(tq, heads, 512).to(kind), q_pe.to(kind), latent[:, None].to(kind), k_pe[:, None].to(kind), *ptr,
+    args = [torch.zeros(tq, heads, ckv).to(kind), q_pe.to(kind), latent[:, None].to(kind), k_pe[:, None].to(kind), *ptr,
             torch.arange(live + tail, dtype=torch.int32), float(np.log(2.0))]
     s = torch.einsum("qhd,kd->qhk", args[1].double(), args[3][:, 0].double())
     w = torch.exp2(s) * (torch.arange(live + tail)[None, None] <= (live + torch.arange(tq))[:, None, None])
@@ -240,6 +241,6 @@ def test_weights_are_rounded_once_where_one_token_half_raises_the_reference_poin
         out = kernel(*[a.cuda() if isinstance(a, torch.Tensor) else a for a in args])[0]
         return float((out.double().cpu() - want).pow(2).mean().sqrt())
 
-    once, here = error(mla_prefill_kernel(heads, dtype=dtype)), error(mla_duo_prefill_kernel(heads, 512, dtype))
-    print(f"{dtype}: rounded once {once:.3e}, score and value waves {here:.3e}", flush=True)
+    once, here = error(mla_prefill_kernel(heads, ckv, dtype=dtype)), error(mla_duo_prefill_kernel(heads, ckv, dtype))
+    print(f"{dtype} {ckv} {first}: rounded once {once:.3e}, score and value waves {here:.3e}", flush=True)
     assert here <= 1.15 * once
