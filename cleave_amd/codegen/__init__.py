@@ -34,7 +34,8 @@ LOG2E = 1.4426950408889634
 # The operands that a template moves from global memory straight into LDS in 16-byte pieces.  Such a load needs its pieces
 # at multiples of 16 bytes; everything else is read through registers, which takes any element's address.
 DIRECT_TO_LDS = {"gemm_tile.hip": ("A", "B", "C"), "mla_decode.hip": ("KV", "KPE"), "mla_paged_decode.hip": ("KV", "KPE"),
-                 "mla_decode_duo.hip": ("Q", "QPE", "KV", "KPE"), "attn_prefill_lds.hip": ("K", "V")}
+                 "mla_decode_duo.hip": ("Q", "QPE", "KV", "KPE"), "attn_prefill_lds.hip": ("K", "V"),
+                 "attn_phased.hip": ("K", "V")}
 
 _C_TYPES = {"float16": "elem_t", "bfloat16": "elem_t", "float32": "float", "int32": "int"}
 
@@ -537,6 +538,13 @@ class HipCodeGen:
             params.insert(at, ParamSpec("Scratch_kn", key.dtype, key.shape, "scratch"))
             unit.direct["K"] = "Scratch_kn"
         self._attn_common(unit, plan, params, partial, combine, False, p["vdim"], p["units"] * rows, False)
+        phased = int(plan.tiling.get("PHASED", 0))
+        if phased:
+            from ..schedule.policy import attn_phased_ok
+
+            if splits > 1 or ("k" in norm and not kpre) or not attn_phased_ok(p):
+                raise CodegenError("the phased attention kernel: unsplit, row-major keys without a norm of their own (or KPRE), "
+                                   "values up to 128 wide, key and value widths of at most five 64-feature panels together")
         for k, v in (("CL_DENSE", 1), ("CL_RAGGED", 1), ("CL_HEAD_DIM", d), ("CL_KV_HEADS", 1), ("CL_Q_HEADS", 1),
                      ("CL_ROWS", rows), ("CL_SKV", p["skv"])):
             unit.define(k, v)
@@ -552,10 +560,10 @@ class HipCodeGen:
         for role, macro in (("Q", "CL_ARG_Q"), ("K", "CL_ARG_K"), ("V", "CL_ARG_V")):
             unit.define(macro, "Scratch_kn" if kpre and role == "K" else op[role])
         for k, v in plan.tiling.items():
-            if k not in ("SHARED", "KPRE"):
+            if k not in ("SHARED", "KPRE", "PHASED"):
                 unit.define(f"CL_PF_{k}", int(v))
         unit.define("CL_EMIT_KPRE", kpre)
-        unit.templates += ["attn_prefill_lds.hip", "attn_combine.hip"]
+        unit.templates += ["attn_tile.hip", "attn_phased.hip" if phased else "attn_prefill_lds.hip", "attn_combine.hip"]
         if kpre:
             by_name = self._by_name(params)
             key_rows = p["units"] * p["skv"]
@@ -566,8 +574,9 @@ class HipCodeGen:
             unit.templates.append("rows_norm.hip")
             unit.launch(ENTRY + "_keys", (-(-(key_rows * (d // 8)) // 256), 1, 1), 256, 0, args)
         if partial:
-            items = -(-(-(-rows // 128)) // 8) * 8              # padded to a multiple of 8 (one eighth of the space per XCD)
-            unit.launch(ENTRY, (items, p["units"], splits), 256, 0, self._partial_args)
+            # (the item axis is padded to a multiple of 8: one eighth of the space per XCD)
+            items = -(-(-(-rows // (256 if phased else 128))) // 8) * 8
+            unit.launch(ENTRY, (items, p["units"], splits), 512 if phased else 256, 0, self._partial_args)
         if combine:
             entry, args = self._combine_args
             unit.launch(entry, (-(-(p["units"] * rows * (p["vdim"] // 4)) // 256), 1, 1), 256, 0, args)
@@ -596,7 +605,7 @@ class HipCodeGen:
             # four waves share every key tile through LDS: 128 query rows per workgroup and kv head
             if d % 64 or d > 256:
                 raise CodegenError("the LDS-shared prefill kernel needs a head dim of whole 64-feature panels (<= 256)")
-            unit.templates.append("attn_prefill_lds.hip")
+            unit.templates += ["attn_tile.hip", "attn_prefill_lds.hip"]
             for k, v in plan.tiling.items():
                 if k != "SHARED":
                     unit.define(f"CL_PF_{k}", int(v))

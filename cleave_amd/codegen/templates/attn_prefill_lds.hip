@@ -9,13 +9,17 @@
 //   image [D/64][32][64]   64-feature panels, 128-byte key rows, 16-byte chunk ^ (key & 6)
 // K is read as the A operand of scores^T = K Q^T with 16-byte reads, V with transposing reads as
 // the A operand of out^T += V^T P^T; each operand read feeds both row tiles of the wave.  Three
-// stages rotate (two steps of loads in flight), one barrier per step.  The softmax is the exact
-// online one (running max per query row, accumulators rescaled only when a max moved), slimmed
-// for the vector unit, which is the busiest unit of this kernel: the loop is unrolled over the
-// three stages so that LDS addresses are immediates, steps below every row's causal limit run a
-// body without mask arithmetic, scale and max subtraction are one multiply-add per score, the
-// row maximum crosses the four key groups with two row-swap instructions, and one sum of the
-// unrounded weights serves both the normalisation and the lse.
+// stages of each rotate (two steps of loads in flight), one barrier per step; the loop is unrolled
+// over them so that LDS addresses are immediates.  The softmax is the exact online one, slimmed for
+// the vector unit: steps below every row's causal limit run a body without mask arithmetic, scale
+// and reference point are one multiply-add per score, a row's maximum is taken only where its weights
+// outgrow their reference point (seen from their sum), and one sum of the unrounded weights serves
+// the normalisation and the lse.
+//
+// What bounds it: the loop runs at the power cap (the clock falls to 1.9 GHz and time follows the work done, not the
+// stalls).  Dense, 32 heads x 4096 x 4096 at 128 wide: 248 -> 239 us when the maxima (ten vector instructions of a
+// step's eighty) went and the operand reads moved ahead of their use; with parts switched off: no tile loads 220, no value
+// reads 228, no key reads 232, no exponentials 212.  attn_phased.hip loads half as much per row.
 //
 // Work items: a new item at every multiple of PL_QT packed query tokens and at every request
 // boundary (item t = chunk w + request b for the one pair that overlaps); an item stops at the
@@ -96,7 +100,8 @@
 #define PL_PANEL (PL_STEP * 64)               // elements of one 64-feature panel
 #define PL_KIMG (PL_KPANELS * PL_PANEL)       // elements of the K image
 #define PL_STAGE ((PL_KPANELS + PL_VPANELS) * PL_PANEL)   // K image, then V image
-#define PL_STAGES 4
+#define PL_VIMG (PL_VPANELS * PL_PANEL)       // elements of the V image
+#define PL_STAGES (CL_HEAD_DIM > 192 ? 4 : 3)     // (the widest keys are read in two halves, the second out of an image still held)
 #define PL_KJ (CL_HEAD_DIM / 32)
 #define PL_FB (CL_VDIM / 16)
 #define PL_UNITS_PER (PL_KPANELS + PL_VPANELS)   // 1 KiB loads per wave and step: its 8-key group of every panel of K and V
@@ -109,59 +114,6 @@ __shared__ __attribute__((aligned(1024))) elem_t pl_tiles[PL_STAGES * PL_STAGE];
 #if !CL_RAGGED
 __shared__ __attribute__((aligned(256))) int pl_ids[2][4][64];   // table entries on their way in: [step parity][wave][lane]
 #endif
-
-typedef short pl_s16x4 __attribute__((ext_vector_type(4)));
-typedef short pl_s16x8 __attribute__((ext_vector_type(8)));
-typedef __attribute__((address_space(3))) pl_s16x4 pl_lds_s16x4;
-
-CL_DEVICE int pl_swz(int key) { return key & 6; }
-CL_DEVICE int pl_clamp(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
-
-// 16 bytes per lane, global -> LDS (see the MLA kernels): not counted by the compiler, the kernel
-// waits for it itself
-template <int OFF>
-CL_DEVICE void pl_dma16(const void* gptr, unsigned lds_byte) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off offset:%2"
-               :: "v"(gptr), "s"(__builtin_amdgcn_readfirstlane(lds_byte)), "n"(OFF) : "memory", "m0");
-}
-// 4 bytes per lane, the same way
-CL_DEVICE void pl_dma4(const void* gptr, unsigned lds_byte) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off"
-               :: "v"(gptr), "s"(__builtin_amdgcn_readfirstlane(lds_byte)) : "memory", "m0");
-}
-
-template <int I> struct PlC { static constexpr int value = I; };
-
-// max of x over the four lanes that share lane % 16 (the key groups of one query row): the two
-// row-swap instructions exchange 16-lane rows 1<->0', 3<->2' and then 2,3<->0',1' of a register pair
-// rows (16 lanes) 1 and 3 of `a` trade places with rows 0 and 2 of `b`
-CL_DEVICE void pl_swap_rows16(unsigned& a, unsigned& b) {
-  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 0" : "+v"(a), "+v"(b));
-}
-CL_DEVICE float pl_max_over_groups(float x) {
-  float a = x, b = x;
-  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 0\n\tv_max_f32 %0, %0, %1\n\tv_mov_b32 %1, %0\n\t"
-               "s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 0\n\tv_max_f32 %0, %0, %1"
-               : "+v"(a), "+v"(b));
-  return a;
-}
-
-// the largest of three (one instruction, and none of the canonicalising copies fmaxf brings along)
-CL_DEVICE float pl_max3(float a, float b, float c) {
-  float r;
-  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-  return r;
-}
-// Row sums of the weights on the matrix unit (a product with a fragment of ones beside the value
-// products: the sum of exactly the rounded weights the values are multiplied by) instead of one
-// vector add per weight -- where the vector unit is the busier one, i.e. 64-wide heads (measured
-// on dense attention over 4096 keys: 151 against 158 us at 64 / 64, 256 against 253 at 128 / 128, 1673
-// against 1527 at 192 / 128).  Not where the log-sum-exp is an output: that is held to 1e-3, which the
-// rounding of a handful of 16-bit weights would show, so there the unrounded weights are added up.
-#ifndef CL_PF_MSUMS
-#define CL_PF_MSUMS (CL_HEAD_DIM <= 64 && CL_VDIM <= 64)
-#endif
-#define PL_MATRIX_SUMS (CL_PF_MSUMS && !CL_EMIT_LSE && !CL_LINEAR)
 
 #if CL_EMIT_PARTIAL
 extern "C" __global__ void __launch_bounds__(256, 2)
@@ -292,25 +244,69 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
   const int n_steps = (ext + PL_STEP - 1) / PL_STEP;
   const unsigned tiles_byte = (unsigned)(size_t)(__attribute__((address_space(3))) elem_t*)pl_tiles;
 
-  // This wave's share of step s (clamped onto the last step: a step past the end reloads the last
-  // one into an image nobody reads, so the load counter holds the same number of steps at every
-  // wait): key rows 8 wave + lane / 8 of every panel of K and V, the chunk for slot lane % 8.
-  // The lane's key row is kv0 + position (packed keys) or its table entry, which `row_of` reads
-  // (positions past the item's last key repeat it; ids outside the pool are clamped into it).
+  // Loads of one step, this wave's share: key rows 8 wave + lane / 8 of every 64-feature panel, the chunk for slot
+  // lane % 8.  A step past the end repeats the last one into an image nobody reads, so that the load counter holds the
+  // same number of loads at every wait; positions past the item's last key repeat it.
   const int my_r = 8 * wave + (lane >> 3);
-  auto key_pos = [&](int s) __attribute__((always_inline)) {
-    s = s < n_steps - 1 ? s : n_steps - 1;
-    const int t = s * PL_STEP + my_r;
-    return t < ext - 1 ? t : ext - 1;
-  };
-  auto row_of = [&](int s) __attribute__((always_inline)) {
+  const int chunk_byte = 16 * ((lane & 7) ^ pl_swz(my_r));
+  const int last_step = n_steps - 1, tail_r = ext - 1 - PL_STEP * last_step;      // last row of the last step
+  const int row_tail = my_r < tail_r ? my_r : tail_r;
 #if CL_RAGGED
-    return kv0 + key_pos(s);
-#else
-    return pl_clamp(CL_ARG_INDICES[kv0 + key_pos(s)], 0, num_pages - 1);
+  // consecutive rows: a scalar base per step and one of two lane offsets (whole step / last step)
+  const unsigned koff[2] = {(unsigned)(my_r * (int)krow_bytes + chunk_byte), (unsigned)(row_tail * (int)krow_bytes + chunk_byte)};
+  const unsigned voff[2] = {(unsigned)(my_r * (int)vrow_bytes + chunk_byte), (unsigned)(row_tail * (int)vrow_bytes + chunk_byte)};
 #endif
+  auto issue_k = [&](int s, int slot, auto lo_c, auto hi_c, int row) __attribute__((always_inline)) {
+    s = s < last_step ? s : last_step;
+    const unsigned dst = tiles_byte + (unsigned)(slot * PL_KIMG * 2 + wave * 1024);
+#if CL_KT
+    // feature row 64 P + 16 wave + lane / 4 of the (d, keys) matrix, the step's 32 keys as four 16-byte chunks
+    pl_static_for<decltype(lo_c)::value, decltype(hi_c)::value>([&](auto p) __attribute__((always_inline)) {
+      constexpr int P = decltype(p)::value;
+      const int feat = 64 * P + 16 * wave + (lane >> 2);
+      const int piece = (lane & 3) ^ ((lane >> 4) & 2);            // halves swapped where feature bit 3 is set
+      pl_dma16<0>(kbase + ((i64)feat * CL_SKV + s * PL_STEP) * 2 + 16 * piece, dst + (unsigned)(P * PL_PANEL * 2));
+    });
+#elif CL_RAGGED
+    const char* base = kbase + (i64)(kv0 + s * PL_STEP) * krow_bytes;
+    const unsigned off = s == last_step ? koff[1] : koff[0];
+    pl_static_for<decltype(lo_c)::value, decltype(hi_c)::value>([&](auto p) __attribute__((always_inline)) {
+      constexpr int P = decltype(p)::value;
+      pl_dma16s<128 * P>(base, off, dst + (unsigned)(P * PL_PANEL * 2) - 128 * P);
+    });
+#else
+    const char* src = kbase + (i64)row * krow_bytes + chunk_byte;
+    pl_static_for<decltype(lo_c)::value, decltype(hi_c)::value>([&](auto p) __attribute__((always_inline)) {
+      constexpr int P = decltype(p)::value;
+      pl_dma16<128 * P>(src, dst + (unsigned)(P * PL_PANEL * 2) - 128 * P);
+    });
+#endif
+    (void)row;
+  };
+  auto issue_v = [&](int s, int slot, auto lo_c, auto hi_c, int row) __attribute__((always_inline)) {
+    s = s < last_step ? s : last_step;
+    const unsigned dst = tiles_byte + (unsigned)((PL_STAGES * PL_KIMG + slot * PL_VIMG) * 2 + wave * 1024);
+#if CL_RAGGED
+    const char* base = vbase + (i64)(kv0 + s * PL_STEP) * vrow_bytes;
+    const unsigned off = s == last_step ? voff[1] : voff[0];
+    pl_static_for<decltype(lo_c)::value, decltype(hi_c)::value>([&](auto p) __attribute__((always_inline)) {
+      constexpr int P = decltype(p)::value;
+      pl_dma16s<128 * P>(base, off, dst + (unsigned)(P * PL_PANEL * 2) - 128 * P);
+    });
+#else
+    const char* src = vbase + (i64)row * vrow_bytes + chunk_byte;
+    pl_static_for<decltype(lo_c)::value, decltype(hi_c)::value>([&](auto p) __attribute__((always_inline)) {
+      constexpr int P = decltype(p)::value;
+      pl_dma16<128 * P>(src, dst + (unsigned)(P * PL_PANEL * 2) - 128 * P);
+    });
+#endif
+    (void)row;
   };
 #if !CL_RAGGED
+  auto key_pos = [&](int s) __attribute__((always_inline)) {
+    return PL_STEP * (s < last_step ? s : last_step) + (s < last_step ? my_r : row_tail);
+  };
+  auto row_of = [&](int s) __attribute__((always_inline)) { return pl_clamp(CL_ARG_INDICES[kv0 + key_pos(s)], 0, num_pages - 1); };
   // In the loop the lane's table entry travels like the tiles do, global -> LDS on the kernel's
   // own load counter, a step ahead of the loads that need it (a load the compiler tracks would
   // make it wait for every load in flight): entry of step s into pl_ids[s & 1][wave][lane].
@@ -322,51 +318,27 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
     return pl_clamp(pl_ids[s & 1][wave][lane], 0, num_pages - 1);
   };
 #endif
-  // load `part` of a step (its K panels, then its V panels) into stage `slot`
-  auto issue_part = [&](int row, int slot, auto part_c) __attribute__((always_inline)) {
-    constexpr int PART = decltype(part_c)::value;
-    constexpr bool IS_K = PART < PL_KPANELS;
-    constexpr int P = IS_K ? PART : PART - PL_KPANELS;
-    const unsigned group_byte = tiles_byte + (unsigned)(slot * PL_STAGE * 2 + wave * 1024) + (IS_K ? 0 : PL_KIMG * 2);
-#if CL_KT
-    if constexpr (IS_K) {
-      // feature row 64 P + 16 wave + lane / 4 of the (d, keys) matrix, the step's 32 keys as four
-      // 16-byte chunks; `row` is the lane's key row of the step, so the step starts at row - my_r
-      const int feat = 64 * P + 16 * wave + (lane >> 2);
-      const int piece = (lane & 3) ^ ((lane >> 4) & 2);            // halves swapped where feature bit 3 is set
-      const char* src = kbase + ((i64)feat * CL_SKV + (row - my_r)) * 2 + 16 * piece;
-      pl_dma16<0>(src, group_byte + (unsigned)(P * PL_PANEL * 2));
-      return;
-    }
-#endif
-    const int chunk = (lane & 7) ^ pl_swz(my_r);
-    const char* src = (IS_K ? kbase + (i64)row * krow_bytes : vbase + (i64)row * vrow_bytes) + 16 * chunk;
-    pl_dma16<128 * P>(src, group_byte + (unsigned)(P * PL_PANEL * 2) - 128 * P);
-  };
-  // the quarter `place` (0..3) of a step's loads: the body spreads them between its matrix work,
-  // because a wave stands still while a load waits for the path into the CU
-  auto issue_quarter = [&](int row, int slot, auto place_c) __attribute__((always_inline)) {
-    constexpr int PLACE = decltype(place_c)::value, LO = PLACE * PL_UNITS_PER / 4, HI = (PLACE + 1) * PL_UNITS_PER / 4;
-    if constexpr (HI > LO) issue_part(row, slot, PlC<LO>{});
-    if constexpr (HI > LO + 1) issue_part(row, slot, PlC<LO + 1>{});
-  };
-  auto issue_step = [&](int row, int slot) __attribute__((always_inline)) {
-    issue_quarter(row, slot, PlC<0>{});
-    issue_quarter(row, slot, PlC<1>{});
-    issue_quarter(row, slot, PlC<2>{});
-    issue_quarter(row, slot, PlC<3>{});
-  };
-#define PL_WAITCNT(n) __builtin_amdgcn_s_waitcnt(0x0F70 | ((n) & 15) | (((n) >> 4) << 14))
 
-  {
-    const int row0 = row_of(0), row1 = row_of(1), row2 = row_of(2);
-    issue_step(row0, 0);
-    issue_step(row1, 1);
-#if !CL_RAGGED
-    fetch_id(3);
+  // Ahead of the loop, in the order the bodies wait for them: K 0, K 1, then V 0 and K 2, V 1 and (behind the first score
+  // products where its image is that of K 0) K 3.
+  using AllK = PlC<PL_KPANELS>;
+  using AllV = PlC<PL_VPANELS>;
+  int rows[2] = {0, 0};                        // table form: the lane's key rows of V of the next two bodies
+#if CL_RAGGED
+  constexpr int row0 = 0, row1 = 0, row3 = 0;
+#else
+  const int row0 = row_of(0), row1 = row_of(1), row3 = row_of(3);
+  rows[0] = row_of(2);
+  rows[1] = row3;
 #endif
-    issue_step(row2, 2);
-  }
+  issue_k(0, 0, PlC<0>{}, AllK{}, row0);
+  issue_k(1, 1, PlC<0>{}, AllK{}, row1);
+  issue_v(0, 0, PlC<0>{}, AllV{}, row0);
+  issue_k(2, 2, PlC<0>{}, AllK{}, rows[0]);
+#if !CL_RAGGED
+  fetch_id(4);
+#endif
+  issue_v(1, 1, PlC<0>{}, AllV{}, row1);
 
   // Query rows as the B operand: lane (c, g) holds Q[row][32 j + 8 g .. +8]; padded rows are 0.
   elem8 qf[2][PL_KJ];
@@ -397,22 +369,31 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
 
   float m_run[2] = {CL_NEG_BIG, CL_NEG_BIG};   // running max of the scaled scores (log2 domain), uniform over g
   float l_run[2] = {0.f, 0.f};                 // this lane's share of the sum of the weights
-#if PL_MATRIX_SUMS
-  f32x4 l_acc[2] = {(f32x4){0.f, 0.f, 0.f, 0.f}, (f32x4){0.f, 0.f, 0.f, 0.f}};   // every component: the sum of row c's weights
-  elem8 ones;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) ones[i] = to_elem(1.0f);
-#endif
   f32x4 acc[2][PL_FB];                         // acc[rt][fb][r] = O[row][16 fb + 4 g + r]
 #pragma unroll
   for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
     for (int fb = 0; fb < PL_FB; ++fb) acc[rt][fb] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
-  // this lane's operand offsets inside an image (elements)
-  const int a_lo = c * 64 + ((g ^ pl_swz(c)) << 3);
-  const int vtok = 4 * g + (c >> 2);
-  const int v_lo = vtok * 64 + (((((c & 3) >> 1)) ^ pl_swz(vtok)) << 3) + 4 * (c & 1);
+  // This lane's operand addresses in the first K and the first V image (LDS bytes), one per XOR pattern of a block: what
+  // is left of every read is its immediate.  Hidden from the optimiser once a body: it formed a register for each sum,
+  // kept them all across the loop and spilled them.
+  unsigned ka[2], va[4];
+  {
+    const int a_lo = c * 64 + ((g ^ pl_swz(c)) << 3);
+    const int vtok = 4 * g + (c >> 2);
+    const int v_lo = vtok * 64 + (((((c & 3) >> 1)) ^ pl_swz(vtok)) << 3) + 4 * (c & 1);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) ka[i] = tiles_byte + 2 * (a_lo ^ (32 * i));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) va[i] = tiles_byte + 2 * (PL_STAGES * PL_KIMG + (v_lo ^ (16 * i)));
+  }
+  auto keep_addresses = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) asm volatile("" : "+v"(ka[i]));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(va[i]));
+  };
   // causal limit of the lane's rows relative to its first key slot (slot q of half h is key t0 + 16 h + 4 g + q)
   const int lim_rel[2] = {limit[0] - 4 * g, limit[1] - 4 * g};
   // Steps every key of which every live row of this wave sees need no mask: the wave's first
@@ -425,31 +406,29 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
   }
   n_full = __builtin_amdgcn_readfirstlane(n_full);
 
-  // scores^T of one step out of the K image in stage SLOT: a 16-byte read per 16-key half and
-  // 32-feature block, each feeding the wave's two row tiles
-  // (`lo`: the lane's operand offset a_lo / v_lo, or a body's own copy of it, see do_step)
-  auto k_frag = [&](auto slot_c, int j, int h, int lo) __attribute__((always_inline)) {
+  // key fragment of 16-key half h and 32-feature block j out of the K image in stage SLOT: a 16-byte read, which feeds the
+  // wave's two row tiles
+  auto k_frag = [&](auto slot_c, int j, int h) __attribute__((always_inline)) {
     constexpr int SLOT = decltype(slot_c)::value;
 #if CL_KT
     // sixteen lanes address a 4 (feature) x 16 (key) patch, lane c: feature row c / 4, keys 4 (c % 4) .. + 3,
     // and lane c receives the four features of key c; two reads give features 8 g .. 8 g + 7 of block j
-    const elem_t* p = pl_tiles + SLOT * PL_STAGE + (j >> 1) * PL_PANEL + (32 * (j & 1) + 8 * g + (c >> 2)) * 32 +
+    const elem_t* p = pl_tiles + SLOT * PL_KIMG + (j >> 1) * PL_PANEL + (32 * (j & 1) + 8 * g + (c >> 2)) * 32 +
                       16 * (h ^ (g & 1)) + 4 * (c & 3);
     const pl_s16x4 lo4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((pl_lds_s16x4*)(p));
     const pl_s16x4 hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((pl_lds_s16x4*)(p + 4 * 32));
     return __builtin_bit_cast(elem8, (pl_s16x8)__builtin_shufflevector(lo4, hi4, 0, 1, 2, 3, 4, 5, 6, 7));
 #else
-    return *reinterpret_cast<const elem8*>(pl_tiles + SLOT * PL_STAGE + (j >> 1) * PL_PANEL + 16 * h * 64 +
-                                           (lo ^ ((4 * (j & 1)) << 3)));
+    return *(const pl_lds_elem8*)(ka[j & 1] + (unsigned)((SLOT * PL_KIMG + (j >> 1) * PL_PANEL + 16 * h * 64) * 2));
 #endif
   };
   // value operand for feature block fb out of the V image in stage SLOT: rows = features
   // 16 fb + (0..15), slots = keys 4 g + (0..3), 16 + 4 g + (0..3)
-  auto v_frag = [&](auto slot_c, int fb, int lo) __attribute__((always_inline)) {
+  auto v_frag = [&](auto slot_c, int fb) __attribute__((always_inline)) {
     constexpr int SLOT = decltype(slot_c)::value;
-    const elem_t* p = pl_tiles + SLOT * PL_STAGE + PL_KIMG + (fb >> 2) * PL_PANEL + (lo ^ (((2 * fb) & 7) << 3));
+    const unsigned p = va[fb & 3] + (unsigned)((SLOT * PL_VIMG + (fb >> 2) * PL_PANEL) * 2);
     const pl_s16x4 lo4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((pl_lds_s16x4*)(p));
-    const pl_s16x4 hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((pl_lds_s16x4*)(p + 16 * 64));
+    const pl_s16x4 hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((pl_lds_s16x4*)(p + 16 * 64 * 2));
     return __builtin_bit_cast(elem8, (pl_s16x8)__builtin_shufflevector(lo4, hi4, 0, 1, 2, 3, 4, 5, 6, 7));
   };
 
@@ -475,240 +454,234 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
   };
 #endif
 
-  // The loop is skewed by one step: body s turns the scores of step s (made in body s - 1) into
-  // weights and adds their value product, and between those vector instructions it issues the
-  // score products of step s + 1, so that the matrix unit works in the shadow of the softmax.
+  // The loop is skewed.  Body s turns the scores of step s (made in body s - 1) into weights, adds their value product and
+  // makes the scores of step s + 1 from key fragments that are in registers when it begins; the value fragments are
+  // read beside the score products and the key fragments of step s + 2 beside the value products, so that no matrix op
+  // waits for a read that has just been asked for (that wait was 8 LDS reads deep behind every barrier).
   f32x4 st[2][2];                              // raw scores^T of the step the next body weighs
-#if CL_RAGGED
-  PL_WAITCNT(2 * PL_UNITS_PER);
-#else
-  PL_WAITCNT(2 * PL_UNITS_PER + 1);
-#endif
-  __syncthreads();
-  {
-#pragma unroll
-    for (int rt = 0; rt < 2; ++rt) st[rt][0] = st[rt][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#if CL_KNORM
-    f32x4 gram[2] = {(f32x4){0.f, 0.f, 0.f, 0.f}, (f32x4){0.f, 0.f, 0.f, 0.f}};
-#endif
-#pragma unroll
-    for (int j = 0; j < PL_KJ; ++j)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const elem8 a = k_frag(PlC<0>{}, j, h, a_lo);
-#pragma unroll
-        for (int rt = 0; rt < 2; ++rt) st[rt][h] = mfma16(a, qf[rt][j], st[rt][h]);
-#if CL_KNORM
-        gram[h] = mfma16(a, a, gram[h]);
-#endif
-      }
-#if CL_KNORM
-    scale_by_key_norms(gram, st);
-#endif
-  }
-
-  // Body of step `step`, whose images are in stage SLOT (compile-time: every LDS address is a
-  // register plus an immediate).
-  auto do_step = [&](auto slot_c, const int step) __attribute__((always_inline)) {
-    constexpr int SLOT = decltype(slot_c)::value;
-    // the images of step + 1 have landed when at most the loads of step + 2 are outstanding; the
-    // barrier makes that everybody's share and frees the stage step - 1 has left, which the
-    // loads of step + 3 fill
-    PL_WAITCNT(PL_UNITS_PER);
-    __syncthreads();
-#if CL_RAGGED
-    const int row_ahead = row_of(step + 3);
-#else
-    // (the entry of step + 3 was asked for a body ago, before the loads the wait above left out)
-    const int row_ahead = fetched_row(step + 3);
-    fetch_id(step + 4);
-#endif
-#define PL_ISSUE(place) issue_quarter(row_ahead, (SLOT + 3) % PL_STAGES, PlC<place>{})
-    PL_ISSUE(0);
-
-    // operands of this body's matrix work: K of step + 1, V of step (8 + 16 LDS reads).
-    // With more than 64 KiB of images (keys wider than 128) the offset field of an LDS instruction no
-    // longer reaches every stage from one register per lane pattern, and the dozen address registers
-    // the optimiser then kept across the loop were spilled, every reload waiting for the tile loads
-    // in flight: each body forms its addresses from a copy of the two lane offsets that the
-    // optimiser cannot see through, so none of them lives longer than the body's reads (192-wide
-    // keys: 14 spilled registers -> none, 8 % faster; at exactly 64 KiB, 128-wide heads, the same
-    // step takes the one spilled register away and costs 4 %: not done there).
-    int a_lo_b = a_lo, v_lo_b = v_lo;
-    if constexpr (PL_STAGES * PL_STAGE * 2 > 65536) asm volatile("" : "+v"(a_lo_b), "+v"(v_lo_b));
-    // (256-wide keys: the fragments of the key image are held half at a time -- the second half is
-    // read once the score products of the first have gone out -- or query fragments are spilled)
-    constexpr int KH = (PL_KJ > 6 && !CL_KNORM) ? PL_KJ / 2 : PL_KJ;
-    elem8 kf[KH][2];
+  // (256-wide keys: fragments are held half a step at a time, or query fragments are spilled)
+  constexpr int KH = PL_KJ > 6 ? PL_KJ / 2 : PL_KJ;
+  static_assert(KH == PL_KJ || PL_STAGES == 4, "K of the step in hand keeps its image where it is read in two halves");
+  elem8 kf[KH][2];                             // key fragments of the step the next body scores
+  auto read_keys = [&](auto slot_c, int j0) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < KH; ++j)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) kf[j][h] = k_frag(PlC<(SLOT + 1) % PL_STAGES>{}, j, h, a_lo_b);
-    elem8 vf[PL_FB];
+      for (int h = 0; h < 2; ++h) kf[j][h] = k_frag(slot_c, j0 + j, h);
+  };
+#if CL_KNORM
+  f32x4 gram[2];
+#endif
+  // scores (and Gram diagonals) of the fragments in hand: feature blocks j0 ..
+  auto score = [&](f32x4 (&sc)[2][2], int j0) __attribute__((always_inline)) {
+    if (j0 == 0) {
 #pragma unroll
-    for (int fb = 0; fb < PL_FB; ++fb) vf[fb] = v_frag(slot_c, fb, v_lo_b);
-    __builtin_amdgcn_sched_barrier(0);
-
-    // ---- maxima of the step's scores; raise a row's reference when they pass it by 2^8 -------
-    float s[2][8];
+      for (int rt = 0; rt < 2; ++rt) sc[rt][0] = sc[rt][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#if CL_KNORM
+      gram[0] = gram[1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#endif
+    }
 #pragma unroll
-    for (int rt = 0; rt < 2; ++rt)
+    for (int j = 0; j < KH; ++j)
 #pragma unroll
-      for (int i = 0; i < 8; ++i) s[rt][i] = st[rt][i >> 2][i & 3];
-    if (step >= n_full) {
-      // slot i of the lane is key 32 step + 16 (i / 4) + 4 g + i % 4; a masked slot scores -inf,
-      // which a finite reference turns into a weight of exactly 0
+      for (int h = 0; h < 2; ++h) {
 #pragma unroll
-      for (int rt = 0; rt < 2; ++rt) {
-        const int room = lim_rel[rt] - step * PL_STEP;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) s[rt][i] = 16 * (i >> 2) + (i & 3) <= room ? s[rt][i] : (CL_LINEAR ? 0.f : CL_NEG_INF);
+        for (int rt = 0; rt < 2; ++rt) sc[rt][h] = mfma16(kf[j][h], qf[rt][j0 + j], sc[rt][h]);
+#if CL_KNORM
+        gram[h] = mfma16(kf[j][h], kf[j][h], gram[h]);
+#endif
       }
-    }
-    // (first half of the score products of step + 1 in the shadow of the maxima)
-    f32x4 sn[2][2];
-#pragma unroll
-    for (int rt = 0; rt < 2; ++rt) sn[rt][0] = sn[rt][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int j = 0; j < PL_KJ / 2; ++j)
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int rt = 0; rt < 2; ++rt) sn[rt][h] = mfma16(kf[j][h], qf[rt][j], sn[rt][h]);
-    if constexpr (KH < PL_KJ) {
-#pragma unroll
-      for (int j = KH; j < PL_KJ; ++j)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) kf[j - KH][h] = k_frag(PlC<(SLOT + 1) % PL_STAGES>{}, j, h, a_lo_b);
-    }
-#if !CL_LINEAR
-    // (the lane's own eight scores of each row; a row's four lane groups are compared only when
-    // some lane passes its row's reference: no row does unless one of its lanes does)
-    float mx[2];
+  };
+  // slot i of the lane is key 32 step + 16 (i / 4) + 4 g + i % 4; a masked slot scores -inf, which a finite reference turns
+  // into a weight of exactly 0
+  auto mask = [&](f32x4 (&sc)[2][2], int step) __attribute__((always_inline)) {
 #pragma unroll
     for (int rt = 0; rt < 2; ++rt) {
-      float v = pl_max3(s[rt][0], s[rt][1], s[rt][2]);
-      v = pl_max3(v, s[rt][3], s[rt][4]);
-      v = pl_max3(v, s[rt][5], s[rt][6]);
-      mx[rt] = pl_max3(v, s[rt][7], s[rt][7]) * scale2;
-    }
+      const int room = lim_rel[rt] - step * PL_STEP;
 #pragma unroll
-    for (int i = 0; i < 2 * PL_KJ; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+      for (int i = 0; i < 8; ++i) sc[rt][i >> 2][i & 3] = 16 * (i >> 2) + (i & 3) <= room ? sc[rt][i >> 2][i & 3] : (CL_LINEAR ? 0.f : CL_NEG_INF);
     }
-    if constexpr (KH < PL_KJ) __builtin_amdgcn_sched_group_barrier(0x100, 2 * (PL_KJ - KH), 0);
-    if (__builtin_amdgcn_ballot_w64(mx[0] > m_run[0] + 8.0f || mx[1] > m_run[1] + 8.0f)) {
-      // cold after the first steps of an item: weights stay below 2^8 against a reference that
-      // lags the running maximum by less than 8 (log2 domain)
+  };
+  // the largest of this lane's eight scores of a row (in the compiler's sight: it keeps the wait states between a matrix op
+  // and a reader of its result, which it does not see in assembly)
+  auto step_max = [&](const f32x4 (&sc)[2]) __attribute__((always_inline)) {
+    float v = sc[0][0];
 #pragma unroll
-      for (int rt = 0; rt < 2; ++rt) {
-        mx[rt] = pl_max_over_groups(mx[rt]);
-        const float m_new = mx[rt] > m_run[rt] + 8.0f ? mx[rt] : m_run[rt];
-        const float alpha = fast_exp2(m_run[rt] - m_new);
-        m_run[rt] = m_new;
-        l_run[rt] *= alpha;
-#if PL_MATRIX_SUMS
-        l_acc[rt] *= alpha;
+    for (int i = 1; i < 8; ++i) v = fmaxf(v, sc[i >> 2][i & 3]);
+    return v;
+  };
+  PL_WAITCNT(PL_KPANELS + 2 * PL_VPANELS + !CL_RAGGED);
+  pl_barrier();
+#pragma unroll
+  for (int j0 = 0; j0 < PL_KJ; j0 += KH) {
+    read_keys(PlC<0>{}, j0);
+    score(st, j0);
+  }
+#if CL_KNORM
+  scale_by_key_norms(gram, st);
 #endif
+  read_keys(PlC<1>{}, 0);
+#if !CL_LINEAR && CL_HEAD_DIM <= 192
+  // (the first reference points, so that the first weights need not be taken twice; the widest heads have no registers for it)
+  if (n_full == 0) mask(st, 0);
 #pragma unroll
-        for (int fb = 0; fb < PL_FB; ++fb) acc[rt][fb] *= alpha;
-      }
-    }
-#endif  // !CL_LINEAR
-    __builtin_amdgcn_sched_barrier(0);
-    PL_ISSUE(1);
+  for (int rt = 0; rt < 2; ++rt) {
+    const float mx = pl_max_over_groups(step_max(st[rt])) * scale2;
+    m_run[rt] = mx > CL_NEG_BIG ? mx : CL_NEG_BIG;
+  }
+#endif
+  // the images of body 0 (V 0, K 2) have landed; K 0 has been read by everybody
+  PL_WAITCNT(PL_VPANELS);
+  pl_barrier();
+  issue_k(3, 3 % PL_STAGES, PlC<0>{}, AllK{}, row3);
 
-    // ---- weights of the first row tile beside the rest of the score products -----------------
+  // Body of step `step`, step % PL_STAGES == S.
+  auto do_step = [&](auto s_c, const int step) __attribute__((always_inline)) {
+    constexpr int S = decltype(s_c)::value;
+    keep_addresses();
+#if CL_RAGGED
+    constexpr int row_v = 0, row_k = 0;
+#else
+    // (V of step + 2, whose row was looked up two bodies ago; K of step + 4, whose entry was asked for in the last body
+    // ahead of the loads that the wait before this one left out)
+    const int row_v = rows[0], row_k = fetched_row(step + 4);
+    rows[0] = rows[1];
+    rows[1] = row_k;
+    fetch_id(step + 5);
+#endif
+    // the loads of this body, in four shares between its matrix work (a wave stands still while a load waits for the path
+    // into the compute unit): V of step + 2, K of step + 4
+    auto ask = [&](auto place_c) __attribute__((always_inline)) {
+      constexpr int LO = decltype(place_c)::value * PL_UNITS_PER / 4, HI = (decltype(place_c)::value + 1) * PL_UNITS_PER / 4;
+      constexpr int VL = LO < PL_VPANELS ? LO : PL_VPANELS, VH = HI < PL_VPANELS ? HI : PL_VPANELS;
+      issue_v(step + 2, (S + 2) % PL_STAGES, PlC<VL>{}, PlC<VH>{}, row_v);
+      issue_k(step + 4, (S + 4) % PL_STAGES, PlC<LO - VL>{}, PlC<HI - VH>{}, row_k);
+    };
+    __builtin_amdgcn_sched_barrier(0);
+    if (step >= n_full) mask(st, step);
+    __builtin_amdgcn_sched_barrier(0);
+
     elem8 pf[2];
+    float psum[2] = {0.f, 0.f};
     auto weigh = [&](int rt) __attribute__((always_inline)) {
-      float psum = 0.f;
+      float sum = 0.f;
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
 #if CL_LINEAR
-        const float p = s[rt][i] * sm_scale;
+        const float p = st[rt][i >> 2][i & 3] * sm_scale;
 #else
-        const float p = fast_exp2(__builtin_fmaf(s[rt][i], scale2, -m_run[rt]));
-#endif
-#if !PL_MATRIX_SUMS
-        psum += p;
+        const float p = fast_exp2(__builtin_fmaf(st[rt][i >> 2][i & 3], scale2, -m_run[rt]));
+        sum += p;
 #endif
         pf[rt][i] = to_elem(p);
       }
-      l_run[rt] += psum;
+      psum[rt] = sum;
     };
+    // The weights are taken against the row's reference first and looked at afterwards: where a lane's eight sum to more
+    // than 2^8 (none passes 2^8 then), the row's reference is raised to its running maximum and the weights are taken
+    // again.  Cold, so that maxima cost the other steps nothing.
+    auto settle = [&](int rt) __attribute__((always_inline)) {
+#if !CL_LINEAR
+      if (__builtin_expect(__builtin_amdgcn_ballot_w64(psum[rt] > 256.0f) != 0, 0)) {
+        const float mx = pl_max_over_groups(step_max(st[rt])) * scale2;
+        const float m_new = mx > m_run[rt] ? mx : m_run[rt];
+        const float alpha = fast_exp2(m_run[rt] - m_new);
+        m_run[rt] = m_new;
+        l_run[rt] *= alpha;
 #pragma unroll
-    for (int j = PL_KJ / 2; j < PL_KJ; ++j)
+        for (int fb = 0; fb < PL_FB; ++fb) acc[rt][fb] *= alpha;
+        weigh(rt);
+      }
+      l_run[rt] += psum[rt];
+#endif
+    };
+
+    // ---- score products of step + 1 and value fragments of this step beside the weights of the first row tile --------
+    f32x4 sn[2][2];
+    ask(PlC<0>{});
+    if constexpr (KH < PL_KJ) {
+      score(sn, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      read_keys(PlC<(S + 1) % PL_STAGES>{}, KH);
+      score(sn, KH);
+    } else {
+      score(sn, 0);
+    }
+    elem8 vf[PL_FB];
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int rt = 0; rt < 2; ++rt) sn[rt][h] = mfma16(kf[KH < PL_KJ ? j - KH : j][h], qf[rt][j], sn[rt][h]);
+    for (int fb = 0; fb < PL_FB; ++fb) vf[fb] = v_frag(PlC<S>{}, fb);
     weigh(0);
+    if constexpr (KH == PL_KJ) {
 #pragma unroll
-    for (int i = 0; i < 2 * PL_KJ; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+      for (int i = 0; i < 4 * PL_KJ; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, (2 * PL_FB + 4 * PL_KJ - 1) / (4 * PL_KJ), 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+      }
     }
     __builtin_amdgcn_sched_barrier(0);
-    PL_ISSUE(2);
+#if CL_KNORM
+    scale_by_key_norms(gram, sn);
+#endif
+    settle(0);
+    __builtin_amdgcn_sched_barrier(0);
+    ask(PlC<1>{});
 
-    // ---- weights of the second row tile beside the value product of the first ----------------
+    // ---- value product of the first row tile and key fragments of step + 2 beside the weights of the second ----------
 #pragma unroll
     for (int fb = 0; fb < PL_FB; ++fb) acc[0][fb] = mfma16(vf[fb], pf[0], acc[0][fb]);
-#if PL_MATRIX_SUMS
-    l_acc[0] = mfma16(ones, pf[0], l_acc[0]);
-#endif
+    read_keys(PlC<(S + 2) % PL_STAGES>{}, 0);
     weigh(1);
 #pragma unroll
     for (int i = 0; i < PL_FB; ++i) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, (2 * KH * (CL_KT ? 2 : 1) + PL_FB - 1) / PL_FB, 0);
       __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
     }
     __builtin_amdgcn_sched_barrier(0);
-    PL_ISSUE(3);
+    settle(1);
+    __builtin_amdgcn_sched_barrier(0);
+    ask(PlC<2>{});
 
     // ---- value product of the second row tile ------------------------------------------------
 #pragma unroll
     for (int fb = 0; fb < PL_FB; ++fb) acc[1][fb] = mfma16(vf[fb], pf[1], acc[1][fb]);
-#if PL_MATRIX_SUMS
-    l_acc[1] = mfma16(ones, pf[1], l_acc[1]);
-#endif
-#if CL_KNORM
-    // (and the sums of squares of the keys of step + 1, whose factors go onto its scores)
-    f32x4 gram[2] = {(f32x4){0.f, 0.f, 0.f, 0.f}, (f32x4){0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-    for (int j = 0; j < PL_KJ; ++j)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) gram[h] = mfma16(kf[j][h], kf[j][h], gram[h]);
-    __builtin_amdgcn_sched_barrier(0);
-    scale_by_key_norms(gram, sn);
-#endif
+    ask(PlC<3>{});
 #pragma unroll
     for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
       for (int h = 0; h < 2; ++h) st[rt][h] = sn[rt][h];
   };
+  // Between two bodies: the loads of all bodies but the last have landed, everybody's (V of the next step and the keys that
+  // it reads ahead), and the images that the last body read last are free for what the next one asks for.
+  auto turn = [&]() __attribute__((always_inline)) {
+    __builtin_amdgcn_sched_barrier(0);
+    PL_WAITCNT(PL_UNITS_PER);
+    pl_barrier();
+  };
 
-  // (where the trip count is a small constant it is kept from the optimiser: a handful of steps
-  // would otherwise be laid out in a straight line, and at a 256-wide head that form, short of
-  // registers, came back from the compiler with one register of a spilled query fragment not
-  // restored; with many steps the counted loop stays a loop and runs 1 - 4 % faster than the
-  // one the optimiser cannot count, except at 256-wide heads, where it spills four times as much,
-  // and at counts that are not whole turns of the four bodies, where the optimiser peels the rest
-  // off and spills sixty registers doing so)
+  // (the trip count is kept from the optimiser where it is a constant: a handful of steps would be laid out in a straight
+  // line, and counts that are not whole turns of the bodies peeled, both short of registers -- at a 256-wide head the
+  // straight line once came back from the compiler with one register of a spilled query fragment not restored)
   int trips = n_steps;
 #if CL_DENSE
-  if constexpr (steps_per_split <= 16 || steps_per_split % 4 != 0 || CL_HEAD_DIM > 192) asm volatile("" : "+s"(trips));
+  asm volatile("" : "+s"(trips));
 #endif
   for (int step = 0;;) {
     do_step(PlC<0>{}, step);
     if (++step >= trips) break;
+    turn();
     do_step(PlC<1>{}, step);
     if (++step >= trips) break;
+    turn();
     do_step(PlC<2>{}, step);
     if (++step >= trips) break;
-    do_step(PlC<3>{}, step);
-    if (++step >= trips) break;
+    turn();
+    if constexpr (PL_STAGES > 3) {
+      do_step(PlC<3>{}, step);
+      if (++step >= trips) break;
+      turn();
+    }
   }
   // no load may still be on its way into LDS when the workgroup ends
   PL_WAITCNT(0);
@@ -721,13 +694,9 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
   const int c_e = lane_e & 15, g_e = lane_e >> 4;
 #pragma unroll
   for (int rt = 0; rt < 2; ++rt) {
-#if PL_MATRIX_SUMS
-    const float l = l_acc[rt][0];
-#else
     float l = l_run[rt];
     l += lane_xor(l, lane_e, 16);
     l += lane_xor(l, lane_e, 32);
-#endif
     const int m = 32 * wave + 16 * rt + c_e;
     if (m >= n_rows) continue;
 #if CL_LINEAR
@@ -755,25 +724,7 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
       (void)inv;
     }
 #else
-    // A lane holds features 16 fb + 4 g .. + 3 of its row for every block fb.  Lanes g and g ^ 1
-    // trade halves of a pair of blocks (one row swap per register), so that each stores 16
-    // contiguous bytes: even g the 8 features from 4 g of the even block, odd g those from
-    // 4 (g - 1) of the odd one.
-    elem_t* dst = CL_ARG_OUT + orow * CL_VDIM + 16 * (g_e & 1) + 4 * (g_e & 2);
-#pragma unroll
-    for (int fp = 0; fp < PL_FB / 2; ++fp) {
-      elem4 y0, y1;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        y0[r] = to_elem(acc[rt][2 * fp][r] * inv);
-        y1[r] = to_elem(acc[rt][2 * fp + 1][r] * inv);
-      }
-      const u32x2 a = __builtin_bit_cast(u32x2, y0), b = __builtin_bit_cast(u32x2, y1);
-      unsigned a0 = a[0], a1 = a[1], b0 = b[0], b1 = b[1];
-      pl_swap_rows16(a0, b0);
-      pl_swap_rows16(a1, b1);
-      *reinterpret_cast<u32x4*>(dst + 32 * fp) = (u32x4){a0, a1, b0, b1};
-    }
+    pl_store_row<PL_FB>(CL_ARG_OUT + orow * CL_VDIM, acc[rt], inv, g_e);
 #if CL_EMIT_LSE
     if (g_e == 0) CL_ARG_LSE[orow] = l > 0.f ? m_run[rt] + fast_log2(l) : CL_NEG_INF;
 #endif

@@ -97,7 +97,17 @@ def search_tiling(graph, topk: int = 10, force_fusion: bool = False, accept=None
             seen.add(c.key())
             c.flat_graph = graph
             unique.append(c)
-    return _cut(unique, max(1, int(topk)))
+    return _with_late(_cut([c for c in unique if not c.late], max(1, int(topk))), [c for c in unique if c.late], max(1, int(topk)))
+
+
+def _with_late(ranked, late, topk):
+    """``ranked`` with the ``late`` candidates behind its first four, ``topk`` in all: forms of a kernel that win by margins
+    the cost model does not resolve, which the search times wherever its pool is that large."""
+    late = late[:max(0, topk - 4)]
+    gone = [(c.template, c.displaces) for c in late if c.displaces is not None]
+    ranked = [c for c in ranked if (c.template, c.tiling) not in gone]
+    ranked = ranked[:max(min(4, topk), topk - len(late))]
+    return ranked[:4] + late + ranked[4:]
 
 
 def _cut(ranked, topk):

@@ -17,6 +17,8 @@ class TileDict:
     score: float = 0.0            # modelled cost, lower is better
     lds_bytes: int = 0
     est_vgprs: int = 0
+    late: bool = False            # joins a pool behind its first four: the cost model does not place it among them
+    displaces: dict | None = None # (late) the tiling of the same template that leaves the pool where this one joins it
     flat_graph: object = field(default=None, repr=False)   # the StageGraph this tiles
 
     @property

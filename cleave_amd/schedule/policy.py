@@ -502,11 +502,32 @@ def attn_many_rows_candidates(low, role, factor, arch: Arch):
     # normalised keys: every workgroup of a unit normalises all of its keys again (a quarter more
     # matrix ops per step and the scaling of the scores); with many row blocks per unit a launch
     # that normalises them once into a scratch copy is cheaper
-    if "k" in (p.get("norm_eps") or {}) and not p.get("k_major") and d in (64, 128, 256) and rows >= 512:
+    kpre = "k" in (p.get("norm_eps") or {}) and not p.get("k_major") and d in (64, 128, 256) and rows >= 512
+    if kpre:
         out.append(TileDict("attn_prefill", role, dict(SHARED=1, KPRE=1), output_tile=[128, vd], rstep_map={"kv": 32},
                             n_threads=256, split_factor=factor, score=0.8 * score, lds_bytes=4 * 32 * (d + vd) * 2,
                             est_vgprs=230))
+    if role != "main":
+        return out
+    # 256 rows on two wave groups half a step apart: half the tile bytes per row, but one workgroup per compute unit
+    # and nothing beside its first loads.  Measured ahead from about 1500 keys (128 wide, us: 4096 keys 239 -> 228, 1024 keys
+    # 65.8 -> 67.2) where its workgroups keep most compute units busy, so it is proposed from half of either on; where it is ahead for certain -- keys in plenty and a workgroup for
+    # every compute unit -- instead of the other: a search times each for some milliseconds, in which the clock has not settled
+    # where the power cap holds it, and picked the slower one every other time.
+    if attn_phased_ok(p) and p["skv"] >= 768 and p["units"] * _ceil(rows, 256) >= arch.compute_units // 2:
+        out.append(TileDict("attn_prefill", role, dict(SHARED=1, PHASED=1, **({"KPRE": 1} if kpre else {})), output_tile=[256, vd],
+                            rstep_map={"kv": 64}, n_threads=512, split_factor=factor, score=score,
+                            lds_bytes=4 * 64 * (d + vd) * 2, est_vgprs=216, late=True,
+                            displaces=out[-1].tiling if d >= 128 and p["skv"] >= 2048 and p["units"] * _ceil(rows, 256) >= arch.compute_units else None))
     return out
+
+
+def attn_phased_ok(p) -> bool:
+    """Whether the two-group kernel takes an attention: four 64-key images of K and V in 160 KiB of LDS, its accumulators and
+    query rows in half a SIMD's registers, row-major keys that need no norm on the way."""
+    d, vd = p["head_dim"], p["vdim"]
+    return (d % 64 == 0 and vd % 64 == 0 and vd <= 128 and (d + vd) // 64 <= 5 and not p.get("k_major")
+            and (not (p.get("norm_eps") or {}).get("k") or d in (64, 128)))
 
 
 # ----------------------------------------------------------------------------- MLA decode

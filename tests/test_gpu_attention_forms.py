@@ -1,0 +1,96 @@
+"""GPU parity of the many-row attention kernels where a turn of their loops, a row block or a key range ends: step counts
+around the rotation of the LDS images, workgroups of one row, partly filled and empty key ranges, scores that raise every
+row's reference point on the way."""
+
+import numpy as np
+import pytest
+import torch
+
+import cleave_amd.lang as cl
+from cleave_amd import examples as C
+from cleave_amd.pipeline.direct import kernel_for
+from oracle import program_oracle
+
+pytestmark = pytest.mark.gpu
+
+LOCKSTEP, PHASED = dict(SHARED=1), dict(SHARED=1, PHASED=1)
+# outputs are averages of unit-variance values, below 4 in magnitude: a rounding of the result is 2^-9 (f16) or 2^-6 (bf16) of that
+# scale at most; the weights' own roundings average out below it
+ATOL = {"f16": 4e-3, "bf16": 2.5e-2}
+
+
+def check(fn, dtype, shapes, tiling, args=None, seed=11):
+    prog = fn.trace(getattr(cl, dtype), **shapes)
+    args = prog.random_inputs(seed=seed) if args is None else args(prog)
+    print(f"attention form {prog.name} {dtype} {shapes} {tiling}", flush=True)
+    out = kernel_for(prog, template="attn_prefill", tiling=tiling)(*args)
+    torch.cuda.synchronize()
+    want = program_oracle.evaluate(prog, list(args))[0]
+    np.testing.assert_allclose(out.float().cpu().numpy(), want, rtol=1e-2, atol=ATOL[dtype])
+
+
+@pytest.mark.parametrize("tiling", [LOCKSTEP, PHASED], ids=["lockstep", "phased"])
+@pytest.mark.parametrize("keys", [1, 31, 32, 33, 64, 65, 97, 128, 160, 193, 256, 257, 321, 449])
+def test_key_counts_around_the_rotation_of_the_images(tiling, keys):
+    check(C.gqa_decode_exact, "f16", dict(HQ=2, HKV=1, SQ=70, SKV=keys, D=128), tiling)
+    check(C.gqa_decode_exact, "bf16", dict(HQ=2, HKV=2, SQ=33, SKV=keys, D=64), tiling)
+
+
+@pytest.mark.parametrize("tiling", [LOCKSTEP, PHASED], ids=["lockstep", "phased"])
+def test_every_row_of_a_chip_full_of_workgroups(tiling):
+    """All outputs against float64 on the card: 2^-11 of the output for its rounding and as much for the weights'."""
+    shapes = dict(HQ=16, HKV=8, SQ=2048, SKV=1100, D=128)
+    q, k, v = C.gqa_decode_exact.trace(cl.f16, **shapes).random_inputs(seed=3)
+    out = kernel_for(C.gqa_decode_exact.trace(cl.f16, **shapes), template="attn_prefill", tiling=tiling)(q, k, v)
+    for h in range(16):
+        w = torch.softmax((q[h].double() @ k[h // 2].double().T) * 128 ** -0.5, dim=-1)
+        want = w @ v[h // 2].double()
+        assert ((out[h].double() - want).norm() / want.norm()).item() < 2.0 ** -10
+
+
+@pytest.mark.parametrize("rows", [1, 16, 127, 128, 129, 255, 256, 257, 513])
+def test_row_counts_around_a_workgroup(rows):
+    for tiling in (LOCKSTEP, PHASED):
+        check(C.gqa_decode_exact, "f16", dict(HQ=3, HKV=3, SQ=rows, SKV=100, D=128), tiling)
+
+
+@pytest.mark.parametrize("widths", [(64, 128), (128, 64), (192, 128), (192, 64)])
+def test_phased_widths(widths):
+    check(C.mla_prefill, "f16", dict(H=2, SQ=300, SKV=200, DK=widths[0], DV=widths[1]), PHASED)
+
+
+def test_phased_with_normalised_queries_and_keys_and_without_a_softmax():
+    check(C.qknorm, "f16", dict(HQ=8, HKV=2, SQ=100, SKV=300, D=128), dict(PHASED, KPRE=1))
+    scaled = lambda prog: [(t.float() / 8).to(t.dtype) if i == 0 else t for i, t in enumerate(prog.random_inputs(seed=29))]  # noqa: E731
+    prog = C.matmul_matmul.trace(cl.f16, H=2, SQ=300, SKV=130, D=64)
+    args = scaled(prog)
+    want = program_oracle.evaluate(prog, list(args))[0]
+    out = kernel_for(prog, template="attn_prefill", tiling=PHASED)(*args)
+    # weights are raw scores here, rounded to 11 bits, and their sums cancel
+    np.testing.assert_allclose(out.float().cpu().numpy(), want, rtol=1e-2, atol=1e-2 + np.abs(want).max() * 2.0 ** -9)
+
+
+@pytest.mark.parametrize("tiling", [LOCKSTEP, PHASED], ids=["lockstep", "phased"])
+def test_scores_that_rise_along_the_keys(tiling):
+    """Every row's reference point is raised several times on the way (weights taken again, sums and accumulators moved)."""
+    def rising(prog):
+        q, k, v = prog.random_inputs(seed=5)
+        q[..., 0] = 4.0
+        k[..., 0] = torch.linspace(0.0, 35.0 * 128 ** 0.5 / (4 * 1.4427), k.shape[1], device=k.device).to(k.dtype)
+        return q, k, v
+
+    check(C.gqa_decode_exact, "f16", dict(HQ=4, HKV=2, SQ=150, SKV=600, D=128), tiling, args=rising)
+
+
+def test_search_proposes_them_behind_the_first_four():
+    from cleave_amd.pipeline.direct import stage_graph
+    from cleave_amd.schedule import search_tiling
+
+    def forms(topk, **shapes):
+        return [c.tiling for c in search_tiling(stage_graph(C.gqa_decode_exact.trace(cl.f16, **shapes)), topk=topk)]
+
+    many = dict(HQ=32, HKV=8, SQ=4096, SKV=4096, D=128)
+    assert PHASED in forms(8, **many) and LOCKSTEP not in forms(8, **many)
+    assert PHASED not in forms(4, **many)
+    shorter = dict(many, SKV=1024)
+    assert PHASED in forms(8, **shorter) and LOCKSTEP in forms(8, **shorter)
