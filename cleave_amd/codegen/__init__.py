@@ -16,6 +16,7 @@ and outputs, then ``OutputNode_<i>``; ``python/cleave/codegen/kernel.py:576-612`
 
 from __future__ import annotations
 
+import dataclasses
 import json
 import math
 from pathlib import Path
@@ -537,6 +538,21 @@ class HipCodeGen:
             at = next(i for i, q in enumerate(params) if q.role in ("scratch", "output"))
             params.insert(at, ParamSpec("Scratch_kn", key.dtype, key.shape, "scratch"))
             unit.direct["K"] = "Scratch_kn"
+        # KEYS: the keys are dealt out to that many ranges inside an unsplit operator: the split form's two launches, partials in scratch
+        keys = int(plan.tiling.get("KEYS", 0))
+        if keys:
+            if plan.role != "main" or kpre or keys < 2 or p.get("emit_lse"):
+                raise CodegenError("KEYS shares the keys of an unsplit attention without lse out to two or more ranges")
+            total = p["units"] * rows
+            at = next(i for i, q in enumerate(params) if q.role == "output")
+            operands, scratch = dict(op), []
+            for role, extents in (("PM", (keys, total)), ("PL", (keys, total)), ("PO", (keys, total, p["vdim"]))):
+                names = [f"Partial_{role}_split", f"Partial_{role}_combine"]
+                scratch += [ParamSpec(names[0], "float32", extents, "scratch"), ParamSpec(names[1], "float32", extents, "scratch", alias=names[0])]
+                operands[role], operands[f"{role}_COMBINE"] = names
+            params[at:at] = scratch
+            plan = dataclasses.replace(plan, role="fused", operands=operands, split_factor=keys)
+            op, splits, combine = operands, keys, True
         self._attn_common(unit, plan, params, partial, combine, False, p["vdim"], p["units"] * rows, False)
         phased = int(plan.tiling.get("PHASED", 0))
         if phased:
@@ -560,7 +576,7 @@ class HipCodeGen:
         for role, macro in (("Q", "CL_ARG_Q"), ("K", "CL_ARG_K"), ("V", "CL_ARG_V")):
             unit.define(macro, "Scratch_kn" if kpre and role == "K" else op[role])
         for k, v in plan.tiling.items():
-            if k not in ("SHARED", "KPRE", "PHASED"):
+            if k not in ("SHARED", "KPRE", "PHASED", "KEYS"):
                 unit.define(f"CL_PF_{k}", int(v))
         unit.define("CL_EMIT_KPRE", kpre)
         unit.templates += ["attn_tile.hip", "attn_phased.hip" if phased else "attn_prefill_lds.hip", "attn_combine.hip"]

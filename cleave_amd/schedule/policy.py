@@ -497,6 +497,8 @@ def attn_many_rows_candidates(low, role, factor, arch: Arch):
     steps = _ceil(_ceil(p["skv"], 32), splits)
     # a workgroup-step is 32 matrix ops per wave beside as many vector ops; two workgroups per CU
     score = _waves_time(items, 2, arch) * (steps * 2200 + 9000)
+    stages = 4 if d > 192 else 3
+    lds = stages * 32 * (d + vd) * 2
     out = [TileDict("attn_prefill", role, dict(SHARED=1), output_tile=[128, vd], rstep_map={"kv": 32}, n_threads=256,
                     split_factor=factor, score=score, lds_bytes=4 * 32 * (d + vd) * 2, est_vgprs=230)]
     # normalised keys: every workgroup of a unit normalises all of its keys again (a quarter more
@@ -519,7 +521,25 @@ def attn_many_rows_candidates(low, role, factor, arch: Arch):
                             rstep_map={"kv": 64}, n_threads=512, split_factor=factor, score=score,
                             lds_bytes=4 * 64 * (d + vd) * 2, est_vgprs=216, late=True,
                             displaces=out[-1].tiling if d >= 128 and p["skv"] >= 2048 and p["units"] * _ceil(rows, 256) >= arch.compute_units else None))
+    # Too few workgroups for the chip and keys enough to share out among more: the key ranges of the split form inside one
+    # operator (partials in scratch, folded by a second launch).  Measured, us, unsplit / ranges: 56 items of 122 steps
+    # 61.5 / 31.3 (4), 16 items of 76 steps 40.3 / 17.1 (8; 20.3 with 16), 64 items of 63 steps 64 wide 26.2 / 16.8 (4); behind
+    # from about a hundred items on or a range of fewer than six steps: 80 items of 14 steps 11.5 / 16.8.
+    if not p.get("emit_lse") and not kpre:
+        for fill in (256, 128):
+            n = min(fill // items, steps // 6)
+            if n > 1 and attn_keys_scratch(p, n) <= FIXED_SCRATCH:
+                out.append(TileDict("attn_prefill", role, dict(SHARED=1, KEYS=n), output_tile=[128, vd], rstep_map={"kv": 32},
+                                    n_threads=256, split_factor=factor, score=score / n, lds_bytes=lds, est_vgprs=230, late=True))
     return out
+
+
+FIXED_SCRATCH = 64 << 20         # what a call without allocations has for scratch: plans of its own that need more are not proposed
+
+
+def attn_keys_scratch(p, n) -> int:
+    """Bytes of the partials of ``n`` key ranges: reference point, sum and unnormalised values of every row."""
+    return n * p["units"] * p["group"] * p["sq"] * (p["vdim"] + 2) * 4 + 3 * 256
 
 
 def attn_phased_ok(p) -> bool:

@@ -36,7 +36,7 @@ def test_key_counts_around_the_rotation_of_the_images(tiling, keys):
     check(C.gqa_decode_exact, "bf16", dict(HQ=2, HKV=2, SQ=33, SKV=keys, D=64), tiling)
 
 
-@pytest.mark.parametrize("tiling", [LOCKSTEP, PHASED], ids=["lockstep", "phased"])
+@pytest.mark.parametrize("tiling", [LOCKSTEP, PHASED, dict(SHARED=1, KEYS=3)], ids=["lockstep", "phased", "ranges"])
 def test_every_row_of_a_chip_full_of_workgroups(tiling):
     """All outputs against float64 on the card: 2^-11 of the output for its rounding and as much for the weights'."""
     shapes = dict(HQ=16, HKV=8, SQ=2048, SKV=1100, D=128)
@@ -65,12 +65,20 @@ def test_phased_with_normalised_queries_and_keys_and_without_a_softmax():
     prog = C.matmul_matmul.trace(cl.f16, H=2, SQ=300, SKV=130, D=64)
     args = scaled(prog)
     want = program_oracle.evaluate(prog, list(args))[0]
-    out = kernel_for(prog, template="attn_prefill", tiling=PHASED)(*args)
-    # weights are raw scores here, rounded to 11 bits, and their sums cancel
-    np.testing.assert_allclose(out.float().cpu().numpy(), want, rtol=1e-2, atol=1e-2 + np.abs(want).max() * 2.0 ** -9)
+    for tiling in (PHASED, dict(SHARED=1, KEYS=3)):
+        out = kernel_for(prog, template="attn_prefill", tiling=tiling)(*args)
+        # weights are raw scores here, rounded to 11 bits, and their sums cancel
+        np.testing.assert_allclose(out.float().cpu().numpy(), want, rtol=1e-2, atol=1e-2 + np.abs(want).max() * 2.0 ** -9)
 
 
-@pytest.mark.parametrize("tiling", [LOCKSTEP, PHASED], ids=["lockstep", "phased"])
+@pytest.mark.parametrize("keys,ranges", [(256, 2), (257, 2), (300, 4), (290, 8), (1000, 5)])
+def test_key_ranges_inside_an_operator(keys, ranges):
+    """Ranges of whole 32-key steps: equal, with a partly filled last step, shorter and empty last ones."""
+    check(C.gqa_decode_exact, "f16", dict(HQ=4, HKV=2, SQ=75, SKV=keys, D=128), dict(SHARED=1, KEYS=ranges))
+    check(C.gqa_decode_exact, "bf16", dict(HQ=2, HKV=2, SQ=130, SKV=keys, D=64), dict(SHARED=1, KEYS=ranges))
+
+
+@pytest.mark.parametrize("tiling", [LOCKSTEP, PHASED, dict(SHARED=1, KEYS=3)], ids=["lockstep", "phased", "ranges"])
 def test_scores_that_rise_along_the_keys(tiling):
     """Every row's reference point is raised several times on the way (weights taken again, sums and accumulators moved)."""
     def rising(prog):
@@ -91,6 +99,8 @@ def test_search_proposes_them_behind_the_first_four():
 
     many = dict(HQ=32, HKV=8, SQ=4096, SKV=4096, D=128)
     assert PHASED in forms(8, **many) and LOCKSTEP not in forms(8, **many)
-    assert PHASED not in forms(4, **many)
+    assert PHASED not in forms(4, **many) and not any("KEYS" in t for t in forms(8, **many))
     shorter = dict(many, SKV=1024)
     assert PHASED in forms(8, **shorter) and LOCKSTEP in forms(8, **shorter)
+    few = forms(8, HQ=32, HKV=8, SQ=193, SKV=3897, D=128)
+    assert dict(SHARED=1, KEYS=4) in few
