@@ -293,14 +293,31 @@ class HipCodeGen:
                                    "row-major A, unsplit")
         elif plan.family not in ("matmul", "swiglu", "matmul_rowsum"):
             raise CodegenError(f"the direct-to-LDS matmul template has no {plan.family} form")
+        # KS: the contraction dealt out to that many ranges inside an unsplit product: the split form's two launches, partials in
+        # scratch
+        ks = int(t.get("KS", 0))
+        if ks:
+            from ..schedule.policy import k_range
+
+            if plan.role != "main" or plan.family not in ("matmul", "swiglu") or "TAIL" in t or "KW" in t or not k_range(p["K"], ks):
+                raise CodegenError("KS shares K of an unsplit product or SwiGLU out to ranges walked in the same two or more 64-wide steps, of "
+                                   "which only the last range's last one may be short of the others'")
+            at = next(i for i, q in enumerate(params) if q.role == "output")
+            rows, cols = max(p["batch_A"], p["batch_B"]) * p["M"], p["N"] * (2 if plan.family == "swiglu" else 1)
+            params[at:at] = [ParamSpec("Partial_PACC_split", "float32", (ks, rows, cols), "scratch"),
+                             ParamSpec("Partial_PACC_combine", "float32", (ks, rows, cols), "scratch", alias="Partial_PACC_split")]
+            plan = dataclasses.replace(plan, role="fused", split_factor=ks, operands=dict(
+                plan.operands, PACC="Partial_PACC_split", PACC_COMBINE="Partial_PACC_combine"))
+            combine = True
+            unit.define("CL_K_RANGE", k_range(p["K"], ks))
         self._matmul_common(unit, plan, params, partial, combine, fused)
         tile = dict(BM=128, BN=128, BK=64, WM=2, WN=2)
-        tile.update({k: v for k, v in t.items() if k != "DMA"})
+        tile.update({k: v for k, v in t.items() if k not in ("DMA", "KS")})
         for k, v in tile.items():
             unit.define(f"CL_{k}", v)
         splits = plan.split_factor or 1
         swiglu = plan.family == "swiglu"
-        if swiglu != bool(tile.get("SWIGLU")) or (swiglu and (splits > 1 or combine)):
+        if swiglu != bool(tile.get("SWIGLU")) or (swiglu and not ks and (splits > 1 or combine)):
             raise CodegenError("SwiGLU is the SWIGLU tiling of the direct-to-LDS matmul, unsplit")
         rowsum = plan.family == "matmul_rowsum"
         if rowsum != bool(tile.get("ROWSUM")) or (rowsum and (splits > 1 or combine or p["N"] % tile["BN"])):
@@ -315,7 +332,7 @@ class HipCodeGen:
         kw = int(tile.get("KW", 0))
         unit.templates += ["gemm_tile.hip", "gemm_kwaves.hip" if kw else "gemm_phased.hip" if phased_matmul(plan.family, p, splits, tile) else "gemm_dma.hip"]
         if partial:
-            if tile["BK"] != 64 or (p["K"] % (splits * 64) and (splits > 1 or p["K"] % 8 or plan.family not in ("matmul", "rmsnorm_matmul"))):
+            if tile["BK"] != 64 or (p["K"] % (splits * 64) and not ks and (splits > 1 or p["K"] % 8 or plan.family not in ("matmul", "rmsnorm_matmul"))):
                 raise CodegenError(f"K={p['K']} is neither a multiple of splits*64={splits * 64} nor, for an unsplit product, of 8")
             if (not p["trans_B"] and p["N"] % 8) or (p["trans_A"] and p["M"] % 8) or p["K"] % 8:
                 raise CodegenError("16-byte global chunks need the minor extent of each operand to be a multiple of 8")

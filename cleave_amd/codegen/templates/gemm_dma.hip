@@ -132,9 +132,8 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
   const GdTile at = gd_tile();
   const int tile_m0 = at.m0, n0 = at.n0, half = at.half;
   const int batch = blockIdx.z / CL_SPLITS, split = blockIdx.z % CL_SPLITS;
-  constexpr int k_per_split = CL_K / CL_SPLITS;
-  const int k_begin = split * k_per_split;
-  constexpr int KT_K = (k_per_split + GD_BK - 1) / GD_BK;       // steps along K (the last one partly filled: GD_K_LEFT)
+  const int k_begin = split * CL_K_RANGE;
+  constexpr int KT_K = GD_KT;                                   // steps along K (the last one may be partly filled: GD_LEFT)
   constexpr int KT = KT_K * (CL_ROWSUM ? CL_N / CL_BN : 1);     // ... times the column tiles one workgroup walks
 #if CL_ROWSUM
   static_assert(CL_N % CL_BN == 0 && CL_SPLITS == 1 && GD_BATCH == 1, "row sums walk whole column tiles, unsplit");
@@ -277,7 +276,7 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
 #define GD_A_AT(kt) (a_base + (i64)(kt) * a_step)
 #define GD_B_AT(kt) (b_base + (i64)(kt) * b_step)
 #endif
-#define GD_LEFT_AT(kt) (GD_K_LEFT > 0 && (kt) % KT_K == KT_K - 1)
+#define GD_LEFT_AT(kt) (GD_LEFT && (kt) % KT_K == KT_K - 1)
 #define GD_ISSUE(kt, a_lds, b_lds)                                  \
   if (GD_LEFT_AT(kt)) {                                             \
     opa.issue_left(GD_A_AT(kt), GD_LDS_BYTE(a_lds), wave_byte);     \
@@ -407,14 +406,22 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
     for (int j = 0; j < GD_TN / 2; ++j) {
       const int n = n0 + bn + 16 * j + 4 * g;
       if (n >= CL_N) continue;
-      elem4 y;
       const f32x4 up = gd_acc_read(acc[i][j]), gates = gd_acc_read(acc[i][j + GD_TN / 2]);
+#if CL_SPLITS > 1
+      // (a row of partials holds both weights' products, the gate's after the bare one's)
+      float* part = CL_ARG_PACC + ((i64)split * CL_M + m) * (2 * CL_N) + n;
+      *reinterpret_cast<f32x4*>(part) = up;
+      *reinterpret_cast<f32x4*>(part + CL_N) = gates;
+      continue;
+#else
+      elem4 y;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float gate = gates[r];
         y[r] = to_elem(up[r] * gate / (1.0f + __expf(-gate)));
       }
       *reinterpret_cast<elem4*>(CL_ARG_OUT + (i64)m * CL_N + n) = y;
+#endif
     }
 #else
 #pragma unroll

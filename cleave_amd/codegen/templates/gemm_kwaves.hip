@@ -47,7 +47,7 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
   const GdTile at = gd_tile();
   const int m0 = at.m0, n0 = at.n0;
   const int batch = blockIdx.z;
-  constexpr int KT = (CL_K + GD_BK - 1) / GD_BK;       // (the last step partly filled: GD_K_LEFT)
+  constexpr int KT = GD_KT;                            // (the last step may be partly filled: GD_LEFT)
   const elem_t* A = CL_ARG_A + (i64)(batch / (GD_BATCH / CL_BATCH_A)) * CL_M * CL_K;
   const elem_t* B = CL_ARG_B + (i64)(batch / (GD_BATCH / CL_BATCH_B)) * CL_K * CL_N;
 
@@ -104,7 +104,7 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
     const int kt = t * CL_KW + wave;
     const unsigned lds = (unsigned)(area + (t & 1) * GK_STEP);
     const elem_t *pa = a_base + (i64)kt * a_step, *pb = b_base + (i64)kt * b_step;
-    if (GD_K_LEFT > 0 && kt == KT - 1) {
+    if (GD_LEFT && kt == KT - 1) {
       opa.issue_left(pa, lds, 0u);
       opb.issue_left(pb, lds + CL_BM * GD_BK * 2, 0u);
     } else {

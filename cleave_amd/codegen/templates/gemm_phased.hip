@@ -93,9 +93,8 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
   const GdTile at = gd_tile();
   const int n0 = at.n0;
   const int batch = blockIdx.z / CL_SPLITS, split = blockIdx.z % CL_SPLITS;
-  constexpr int k_per_split = CL_K / CL_SPLITS;
-  const int k_begin = split * k_per_split;
-  constexpr int KT = (k_per_split + GD_BK - 1) / GD_BK;   // (the last one partly filled: GD_K_LEFT)
+  const int k_begin = split * CL_K_RANGE;
+  constexpr int KT = GD_KT;                            // (the last one may be partly filled: GD_LEFT)
   static_assert(KT >= 2, "two stages are asked for ahead of the loop");
 
   const elem_t* A = CL_ARG_A + (i64)(batch / (GD_BATCH / CL_BATCH_A)) * CL_M * CL_K;
@@ -240,7 +239,7 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
   LOAD(opb0, pb0, stage, GP_B0) LOAD(opa0, pa, stage, GP_A0) LOAD(opb1, pb1, stage, GP_B1) LOAD(opa1, pa, stage, GP_A1) \
   pa += a_step; pb0 += b_step; pb1 += b_step;
   GP_ASK(0, GP_LOAD)
-  if constexpr (GD_K_LEFT > 0 && KT == 2) { GP_ASK(1, GP_LOAD_LEFT) } else { GP_ASK(1, GP_LOAD) }
+  if constexpr (GD_LEFT && KT == 2) { GP_ASK(1, GP_LOAD_LEFT) } else { GP_ASK(1, GP_LOAD) }
   constexpr int ahead = 3 * (la + lb);                 // loads still out when a phase's operands have landed
 #else
   // One phase: the memory part (operand reads, loads, the wait for both the reads and what the next
@@ -276,7 +275,7 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
   GP_PHASE(GP_READ_A(S, GP_A1), GP_NONE, 0, 1, p)
 
 #define GP_END(S, p, q)                                                                             \
-  if constexpr (GD_K_LEFT > 0) { GP_STEP_LAST2(S, p, q, GP_LOAD_LEFT) } else { GP_STEP_LAST2(S, p, q, GP_LOAD) } \
+  if constexpr (GD_LEFT) { GP_STEP_LAST2(S, p, q, GP_LOAD_LEFT) } else { GP_STEP_LAST2(S, p, q, GP_LOAD) } \
   GP_STEP_LAST(1 - (S), q)
 
   // Ahead of the loop, in the order the steps ask: everything of step 0, and B0, A0, B1 of step 1.
@@ -285,7 +284,7 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
     GP_LOAD(opb0, pb0, 0, GP_B0)
     GP_LOAD(opa0, pa, 0, GP_A0) GP_LOAD(opb1, pb1, 0, GP_B1)
     GP_LOAD(opa1, pa, 0, GP_A1)
-    if constexpr (GD_K_LEFT > 0 && KT == 2) {
+    if constexpr (GD_LEFT && KT == 2) {
       GP_LOAD_LEFT(opb0, pb01, 1, GP_B0) GP_LOAD_LEFT(opa0, pa1, 1, GP_A0) GP_LOAD_LEFT(opb1, pb11, 1, GP_B1)
     } else {
       GP_LOAD(opb0, pb01, 1, GP_B0) GP_LOAD(opa0, pa1, 1, GP_A0) GP_LOAD(opb1, pb11, 1, GP_B1)
@@ -303,7 +302,7 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
   if (late) gp_barrier();
 
   // (F steps ask for whole steps; with a partly filled last step, one more asks for that one)
-  constexpr int F = KT - 2 - (GD_K_LEFT > 0 && KT > 2);
+  constexpr int F = KT - 2 - (GD_LEFT && KT > 2);
   for (int pair = 0; pair < F / 2; ++pair) {
     keep_addresses();
     GP_STEP(0, fx, fy, GP_LOAD, GP_LOAD, GP_LOAD)
@@ -342,9 +341,11 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
       for (int v = 0; v < 2; ++v)
 #pragma unroll
         for (int j = 0; j < GP_TNH; ++j) {
-          const int n = n0 + GP_HN * v + ecol + 16 * j + 4 * eg;
+          // (SwiGLU: a row of partials holds both weights' products, the gate's after the bare one's)
+          const int n = n0 + (CL_SWIGLU ? 0 : GP_HN * v) + ecol + 16 * j + 4 * eg;
           if (m < CL_M && n < CL_N)
-            *reinterpret_cast<f32x4*>(CL_ARG_PACC + (((i64)split * GD_BATCH + batch) * CL_M + m) * CL_N + n) = acc[h][i][v][j];
+            *reinterpret_cast<f32x4*>(CL_ARG_PACC + (((i64)split * GD_BATCH + batch) * CL_M + m) * (CL_SWIGLU ? 2 * CL_N : CL_N) +
+                                      (CL_SWIGLU ? v * CL_N : 0) + n) = acc[h][i][v][j];
         }
 #else
       // neighbouring column fragments trade rows of lanes: 16 contiguous bytes per lane, 64 per row of C

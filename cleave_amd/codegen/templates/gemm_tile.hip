@@ -53,11 +53,21 @@ static_assert(CL_BK == 64, "K steps are 64 wide (128-byte K-minor rows)");
 static_assert((GD_TM & (GD_TM - 1)) == 0 && (GD_TN & (GD_TN - 1)) == 0, "wave tiles are powers of two");
 static_assert(CL_BM % 16 == 0 && CL_BN % 16 == 0, "tiles are multiples of 16");
 
-// A contraction that is not whole 64-wide steps (unsplit, a multiple of 8) ends on a step whose 16-byte chunks past
-// K are fetched from here instead, for both operands: the image holds zeros there and the step is one more
-// whole step.  (Such products ran on the register-staged kernel, which zeroes on the way to LDS: 2016 x 2560 x 7640
-// with a (N, K) weight 152 us there, 103 here; 2201 x 1408 x 2288 34 and 25; 100 x 64 x 4104 21.7 and 11.2.)
-#define GD_K_LEFT (CL_SPLITS == 1 ? CL_K % GD_BK : 0)
+// The contraction is dealt out to CL_SPLITS ranges of CL_K_RANGE, walked in GD_KT 64-wide steps each; the last step of a
+// range may be partly filled (and, of the last range, empty): GD_FILL columns of it lie inside, GD_FILL_LAST in the last
+// range.  That step's 16-byte chunks past the range are fetched from here instead, for both operands: the image holds
+// zeros there and the step is one more whole step.  (Unsplit products of such lengths ran on the register-staged kernel,
+// which zeroes on the way to LDS: 2016 x 2560 x 7640 with a (N, K) weight 152 us there, 103 here; 2201 x 1408 x 2288 34 and
+// 25; 100 x 64 x 4104 21.7 and 11.2.)
+#ifndef CL_K_RANGE
+#define CL_K_RANGE (CL_K / CL_SPLITS)
+#endif
+#define GD_KT ((CL_K_RANGE + GD_BK - 1) / GD_BK)
+#define GD_FILL (CL_K_RANGE - (GD_KT - 1) * GD_BK)
+#define GD_FILL_LAST (CL_K - (CL_SPLITS - 1) * CL_K_RANGE - (GD_KT - 1) * GD_BK)
+#define GD_LEFT (GD_FILL < GD_BK || GD_FILL_LAST < GD_BK)
+static_assert(GD_FILL_LAST >= 0 && GD_FILL_LAST <= GD_FILL && CL_K % 8 == 0 && CL_K_RANGE % 8 == 0,
+              "ranges are whole chunks, and only the last step of the last one is short of the others");
 static __device__ const u32x4 gd_zeros = {0u, 0u, 0u, 0u};
 
 typedef __attribute__((address_space(3))) void gd_lds_void;
@@ -166,7 +176,8 @@ struct GdOperand {
       const int lane = threadIdx.x & 63;
       constexpr int RPU = 64 / CPR > 0 ? 64 / CPR : 1;
       const int k = KMAJOR ? u * RPU + lane / CPR : 8 * ((lane & 7) ^ gd_swz_kmin(lane >> 3));
-      const char* src = k < GD_K_LEFT ? reinterpret_cast<const char*>(base) + goff[i] : reinterpret_cast<const char*>(&gd_zeros);
+      const int left = (int)(blockIdx.z % CL_SPLITS) != CL_SPLITS - 1 ? GD_FILL : GD_FILL_LAST;
+      const char* src = k < left ? reinterpret_cast<const char*>(base) + goff[i] : reinterpret_cast<const char*>(&gd_zeros);
       asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
                    :: "v"(src), "s"(lds_byte + i * GD_WAVES * 1024 + wave_byte)
                    : "memory", "m0");
@@ -174,7 +185,7 @@ struct GdOperand {
   }
   // ... of the step `base` starts, or of the partly filled last one
   CL_METHOD void issue_unit_of(int i, const elem_t* base, unsigned lds_byte, unsigned wave_byte, bool left) const {
-    if (GD_K_LEFT > 0 && left) issue_unit_left(i, base, lds_byte, wave_byte);
+    if (GD_LEFT && left) issue_unit_left(i, base, lds_byte, wave_byte);
     else issue_unit(i, base, lds_byte, wave_byte);
   }
   CL_METHOD void issue_left(const elem_t* base, unsigned lds_byte, unsigned wave_byte) const {

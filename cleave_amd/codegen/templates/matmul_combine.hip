@@ -8,8 +8,12 @@
 // the input of the reference's second product is) and LB (CL_R, N).  A workgroup's 256 threads
 // share one row of C (the emitter picks the column count so that N / cols is a multiple of
 // 256), so the row of D is summed once per workgroup into LDS.
+// CL_SWIGLU: a partial row holds the products of the bare weight and, behind them, of the gate weight: C = up * silu(gate).
 #ifndef CL_LORA
 #define CL_LORA 0
+#endif
+#ifndef CL_SWIGLU
+#define CL_SWIGLU 0
 #endif
 #if CL_SPLITS > 1 && CL_EMIT_COMBINE
 extern "C" __global__ void __launch_bounds__(256)
@@ -39,18 +43,27 @@ CL_COMBINE_NAME(CL_COMBINE_PARAMS) {
   float a[CL_COMBINE_COLS];
 #pragma unroll
   for (int r = 0; r < CL_COMBINE_COLS; ++r) a[r] = 0.f;
+#if CL_SWIGLU
+  float gate[CL_COMBINE_COLS];
+#pragma unroll
+  for (int r = 0; r < CL_COMBINE_COLS; ++r) gate[r] = 0.f;
+#endif
 #if CL_NORM
   float tot = 0.f;
 #endif
 #pragma unroll
   for (int s = 0; s < CL_SPLITS; ++s) {
-    const float* p = CL_CARG_PACC + ((i64)s * rows + row) * CL_N + n;
+    const float* p = CL_CARG_PACC + ((i64)s * rows + row) * (CL_SWIGLU ? 2 * CL_N : CL_N) + n;
 #if CL_COMBINE_COLS == 1
     a[0] += p[0];
 #else
     const mc_f32 v = *reinterpret_cast<const mc_f32*>(p);
 #pragma unroll
     for (int r = 0; r < CL_COMBINE_COLS; ++r) a[r] += v[r];
+#endif
+#if CL_SWIGLU
+#pragma unroll
+    for (int r = 0; r < CL_COMBINE_COLS; ++r) gate[r] += p[CL_N + r];
 #endif
 #if CL_NORM
     tot += CL_CARG_PSS[(i64)s * rows + row];
@@ -60,6 +73,10 @@ CL_COMBINE_NAME(CL_COMBINE_PARAMS) {
   const float rs = fast_rsqrt(tot * (1.0f / CL_K) + CL_EPS);
 #else
   const float rs = 1.0f;
+#endif
+#if CL_SWIGLU
+#pragma unroll
+  for (int r = 0; r < CL_COMBINE_COLS; ++r) a[r] = a[r] * gate[r] / (1.0f + __expf(-gate[r]));
 #endif
 #if CL_LORA
   for (int rr = 0; rr < CL_R; ++rr) {

@@ -217,10 +217,56 @@ def gemm_dma_candidates(low, role, factor, arch: Arch, twin_of=None):
         for c in kwaves_candidates(low, role, factor, arch):
             c.score = max([c.score] + [math.nextafter(s, math.inf) for s in second])
             out.append(c)
+    if not twin_of and low.family == "matmul" and splits == 1:
+        out += k_range_candidates(low, role, arch)
     if K % 64:
         # (under the name of the template that takes such lengths; DMA picks its direct-to-LDS form)
         for c in out:
             c.template, c.tiling = "gemm", dict(c.tiling, DMA=1)
+    return out
+
+
+def k_range(K, n) -> int:
+    """The extent of ``n`` ranges that K is dealt out to inside an unsplit product, or 0 where it cannot be: whole 64-wide steps
+    if the last range is then less than a step short, else whole 16-byte chunks.  Every range is walked in the same number of
+    steps, two or more, and the kernels fetch zeros for the rest of a range's last step only."""
+    if n < 2 or K % 8:
+        return 0
+    for unit in (64, 8):
+        extent = _ceil(_ceil(K, unit), n) * unit
+        steps = _ceil(extent, 64)
+        if steps >= 2 and K - (n - 1) * extent - (steps - 1) * 64 >= 0:
+            return extent
+    return 0
+
+
+def k_range_candidates(low, role, arch: Arch, twin=False):
+    """Products of too few tiles for the chip and a long contraction: K dealt out to ranges inside an unsplit operator, f32
+    partials in scratch folded by a second launch (SwiGLU's gate there too).  Two tilings, with as many ranges as give
+    every compute unit one 128 x 256 tile (two of 128 x 128, at most five ranges) and a range eight steps.  Measured, us, best unsplit /
+    ranges: 655 x 3264 x 6912 53.1 / 41.6, 3000 x 1000 x 8000 67.0 / 53.1, 290 x 1968 x 5056 32.6 / 18.8, SwiGLU 156 x 3968 x
+    8064 89.8 / 44.3 and 700 x 1024 x 4096 32.4 / 23.5; behind where the contraction is short (906 x 1152 x 1024 9.7 / 13.1)
+    or the tiles fill the chip (SwiGLU 507 x 7040 x 2240 32.3 / 49.7)."""
+    p = low.problem
+    M, N, K = p["M"], p["N"], p["K"]
+    width = 2 * N if twin else N
+    batch = max(p["batch_A"], p["batch_B"])
+    steps = _ceil(K, 64)
+    if role != "main" or steps < 24 or K % 8 or (not p["trans_B"] and N % 8) or (p["trans_A"] and M % 8):
+        return []
+    out = []
+    for (bm, bn), fill in (((128, 256), 1), ((128, 128), 2)):
+        if twin and N % (bn // 2) or not twin and bn > 2 * N:
+            continue
+        blocks = _ceil(M, bm) * _ceil(width, bn) * batch
+        most = min(fill * arch.compute_units // blocks, 8 if fill == 1 else 5, steps // 8)
+        fits = [n for n in range(2, most + 1) if k_range(K, n) and 4 * n * batch * M * width + 512 <= FIXED_SCRATCH]
+        # (ranges that start on a 128-byte line ahead of one range more)
+        n = max((n for n in fits[-2:] if k_range(K, n) % 64 == 0), default=fits[-1] if fits else 0)
+        if n and _ceil(M, 128) * _ceil(width, 256) * batch <= arch.compute_units // 2:
+            tiling = dict(BM=bm, BN=bn, BK=64, WM=2, WN=4, KS=n, **({"SWIGLU": 1} if twin else {}))
+            out.append(TileDict("gemm_dma", role, tiling, output_tile=[bm, bn // 2 if twin else bn], rstep_map={"k": 64}, n_threads=512,
+                                score=float(steps // n), lds_bytes=gemm_lds_bytes(bm, bn, 64), est_vgprs=200, late=True))
     return out
 
 
@@ -282,7 +328,7 @@ def swiglu_candidates(low, role, factor, arch: Arch):
         c.tiling = dict(t, SWIGLU=1)
         c.output_tile = [t["BM"], t["BN"] // 2]
         out.append(c)
-    return out
+    return out + (k_range_candidates(low, role, arch, twin=True) if out else [])
 
 
 def rowsum_candidates(low, role, factor, arch: Arch):
