@@ -789,7 +789,8 @@ class HipCodeGen:
                                    "latent width in multiples of 128, a rope width of an odd number of 64s, and four images "
                                    "within 160 KiB of LDS")
             unit.templates += ["mla_decode_duo.hip", "attn_combine.hip"]
-            unit.launch(ENTRY, (f"ceildiv({p['dim_names']['total_q']}, 4) + batch", p["heads"] // 16, 1), 512, 0, self._partial_args)
+            # (the item axis is padded to a multiple of 8: the kernel deals runs of items out to the XCDs)
+            unit.launch(ENTRY, (f"ceildiv(ceildiv({p['dim_names']['total_q']}, 4) + batch, 8) * 8", p["heads"] // 16, 1), 512, 0, self._partial_args)
             return
         unit.templates += ["mla_paged_decode.hip", "attn_combine.hip"]
         if partial:
