@@ -374,7 +374,7 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
     l += lane_xor(l, lane_e, 32);
     const float inv = 1.0f / fmaxf(l, 1.0e-30f);
 #endif
-    pl_store_row<AP_FB>(CL_ARG_OUT + row_of(rt, c_e) * CL_VDIM, acc[rt], inv, g_e);
+    pl_store_row<AP_FB, true>(CL_ARG_OUT + row_of(rt, c_e) * CL_VDIM, acc[rt], inv, g_e);
   }
   if (!late) ap_barrier();                               // (the late group's last one)
 }

@@ -724,7 +724,7 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
       (void)inv;
     }
 #else
-    pl_store_row<PL_FB>(CL_ARG_OUT + orow * CL_VDIM, acc[rt], inv, g_e);
+    pl_store_row<PL_FB, CL_DENSE>(CL_ARG_OUT + orow * CL_VDIM, acc[rt], inv, g_e);
 #if CL_EMIT_LSE
     if (g_e == 0) CL_ARG_LSE[orow] = l > 0.f ? m_run[rt] + fast_log2(l) : CL_NEG_INF;
 #endif

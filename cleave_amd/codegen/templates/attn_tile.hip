@@ -64,7 +64,10 @@ CL_DEVICE float pl_max_over_groups(float x) {
 // One row tile's results: a lane holds features 16 fb + 4 g .. + 3 of its row for every block fb.  Lanes g and g ^ 1 trade
 // halves of a pair of blocks (one row swap per register), so that each stores 16 contiguous bytes: even g the 8 features
 // from 4 g of the even block, odd g those from 4 (g - 1) of the odd one.  `row`: the row's first feature.
-template <int FB>
+// STREAM: past the caches' retention (64-byte pieces of rows that nothing in the kernel reads again: dense, 32 heads x 4096
+// rows at 128 wide, us, 128 keys 23.2 -> 20.0, 512 keys 41.3 -> 38.6, 4096 keys 253 -> 250; packed prompts, whose rows of all heads
+// lie together, 131.8 -> 134.6: not there).
+template <int FB, bool STREAM>
 CL_DEVICE void pl_store_row(elem_t* row, const f32x4 (&acc)[FB], float inv, int g) {
   elem_t* dst = row + 16 * (g & 1) + 4 * (g & 2);
 #pragma unroll
@@ -79,6 +82,8 @@ CL_DEVICE void pl_store_row(elem_t* row, const f32x4 (&acc)[FB], float inv, int 
     unsigned a0 = a[0], a1 = a[1], b0 = b[0], b1 = b[1];
     pl_swap_rows16(a0, b0);
     pl_swap_rows16(a1, b1);
-    *reinterpret_cast<u32x4*>(dst + 32 * fp) = (u32x4){a0, a1, b0, b1};
+    u32x4* at = reinterpret_cast<u32x4*>(dst + 32 * fp);
+    if constexpr (STREAM) __builtin_nontemporal_store((u32x4){a0, a1, b0, b1}, at);
+    else *at = (u32x4){a0, a1, b0, b1};
   }
 }
