@@ -15,8 +15,12 @@
 // allocator hands it out again in stream order only).
 #include <Python.h>
 
+#include <ATen/Context.h>
+#include <ATen/EmptyTensor.h>
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
+#include <ATen/record_function.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/VirtualGuardImpl.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -153,6 +157,23 @@ bool plain(const at::Tensor& t) {
   return t.defined() && !t.key_set().has_any(others) && t.has_storage();
 }
 
+// Whether an allocation may go to torch's allocator without passing its dispatcher: nobody listens there -- no mode, transform
+// or tracer on this thread, no profiler -- and fresh memory needs no fill.  A call of a paged decode operator (two outputs)
+// takes 5.6 us of host time instead of 6.2 with this and its split / single rule in plain integers, a small matmul 4.0 instead of
+// 4.2; both are what such calls are bound by.
+bool dispatcher_idle() {
+  const auto included = c10::impl::tls_local_dispatch_key_set().included_ - c10::default_included_set;
+  return included.empty() && !at::hasCallbacks() &&
+         !(at::globalContext().deterministicAlgorithms() && at::globalContext().deterministicFillUninitializedMemory());
+}
+
+// The allocator behind torch's device tensors, one for the life of the process: asked of a tensor, because the one registered
+// for the device type makes storage of the type's HIP twin.
+c10::Allocator* device_allocator(int device) {
+  static c10::Allocator* const its = at::empty({1}, at::TensorOptions().device(at::kCUDA, device).dtype(at::kByte)).storage().allocator();
+  return its;
+}
+
 PyObject* call_plain(PyObject* self_, PyObject* const* argv, size_t nargsf, PyObject* kwnames) {
   Plan* self = reinterpret_cast<Plan*>(self_);
   const size_t n = PyVectorcall_NARGS(nargsf);
@@ -237,6 +258,13 @@ PyObject* call_plain(PyObject* self_, PyObject* const* argv, size_t nargsf, PyOb
 
   if (c10::impl::VirtualGuardImpl(c10::DeviceType::CUDA).getDevice().index() != device) MISS();
   const auto on_device = at::TensorOptions().device(at::kCUDA, device);
+  const bool direct = dispatcher_idle() && device_allocator(device);
+  c10::Allocator* const allocator = direct ? device_allocator(device) : nullptr;
+  constexpr c10::DispatchKeySet cuda_keys(c10::DispatchKey::CUDA);
+  auto fresh = [&](at::IntArrayRef shape, at::ScalarType dtype) -> at::Tensor {
+    if (!direct) return at::empty(shape, on_device.dtype(dtype));
+    return at::Tensor(at::detail::empty_generic(shape, allocator, cuda_keys, dtype, std::nullopt));
+  };
   at::Tensor outs[kMaxOuts];
   void* out_ptr[kMaxOuts];
   for (size_t i = 0; i < self->outs->size(); ++i) {
@@ -244,7 +272,7 @@ PyObject* call_plain(PyObject* self_, PyObject* const* argv, size_t nargsf, PyOb
     int64_t shape[8];
     for (size_t k = 0; k < o.shape.size(); ++k)
       if (!evaluate(o.shape[k], dims, &shape[k]) || shape[k] < 0) MISS();
-    outs[i] = at::empty(at::IntArrayRef(shape, o.shape.size()), on_device.dtype(o.dtype));
+    outs[i] = fresh(at::IntArrayRef(shape, o.shape.size()), o.dtype);
     out_ptr[i] = outs[i].data_ptr();
   }
   at::Tensor scratch;
@@ -257,7 +285,7 @@ PyObject* call_plain(PyObject* self_, PyObject* const* argv, size_t nargsf, PyOb
       at_byte[i] = total;
       total += (v + 255) / 256 * 256;
     }
-    scratch = at::empty({total}, on_device.dtype(at::kByte));
+    scratch = fresh({total}, at::kByte);
     for (size_t i = 0; i < self->temps->size(); ++i) temp_ptr[i] = static_cast<char*>(scratch.data_ptr()) + at_byte[i];
   }
   if (!empty) {

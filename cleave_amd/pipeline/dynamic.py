@@ -474,18 +474,20 @@ class PagedKernel(Kernel):
         """``"split"`` or ``"single"`` for a batch of ``requests`` requests whose longest spans ``longest``
         page-table units, by the calibrated rule (kv tiles of the longest request against ``min_tiles``, or
         ``lone_tiles`` where the requests are too few to fill the chip)."""
-        if not self.dispatch or set(self.dispatch_sources) < {"split", "single"}:
+        rule, sources = self.dispatch, self.dispatch_sources
+        if not rule or "split" not in sources or "single" not in sources:
             raise CleaveError(f"{self.name}: no split / single calibration was made (or saved) for this operator")
-        tiles = math.ceil(int(longest) * int(self.dispatch["page_size"]) / int(self.dispatch["kv_tile"]))
-        few = requests is not None and requests < int(self.dispatch.get("few_requests", 0))
-        return "split" if tiles >= int(self.dispatch["lone_tiles" if few else "min_tiles"]) else "single"
+        few = requests is not None and requests < rule.get("few_requests", 0)
+        # (tiles of the longest request, rounded up, against a whole number of them)
+        return "split" if int(longest) * rule["page_size"] > (rule["lone_tiles" if few else "min_tiles"] - 1) * rule["kv_tile"] else "single"
 
     def token_role(self, tokens: int):
         """``"few"`` or ``"many"`` for a call with ``tokens`` packed query tokens, by the rule
         calibrated for a prefill layer; None when no such rule was made (or saved)."""
-        if not self.dispatch or self.dispatch.get("by") != "query_tokens" or set(self.dispatch_sources) < {"few", "many"}:
+        rule, sources = self.dispatch, self.dispatch_sources
+        if not rule or rule.get("by") != "query_tokens" or "few" not in sources or "many" not in sources:
             return None
-        return "few" if int(tokens) <= int(self.dispatch["max_tokens"]) else "many"
+        return "few" if int(tokens) <= rule["max_tokens"] else "many"
 
     def _dispatched(self, longest: int, role=None):
         role = role or self.dispatch_role(longest)
