@@ -59,7 +59,7 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
   const int lin = (launch % 8) * (gx * (int)gridDim.y / 8) + launch / 8;
   const int unit = lin / gx, lo = (lin % gx) * AP_ROWS;
   if (lo >= CL_ROWS) return;
-  // row of the unit that lane `col` of row tile rt works on (rows past the last repeat it: they store the same values)
+  // row of the unit that lane `col` of row tile rt works on (rows past the last repeat it and are not stored)
   auto row_of = [&](int rt, int col) __attribute__((always_inline)) {
     const int m = lo + 32 * wave + 16 * rt + col;
     return (i64)unit * CL_ROWS + (m < CL_ROWS ? m : CL_ROWS - 1);
@@ -374,7 +374,8 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
     l += lane_xor(l, lane_e, 32);
     const float inv = 1.0f / fmaxf(l, 1.0e-30f);
 #endif
-    pl_store_row<AP_FB, true>(CL_ARG_OUT + row_of(rt, c_e) * CL_VDIM, acc[rt], inv, g_e);
+    if (lo + 32 * wave + 16 * rt + c_e < CL_ROWS)        // (all lanes of a row or none)
+      pl_store_row<AP_FB, true>(CL_ARG_OUT + row_of(rt, c_e) * CL_VDIM, acc[rt], inv, g_e);
   }
   if (!late) ap_barrier();                               // (the late group's last one)
 }
