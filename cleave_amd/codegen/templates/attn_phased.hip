@@ -229,11 +229,11 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
         const float p = AP_S(rt, i) * sm_scale;
 #else
         const float p = fast_exp2(__builtin_fmaf(AP_S(rt, i), scale2, -m_run[rt]));
-        sum += p;
+        if (!PL_ROUNDED_SUMS) sum += p;
 #endif
         pf[rt][i >> 3][i & 7] = to_elem(p);
       }
-      psum[rt] = sum;
+      psum[rt] = PL_ROUNDED_SUMS ? pl_sum_weights(pf[rt][1], pl_sum_weights(pf[rt][0], 0.f)) : sum;
     };
     auto settle = [&](int rt) __attribute__((always_inline)) {
 #if !CL_LINEAR

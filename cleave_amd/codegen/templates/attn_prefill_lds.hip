@@ -13,8 +13,8 @@
 // over them so that LDS addresses are immediates.  The softmax is the exact online one, slimmed for
 // the vector unit: steps below every row's causal limit run a body without mask arithmetic, scale
 // and reference point are one multiply-add per score, a row's maximum is taken only where its weights
-// outgrow their reference point (seen from their sum), and one sum of the unrounded weights serves
-// the normalisation and the lse.
+// outgrow their reference point (seen from their sum), and one sum of the weights serves the normalisation
+// and the lse (of 64-wide heads without an lse the rounded weights', see PL_ROUNDED_SUMS).
 //
 // What bounds it: the loop runs at the power cap (the clock falls to 1.9 GHz and time follows the work done, not the
 // stalls).  Dense, 32 heads x 4096 x 4096 at 128 wide: 248 -> 239 us when the maxima (ten vector instructions of a
@@ -571,11 +571,11 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
         const float p = st[rt][i >> 2][i & 3] * sm_scale;
 #else
         const float p = fast_exp2(__builtin_fmaf(st[rt][i >> 2][i & 3], scale2, -m_run[rt]));
-        sum += p;
+        if (!PL_ROUNDED_SUMS) sum += p;
 #endif
         pf[rt][i] = to_elem(p);
       }
-      psum[rt] = sum;
+      psum[rt] = PL_ROUNDED_SUMS ? pl_sum_weights(pf[rt], 0.f) : sum;
     };
     // The weights are taken against the row's reference first and looked at afterwards: where a lane's eight sum to more
     // than 2^8 (none passes 2^8 then), the row's reference is raised to its running maximum and the weights are taken

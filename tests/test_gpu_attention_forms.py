@@ -90,6 +90,18 @@ def test_scores_that_rise_along_the_keys(tiling):
     check(C.gqa_decode_exact, "f16", dict(HQ=4, HKV=2, SQ=150, SKV=600, D=128), tiling, args=rising)
 
 
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("tiling", [LOCKSTEP, PHASED, dict(SHARED=1, KEYS=3)], ids=["lockstep", "phased", "ranges"])
+def test_a_value_that_is_the_same_for_every_key_comes_back_exactly(tiling, dtype):
+    """64-wide heads add the weights up as they multiply them, rounded: what is left of a constant value's error is that of two
+    sums of 600 positive terms in 32 bits, far below the 2^-12 and 2^-9 that would reach the next 16-bit number."""
+    prog = C.gqa_decode_exact.trace(getattr(cl, dtype), HQ=4, HKV=2, SQ=150, SKV=600, D=64)
+    q, k, v = prog.random_inputs(seed=21)
+    v[:] = (1.9 - torch.arange(64, device=v.device) / 128).to(v.dtype)
+    out = kernel_for(prog, template="attn_prefill", tiling=tiling)((q.float() * 4).to(q.dtype), k, v)
+    assert torch.equal(out, v[:1, :1].expand_as(out))
+
+
 def test_search_proposes_them_behind_the_first_four():
     from cleave_amd.pipeline.direct import stage_graph
     from cleave_amd.schedule import search_tiling
