@@ -367,7 +367,7 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
 #endif
   }
 
-  float m_run[2] = {CL_NEG_BIG, CL_NEG_BIG};   // running max of the scaled scores (log2 domain), uniform over g
+  float m_run[2] = {CL_NEG_BIG, CL_NEG_BIG};   // reference point of a row's weights (log2 domain, the row's running max or up to 8 below it), uniform over g
   float l_run[2] = {0.f, 0.f};                 // this lane's share of the sum of the weights
   f32x4 acc[2][PL_FB];                         // acc[rt][fb][r] = O[row][16 fb + 4 g + r]
 #pragma unroll
@@ -578,13 +578,14 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
       psum[rt] = PL_ROUNDED_SUMS ? pl_sum_weights(pf[rt], 0.f) : sum;
     };
     // The weights are taken against the row's reference first and looked at afterwards: where a lane's eight sum to more
-    // than 2^8 (none passes 2^8 then), the row's reference is raised to its running maximum and the weights are taken
-    // again.  Cold, so that maxima cost the other steps nothing.
+    // than 2^8 (none passes 2^8 then), the row's reference is raised to the step's maximum and the weights are taken
+    // again.  Only that row's: a row's bits do not depend on the rows beside it in the wave.  Cold, so that maxima cost the
+    // other steps nothing.
     auto settle = [&](int rt) __attribute__((always_inline)) {
 #if !CL_LINEAR
       if (__builtin_expect(__builtin_amdgcn_ballot_w64(psum[rt] > 256.0f) != 0, 0)) {
         const float mx = pl_max_over_groups(step_max(st[rt])) * scale2;
-        const float m_new = mx > m_run[rt] ? mx : m_run[rt];
+        const float m_new = pl_max_over_groups(psum[rt]) > 256.0f && mx > m_run[rt] ? mx : m_run[rt];
         const float alpha = fast_exp2(m_run[rt] - m_new);
         m_run[rt] = m_new;
         l_run[rt] *= alpha;

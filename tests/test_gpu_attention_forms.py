@@ -102,6 +102,23 @@ def test_a_value_that_is_the_same_for_every_key_comes_back_exactly(tiling, dtype
     assert torch.equal(out, v[:1, :1].expand_as(out))
 
 
+@pytest.mark.parametrize("d,tiling", [(d, t) for t in (LOCKSTEP, PHASED, dict(SHARED=1, KEYS=3)) for d in (64, 128, 256)
+                                      if d < 256 or "PHASED" not in t])
+def test_a_row_does_not_depend_on_the_rows_beside_it(d, tiling):
+    """Every other row's scores rise along the keys, so that its reference point is raised on the way; the rows between them keep
+    their bits whether that happens beside them or not."""
+    prog = C.gqa_decode_exact.trace(cl.f16, HQ=2, HKV=2, SQ=290, SKV=700, D=d)
+    q, k, v = prog.random_inputs(seed=8)
+    q = (q.float() * 2).to(q.dtype)
+    q[..., 0] = 0.0
+    k[..., 0] = torch.linspace(0.0, 40.0 * d ** 0.5 / (4 * 1.4427), k.shape[1], device=k.device).to(k.dtype)
+    kernel = kernel_for(prog, template="attn_prefill", tiling=tiling)
+    calm = kernel(q, k, v)
+    q[:, 1::2, 0] = 4.0
+    beside = kernel(q, k, v)
+    assert torch.equal(calm[:, ::2], beside[:, ::2]) and not torch.equal(calm[:, 1::2], beside[:, 1::2])
+
+
 def test_search_proposes_them_behind_the_first_four():
     from cleave_amd.pipeline.direct import stage_graph
     from cleave_amd.schedule import search_tiling
