@@ -196,8 +196,8 @@ def gemm_dma_candidates(low, role, factor, arch: Arch, twin_of=None):
                             split_factor=factor, score=place, lds_bytes=lds, est_vgprs=vgprs))
         # Three LDS stages where three images fit beside as many workgroups per compute unit as two
         # allow: the loads of a step asked for two steps ahead and spread over the whole step
-        # (256 x 128 tiles on 4096 x 14336 x 4096: 426 us against 526).
-        if ((twin_of or not phased) and 3 * (bm + bn) * 128 * per_cu <= arch.lds_bytes and units_a % (wm * wn) == 0 and units_b % (wm * wn) == 0
+        # (256 x 128 tiles on 4096 x 14336 x 4096: 426 us against 526).  The row-sum walk has no such form.
+        if (twin_of != "matmul_rowsum" and (twin_of or not phased) and 3 * (bm + bn) * 128 * per_cu <= arch.lds_bytes and units_a % (wm * wn) == 0 and units_b % (wm * wn) == 0
                 and not post_norm):
             out.append(TileDict("gemm_dma", role, dict(tiling, STAGES=3), output_tile=[bm, bn], rstep_map={"k": 64},
                                 n_threads=threads, split_factor=factor, score=0.85 * score, lds_bytes=3 * lds // 2,

@@ -471,3 +471,10 @@ def test_score_wave_mla_kernels_are_offered_where_they_compile(ckv, kpe, fits):
         else:
             with pytest.raises(CodegenError, match="latent width"):
                 make()
+
+
+def test_row_sum_searches_propose_only_what_the_emitter_takes():
+    """The row-sum walk of the direct-to-LDS matmul has no three-stage form."""
+    for shapes in (dict(M=558, N=1024, K=2944), dict(M=4096, N=4096, K=64), dict(M=4000, N=7168, K=2048)):
+        for cand in search_tiling(stage_graph(C.matmul_rowsum.trace(cl.f16, **shapes)), topk=1000):
+            HipCodeGen().gen(apply_tiling(cand))
