@@ -575,7 +575,7 @@ class HipCodeGen:
         if phased:
             from ..schedule.policy import attn_phased_ok
 
-            if splits > 1 or ("k" in norm and not kpre) or not attn_phased_ok(p):
+            if splits > 1 or not attn_phased_ok(p, kpre):
                 raise CodegenError("the phased attention kernel: unsplit, row-major keys without a norm of their own (or KPRE), "
                                    "values up to 128 wide, key and value widths of at most five 64-feature panels together")
         for k, v in (("CL_DENSE", 1), ("CL_RAGGED", 1), ("CL_HEAD_DIM", d), ("CL_KV_HEADS", 1), ("CL_Q_HEADS", 1),

@@ -562,7 +562,7 @@ def attn_many_rows_candidates(low, role, factor, arch: Arch):
     # 65.8 -> 67.2) where its workgroups keep most compute units busy, so it is proposed from half of either on; where it is ahead for certain -- keys in plenty and a workgroup for
     # every compute unit -- instead of the other: a search times each for some milliseconds, in which the clock has not settled
     # where the power cap holds it, and picked the slower one every other time.
-    if attn_phased_ok(p) and p["skv"] >= 768 and p["units"] * _ceil(rows, 256) >= arch.compute_units // 2:
+    if attn_phased_ok(p, kpre) and p["skv"] >= 768 and p["units"] * _ceil(rows, 256) >= arch.compute_units // 2:
         out.append(TileDict("attn_prefill", role, dict(SHARED=1, PHASED=1, **({"KPRE": 1} if kpre else {})), output_tile=[256, vd],
                             rstep_map={"kv": 64}, n_threads=512, split_factor=factor, score=score,
                             lds_bytes=4 * 64 * (d + vd) * 2, est_vgprs=216, late=True,
@@ -588,12 +588,12 @@ def attn_keys_scratch(p, n) -> int:
     return n * p["units"] * p["group"] * p["sq"] * (p["vdim"] + 2) * 4 + 3 * 256
 
 
-def attn_phased_ok(p) -> bool:
+def attn_phased_ok(p, kpre) -> bool:
     """Whether the two-group kernel takes an attention: four 64-key images of K and V in 160 KiB of LDS, its accumulators and
-    query rows in half a SIMD's registers, row-major keys that need no norm on the way."""
+    query rows in half a SIMD's registers, row-major keys that need no norm on the way (``kpre``: a launch ahead normalises them)."""
     d, vd = p["head_dim"], p["vdim"]
     return (d % 64 == 0 and vd % 64 == 0 and vd <= 128 and (d + vd) // 64 <= 5 and not p.get("k_major")
-            and (not (p.get("norm_eps") or {}).get("k") or d in (64, 128)))
+            and (kpre or "k" not in (p.get("norm_eps") or {})))
 
 
 # ----------------------------------------------------------------------------- MLA decode

@@ -478,3 +478,53 @@ def test_row_sum_searches_propose_only_what_the_emitter_takes():
     for shapes in (dict(M=558, N=1024, K=2944), dict(M=4096, N=4096, K=64), dict(M=4000, N=7168, K=2048)):
         for cand in search_tiling(stage_graph(C.matmul_rowsum.trace(cl.f16, **shapes)), topk=1000):
             HipCodeGen().gen(apply_tiling(cand))
+
+
+def test_every_candidate_of_a_search_emits():
+    """Drawn sizes of every dense family, and QK-norm attention of few rows per unit and many units (the two-group kernel takes its
+    keys only normalised ahead, which is not done for so few rows): what the search proposes, the emitter takes."""
+    import math
+    import random
+
+    rng = random.Random(5)
+
+    def size(lo, hi, step=1):
+        return max(step, round(math.exp(rng.uniform(math.log(lo), math.log(hi))) / step) * step)
+
+    def draw(op):
+        if op in (C.matmul, C.matmul_nt, C.rmsnorm_matmul, C.swiglu, C.matmul_rowsum):
+            return dict(M=size(1, 9000), N=size(8, 9000, rng.choice([8, 64])), K=size(8, 9000, rng.choice([8, 64])))
+        if op is C.batched_matmul:
+            return dict(BX=2, BW=rng.choice([1, 2]), M=size(1, 2000), N=size(8, 2000, 8), K=size(8, 9000, 8))
+        if op is C.lora:
+            return dict(M=size(1, 64), N=size(256, 4096, 256), K=size(32, 4096, 32), R=rng.choice([8, 16, 64]))
+        if op is C.matmul_matmul_2d:
+            return dict(M=size(1, 5000), N=size(32, 5000, 32), K=rng.choice([64, 128, 192, 256]))
+        if op is C.mla_decode:
+            return dict(B=size(1, 32), H=rng.choice([16, 64, 128]), D=512, PE=64, SKV=size(1, 8192))
+        d, units, keys = rng.choice([64, 128, 192, 256]), size(1, 256), size(1, 5000)
+        if op is C.mla_prefill:
+            return dict(H=units, SQ=size(1, 3000), SKV=keys, DK=d, DV=rng.choice([64, 128, 192, 256]))
+        if op is C.matmul_matmul:
+            return dict(H=units, SQ=size(1, 3000), SKV=keys, D=d)
+        return dict(HQ=units * rng.choice([1, 4, 8]), HKV=units, SQ=size(1, 3000), SKV=keys, D=d)
+
+    ops = [C.matmul, C.matmul_nt, C.rmsnorm_matmul, C.swiglu, C.matmul_rowsum, C.batched_matmul, C.lora, C.matmul_matmul_2d, C.mla_decode,
+           C.mla_prefill, C.matmul_matmul, C.gqa_decode_exact, C.qknorm]
+    cases = [(op, draw(op)) for op in ops for _ in range(20)]
+    cases += [(C.qknorm, dict(HQ=units * group, HKV=units, SQ=rng.randint(1, 511 // group), SKV=keys, D=d))
+              for units in (128, 256) for group in (1, 2) for keys in (768, 2048, 4096) for d in (64, 128)]
+    cases += [(C.qknorm, dict(HQ=128, HKV=128, SQ=400, SKV=2048, D=128)), (C.qknorm, dict(HQ=512, HKV=256, SQ=150, SKV=2048, D=128))]
+    emitted = 0
+    for op, shapes in cases:
+        graph = stage_graph(op.trace(rng.choice([cl.f16, cl.bf16]), **shapes))
+        for topk in (4, 8, 32):
+            try:
+                candidates = search_tiling(graph, topk=topk)
+            except ScheduleRejected:
+                break
+            assert candidates, (op, shapes, topk)
+            for cand in candidates:
+                HipCodeGen().gen(apply_tiling(cand))
+                emitted += 1
+    assert emitted > 3000
