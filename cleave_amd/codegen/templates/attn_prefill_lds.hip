@@ -101,7 +101,11 @@
 #define PL_KIMG (PL_KPANELS * PL_PANEL)       // elements of the K image
 #define PL_STAGE ((PL_KPANELS + PL_VPANELS) * PL_PANEL)   // K image, then V image
 #define PL_VIMG (PL_VPANELS * PL_PANEL)       // elements of the V image
-#define PL_STAGES (CL_HEAD_DIM > 192 ? 4 : 3)     // (the widest keys are read in two halves, the second out of an image still held)
+// Images of K and of V: three, and four where the widest keys are read in two halves, the second out of an image still held, or
+// where three would let two workgroups onto a compute unit that 256 registers a wave do not hold (192 / 192 and 128 / 256 wide,
+// 32 heads x 2048 x 2048, us: three images and 40 / 146 spilled registers 177 / 357, four and none 105 / 117).
+#define PL_STAGES (CL_HEAD_DIM > 192 || CL_HEAD_DIM + CL_VDIM == 384 ? 4 : 3)
+#define PL_ALONE (PL_STAGES * PL_STAGE * 4 > 163840)       // one workgroup of a compute unit: 512 registers a wave
 #define PL_KJ (CL_HEAD_DIM / 32)
 #define PL_FB (CL_VDIM / 16)
 #define PL_UNITS_PER (PL_KPANELS + PL_VPANELS)   // 1 KiB loads per wave and step: its 8-key group of every panel of K and V
@@ -589,6 +593,13 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
         const float alpha = fast_exp2(m_run[rt] - m_new);
         m_run[rt] = m_new;
         l_run[rt] *= alpha;
+#if PL_ALONE
+        // (512 registers: the accumulators live in the half that only matrix ops reach, and their way to these multiplications
+        // begins here: the compiler had moved all of them out and back in every step.  Us: 256 / 256 wide 187 -> 143, 192 / 256
+        // 162 -> 117, 192 / 192 133 -> 105)
+#pragma unroll
+        for (int fb = 0; fb < PL_FB; ++fb) asm volatile("" : "+a"(acc[rt][fb]));
+#endif
 #pragma unroll
         for (int fb = 0; fb < PL_FB; ++fb) acc[rt][fb] *= alpha;
         weigh(rt);

@@ -130,6 +130,22 @@ def test_both_kernels_round_the_weights_at_the_same_places(d, dtype):
     assert (a != b).float().mean().item() < 0.01
 
 
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("widths", [(192, 192), (128, 256), (192, 256), (256, 256)], ids=lambda w: f"{w[0]}_{w[1]}")
+def test_widths_with_a_compute_unit_to_themselves(widths, dtype):
+    """Key counts around a turn of four (192 / 256: three) images, and scores that rise along the keys, so that the accumulators are
+    moved out of the matrix half of the registers and back."""
+    def rising(prog):
+        q, k, v = prog.random_inputs(seed=5)
+        q[..., 0] = 4.0
+        k[..., 0] = torch.linspace(0.0, 35.0 * widths[0] ** 0.5 / (4 * 1.4427), k.shape[1], device=k.device).to(k.dtype)
+        return q, k, v
+
+    for keys in (1, 33, 97, 128, 129, 300):
+        check(C.mla_prefill, dtype, dict(H=2, SQ=140, SKV=keys, DK=widths[0], DV=widths[1]), LOCKSTEP)
+    check(C.mla_prefill, dtype, dict(H=2, SQ=140, SKV=600, DK=widths[0], DV=widths[1]), LOCKSTEP, args=rising)
+
+
 def test_search_proposes_them_behind_the_first_four():
     from cleave_amd.pipeline.direct import stage_graph
     from cleave_amd.schedule import search_tiling

@@ -423,6 +423,21 @@ def test_hot_kernels_keep_their_values_in_registers():
                 assert entry["vgprs"] <= 512 and entry["lds_bytes"] <= 160 * 1024, (label, entry)
 
 
+def test_wide_attention_keeps_its_values_in_registers():
+    """Widths whose accumulators and fragments do not fit 256 registers are left a compute unit to themselves: nothing spills where
+    three LDS images would have let a second workgroup in."""
+    from cleave_amd.pipeline.direct import kernel_for
+    from cleave_amd.runtime import shim
+    shim.load()
+    progs = [C.mla_prefill.trace(cl.f16, H=2, SQ=300, SKV=300, DK=dk, DV=dv)
+             for dk, dv in ((128, 128), (192, 128), (192, 192), (128, 256), (192, 256), (256, 64), (256, 128), (256, 256))]
+    progs += [op.trace(cl.f16, **sizes) for d in (192, 256) for op, sizes in ((C.qknorm, dict(HQ=4, HKV=2, SQ=300, SKV=300, D=d)),
+                                                                              (C.matmul_matmul, dict(H=2, SQ=300, SKV=300, D=d)))]
+    for prog in progs:
+        for entry in kernel_for(prog, template="attn_prefill", tiling=dict(SHARED=1)).stats:
+            assert entry["spilled_vgprs"] == 0 and entry["scratch_bytes"] == 0, (prog.name, entry)
+
+
 def test_a_split_of_a_family_without_a_contraction_is_refused_with_its_reason():
     """Row reductions have nothing to split: asking for a split is a refusal that says so (it
     was a KeyError from inside the lowering)."""
