@@ -95,6 +95,17 @@ CL_DEVICE ClRequest cl_find_request(const int* __restrict__ ptr, int batch, int 
 // 16-byte global load / store of eight elements.
 CL_DEVICE u32x4 ld16(const elem_t* p) { return *reinterpret_cast<const u32x4*>(p); }
 CL_DEVICE void st16(elem_t* p, u32x4 v) { *reinterpret_cast<u32x4*>(p) = v; }
+// Columns n .. n + 3 of a row of COLS: one store where rows are whole pieces of four, else element by element and none past the
+// row's end (the piece that crosses it would land in the next row, which another workgroup may own, or behind the tensor)
+template <int COLS, class T, class V> CL_DEVICE void st_cols4(T* row, int n, V v) {
+  if constexpr (COLS % 4 == 0) {
+    *reinterpret_cast<V*>(row + n) = v;
+  } else {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (n + r < COLS) row[n + r] = v[r];
+  }
+}
 CL_DEVICE elem8 as_elem8(u32x4 v) { return __builtin_bit_cast(elem8, v); }
 CL_DEVICE u32x4 as_u32x4(elem8 v) { return __builtin_bit_cast(u32x4, v); }
 

@@ -420,7 +420,7 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
       const int n = n0 + wn * (CL_BN / CL_WN) + 16 * j + 4 * g;
       if (n >= CL_N) continue;
 #if CL_SPLITS > 1
-      *reinterpret_cast<f32x4*>(CL_ARG_PACC + (((i64)split * GM_BATCH + batch) * CL_M + m) * CL_N + n) = acc[i][j];
+      st_cols4<CL_N>(CL_ARG_PACC + (((i64)split * GM_BATCH + batch) * CL_M + m) * CL_N, n, acc[i][j]);
 #if CL_NORM
       if (n0 == 0 && wn == 0 && j == 0 && g == 0) CL_ARG_PSS[((i64)split * GM_BATCH + batch) * CL_M + m] = tot;
 #endif
@@ -433,7 +433,7 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
       elem4 y;
 #pragma unroll
       for (int r = 0; r < 4; ++r) y[r] = to_elem(acc[i][j][r] * rs);
-      *reinterpret_cast<elem4*>(CL_ARG_OUT + ((i64)batch * CL_M + m) * CL_N + n) = y;
+      st_cols4<CL_N>(CL_ARG_OUT + ((i64)batch * CL_M + m) * CL_N, n, y);
 #endif
     }
   }

@@ -430,7 +430,7 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
       if (n >= CL_N) continue;
       const f32x4 v = gd_acc_read(acc[i][j]);
 #if CL_SPLITS > 1
-      *reinterpret_cast<f32x4*>(CL_ARG_PACC + (((i64)split * GD_BATCH + batch) * CL_M + m) * CL_N + n) = v;
+      st_cols4<CL_N>(CL_ARG_PACC + (((i64)split * GD_BATCH + batch) * CL_M + m) * CL_N, n, v);
 #else
       elem4 y;
 #pragma unroll
@@ -439,7 +439,7 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
 #else
       for (int r = 0; r < 4; ++r) y[r] = to_elem(v[r]);
 #endif
-      *reinterpret_cast<elem4*>(CL_ARG_OUT + ((i64)batch * CL_M + m) * CL_N + n) = y;
+      st_cols4<CL_N>(CL_ARG_OUT + ((i64)batch * CL_M + m) * CL_N, n, y);
 #endif
     }
 #endif  // CL_SWIGLU

@@ -1,5 +1,6 @@
 """GPU parity of products whose contraction is dealt out to ranges inside an unsplit operator: ranges of whole steps, ranges that end
-on a partly filled or an empty step, ragged rows and columns, both weight layouts, batches, SwiGLU."""
+on a partly filled or an empty step, ragged rows and columns, both weight layouts, batches, SwiGLU; row lengths that are no whole
+pieces of a store."""
 
 import numpy as np
 import pytest
@@ -7,7 +8,8 @@ import torch
 
 import cleave_amd.lang as cl
 from cleave_amd import examples as C
-from cleave_amd.pipeline.direct import kernel_for, stage_graph
+from cleave_amd.pipeline.direct import kernel_for, source_for, stage_graph
+from cleave_amd.runtime.compile import _compile, _load_main_kernel_from_code
 from cleave_amd.schedule import search_tiling
 from cleave_amd.schedule.policy import k_range
 from oracle import program_oracle
@@ -51,6 +53,29 @@ def test_batched_ranges():
     out = kernel_for(prog, template="gemm_dma", tiling=dict(BM=128, BN=128, BK=64, WM=2, WN=4, KS=4))(*args)
     want = program_oracle.evaluate(prog, list(args))[0]
     assert np.linalg.norm(out.float().cpu().numpy() - want) / np.linalg.norm(want) < 2.0 ** -10
+
+
+FORMS = [("gemm", dict(BM=64, BN=64, BK=64, WM=2, WN=2), None), ("gemm", dict(BM=32, BN=32, BK=64, WM=1, WN=1), 2),
+         ("gemm_dma", dict(BM=64, BN=128, BK=64, WM=2, WN=2), None), ("gemm_dma", dict(BM=256, BN=256, BK=64, WM=2, WN=2), None),
+         ("gemm_dma", dict(BM=128, BN=128, BK=64, WM=2, WN=4), 2), ("gemm_dma", dict(BM=128, BN=256, BK=64, WM=2, WN=4, KS=2), None)]
+
+
+@pytest.mark.parametrize("N", [1, 2, 7, 261, 262, 263, 264])
+@pytest.mark.parametrize("template,tiling,split", FORMS)
+def test_columns_that_are_no_whole_pieces(template, tiling, split, N):
+    """A (N, K) weight leaves N free: no store of a row's last columns reaches the next row, which is another workgroup's where a
+    row ends on a tile's edge, or the memory behind the last one."""
+    prog = C.matmul_nt.trace(cl.f16, M=70, N=N, K=512)
+    args = prog.random_inputs(seed=13)
+    print(f"columns {template} {tiling} split {split} N {N}", flush=True)
+    loaded = _load_main_kernel_from_code(source_for(prog, template=template, tiling=tiling, split=split))
+    room = torch.full((70 * N + 64,), 7.0, device="cuda", dtype=torch.float16)
+    _compile(loaded, None)(*args, room[:70 * N].view(70, N))
+    torch.cuda.synchronize()
+    want = program_oracle.evaluate(prog, list(args))[0]
+    got = room.float().cpu().numpy()
+    assert (got[70 * N:] == 7.0).all()
+    np.testing.assert_allclose(got[:70 * N].reshape(70, N), want, rtol=2e-3, atol=2e-3 * np.abs(want).max())
 
 
 def test_search_proposes_them_where_tiles_are_few():
