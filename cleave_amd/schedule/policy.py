@@ -556,15 +556,21 @@ def attn_many_rows_candidates(low, role, factor, arch: Arch):
     if role != "main":
         return out
     # 256 rows on two wave groups half a step apart: half the tile bytes per row, but one workgroup per compute unit
-    # and nothing beside its first loads.  Measured ahead from about 1500 keys (128 wide, us: 4096 keys 239 -> 228, 1024 keys
-    # 65.8 -> 67.2) where its workgroups keep most compute units busy, so it is proposed from half of either on; where it is ahead for certain -- keys in plenty and a workgroup for
-    # every compute unit -- instead of the other: a search times each for some milliseconds, in which the clock has not settled
-    # where the power cap holds it, and picked the slower one every other time.
-    if attn_phased_ok(p, kpre) and p["skv"] >= 768 and p["units"] * _ceil(rows, 256) >= arch.compute_units // 2:
+    # and nothing beside its first loads.  Measured ahead from about 1500 keys (128 wide, us: 4096 keys 246 -> 229, 1024 keys
+    # 68.1 -> 66.3) where its workgroups keep most compute units busy, so it is proposed from half of either on.  Where it is ahead for
+    # certain -- keys in plenty, wide keys, and rows that fill seven eighths of its rounds of one workgroup per compute unit --
+    # instead of the other: a search times each for some milliseconds, in which the clock has not settled where the power cap
+    # holds it, and picked the slower one every other time.  us over 2048 keys, 128 wide, the other / this one, by the share of its
+    # rounds that 32 / 8 heads fill: 2048 rows (all of one) 66.2 / 61.7, 2112 (0.52 of two) 90.1 / 108.1, 3072 (0.75) 98.4 / 108.6,
+    # 3584 (0.88) 115 / 106, 4096 (all) 128.8 / 122.2, 4160 (0.68 of three) 150 / 168, 5120 (0.83) 159.4 / 168.7, 5376 (0.88) 172 / 161,
+    # 7200 (0.88 of four) 229 / 217; 3584 rows at 192 / 128, 192 / 64 and 128 / 64 wide 138 / 127, 119 / 105, 94 / 85.
+    blocks = p["units"] * _ceil(rows, 256)
+    filled = p["units"] * rows / (256 * arch.compute_units * _ceil(blocks, arch.compute_units))
+    if attn_phased_ok(p, kpre) and p["skv"] >= 768 and blocks >= arch.compute_units // 2:
         out.append(TileDict("attn_prefill", role, dict(SHARED=1, PHASED=1, **({"KPRE": 1} if kpre else {})), output_tile=[256, vd],
                             rstep_map={"kv": 64}, n_threads=512, split_factor=factor, score=score,
                             lds_bytes=4 * 64 * (d + vd) * 2, est_vgprs=216, late=True,
-                            displaces=out[-1].tiling if d >= 128 and p["skv"] >= 2048 and p["units"] * _ceil(rows, 256) >= arch.compute_units else None))
+                            displaces=out[-1].tiling if d >= 128 and p["skv"] >= 2048 and blocks >= arch.compute_units and filled >= 0.875 else None))
     # Too few workgroups for the chip and keys enough to share out among more: the key ranges of the split form inside one
     # operator (partials in scratch, folded by a second launch).  Measured, us, unsplit / ranges: 56 items of 122 steps
     # 61.5 / 31.3 (4), 16 items of 76 steps 40.3 / 17.1 (8; 20.3 with 16), 64 items of 63 steps 64 wide 26.2 / 16.8 (4); behind

@@ -438,6 +438,16 @@ def test_wide_attention_keeps_its_values_in_registers():
             assert entry["spilled_vgprs"] == 0 and entry["scratch_bytes"] == 0, (prog.name, entry)
 
 
+@pytest.mark.parametrize("rows,alone", [(2048, True), (2049, False), (2112, False), (3000, False), (3584, True), (4096, True), (4160, False),
+                                        (5120, False), (5376, True), (6144, True), (1000, False)])
+def test_the_two_group_attention_takes_the_other_ones_place_only_where_it_fills_its_rounds(rows, alone):
+    """One workgroup of 256 rows per compute unit: just past a whole round the kernel on 128 rows, two workgroups a unit, is ahead."""
+    prog = C.gqa_decode_exact.trace(cl.f16, HQ=32, HKV=8, SQ=rows, SKV=2048, D=128)
+    tilings = [c.tiling for c in search_tiling(stage_graph(prog), topk=8)]
+    assert dict(SHARED=1, PHASED=1) in tilings
+    assert (dict(SHARED=1) in tilings) != alone
+
+
 def test_a_split_of_a_family_without_a_contraction_is_refused_with_its_reason():
     """Row reductions have nothing to split: asking for a split is a refusal that says so (it
     was a KeyError from inside the lowering)."""
