@@ -352,10 +352,11 @@ class CompiledKernel:
 
     def call_fixed_scratch(self, *args, clear: bool = False) -> None:
         """Run with caller-owned outputs and no allocation of device memory: the scratch buffers
-        (split partials) live in the native library's fixed per-GPU array instead of tensors.  The
-        kernel must have been made with ``out_idx=None``; ``args`` are the inputs, scalars and
-        outputs in parameter order.  A layout beyond the array's size is refused by the library.
-        Calls that overlap on one GPU share the array and race.  (One of the ``aligned_inputs`` that starts
+        live in the native library's fixed per-GPU array instead of tensors: the partials of a split, and what an unsplit
+        operator keeps between launches of its own (partials of key or contraction ranges, keys normalised ahead; a search
+        with the hint ``scratch=False`` finds plans without).  The kernel must have been made with ``out_idx=None``; ``args`` are the
+        inputs, scalars and outputs in parameter order.  A layout beyond the array's size is refused by the library.
+        Calls with scratch (``fixed_scratch_layout``'s bytes are not 0) that overlap on one GPU share the array and race.  (One of the ``aligned_inputs`` that starts
         between two 16-byte pieces is copied for the call: the one allocation there can be.)"""
         import torch
 

@@ -80,16 +80,20 @@ def _candidates(graph, arch):
     raise ScheduleRejected(f"no template for family {fam!r}")
 
 
-def search_tiling(graph, topk: int = 10, force_fusion: bool = False, accept=None, arch=None):
+def search_tiling(graph, topk: int = 10, force_fusion: bool = False, accept=None, arch=None, scratch: bool = True):
     """Up to ``topk`` ``TileDict`` candidates for a stage graph, best modelled cost first.
     ``accept(cand) -> bool`` filters before the cut.  ``force_fusion`` is accepted for API
-    compatibility: every template here is already one fused kernel."""
+    compatibility: every template here is already one fused kernel.  ``scratch=False``: no plan of an unsplit
+    operator that keeps scratch memory of its own (key or contraction ranges, keys normalised ahead), which every
+    call allocates and which calls through the fixed array share; ``ScheduleConfig(hints={"scratch": False})`` passes it."""
     arch = arch or current_target().arch
     if not hasattr(graph, "lowered"):
         raise ScheduleRejected("search_tiling needs a recognised stage graph (cleave_amd.lower.to_ir)")
     cands = _candidates(graph, arch)
     if accept is not None:
         cands = [c for c in cands if accept(c)]
+    if not scratch:
+        cands = [c for c in cands if not c.own_scratch]
     cands.sort(key=lambda c: (c.score, c.key()))
     seen, unique = set(), []
     for c in cands:

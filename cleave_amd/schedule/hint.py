@@ -21,6 +21,9 @@ class TileDict:
     displaces: dict | None = None # (late) the tiling of the same template that leaves the pool where this one joins it
     flat_graph: object = field(default=None, repr=False)   # the StageGraph this tiles
 
+    own_scratch = property(lambda self: self.role == "main" and not {"KEYS", "KS", "KPRE"}.isdisjoint(self.tiling),
+                           doc="whether an unsplit operator of this tiling keeps scratch memory between its launches")
+
     @property
     def label(self) -> str:
         knobs = " ".join(f"{k}={v}" for k, v in self.tiling.items())

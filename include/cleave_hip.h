@@ -164,8 +164,9 @@ typedef struct chip_scratch_arg {
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
  * Has no counterpart in the reference, whose callers always allocate the
  * split partials (python/cleave/runtime/autotune.py:164-227).  The scratch
- * buffers of the sequence -- the split partials a partial kernel writes and
- * its combine reads -- live in a fixed array of CHIP_FIXED_SCRATCH_BYTES that
+ * buffers of the sequence -- the partials of a split, and what an unsplit
+ * operator keeps between its own launches (partials of key or contraction
+ * ranges, keys normalised ahead) -- live in a fixed array of CHIP_FIXED_SCRATCH_BYTES that
  * is part of the library and is held by every GPU the library runs on until
  * the process ends; inputs and outputs are still the caller's.  For each of
  * the `nrefs` entries of `refs` the named argument is launched with the

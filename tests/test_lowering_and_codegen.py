@@ -448,6 +448,20 @@ def test_the_two_group_attention_takes_the_other_ones_place_only_where_it_fills_
     assert (dict(SHARED=1) in tilings) != alone
 
 
+@pytest.mark.parametrize("op,shapes", [(C.gqa_decode_exact, dict(HQ=32, HKV=8, SQ=193, SKV=3897, D=128)), (C.matmul, dict(M=655, N=3264, K=6912)),
+                                       (C.swiglu, dict(M=156, N=3968, K=8064)), (C.qknorm, dict(HQ=64, HKV=8, SQ=4096, SKV=4096, D=128))])
+def test_a_search_can_be_kept_to_plans_without_scratch(op, shapes):
+    graph = stage_graph(op.trace(cl.f16, **shapes))
+
+    def scratch(**how):
+        found = search_tiling(graph, topk=8, **how)
+        keeps = [any(q["role"] == "scratch" for q in parse_manifest(HipCodeGen().gen(apply_tiling(c)))["params"]) for c in found]
+        assert keeps == [c.own_scratch for c in found]
+        return keeps
+
+    assert any(scratch()) and not any(scratch(scratch=False))
+
+
 def test_a_split_of_a_family_without_a_contraction_is_refused_with_its_reason():
     """Row reductions have nothing to split: asking for a split is a refusal that says so (it
     was a KeyError from inside the lowering)."""

@@ -62,6 +62,30 @@ def test_split_k_matmul_twice_second_call_smaller():
         assert torch.equal(out, want)
 
 
+@pytest.mark.parametrize("case", ["keys", "matmul", "swiglu", "normed keys"])
+def test_unsplit_operators_with_scratch_of_their_own(case):
+    """Key ranges, contraction ranges and keys normalised ahead, inside operators nobody split: the same launches, twice, the
+    second call of other inputs over what the first left in the array."""
+    fn, shapes, template, tiling = {
+        "keys": (C.gqa_decode_exact, dict(HQ=4, HKV=2, SQ=75, SKV=300, D=128), "attn_prefill", dict(SHARED=1, KEYS=4)),
+        "matmul": (C.matmul, dict(M=77, N=264, K=600), "gemm", dict(BM=128, BN=128, BK=64, WM=2, WN=4, KS=3, DMA=1)),
+        "swiglu": (C.swiglu, dict(M=150, N=384, K=512), "gemm_dma", dict(BM=128, BN=256, BK=64, WM=2, WN=4, KS=2, SWIGLU=1)),
+        "normed keys": (C.qknorm, dict(HQ=4, HKV=2, SQ=75, SKV=300, D=128), "attn_prefill", dict(SHARED=1, KPRE=1))}[case]
+    prog = fn.trace(C.cl.f16, **shapes)
+    loaded = _load_main_kernel_from_code(source_for(prog, template=template, tiling=tiling))
+    own, caller = _compile(loaded, loaded.manifest["out_idx"]), _compile(loaded, None)
+    for seed in (1, 2):
+        ins = prog.random_inputs(seed=seed)
+        want = own(*ins)
+        out = torch.full_like(want, float("nan"))
+        print(f"fixed scratch: unsplit {case} {shapes}", flush=True)
+        caller.call_fixed_scratch(*ins, out)
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        _, dims, _ = caller._bind([*ins, out])
+        assert caller.fixed_scratch_layout(dims)[1] > 0
+
+
 def test_sizes_beyond_the_array_are_refused():
     own, caller = _paged_pair()
     args = [a.cuda() if isinstance(a, torch.Tensor) else a for a in C.paged_workload([64, 64], page_size=64, num_pages=8)]
