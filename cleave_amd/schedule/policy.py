@@ -574,10 +574,13 @@ def attn_many_rows_candidates(low, role, factor, arch: Arch):
     # Too few workgroups for the chip and keys enough to share out among more: the key ranges of the split form inside one
     # operator (partials in scratch, folded by a second launch).  Measured, us, unsplit / ranges: 56 items of 122 steps
     # 61.5 / 31.3 (4), 16 items of 76 steps 40.3 / 17.1 (8; 20.3 with 16), 64 items of 63 steps 64 wide 26.2 / 16.8 (4); behind
-    # from about a hundred items on or a range of fewer than six steps: 80 items of 14 steps 11.5 / 16.8.
+    # from about a hundred items on or a range of fewer than six steps: 80 items of 14 steps 11.5 / 16.8.  At most 32 ranges: the
+    # combine reads every range's partial of a row at once, and from 64 on that is slower than what they save -- two items of
+    # 512 steps, 128 wide, us by ranges: 1 225, 20 30.3, 32 25.2, 48 29.8, 64 59.5, 128 120.  (Where the steps do not divide, the
+    # last ranges are empty: eight items of 97 steps take 19.6 in 16 ranges, two of them empty, and 21.6 in 14.)
     if not p.get("emit_lse") and not kpre:
-        for fill in (256, 128):
-            n = min(fill // items, steps // 6)
+        most = [min(fill // items, steps // 6, 32) for fill in (arch.compute_units, arch.compute_units // 2)]
+        for n in (most[0], most[1] if most[1] < most[0] else most[0] // 2):
             if n > 1 and attn_keys_scratch(p, n) <= FIXED_SCRATCH:
                 out.append(TileDict("attn_prefill", role, dict(SHARED=1, KEYS=n), output_tile=[128, vd], rstep_map={"kv": 32},
                                     n_threads=256, split_factor=factor, score=score / n, lds_bytes=lds, est_vgprs=230, late=True))

@@ -462,6 +462,13 @@ def test_a_search_can_be_kept_to_plans_without_scratch(op, shapes):
     assert any(scratch()) and not any(scratch(scratch=False))
 
 
+@pytest.mark.parametrize("heads,rows,keys,want", [(1, 128, 16384, [32, 16]), (2, 128, 16384, [32, 16]), (8, 128, 3104, [16, 8]), (8, 128, 16384, [32, 16]),
+                                                  (56, 100, 3897, [4, 2]), (16, 100, 2409, [12, 8]), (100, 100, 4096, [2]), (8, 128, 200, [])])
+def test_key_ranges_are_few_enough_for_one_combine_and_two_different_numbers(heads, rows, keys, want):
+    found = search_tiling(stage_graph(C.gqa_decode_exact.trace(cl.f16, HQ=heads, HKV=heads, SQ=rows, SKV=keys, D=128)), topk=8)
+    assert [c.tiling["KEYS"] for c in found if "KEYS" in c.tiling] == want
+
+
 def test_a_split_of_a_family_without_a_contraction_is_refused_with_its_reason():
     """Row reductions have nothing to split: asking for a split is a refusal that says so (it
     was a KeyError from inside the lowering)."""
