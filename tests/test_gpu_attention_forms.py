@@ -130,6 +130,25 @@ def test_both_kernels_round_the_weights_at_the_same_places(d, dtype):
     assert (a != b).float().mean().item() < 0.01
 
 
+@pytest.mark.parametrize("place", [0, 40, 130, 261])
+@pytest.mark.parametrize("d,tiling", [(d, t) for t in (LOCKSTEP, PHASED, dict(SHARED=1, KEYS=3)) for d in (64, 128, 256)
+                                      if d < 256 or "PHASED" not in t])
+def test_infinite_and_undefined_scores(d, tiling, place):
+    """A key with an infinite feature, in the first step, the second, a middle one and the last: rows that see it at +inf or as a NaN
+    are NaN, rows that see it at -inf give it no weight, and a NaN in a query row stays in that row."""
+    prog = C.gqa_decode_exact.trace(cl.f16, HQ=2, HKV=2, SQ=150, SKV=262, D=d)
+    q, k, v = prog.random_inputs(seed=9)
+    q[0, :, 0] = torch.where(torch.arange(150, device=q.device) % 3 == 0, 1.0, -1.0).to(q.dtype)
+    q[0, 7, 0] = 0.0
+    q[1, 5, 3] = float("nan")
+    k[0, place, 0] = float("inf")
+    out = kernel_for(prog, template="attn_prefill", tiling=tiling)(q, k, v).double().cpu()
+    want = torch.softmax((q.double().cpu() @ k.double().cpu().transpose(1, 2).contiguous()) * d ** -0.5, dim=-1) @ v.double().cpu()
+    assert torch.isnan(want[0, ::3]).all() and torch.isnan(want[0, 7]).all() and torch.isnan(want[1, 5]).all()
+    assert torch.equal(torch.isnan(out), torch.isnan(want)) and torch.isnan(want).any(dim=-1).sum() == 52
+    np.testing.assert_allclose(out.nan_to_num(0).numpy(), want.nan_to_num(0).numpy(), rtol=1e-2, atol=ATOL["f16"])
+
+
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 @pytest.mark.parametrize("widths", [(192, 192), (128, 256), (192, 256), (256, 256)], ids=lambda w: f"{w[0]}_{w[1]}")
 def test_widths_with_a_compute_unit_to_themselves(widths, dtype):

@@ -85,6 +85,54 @@ def test_drawn_shapes_and_tilings_against_the_oracle(seed):
     assert 3 * ran >= 2 * DRAWS, f"only {ran} of {DRAWS} draws ran"
 
 
+def _draw_ranges(rng, n):
+    """Forms that need long contractions, many keys or tall workgroups: K or the keys dealt out to ranges inside an unsplit
+    operator, attention on two groups of waves and on widths that differ."""
+    from cleave_amd.schedule.policy import k_range
+
+    family = rng.choice(["matmul", "matmul_nt", "swiglu", "attention", "attention", "widths"])
+    if family in ("matmul", "matmul_nt", "swiglu"):
+        bm, bn, wm, wn = rng.choice([(128, 256, 2, 4), (256, 256, 2, 4), (128, 128, 2, 4), (64, 128, 2, 2), (64, 64, 2, 2)])
+        columns = rng.randrange(1, 500) if family == "matmul_nt" else (bn // 2 if family == "swiglu" else 8) * rng.randrange(1, 5)
+        shapes = dict(M=rng.randrange(1, 400), N=columns, K=64 * rng.randrange(4, 60) if family == "swiglu" else 8 * rng.randrange(40, 500))
+        ranges = rng.choice([r for r in range(2, 9) if k_range(shapes["K"], r)])
+        tiling = dict(BM=bm, BN=bn, BK=64, WM=wm, WN=wn, KS=ranges)
+        tiling.update({"SWIGLU": 1} if family == "swiglu" else {}, **({"DMA": 1} if shapes["K"] % 64 else {}))
+        make = {"matmul": C.inputs_c1, "matmul_nt": C.inputs_nt, "swiglu": C.inputs_swiglu}[family]
+        return (f"{family} {shapes}", getattr(C, family).trace(cl.f16, **shapes), make(shapes, seed=n),
+                dict(template="gemm" if shapes["K"] % 64 else "gemm_dma", tiling=tiling))
+    keys, rows = rng.randrange(1, 1500), rng.randrange(1, 700)
+    if family == "widths":
+        shapes = dict(H=rng.choice([1, 2, 3]), SQ=rows, SKV=keys, DK=64 * rng.randrange(1, 5), DV=64 * rng.randrange(1, 5))
+        forms = [dict(SHARED=1), dict(SHARED=1, KEYS=rng.randrange(2, 9))] + ([dict(SHARED=1, PHASED=1)] if shapes["DV"] <= 128 else [])
+        return f"mla_prefill {shapes}", C.mla_prefill.trace(cl.f16, **shapes), C.inputs_mla_prefill(shapes, seed=n), \
+            dict(template="attn_prefill", tiling=rng.choice(forms))
+    group, kv_heads = rng.choice([1, 2, 4, 8]), rng.choice([1, 2, 4])
+    shapes = dict(HQ=kv_heads * group, HKV=kv_heads, SQ=max(1, rows // group), SKV=keys, D=rng.choice([64, 128]))
+    tiling = rng.choice([dict(SHARED=1, PHASED=1), dict(SHARED=1, PHASED=1), dict(SHARED=1, KEYS=rng.randrange(2, 33))])
+    return (f"attention {shapes}", C.gqa_decode_exact.trace(cl.f16, **shapes), C.inputs_c3(shapes, seed=n),
+            dict(template="attn_prefill", tiling=tiling))
+
+
+@pytest.mark.parametrize("seed", [41, 42, 43])
+def test_drawn_ranges_and_two_group_attention_against_the_oracle(seed):
+    rng = random.Random(seed)
+    ran = 0
+    for n in range(DRAWS):
+        label, program, inputs, how = _draw_ranges(rng, 1000 * seed + n)
+        print(f"case drawn {label} {how}", flush=True)
+        try:
+            kernel = kernel_for(program, **how)
+        except CleaveError as refusal:
+            print(f"    refused: {str(refusal)[:120]}", flush=True)
+            continue
+        got = kernel(*[t.cuda() for t in inputs]).float().cpu().numpy()
+        want = po.evaluate(program, inputs)[0]
+        np.testing.assert_allclose(got.reshape(want.shape), want, rtol=1e-2, atol=1e-2, err_msg=f"{label} {how}")
+        ran += 1
+    assert 10 * ran >= 9 * DRAWS, f"only {ran} of {DRAWS} draws ran"
+
+
 @pytest.mark.parametrize("seed", [21, 22])
 def test_drawn_paged_decode_requests_against_the_oracle(seed):
     """Paged decode over drawn page sizes, head groups, request lengths (empty, one token, under a
