@@ -242,7 +242,8 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
       // (as in attn_prefill_lds.hip: weights first, the row's maximum only where a lane's sixteen of it sum to more than 2^8)
       if (__builtin_expect(__builtin_amdgcn_ballot_w64(psum[rt] > 256.0f) != 0, 0)) {
         const float mx = part_max(rt, 16) * scale2;
-        const float m_new = pl_max_over_groups(psum[rt]) > 256.0f && mx > m_run[rt] ? mx : m_run[rt];
+        const bool over = pl_max_over_groups(psum[rt]) > 256.0f;
+        const float m_new = over ? fmaxf(mx, m_run[rt]) : m_run[rt];
         const float alpha = fast_exp2(m_run[rt] - m_new);
         m_run[rt] = m_new;
         l_run[rt] *= alpha;
