@@ -1,5 +1,5 @@
 // ---- split-KV combine shared by the decode-attention kernels -------------------------------
-// Partials are (split, row[, d]) f32 with m the running max in the log2 domain, l the sum of
+// Partials are (split, row[, d]) f32 with m the reference point of the row's weights in the log2 domain, l the sum of
 // weights relative to m, and O the unnormalised weighted values.
 #ifndef CL_CHUNK_PAGES
 #define CL_CHUNK_PAGES 0

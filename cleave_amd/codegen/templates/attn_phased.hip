@@ -8,11 +8,12 @@
 // with.  Four images of K and V rotate: a tile is asked for two (V) and three (K) tiles ahead, in the softmax parts.
 //
 // What bounds it: the power cap, as the kernel it stands beside; it moves half the tile bytes into LDS and has no
-// barrier that finds both waves of a SIMD in the same part.  32 heads x 4096 rows at 128 wide, us, attn_prefill_lds.hip /
-// this kernel: 4096 keys 239 / 228, 2048 keys 119.5 / 116.3, 1024 keys 65.8 / 67.2, 512 keys 38.2 / 41.1, 128 keys 20.4 / 24.3
-// (one workgroup of a compute unit: nothing runs beside its first loads and its stores); the search times both.  Workgroups
-// that stay and walk several items, the next one's queries loaded under the last tiles, were 231 at 4096 keys and level
-// with the other kernel on few keys (the queries and outputs of all workgroups are then what memory moves).
+// barrier that finds both waves of a SIMD in the same part.  32 / 8 heads x 4096 rows at 128 wide, us, attn_prefill_lds.hip /
+// this kernel, the two in turn on one card: 4096 keys 245 / 228, 2048 keys 127 / 119.5, 1536 keys 96.7 / 92.5, 1024 keys 67.1 / 65.4, 512 keys
+// 39.7 / 40.0, 128 keys 19.5 / 21.9 (one workgroup of a compute unit: nothing runs beside its first loads and its stores); the
+// search times both.  Workgroups that stay and walk several items, the next one's queries loaded under the last tiles, were
+// 231 at 4096 keys where these took 228, and level with the other kernel on few keys (the queries and outputs of all
+// workgroups are then what memory moves).
 //
 //   CL_HEAD_DIM, CL_VDIM (multiples of 64, (CL_HEAD_DIM + CL_VDIM) / 64 <= 5)  CL_ROWS  CL_SKV  CL_SCALE  CL_LINEAR  CL_QNORM
 #ifndef CL_LINEAR

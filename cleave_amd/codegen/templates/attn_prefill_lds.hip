@@ -17,9 +17,10 @@
 // and the lse (of 64-wide heads without an lse the rounded weights', see PL_ROUNDED_SUMS).
 //
 // What bounds it: the loop runs at the power cap (the clock falls to 1.9 GHz and time follows the work done, not the
-// stalls).  Dense, 32 heads x 4096 x 4096 at 128 wide: 248 -> 239 us when the maxima (ten vector instructions of a
-// step's eighty) went and the operand reads moved ahead of their use; with parts switched off: no tile loads 220, no value
-// reads 228, no key reads 232, no exponentials 212.  attn_phased.hip loads half as much per row.
+// stalls; cards and minutes differ by 5 %, so only pairs timed in turn compare).  Dense, 32 / 8 heads x 4096 x 4096 at 128 wide:
+// 257 -> 246 us when the maxima (ten vector instructions of a step's eighty) went, the operand reads moved ahead of their use
+// and results left past the caches' retention; with parts switched off, of 239: no tile loads 220, no value reads 228, no
+// key reads 232, no exponentials 212.  attn_phased.hip loads half as much per row.
 //
 // Work items: a new item at every multiple of PL_QT packed query tokens and at every request
 // boundary (item t = chunk w + request b for the one pair that overlaps); an item stops at the

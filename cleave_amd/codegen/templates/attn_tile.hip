@@ -87,9 +87,9 @@ CL_DEVICE float pl_sum_weights(const elem8& w, float sum) {
 // One row tile's results: a lane holds features 16 fb + 4 g .. + 3 of its row for every block fb.  Lanes g and g ^ 1 trade
 // halves of a pair of blocks (one row swap per register), so that each stores 16 contiguous bytes: even g the 8 features
 // from 4 g of the even block, odd g those from 4 (g - 1) of the odd one.  `row`: the row's first feature.
-// STREAM: past the caches' retention (64-byte pieces of rows that nothing in the kernel reads again: dense, 32 heads x 4096
-// rows at 128 wide, us, 128 keys 23.2 -> 20.0, 512 keys 41.3 -> 38.6, 4096 keys 253 -> 250; packed prompts, whose rows of all heads
-// lie together, 131.8 -> 134.6: not there).
+// STREAM: past the caches' retention (64-byte pieces of rows that nothing in the kernel reads again: the lock-step kernel, dense,
+// 32 heads x 4096 rows at 128 wide, both in turn, us, 128 keys 23.2 -> 20.0, 512 keys 41.3 -> 38.6, 4096 keys 253 -> 250; packed
+// prompts, whose rows of all heads lie together, 131.8 -> 134.6: not there).
 template <int FB, bool STREAM>
 CL_DEVICE void pl_store_row(elem_t* row, const f32x4 (&acc)[FB], float inv, int g) {
   elem_t* dst = row + 16 * (g & 1) + 4 * (g & 2);

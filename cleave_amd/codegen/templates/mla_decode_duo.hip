@@ -265,9 +265,11 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
   // 24 requests of up to 350 tokens: 92.4 -> 90.6 us.  Ranking the items of all requests by their keys instead lets
   // equally long ones run in lockstep, loading queries and storing outputs all at once: 98 - 103 us)
   // Runs of four neighbouring items go to one XCD (launch index % 8; the grid's extent is a multiple of eight): they read the
-  // same keys, which every XCD that works on a request fetches into its own L2.  One item after the other / runs of 4 / 8 /
-  // 16 / a contiguous eighth of all items for each XCD, us, 24 requests of up to 350 tokens: 95.7 / 92.8 / 95.5 / 102 / 124, 16 of
-  // up to 512: 117.2 / 111.5 / 114.2 / 114.7 / 144: longer runs leave the XCDs unequal work.
+  // same keys, which every XCD that works on a request fetches into its own L2.  The kernel, one item after the other / runs of
+  // 4 / 8, us: 24 requests of up to 350 tokens 87.8 / 87.6 / 87.7, 16 of up to 512 91.2 / 89.8 / 91.4, 32 of up to 512 146.5 / 144.7 /
+  // 145.4, 32 of up to 128 23.4 / 22.8 / 22.4, 8 of up to 512 without a prefix 50.4 / 49.4 / 51.8: up to 2.5 %, and within noise for few
+  // requests.  Runs of 16 and a contiguous eighth of all items for each XCD leave the XCDs unequal work (102 and 124 where runs of
+  // 4 took 93).
   constexpr int RUN = 4;
   const int xcd = (int)blockIdx.x & 7, nth = (int)blockIdx.x >> 3, of_xcd = (int)gridDim.x >> 3, in_runs = of_xcd / RUN * RUN;
   const int place = nth < in_runs ? (nth / RUN * 8 + xcd) * RUN + nth % RUN : 8 * in_runs + xcd * (of_xcd - in_runs) + nth - in_runs;

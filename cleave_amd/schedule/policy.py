@@ -556,8 +556,8 @@ def attn_many_rows_candidates(low, role, factor, arch: Arch):
     if role != "main":
         return out
     # 256 rows on two wave groups half a step apart: half the tile bytes per row, but one workgroup per compute unit
-    # and nothing beside its first loads.  Measured ahead from about 1500 keys (128 wide, us: 4096 keys 246 -> 229, 1024 keys
-    # 68.1 -> 66.3) where its workgroups keep most compute units busy, so it is proposed from half of either on.  Where it is ahead for
+    # and nothing beside its first loads.  Measured ahead from about 1000 keys (128 wide, us: 4096 keys 245 -> 228, 1024 keys
+    # 67.1 -> 65.4, 512 keys 39.7 -> 40.0) where its workgroups keep most compute units busy, so it is proposed from half of either on.  Where it is ahead for
     # certain -- keys in plenty, wide keys, and rows that fill seven eighths of its rounds of one workgroup per compute unit --
     # instead of the other: a search times each for some milliseconds, in which the clock has not settled where the power cap
     # holds it, and picked the slower one every other time.  us over 2048 keys, 128 wide, the other / this one, by the share of its
