@@ -22,6 +22,7 @@ import math
 from pathlib import Path
 
 from ..core.errors import CodegenError
+from ..lower.stages import mla_po_elem
 from ..schedule.plan import KernelPlan, ParamSpec
 
 TEMPLATE_DIR = Path(__file__).resolve().parent / "templates"
@@ -468,6 +469,34 @@ class HipCodeGen:
             args = unit.signature("CL_COMBINE_PARAMS", "CL_COMBINE_NAME", entry, sig, dyn, dyn_c)
             self._combine_args = (entry, args)
 
+    @staticmethod
+    def _key_ranges(plan, params, keys, rows, vdim):
+        """The plan of an unsplit attention whose keys are dealt out to ``keys`` ranges: the split form's two launches, f32 partials in
+        scratch (added to ``params`` ahead of the outputs)."""
+        if plan.role != "main" or keys < 2 or plan.problem.get("emit_lse"):
+            raise CodegenError("KEYS shares the keys of an unsplit attention without lse out to two or more ranges")
+        at = next(i for i, q in enumerate(params) if q.role == "output")
+        operands, scratch = dict(plan.operands), []
+        for role, extents in (("PM", (keys, rows)), ("PL", (keys, rows)), ("PO", (keys, rows, vdim))):
+            names = [f"Partial_{role}_split", f"Partial_{role}_combine"]
+            scratch += [ParamSpec(names[0], "float32", extents, "scratch"), ParamSpec(names[1], "float32", extents, "scratch", alias=names[0])]
+            operands[role], operands[f"{role}_COMBINE"] = names
+        params[at:at] = scratch
+        return dataclasses.replace(plan, role="fused", operands=operands, split_factor=keys)
+
+    def _launch_combine(self, unit, rows, vdim, splits, po_elem=False, plain=None):
+        """The launch that merges the f32 (or, ``po_elem``, element-type) partials of ``splits`` key ranges.
+        ``plain``: the grid of one thread per piece, where it is written otherwise."""
+        from ..schedule.policy import combine_groups
+
+        entry, args = self._combine_args
+        groups = 1 if po_elem else combine_groups(rows, vdim, splits)
+        if groups > 1:
+            unit.define("CL_COMBINE_GROUPS", groups)
+            unit.launch(entry, (rows * (vdim * groups // 1024), 1, 1), 256, 0, args)
+        else:
+            unit.launch(entry, (plain or -(-(rows * (vdim // (8 if po_elem else 4))) // 256), 1, 1), 256, 0, args)
+
     def _emit_attn_decode(self, unit, plan, params, partial, combine, fused):
         p, t, op = plan.problem, plan.tiling, plan.operands
         if partial and (p.get("norm_eps") or p.get("linear")):
@@ -531,8 +560,11 @@ class HipCodeGen:
             lds = 0 if waves == 1 or chunk_pages else attn_lds_bytes(waves, p["vdim"])
             unit.launch(ENTRY, grid, waves * 64, lds, self._partial_args)
         if combine:
-            entry, args = self._combine_args
-            unit.launch(entry, (f"ceildiv({grid_rows} * {p['vdim'] // 4}, 256)", 1, 1), 256, 0, args)
+            plain = f"ceildiv({grid_rows} * {p['vdim'] // 4}, 256)"
+            if paged:
+                unit.launch(self._combine_args[0], (plain, 1, 1), 256, 0, self._combine_args[1])
+            else:
+                self._launch_combine(unit, total_rows, p["vdim"], splits, plain=plain)
 
     def _emit_attn_dense_prefill(self, unit, plan, params, partial, combine):
         """The LDS-shared prefill kernel over the dense attention family's operands: every unit
@@ -558,18 +590,10 @@ class HipCodeGen:
         # KEYS: the keys are dealt out to that many ranges inside an unsplit operator: the split form's two launches, partials in scratch
         keys = int(plan.tiling.get("KEYS", 0))
         if keys:
-            if plan.role != "main" or kpre or keys < 2 or p.get("emit_lse"):
-                raise CodegenError("KEYS shares the keys of an unsplit attention without lse out to two or more ranges")
-            total = p["units"] * rows
-            at = next(i for i, q in enumerate(params) if q.role == "output")
-            operands, scratch = dict(op), []
-            for role, extents in (("PM", (keys, total)), ("PL", (keys, total)), ("PO", (keys, total, p["vdim"]))):
-                names = [f"Partial_{role}_split", f"Partial_{role}_combine"]
-                scratch += [ParamSpec(names[0], "float32", extents, "scratch"), ParamSpec(names[1], "float32", extents, "scratch", alias=names[0])]
-                operands[role], operands[f"{role}_COMBINE"] = names
-            params[at:at] = scratch
-            plan = dataclasses.replace(plan, role="fused", operands=operands, split_factor=keys)
-            op, splits, combine = operands, keys, True
+            if kpre:
+                raise CodegenError("KEYS and KPRE: one launch beside the kernel's own")
+            plan = self._key_ranges(plan, params, keys, p["units"] * rows, p["vdim"])
+            op, splits, combine = plan.operands, keys, True
         self._attn_common(unit, plan, params, partial, combine, False, p["vdim"], p["units"] * rows, False)
         phased = int(plan.tiling.get("PHASED", 0))
         if phased:
@@ -611,8 +635,7 @@ class HipCodeGen:
             items = -(-(-(-rows // (256 if phased else 128))) // 8) * 8
             unit.launch(ENTRY, (items, p["units"], splits), 512 if phased else 256, 0, self._partial_args)
         if combine:
-            entry, args = self._combine_args
-            unit.launch(entry, (-(-(p["units"] * rows * (p["vdim"] // 4)) // 256), 1, 1), 256, 0, args)
+            self._launch_combine(unit, p["units"] * rows, p["vdim"], splits)
 
     def _emit_attn_prefill(self, unit, plan, params, partial, combine, fused):
         if not plan.problem.get("paged"):
@@ -657,6 +680,12 @@ class HipCodeGen:
             return self._emit_mla_paged(unit, plan, params, partial, combine, fused)
         total_rows = p["batch"] * p["heads"]
         emit_lse = bool(p.get("emit_lse"))
+        # KEYS: the keys dealt out to that many ranges inside an unsplit operator.  Its partials are f32, as the accumulators of an
+        # operator without ranges are; those of the split form are in the type that form's buffers have.
+        keys = int(t.get("KEYS", 0))
+        if keys:
+            plan, combine = self._key_ranges(plan, params, keys, total_rows, p["ckv"]), True
+        po_elem = not keys and mla_po_elem(p["heads"])
         self._attn_common(unit, plan, params, partial, combine, fused, p["ckv"], total_rows, emit_lse)
         if int(t.get("XW", 0)):
             # The cross-wave form (64 heads per workgroup, weights exchanged through LDS) was
@@ -664,13 +693,13 @@ class HipCodeGen:
             # wrong result whose cause was never found.
             raise CodegenError("tiling XW=1 (cross-wave MLA decode) is withdrawn; use WAVES/HG/VSPLIT/STAGES")
         if int(t.get("DUO", 0)):
-            return self._emit_mla_duo(unit, plan, partial, combine, total_rows)
-        waves, hg, stages = int(t.get("WAVES", 4)), int(t.get("HG", 1)), int(t.get("STAGES", 3))
+            return self._emit_mla_duo(unit, plan, partial, combine, total_rows, po_elem)
+        waves, hg, stages = int(t.get("WAVES", 4 if partial else 1)), int(t.get("HG", 1)), int(t.get("STAGES", 3))
         vsplit = int(t.get("VSPLIT", 1))
         if waves not in (1, 2, 4, 8):
             raise CodegenError("the MLA template runs 1, 2, 4 or 8 waves per workgroup")
-        # (a combine on its own has no wave grid: held to the default four waves of 16 heads, operators of 16 or 32
-        # heads had no split form at all)
+        # (a combine on its own has no wave grid: held to the default four waves of 16 heads, in the checks below or in the
+        # template's own, operators of 16 or 32 heads had no split form that a search could run)
         if partial and (waves % vsplit or p["heads"] % (16 * hg * waves // vsplit) or (p["ckv"] // 16) % (4 * vsplit)):
             raise CodegenError(f"{p['heads']} heads / {p['ckv']} features do not divide into {waves} waves of "
                                f"{16 * hg} heads sharing a head set by {vsplit}")
@@ -684,8 +713,7 @@ class HipCodeGen:
             unit.define("CL_LDS_AHEAD", int(t["LDS_AHEAD"]))
         if "OCC" in t:
             unit.define("CL_OCC", int(t["OCC"]))
-        # split partials of this family are stored in the element type (normalised per split)
-        unit.define("CL_PO_ELEM", 1)
+        unit.define("CL_PO_ELEM", po_elem)
         unit.define("CL_SCALE_LOG2E", _f(float(p["scale"]) * LOG2E))
         for role, macro in (("Q", "CL_ARG_Q"), ("QPE", "CL_ARG_QPE"), ("KV", "CL_ARG_KV"), ("KPE", "CL_ARG_KPE")):
             if role in op:
@@ -697,11 +725,9 @@ class HipCodeGen:
             # the LDS images are a static array of the kernel: no dynamic LDS at launch
             unit.launch(ENTRY, grid, waves * 64, 0, self._partial_args)
         if combine:
-            entry, args = self._combine_args
-            unit.launch(entry, (-(-(total_rows * (p["ckv"] // 8)) // 256), 1, 1), 256, 0, args)
+            self._launch_combine(unit, total_rows, p["ckv"], splits, po_elem)
 
-
-    def _emit_mla_duo(self, unit, plan, partial, combine, total_rows):
+    def _emit_mla_duo(self, unit, plan, partial, combine, total_rows, po_elem):
         """The score-wave / value-wave form of MLA decode: eight waves own 64 heads, four making the
         scores of 32 heads x half of each step's tokens, four the value products of 32 heads x half
         the latent features."""
@@ -712,7 +738,7 @@ class HipCodeGen:
             raise CodegenError("the score-wave / value-wave MLA kernel needs heads % 64 == 0, a latent width in multiples of 128, "
                                "a rope width of an odd number of 64s, and four images within 160 KiB of LDS")
         for k, v in (("CL_HEADS", p["heads"]), ("CL_CKV", p["ckv"]), ("CL_KPE", p["kpe"]), ("CL_SKV", p["skv"]),
-                     ("CL_BATCH", p["batch"]), ("CL_PO_ELEM", 1)):
+                     ("CL_BATCH", p["batch"]), ("CL_PO_ELEM", po_elem)):
             unit.define(k, v)
         if "LDS_AHEAD" in t:
             ahead = int(t["LDS_AHEAD"])
@@ -733,11 +759,15 @@ class HipCodeGen:
             if role in op:
                 unit.define(macro, op[role])
         unit.templates += ["mla_decode_duo.hip", "attn_combine.hip"]
-        if partial:
-            unit.launch(ENTRY, (p["batch"] * (p["heads"] // 64), plan.split_factor or 1, 1), 512, 0, self._partial_args)
+        splits = plan.split_factor or 1
+        if partial and "KEYS" in t:
+            # (one-dimensional: the head blocks of a range eight launches apart, on one XCD)
+            unit.define("CL_UNITS_1D", 1)
+            unit.launch(ENTRY, (-(-(p["batch"] * splits) // 8) * 8 * (p["heads"] // 64), 1, 1), 512, 0, self._partial_args)
+        elif partial:
+            unit.launch(ENTRY, (p["batch"] * (p["heads"] // 64), splits, 1), 512, 0, self._partial_args)
         if combine:
-            entry, args = self._combine_args
-            unit.launch(entry, (-(-(total_rows * (p["ckv"] // 8)) // 256), 1, 1), 256, 0, args)
+            self._launch_combine(unit, total_rows, p["ckv"], splits, po_elem)
 
     def _emit_mla_paged(self, unit, plan, params, partial, combine, fused):
         """Paged MLA decode (token table, page size 1): one wave per (work item, 16 heads); work

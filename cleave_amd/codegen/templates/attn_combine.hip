@@ -7,6 +7,9 @@
 #ifndef CL_PO_ELEM
 #define CL_PO_ELEM 0
 #endif
+#ifndef CL_COMBINE_GROUPS
+#define CL_COMBINE_GROUPS 1
+#endif
 #if CL_CHUNK_PAGES && CL_EMIT_COMBINE
 // Combine of chunked items: request b owns items b + p0/C .. b + (p1-1)/C (p0, p1 its page-table
 // range); partials are (item, query head[, d]).  One thread per (request, head, 4 d).
@@ -103,6 +106,73 @@ CL_COMBINE_NAME(CL_COMBINE_PARAMS) {
   st16(CL_CARG_OUT + row * CL_VDIM + d, as_u32x4(r));
 #if CL_EMIT_LSE
   if (d == 0) CL_CARG_LSE[row] = l > 0.f ? m + fast_log2(l) : CL_NEG_INF;
+#endif
+}
+#elif CL_SPLITS > 1 && CL_EMIT_COMBINE && CL_COMBINE_GROUPS > 1
+// The rule of the next kernel where rows are few and splits are many: CL_COMBINE_GROUPS groups of threads share the splits of a
+// row's CB_COLS columns (thread t: group t / CB_THREADS, columns 4 (t % CB_THREADS) .. + 3), each adds up its own against the
+// largest of their reference points, and the first group adds the groups' sums up out of LDS.
+// What bounds it: one round trip to memory, which one thread that reads 57 splits makes in parts.  Whole operators, us, one thread /
+// groups: 48 rows x 512 of 57 splits 20.2 / 15.5, 32 x 512 of 20 8.8 / 8.2, 256 x 128 of 32 25.1 / 23.9; behind where splits are
+// fewer or rows enough to fill the chip: 384 x 512 of 18 23.7 / 24.0, 256 x 512 of 16 18.0 / 18.3, 11 x 128 of 8 6.7 / 6.9.
+#define CB_THREADS (256 / CL_COMBINE_GROUPS)
+#define CB_COLS (4 * CB_THREADS)
+#define CB_EACH ((CL_SPLITS + CL_COMBINE_GROUPS - 1) / CL_COMBINE_GROUPS)
+static_assert(256 % CL_COMBINE_GROUPS == 0 && CL_VDIM % CB_COLS == 0, "a workgroup takes whole pieces of one row");
+extern "C" __global__ void __launch_bounds__(256)
+CL_COMBINE_NAME(CL_COMBINE_PARAMS) {
+  __shared__ __attribute__((aligned(16))) f32x4 part_o[CL_COMBINE_GROUPS][CB_THREADS];
+  __shared__ f32x2 part_ml[CL_COMBINE_GROUPS];
+  const i64 row = (i64)blockIdx.x / (CL_VDIM / CB_COLS);
+  const int group = threadIdx.x / CB_THREADS, at = threadIdx.x % CB_THREADS;
+  const int d = (int)(blockIdx.x % (CL_VDIM / CB_COLS)) * CB_COLS + 4 * at;
+  float pm[CB_EACH], pl[CB_EACH];
+  f32x4 po[CB_EACH];
+#pragma unroll
+  for (int u = 0; u < CB_EACH; ++u) {
+    const int s = group + u * CL_COMBINE_GROUPS;
+    const i64 prow = (i64)(s < CL_SPLITS ? s : CL_SPLITS - 1) * CL_TOTAL_ROWS + row;      // (past the last: it again, with weight 0)
+    pm[u] = CL_CARG_PM[prow];
+    pl[u] = CL_CARG_PL[prow];
+    po[u] = *reinterpret_cast<const f32x4*>(CL_CARG_PO + prow * CL_VDIM + d);
+  }
+  float m = pm[0];
+#pragma unroll
+  for (int u = 1; u < CB_EACH; ++u) m = fmaxf(m, pm[u]);
+  float l = 0.f;
+  f32x4 o = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int u = 0; u < CB_EACH; ++u) {
+    const float f = group + u * CL_COMBINE_GROUPS < CL_SPLITS ? fast_exp2(pm[u] - m) : 0.f;
+    l += pl[u] * f;
+    o += po[u] * f;
+  }
+  part_o[group][at] = o;
+  if (at == 0) part_ml[group] = (f32x2){m, l};
+  __syncthreads();
+  if (group != 0) return;
+  f32x2 ml[CL_COMBINE_GROUPS];
+  float top = CL_NEG_BIG;
+#pragma unroll
+  for (int k = 0; k < CL_COMBINE_GROUPS; ++k) {
+    ml[k] = part_ml[k];
+    top = fmaxf(top, ml[k][0]);
+  }
+  l = 0.f;
+  o = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int k = 0; k < CL_COMBINE_GROUPS; ++k) {
+    const float f = fast_exp2(ml[k][0] - top);
+    l += ml[k][1] * f;
+    o += part_o[k][at] * f;
+  }
+  const float inv = 1.0f / fmaxf(l, 1.0e-30f);
+  elem4 r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r[i] = to_elem(o[i] * inv);
+  *reinterpret_cast<elem4*>(CL_CARG_OUT + row * CL_VDIM + d) = r;
+#if CL_EMIT_LSE
+  if (d == 0) CL_CARG_LSE[row] = l > 0.f ? top + fast_log2(l) : CL_NEG_INF;
 #endif
 }
 #elif CL_SPLITS > 1 && CL_EMIT_COMBINE

@@ -55,7 +55,8 @@
 // weights as used).
 //
 //   CL_HEADS (multiple of 64)  CL_CKV (multiple of 128)  CL_KPE (multiple of 64)  CL_SKV  CL_BATCH
-//   CL_SPLITS  CL_SCALE_LOG2E  CL_PO_ELEM (must be 1: split partials normalised, in the element type)
+//   CL_SPLITS  CL_SCALE_LOG2E  CL_PO_ELEM  1: split partials are normalised values in the element type with m = log-sum-exp and
+//   l = 1;  0: unnormalised f32 values with their reference point and sum    CL_UNITS_1D  a one-dimensional grid (key ranges)
 //
 // CL_PREFILL: paged causal prefill over ragged query rows.  The 64 rows of a workgroup are four consecutive
 // query tokens of one request (a new item at every multiple of four packed tokens and at every request boundary) x
@@ -73,8 +74,8 @@
 #ifndef CL_PREFILL
 #define CL_PREFILL 0
 #endif
-#if CL_SPLITS > 1 && !CL_PO_ELEM
-#error "the score-wave / value-wave kernel writes its split partials in the element type"
+#ifndef CL_UNITS_1D
+#define CL_UNITS_1D 0
 #endif
 #define MD_STEP 32
 #define MD_D (CL_CKV + CL_KPE)
@@ -320,7 +321,14 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
   {
     constexpr int per_entry = CL_SPLITS * MD_HEAD_GROUPS;
     const int launch = blockIdx.y * gridDim.x + blockIdx.x;
-    if (CL_BATCH % 8 == 0) {
+    if (CL_UNITS_1D) {
+      // few batch entries and many ranges: (batch entry, range) pairs go round the XCDs, the head blocks of a pair to one of them
+      const int unit = launch % 8 + 8 * (launch / (8 * MD_HEAD_GROUPS));
+      if (unit >= CL_BATCH * CL_SPLITS) return;
+      b = unit / CL_SPLITS;
+      split = unit % CL_SPLITS;
+      hg_block = (launch / 8) % MD_HEAD_GROUPS;
+    } else if (CL_BATCH % 8 == 0) {
       const int k = launch / 8;                              // the k-th workgroup of XCD launch % 8
       b = launch % 8 + 8 * (k / per_entry);
       split = (k % per_entry) / MD_HEAD_GROUPS;
@@ -787,6 +795,17 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
 #else
     const i64 orow = row0 + 16 * t;                                // first head row of this tile
 #endif
+#if CL_SPLITS > 1 && !CL_PO_ELEM
+    // f32 partials: 16 bytes per lane and feature block as they are
+    const i64 prow = (i64)split * CL_TOTAL_ROWS + orow + c;
+    float* dst = CL_ARG_PO + prow * CL_CKV + 16 * MD_FBW * fhalf + 4 * g;
+    if (g == 0 && fhalf == 0) {
+      CL_ARG_PM[prow] = m;
+      CL_ARG_PL[prow] = l;
+    }
+#pragma unroll
+    for (int fb = 0; fb < MD_FBW; ++fb) *reinterpret_cast<f32x4*>(dst + 16 * fb) = acc[t][fb];
+#else
     const float inv = 1.0f / fmaxf(l, 1.0e-30f);
 #if CL_SPLITS > 1
     const i64 prow = (i64)split * CL_TOTAL_ROWS + orow;
@@ -822,6 +841,7 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
       md_swap_rows16(a1, b1);
       *reinterpret_cast<u32x4*>(dst + 32 * fp) = (u32x4){a0, a1, b0, b1};
     }
+#endif
   }
 }
 #endif  // CL_EMIT_PARTIAL

@@ -34,10 +34,16 @@ def to_ir(structure, symbol_map=None, dtype="float16", out_dtype=None, input_nam
     return StageGraph(g, recognize(g))
 
 
+def mla_po_elem(heads: int) -> bool:
+    """Whether the value partials of a split latent attention are in the element type.  Operators of 16 or 32 heads, whose
+    partials are small beside the keys they read, keep f32 ones, as the accumulators they come from are."""
+    return heads % 64 == 0
+
+
 def partial_buffers(low: Lowered, factor: int) -> list:
     """``[(name, shape, dtype)]`` of what a split partial writes and its combine reads, split-major
     like the reference's ``(split, batch, heads[, D])`` layout
-    (``python/cleave/dynamic/paging/tensor_maps.py:41-69``); f32 except the MLA value partials."""
+    (``python/cleave/dynamic/paging/tensor_maps.py:41-69``); f32 except the MLA value partials of 64 heads or more."""
     p = low.problem
     if low.family in ("matmul", "rmsnorm_matmul", "lora"):
         batch = max(p["batch_A"], p["batch_B"])
@@ -55,7 +61,7 @@ def partial_buffers(low: Lowered, factor: int) -> list:
         # split's log-sum-exp in PM and PL = 1 (the reference's partials are in the element type too)
         rows, width = p["batch"] * p["heads"], p["ckv"]
         return [("PM", (factor, rows), "float32"), ("PL", (factor, rows), "float32"),
-                ("PO", (factor, rows, width), low.dtype)]
+                ("PO", (factor, rows, width), low.dtype if mla_po_elem(p["heads"]) else "float32")]
     else:
         raise LoweringRejected(f"family {low.family!r} has no split form")
     return [("PM", (factor, rows), "float32"), ("PL", (factor, rows), "float32"),

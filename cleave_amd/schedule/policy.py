@@ -603,6 +603,14 @@ def attn_phased_ok(p, kpre) -> bool:
             and (kpre or "k" not in (p.get("norm_eps") or {})))
 
 
+def combine_groups(rows, vdim, splits) -> int:
+    """Thread groups that share the splits of a row in the combine of f32 partials, or 1: one thread adds up all of them.  The line
+    lies between 256 x 128 values of 32 splits (25.1 us with one thread each, 23.9 with groups) and 256 x 512 of 16 (18.0 / 18.3)."""
+    if splits <= 16 or vdim % 64 or rows * vdim > 64 * 1024:
+        return 1
+    return 8 if vdim % 128 == 0 else 16
+
+
 # ----------------------------------------------------------------------------- MLA decode
 def mla_lds_bytes(ckv, kpe, stages=3):
     """`stages` token-major images of a 32-token step: (ckv + kpe) / 64 panels of 32 x 64 elements."""
@@ -691,6 +699,30 @@ def mla_candidates(low, role, factor, arch: Arch):
                             (dict(DUO=1, LDS_AHEAD=4, S_PANELS=shared), 0.755)):
             out.append(TileDict("mla_decode", role, tiling, output_tile=[64, p["ckv"]], rstep_map={"kv": 32},
                                 n_threads=512, split_factor=factor, score=rel * best, lds_bytes=duo_lds, est_vgprs=208))
+    if role == "main" and not p.get("emit_lse") and out:
+        out += mla_key_ranges(p, min(out, key=lambda c: (c.score, c.key())), arch)
+    return out
+
+
+def mla_key_ranges(p, base, arch: Arch):
+    """Latent attention of too few workgroups for the chip: the keys dealt out to ranges inside an unsplit operator, f32 partials
+    in scratch, folded by a second launch.  As many ranges as give every compute unit the workgroups it holds, and one or half a
+    workgroup each: requests x heads x keys, us, one range / ranges: 3 x 16 x 7233 345 / 15.5 (57; 30 with 16), 24 x 16 x 2869 156 / 24.1
+    (18; 28.1 with 10, 39.4 with 5), 2 x 16 x 639 34 / 8.2 (20; 9.9 with 10), 6 x 128 x 7649 198 / 28.8 (20; 34.0 as the split form
+    at 8).  The split form, where a program asks for it, stays ahead for 64 heads and more on few keys, whose partials it halves
+    by keeping them in 16 bits: 4 x 64 x 1819 15.7 (8) against 17.7 (12)."""
+    rows, steps = p["batch"] * p["heads"], _ceil(p["skv"], 32)
+    blocks = p["batch"] * _ceil(p["heads"], base.output_tile[0])
+    out, seen = [], set()
+    per_cu = min(2, max(1, arch.blocks_per_cu(base.n_threads, base.lds_bytes, base.est_vgprs)))
+    for fill in sorted({arch.compute_units * per_cu, arch.compute_units, arch.compute_units // 2}, reverse=True):
+        n = min(fill // blocks, steps, 64)
+        n = _ceil(steps, _ceil(steps, n)) if n > 1 else 0              # (no empty ranges)
+        if n > 1 and n not in seen and n * rows * (p["ckv"] + 2) * 4 + 3 * 256 <= FIXED_SCRATCH:
+            seen.add(n)
+            tiling = dict(base.tiling, KEYS=n)
+            out.append(TileDict(base.template, base.role, tiling, output_tile=base.output_tile, rstep_map=base.rstep_map, n_threads=base.n_threads,
+                                score=base.score / n, lds_bytes=base.lds_bytes, est_vgprs=base.est_vgprs, late=True))
     return out
 
 

@@ -1,0 +1,56 @@
+"""Latent attention whose keys are dealt out to ranges inside an unsplit operator: key counts at the edges of a step and of a range,
+workgroups of 16 heads and of score and value waves, one and two head blocks to a range, batches that are and are not whole eights, and
+both forms of the combine (up to 16 ranges one thread adds up, above that groups of threads).  The combine of an operator of 16 or 32
+heads is a kernel by itself."""
+
+import numpy as np
+import pytest
+import torch
+
+import cleave_amd.lang as cl
+from cleave_amd import examples as C
+from cleave_amd.codegen import HipCodeGen
+from cleave_amd.lower.stages import split_stages
+from cleave_amd.pipeline.direct import kernel_for, stage_graph
+from cleave_amd.runtime.compile import _compile, _load_main_kernel_from_code
+from cleave_amd.schedule import apply_tiling, search_tiling
+from cleave_amd.schedule.policy import combine_groups
+from oracle import program_oracle
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("skv,ranges", [(33, 2), (64, 2), (65, 3), (289, 8), (1043, 5), (1043, 33), (703, 22)])
+@pytest.mark.parametrize("batch,heads,tiling", [(3, 16, dict(WAVES=1, STAGES=2)), (1, 32, dict(WAVES=2)), (2, 64, dict(DUO=1)),
+                                                (3, 128, dict(DUO=1, LDS_AHEAD=4, S_PANELS=4)), (8, 64, dict(DUO=1))],
+                         ids=["h16", "h32", "duo", "duo128", "duo8"])
+def test_ranges(batch, heads, tiling, skv, ranges):
+    shapes = dict(B=batch, H=heads, D=512, PE=64, SKV=skv)
+    prog = C.mla_decode.trace(cl.bf16, **shapes)
+    args = prog.random_inputs(seed=skv, device="cpu")
+    print(f"mla ranges {shapes} {tiling} {ranges}", flush=True)
+    got = kernel_for(prog, template="mla_decode", tiling=dict(tiling, KEYS=ranges))(*[a.cuda() for a in args])
+    torch.cuda.synchronize()
+    want = program_oracle.evaluate(prog, args)[0]
+    got = got.float().cpu().numpy().reshape(want.shape)
+    # weights rounded to 8 bits (2^-9 each, of either sign) and one rounding of the result (2^-9)
+    assert np.linalg.norm(got - want) / np.linalg.norm(want) < 2.0 ** -7
+    np.testing.assert_allclose(got, want, rtol=1e-2, atol=1e-2)
+
+
+@pytest.mark.parametrize("heads", [16, 32, 64])
+def test_the_combine_is_a_kernel_by_itself(heads):
+    graph = stage_graph(C.mla_decode.trace(cl.bf16, B=2, H=heads, D=512, PE=64, SKV=640))
+    combine = split_stages(graph, 8)[1]
+    source = HipCodeGen().gen(apply_tiling(search_tiling(combine)[0]))
+    assert _compile(_load_main_kernel_from_code(source), None).stats[0]["spilled_vgprs"] == 0
+
+
+def test_search_proposes_them_where_workgroups_are_few():
+    def ranges(**shapes):
+        return [c.tiling["KEYS"] for c in search_tiling(stage_graph(C.mla_decode.trace(cl.bf16, D=512, PE=64, **shapes)), topk=8) if "KEYS" in c.tiling]
+
+    assert ranges(B=3, H=16, SKV=7233) == [57, 38] and ranges(B=24, H=16, SKV=2869) == [18, 10, 5]
+    assert ranges(B=6, H=128, SKV=7649) == [20, 10] and ranges(B=32, H=128, SKV=8192)[:1] == [4]
+    assert ranges(B=2, H=16, SKV=32) == [] and ranges(B=32, H=16, SKV=40) == [2]
+    assert combine_groups(48, 512, 57) == 8 and combine_groups(48, 64, 17) == 16
+    assert combine_groups(48, 512, 16) == combine_groups(384, 512, 18) == combine_groups(48, 96, 57) == 1
