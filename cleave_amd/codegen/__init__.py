@@ -22,6 +22,7 @@ import math
 from pathlib import Path
 
 from ..core.errors import CodegenError
+from ..core.target import current_target
 from ..lower.stages import mla_po_elem
 from ..schedule.plan import KernelPlan, ParamSpec
 
@@ -36,7 +37,7 @@ LOG2E = 1.4426950408889634
 # The operands that a template moves from global memory straight into LDS in 16-byte pieces.  Such a load needs its pieces
 # at multiples of 16 bytes; everything else is read through registers, which takes any element's address.
 DIRECT_TO_LDS = {"gemm_tile.hip": ("A", "B", "C"), "mla_decode.hip": ("KV", "KPE"), "mla_paged_decode.hip": ("KV", "KPE"),
-                 "mla_decode_duo.hip": ("Q", "QPE", "KV", "KPE"), "attn_prefill_lds.hip": ("K", "V"),
+                 "mla_decode_duo.hip": ("Q", "QPE", "KV", "KPE"), "mla_prefill_duo.hip": ("Q", "QPE", "KV", "KPE"), "attn_prefill_lds.hip": ("K", "V"),
                  "attn_phased.hip": ("K", "V")}
 
 _C_TYPES = {"float16": "elem_t", "bfloat16": "elem_t", "float32": "float", "int32": "int"}
@@ -89,9 +90,10 @@ class _Unit:
         self.define(macro, ", ".join(parts))
         return [p.name for p in params] + list(dyn_dims)
 
-    def launch(self, entry, grid, block, lds, args):
+    def launch(self, entry, grid, block, lds, args, optional=False):
+        """``optional``: left out where its grid is empty (any other empty grid means that the call has nothing to do)."""
         self.launches.append({"entry": entry, "grid": [str(g) for g in grid], "block": [int(block), 1, 1],
-                              "lds": int(lds), "args": list(args)})
+                              "lds": int(lds), "args": list(args), **({"optional": True} if optional else {})})
 
 
 class HipCodeGen:
@@ -818,9 +820,7 @@ class HipCodeGen:
                 raise CodegenError("score waves and value waves on a token table: causal prefill with four query tokens per item, a "
                                    "latent width in multiples of 128, a rope width of an odd number of 64s, and four images "
                                    "within 160 KiB of LDS")
-            unit.templates += ["mla_decode_duo.hip", "attn_combine.hip"]
-            # (the item axis is padded to a multiple of 8: the kernel deals runs of items out to the XCDs)
-            unit.launch(ENTRY, (f"ceildiv(ceildiv({p['dim_names']['total_q']}, 4) + batch, 8) * 8", p["heads"] // 16, 1), 512, 0, self._partial_args)
+            self._mla_prefill_duo(unit, plan, params)
             return
         unit.templates += ["mla_paged_decode.hip", "attn_combine.hip"]
         if partial:
@@ -831,6 +831,35 @@ class HipCodeGen:
         if combine:
             entry, args = self._combine_args
             unit.launch(entry, (f"ceildiv(({batch_name} * {p['heads']}) * {p['ckv'] // 4}, 256)", 1, 1), 256, 0, args)
+
+
+    def _mla_prefill_duo(self, unit, plan, params):
+        """The launches of the score-wave / value-wave prefill: one workgroup an item, or, for more than ``few`` items, workgroups that stay
+        and draw them (a counter in scratch, cleared by a launch of its own).  Either is left out where the other runs.
+
+        The line lies at three rounds of one workgroup per compute unit.  us, one workgroup an item / that stay, 16 heads: 1380 items
+        of 24 requests 95.1 / 86.3, 2336 of 32 149.9 / 137.8, 1136 of 16 68.3 / 65.0; 568 of 8 33.8 / 34.9, 520 of 32 (up to 160 keys)
+        25.7 / 25.8, 464 of 12 24.1 / 26.7: there the clearing launch (2 us) and the last round's uneven ends outweigh what overlaps."""
+        p = plan.problem
+        dyn = tuple(plan.dyn_dims) + tuple(name for name, _ in plan.extra["derived_dims"])
+        groups, units = p["heads"] // 16, current_target().arch.compute_units // 8 * 8
+        # (the item axis is padded to a multiple of 8: the kernels deal runs of items out to the XCDs)
+        items = f"ceildiv(ceildiv({p['dim_names']['total_q']}, 4) + batch, 8) * 8"
+        few = int(plan.tiling.get("FEW", 3 * units)) // groups
+        stay = f"min(max({items} - {few}, 0), 1)"
+        tickets = ParamSpec("Tickets", "int32", (f"64 * {stay}",), "scratch")
+        at = next(i for i, q in enumerate(params) if q.role == "output")
+        params.insert(at, tickets)
+        dyn_c = tuple(p["dim_names"]) + tuple(name for name, _ in plan.extra["derived_dims"])
+        unit.define("CL_EMIT_STAY", 1)
+        unit.define("CL_ARG_TICKETS", tickets.name)
+        zero = unit.signature("CL_TICKETS_PARAMS", "CL_TICKETS_NAME", ENTRY + "_tickets", [tickets], ())
+        walk = unit.signature("CL_STAY_PARAMS", "CL_STAY_NAME", ENTRY + "_stay",
+                              [q for q in params if q.role in ("input", "scalar")] + [tickets] + [q for q in params if q.role == "output"], dyn, dyn_c)
+        unit.templates += ["mla_decode_duo.hip", "mla_prefill_duo.hip"]
+        unit.launch(ENTRY, (f"{items} * (1 - {stay})", groups, 1), 512, 0, self._partial_args, optional=True)
+        unit.launch(ENTRY + "_tickets", (stay, 1, 1), 64, 0, zero, optional=True)
+        unit.launch(ENTRY + "_stay", (f"{units} * {stay}", 1, 1), 512, 0, walk, optional=True)
 
 
 def aligned_inputs(source: str, params) -> frozenset:

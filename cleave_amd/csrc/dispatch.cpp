@@ -115,6 +115,7 @@ struct Launch {
   void* fn;
   Expr grid[3];
   uint32_t block[3], lds;
+  bool optional;                 // left out where its grid is empty; any other empty grid means that the call has nothing to do
   std::vector<Value> values;
 };
 
@@ -246,12 +247,12 @@ PyObject* call_plain(PyObject* self_, PyObject* const* argv, size_t nargsf, PyOb
     dim_value[i] = (int32_t)dims[i];
   }
   uint32_t grids[8][3];
-  bool empty = false;
+  bool empty = false, left_out[8] = {};
   for (size_t l = 0; l < self->launches->size(); ++l)
     for (int k = 0; k < 3; ++k) {
       int64_t v;
       if (!evaluate((*self->launches)[l].grid[k], dims, &v)) MISS();
-      if (v < 1) empty = true;
+      if (v < 1) ((*self->launches)[l].optional ? left_out[l] : empty) = true;
       else if (v > (k == 0 ? (int64_t)INT32_MAX : 65535)) MISS();
       else grids[l][k] = (uint32_t)v;
     }
@@ -285,8 +286,10 @@ PyObject* call_plain(PyObject* self_, PyObject* const* argv, size_t nargsf, PyOb
       at_byte[i] = total;
       total += (v + 255) / 256 * 256;
     }
-    scratch = fresh({total}, at::kByte);
-    for (size_t i = 0; i < self->temps->size(); ++i) temp_ptr[i] = static_cast<char*>(scratch.data_ptr()) + at_byte[i];
+    // (nothing where only launches that are left out have scratch)
+    if (total) scratch = fresh({total}, at::kByte);
+    char* const base = total ? static_cast<char*>(scratch.data_ptr()) : nullptr;
+    for (size_t i = 0; i < self->temps->size(); ++i) temp_ptr[i] = base + at_byte[i];
   }
   if (!empty) {
     PyObject* index = PyLong_FromLong(device);
@@ -302,6 +305,7 @@ PyObject* call_plain(PyObject* self_, PyObject* const* argv, size_t nargsf, PyOb
     int failed = 0;
     for (size_t l = 0; l < self->launches->size() && !failed; ++l) {
       const Launch& q = (*self->launches)[l];
+      if (left_out[l]) continue;
       void* values[kMaxValues];
       int nv = 0;
       for (const Value& v : q.values)
@@ -405,7 +409,9 @@ bool read_plan(Plan* p, PyObject* args, PyObject* derived, PyObject* outs, PyObj
         unsigned long long fn;
         PyObject *grid, *values;
         unsigned bx, by, bz, lds;
-        if (!PyArg_ParseTuple(o, "KO(III)IO", &fn, &grid, &bx, &by, &bz, &lds, &values)) return false;
+        int optional = 0;
+        if (!PyArg_ParseTuple(o, "KO(III)IO|i", &fn, &grid, &bx, &by, &bz, &lds, &values, &optional)) return false;
+        l.optional = optional != 0;
         l.fn = reinterpret_cast<void*>(fn);
         l.block[0] = bx; l.block[1] = by; l.block[2] = bz;
         l.lds = lds;

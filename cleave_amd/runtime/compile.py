@@ -275,6 +275,9 @@ class CompiledKernel:
         into its fixed scratch array."""
         keep, descs = [], []
         for l in self.manifest["launches"]:
+            grid = [eval_extent(g, dims) for g in l["grid"]]
+            if min(grid) < 1 and l.get("optional"):
+                continue           # a launch that this call has no use for
             values = []
             for name in l["args"]:
                 if name in dims and name not in bound:
@@ -292,7 +295,6 @@ class CompiledKernel:
                 else:
                     values.append(("ptr", v.data_ptr()))
             packed = shim.PackedArgs(values)
-            grid = [eval_extent(g, dims) for g in l["grid"]]
             if min(grid) < 1:
                 return None, None  # an empty problem (e.g. batch == 0): nothing to launch
             if grid[1] > 65535 or grid[2] > 65535 or grid[0] > 2 ** 31 - 1:

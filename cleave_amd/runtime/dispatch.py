@@ -178,7 +178,7 @@ def chain_plan(stages, *, arguments=None, output_shapes=None, as_tuple=False):
             block = list(launch["block"]) + [1] * (3 - len(launch["block"]))
             grid = list(launch["grid"]) + [1] * (3 - len(launch["grid"]))
             launches.append((kernel.module.function(launch["entry"]), [postfix(_number(g), dims) for g in grid],
-                             tuple(int(b) for b in block), int(launch["lds"]), values))
+                             tuple(int(b) for b in block), int(launch["lds"]), values, int(bool(launch.get("optional")))))
         before = produced
     lib = shim.load()
     return module.make_plan(args, n_dims, derived, outs, temps, launches, 2 if as_tuple else 1 if outs else 0,
