@@ -486,6 +486,14 @@ class HipCodeGen:
         params[at:at] = scratch
         return dataclasses.replace(plan, role="fused", operands=operands, split_factor=keys)
 
+    def _launch_chunk_combine(self, unit, rows, vdim):
+        """The launch that merges the partials of chunked items: groups of threads share the items of a row."""
+        from ..schedule.policy import COMBINE_GROUPS
+
+        groups = next(n for n in COMBINE_GROUPS if vdim * n % 1024 == 0)
+        unit.define("CL_COMBINE_GROUPS", groups)
+        unit.launch(self._combine_args[0], (f"{rows} * {vdim * groups // 1024}", 1, 1), 256, 0, self._combine_args[1])
+
     def _launch_combine(self, unit, rows, vdim, splits, po_elem=False, plain=None):
         """The launch that merges the f32 (or, ``po_elem``, element-type) partials of ``splits`` key ranges.
         ``plain``: the grid of one thread per piece, where it is written otherwise."""
@@ -563,7 +571,9 @@ class HipCodeGen:
             unit.launch(ENTRY, grid, waves * 64, lds, self._partial_args)
         if combine:
             plain = f"ceildiv({grid_rows} * {p['vdim'] // 4}, 256)"
-            if paged:
+            if chunk_pages:
+                self._launch_chunk_combine(unit, grid_rows, p["vdim"])
+            elif paged:
                 unit.launch(self._combine_args[0], (plain, 1, 1), 256, 0, self._combine_args[1])
             else:
                 self._launch_combine(unit, total_rows, p["vdim"], splits, plain=plain)
@@ -829,8 +839,7 @@ class HipCodeGen:
                 items = f"ceildiv({p['dim_names']['total_q']}, {tok}) + batch"
             unit.launch(ENTRY, (items, p["heads"] // 16, 1), 64 * max(tok, ksplit), 0, self._partial_args)
         if combine:
-            entry, args = self._combine_args
-            unit.launch(entry, (f"ceildiv(({batch_name} * {p['heads']}) * {p['ckv'] // 4}, 256)", 1, 1), 256, 0, args)
+            self._launch_chunk_combine(unit, f"({batch_name} * {p['heads']})", p["ckv"])
 
 
     def _mla_prefill_duo(self, unit, plan, params):

@@ -10,35 +10,74 @@
 #ifndef CL_COMBINE_GROUPS
 #define CL_COMBINE_GROUPS 1
 #endif
+#if CL_EMIT_COMBINE && CL_COMBINE_GROUPS > 1
+// Where CL_COMBINE_GROUPS groups of threads share the partials of a row's CB_COLS columns (thread t: group t / CB_THREADS, columns
+// 4 (t % CB_THREADS) .. + 3): each adds its own up against the largest of their reference points, and the first group adds the
+// groups' sums up out of LDS.
+#define CB_THREADS (256 / CL_COMBINE_GROUPS)
+#define CB_COLS (4 * CB_THREADS)
+static_assert(256 % CL_COMBINE_GROUPS == 0 && CL_VDIM % CB_COLS == 0, "a workgroup takes whole pieces of one row");
+__shared__ __attribute__((aligned(16))) f32x4 cb_o[CL_COMBINE_GROUPS][CB_THREADS];
+__shared__ f32x2 cb_ml[CL_COMBINE_GROUPS];
+// the row's columns from `out` on, and with `lse` (column 0) its log-sum-exp; m, l, o: this group's reference point, sum and values
+CL_DEVICE void cb_finish(float m, float l, f32x4 o, elem_t* out, float* lse) {
+  const int group = threadIdx.x / CB_THREADS, at = threadIdx.x % CB_THREADS;
+  cb_o[group][at] = o;
+  if (at == 0) cb_ml[group] = (f32x2){m, l};
+  __syncthreads();
+  if (group != 0) return;
+  f32x2 ml[CL_COMBINE_GROUPS];
+  float top = CL_NEG_BIG;
+#pragma unroll
+  for (int k = 0; k < CL_COMBINE_GROUPS; ++k) {
+    ml[k] = cb_ml[k];
+    top = fmaxf(top, ml[k][0]);
+  }
+  l = 0.f;
+  o = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int k = 0; k < CL_COMBINE_GROUPS; ++k) {
+    const float f = fast_exp2(ml[k][0] - top);
+    l += ml[k][1] * f;
+    o += cb_o[k][at] * f;
+  }
+  const float inv = 1.0f / fmaxf(l, 1.0e-30f);
+  elem4 r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r[i] = to_elem(o[i] * inv);
+  *reinterpret_cast<elem4*>(out) = r;
+  if (lse) *lse = l > 0.f ? top + fast_log2(l) : CL_NEG_INF;
+}
+#endif
 #if CL_CHUNK_PAGES && CL_EMIT_COMBINE
-// Combine of chunked items: request b owns items b + p0/C .. b + (p1-1)/C (p0, p1 its page-table
-// range); partials are (item, query head[, d]).  One thread per (request, head, 4 d).
+// Combine of chunked items: request b owns items b + p0/C .. b + (p1-1)/C (p0, p1 its page-table range); partials are (item,
+// query head[, d]).  A group takes every CL_COMBINE_GROUPS-th item, CB_EACH of them at a time, every load of a round issued before
+// the first use (the trip count is a run-time value: left alone, each item's loads wait for the previous item's); the running
+// maximum is carried along and the sums rescaled when a round raises it; slots past the end repeat the last item with weight zero.
+// What bounds it: round trips to memory, of which a request of up to CB_EACH * CL_COMBINE_GROUPS items costs one: one thread walking all
+// items of its columns, eight at a time, was most of a call of few long requests.  us, one thread / groups, f16, 32 / 8 heads, pages of 64: one
+// request of 12705 keys (199 items) 34.2 / 16.7, 2 of up to 3644 17.6 / 12.6, 6 of 4345 20.9 / 15.4, 19 of 1787 17.8 / 15.8, 12 of 9000
+// 49.2 / 45.7, 45 of 6963 (seven items each) 119.8 / 119.8.
+#define CB_EACH 4
 extern "C" __global__ void __launch_bounds__(256)
 CL_COMBINE_NAME(CL_COMBINE_PARAMS) {
-  const i64 total = (i64)CL_TOTAL_ROWS * (CL_VDIM / 4);
-  const i64 idx = (i64)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= total) return;
-  const i64 row = idx / (CL_VDIM / 4);
-  const int d = (int)(idx % (CL_VDIM / 4)) * 4;
+  const i64 row = (i64)blockIdx.x / (CL_VDIM / CB_COLS);
+  const int group = threadIdx.x / CB_THREADS, at = threadIdx.x % CB_THREADS;
+  const int d = (int)(blockIdx.x % (CL_VDIM / CB_COLS)) * CB_COLS + 4 * at;
   const int req = (int)(row / CL_Q_HEADS), qh = (int)(row % CL_Q_HEADS);
   int p0 = CL_CARG_INDPTR[req], p1 = CL_CARG_INDPTR[req + 1];
   p0 = p0 < 0 ? 0 : (p0 > n_idx ? n_idx : p0);
   p1 = p1 < 0 ? 0 : (p1 > n_idx ? n_idx : p1);
   const int first = req + p0 / chunk_pages;
   const int count = p1 > p0 ? (p1 - 1) / chunk_pages - p0 / chunk_pages + 1 : 0;
-  // One pass, eight items at a time, every load of a group issued before the first use (the trip
-  // count is a run-time value: left alone, each item's loads wait for the previous item's).  The
-  // running maximum is carried along and the sums rescaled when a group raises it, so a request of
-  // up to eight items costs one round trip to memory; slots past the end repeat the last item with
-  // weight zero.
   float m = CL_NEG_BIG, l = 0.f;
   f32x4 o = (f32x4){0.f, 0.f, 0.f, 0.f};
-  for (int s = 0; s < count; s += 8) {
-    float pm[8], pl[8];
-    f32x4 po[8];
+  for (int s = group; s < count; s += CB_EACH * CL_COMBINE_GROUPS) {
+    float pm[CB_EACH], pl[CB_EACH];
+    f32x4 po[CB_EACH];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int it = s + u < count ? s + u : count - 1;
+    for (int u = 0; u < CB_EACH; ++u) {
+      const int it = s + u * CL_COMBINE_GROUPS < count ? s + u * CL_COMBINE_GROUPS : count - 1;
       const i64 prow = (i64)(first + it) * CL_Q_HEADS + qh;
       pm[u] = CL_CARG_PM[prow];
       pl[u] = CL_CARG_PL[prow];
@@ -46,25 +85,22 @@ CL_COMBINE_NAME(CL_COMBINE_PARAMS) {
     }
     float m_new = m;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) m_new = fmaxf(m_new, pm[u]);   // (a repeated item's maximum is one the group has anyway)
+    for (int u = 0; u < CB_EACH; ++u) m_new = fmaxf(m_new, pm[u]);   // (a repeated item's maximum is one the row has anyway)
     const float keep = fast_exp2(m - m_new);
     m = m_new;
     l *= keep;
     o *= keep;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const float f = s + u < count ? fast_exp2(pm[u] - m) : 0.f;
+    for (int u = 0; u < CB_EACH; ++u) {
+      const float f = s + u * CL_COMBINE_GROUPS < count ? fast_exp2(pm[u] - m) : 0.f;
       l += pl[u] * f;
       o += po[u] * f;
     }
   }
-  const float inv = 1.0f / fmaxf(l, 1.0e-30f);
-  elem4 r;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) r[i] = to_elem(o[i] * inv);
-  *reinterpret_cast<elem4*>(CL_CARG_OUT + row * CL_VDIM + d) = r;
 #if CL_EMIT_LSE
-  if (d == 0) CL_CARG_LSE[row] = l > 0.f ? m + fast_log2(l) : CL_NEG_INF;
+  cb_finish(m, l, o, CL_CARG_OUT + row * CL_VDIM + d, d == 0 ? CL_CARG_LSE + row : nullptr);
+#else
+  cb_finish(m, l, o, CL_CARG_OUT + row * CL_VDIM + d, nullptr);
 #endif
 }
 #elif CL_SPLITS > 1 && CL_EMIT_COMBINE && CL_PO_ELEM
@@ -109,20 +145,13 @@ CL_COMBINE_NAME(CL_COMBINE_PARAMS) {
 #endif
 }
 #elif CL_SPLITS > 1 && CL_EMIT_COMBINE && CL_COMBINE_GROUPS > 1
-// The rule of the next kernel where rows are few and splits are many: CL_COMBINE_GROUPS groups of threads share the splits of a
-// row's CB_COLS columns (thread t: group t / CB_THREADS, columns 4 (t % CB_THREADS) .. + 3), each adds up its own against the
-// largest of their reference points, and the first group adds the groups' sums up out of LDS.
+// The rule of the next kernel where rows are few and splits are many, by groups of threads.
 // What bounds it: one round trip to memory, which one thread that reads 57 splits makes in parts.  Whole operators, us, one thread /
 // groups: 48 rows x 512 of 57 splits 20.2 / 15.5, 32 x 512 of 20 8.8 / 8.2, 256 x 128 of 32 25.1 / 23.9; behind where splits are
 // fewer or rows enough to fill the chip: 384 x 512 of 18 23.7 / 24.0, 256 x 512 of 16 18.0 / 18.3, 11 x 128 of 8 6.7 / 6.9.
-#define CB_THREADS (256 / CL_COMBINE_GROUPS)
-#define CB_COLS (4 * CB_THREADS)
 #define CB_EACH ((CL_SPLITS + CL_COMBINE_GROUPS - 1) / CL_COMBINE_GROUPS)
-static_assert(256 % CL_COMBINE_GROUPS == 0 && CL_VDIM % CB_COLS == 0, "a workgroup takes whole pieces of one row");
 extern "C" __global__ void __launch_bounds__(256)
 CL_COMBINE_NAME(CL_COMBINE_PARAMS) {
-  __shared__ __attribute__((aligned(16))) f32x4 part_o[CL_COMBINE_GROUPS][CB_THREADS];
-  __shared__ f32x2 part_ml[CL_COMBINE_GROUPS];
   const i64 row = (i64)blockIdx.x / (CL_VDIM / CB_COLS);
   const int group = threadIdx.x / CB_THREADS, at = threadIdx.x % CB_THREADS;
   const int d = (int)(blockIdx.x % (CL_VDIM / CB_COLS)) * CB_COLS + 4 * at;
@@ -147,32 +176,10 @@ CL_COMBINE_NAME(CL_COMBINE_PARAMS) {
     l += pl[u] * f;
     o += po[u] * f;
   }
-  part_o[group][at] = o;
-  if (at == 0) part_ml[group] = (f32x2){m, l};
-  __syncthreads();
-  if (group != 0) return;
-  f32x2 ml[CL_COMBINE_GROUPS];
-  float top = CL_NEG_BIG;
-#pragma unroll
-  for (int k = 0; k < CL_COMBINE_GROUPS; ++k) {
-    ml[k] = part_ml[k];
-    top = fmaxf(top, ml[k][0]);
-  }
-  l = 0.f;
-  o = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int k = 0; k < CL_COMBINE_GROUPS; ++k) {
-    const float f = fast_exp2(ml[k][0] - top);
-    l += ml[k][1] * f;
-    o += part_o[k][at] * f;
-  }
-  const float inv = 1.0f / fmaxf(l, 1.0e-30f);
-  elem4 r;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) r[i] = to_elem(o[i] * inv);
-  *reinterpret_cast<elem4*>(CL_CARG_OUT + row * CL_VDIM + d) = r;
 #if CL_EMIT_LSE
-  if (d == 0) CL_CARG_LSE[row] = l > 0.f ? top + fast_log2(l) : CL_NEG_INF;
+  cb_finish(m, l, o, CL_CARG_OUT + row * CL_VDIM + d, d == 0 ? CL_CARG_LSE + row : nullptr);
+#else
+  cb_finish(m, l, o, CL_CARG_OUT + row * CL_VDIM + d, nullptr);
 #endif
 }
 #elif CL_SPLITS > 1 && CL_EMIT_COMBINE

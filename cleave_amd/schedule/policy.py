@@ -603,12 +603,15 @@ def attn_phased_ok(p, kpre) -> bool:
             and (kpre or "k" not in (p.get("norm_eps") or {})))
 
 
+COMBINE_GROUPS = (8, 16)         # of 32 threads, 128 columns; of 16 threads where the values are an odd number of 64s wide
+
+
 def combine_groups(rows, vdim, splits) -> int:
     """Thread groups that share the splits of a row in the combine of f32 partials, or 1: one thread adds up all of them.  The line
     lies between 256 x 128 values of 32 splits (25.1 us with one thread each, 23.9 with groups) and 256 x 512 of 16 (18.0 / 18.3)."""
     if splits <= 16 or vdim % 64 or rows * vdim > 64 * 1024:
         return 1
-    return 8 if vdim % 128 == 0 else 16
+    return next(n for n in COMBINE_GROUPS if vdim * n % 1024 == 0)
 
 
 # ----------------------------------------------------------------------------- MLA decode
