@@ -31,7 +31,8 @@
 //                XCD.  Every step still belongs to exactly one split.  (Even split counts, grid x
 //                a multiple of eight; the search times a few values.)
 //   CL_CHUNK_PAGES  paged only, 0 = off.  1: work is cut into items of at most `chunk_pages`
-//                pages (a run-time argument, 1..64, chosen by the host from the table length)
+//                pages (a run-time argument, 1..64, chosen by the host from the table length; of a
+//                token table, page size 1, up to 2048 entries)
 //                instead of a fixed number of splits per request, and a workgroup holds one wave
 //                per kv head, so that the eight waves together stream whole contiguous token
 //                rows of the cache and a long request costs many items rather than long ones.
@@ -76,7 +77,12 @@ struct AttUnit {
   i64 out_row;          // flattened (unit, row) index of the tile's first row
 };
 
-#if CL_PAGED && CL_CHUNK_PAGES
+#if CL_PAGED && CL_CHUNK_PAGES && CL_PAGE_SIZE == 1
+// Token tables: the (clamped) ids of an item's tokens lie in LDS, read once by all waves, the last one repeated up to a whole step.
+// (A lane's registers hold 64 of them, two steps; a table load per token would sit in the same in-order queue as the rows.)
+#define ATT_MAX_IDS 2048
+__shared__ __attribute__((aligned(16))) int att_ids[ATT_MAX_IDS];
+#elif CL_PAGED && CL_CHUNK_PAGES
 // An item's page ids were read once into one register per lane; a token's page id comes from
 // the lane that holds it.  A page-table load per token would sit in the same in-order load
 // queue as the K/V rows and make every prefetch wait for the rows of the step before it.
@@ -108,6 +114,27 @@ struct AttTile {               // one 32-token step's K and V, as loaded
 // Issue the loads of the step starting at token t0.  Tokens past kv_len are clamped onto the
 // last valid token (their scores are masked later), so no load leaves the tensor.
 CL_DEVICE void att_load(const AttUnit& u, int t0, int c, int g, AttTile& tile) {
+#if CL_PAGED && CL_CHUNK_PAGES && CL_PAGE_SIZE == 1
+  typedef int att_i32x4 __attribute__((ext_vector_type(4)));
+  const int id_k[2] = {att_ids[t0 + c], att_ids[t0 + 16 + c]};
+  const att_i32x4 id_v[2] = {*reinterpret_cast<const att_i32x4*>(&att_ids[t0 + 4 * g]), *reinterpret_cast<const att_i32x4*>(&att_ids[t0 + 16 + 4 * g])};
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const elem_t* row = u.k + (i64)id_k[h] * u.k_stride + 8 * g;
+#pragma unroll
+    for (int j = 0; j < ATT_KJ; ++j) tile.k[h][j] = ld16(row + 32 * j);
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const elem_t* row = u.v + (i64)id_v[e >> 2][e & 3] * u.v_stride;
+#pragma unroll
+    for (int vc = 0; vc < ATT_VC; ++vc) {
+      int col = 128 * vc + 8 * c;
+      if (CL_VDIM % 128 != 0) col = col < CL_VDIM - 8 ? col : CL_VDIM - 8;
+      tile.v[vc][e] = ld16(row + col);
+    }
+  }
+#else
   const int last = u.kv_len - 1;
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
@@ -129,6 +156,7 @@ CL_DEVICE void att_load(const AttUnit& u, int t0, int c, int g, AttTile& tile) {
       tile.v[vc][e] = ld16(row + col);
     }
   }
+#endif
 }
 
 #if CL_CHUNK_PAGES
@@ -194,11 +222,21 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
   u.pages = CL_ARG_INDICES + lo;
   u.n_pages = hi - lo;
   u.pool_pages = num_pages;
+#if CL_PAGE_SIZE == 1
+  for (int i = threadIdx.x; i < (u.n_pages + ATT_STEP - 1) / ATT_STEP * ATT_STEP; i += CL_WAVES * 64) {
+    int pid = u.pages[i < u.n_pages ? i : u.n_pages - 1];
+    pid = pid < num_pages - 1 ? pid : num_pages - 1;
+    att_ids[i] = pid > 0 ? pid : 0;
+  }
+  u.page_reg = 0;
+  __syncthreads();
+#else
   {
     int pid = u.pages[lane < u.n_pages ? lane : u.n_pages - 1];
     pid = pid < num_pages - 1 ? pid : num_pages - 1;
     u.page_reg = pid > 0 ? pid : 0;
   }
+#endif
   u.k_stride = (i64)CL_KV_HEADS * CL_HEAD_DIM;
   u.v_stride = (i64)CL_KV_HEADS * CL_VDIM;
   u.k = CL_ARG_K + (i64)head * CL_HEAD_DIM;

@@ -217,16 +217,23 @@ def _plan(spec, dense, role, params, operands, split=None) -> KernelPlan:
 
 
 MAX_CHUNK_PAGES = 64      # an item's page ids live in one register per lane of a wave
+MAX_CHUNK_TOKENS = 2048   # ... or, of a token table (page size 1), in LDS
+
+
+def max_chunk_pages(spec) -> int:
+    return MAX_CHUNK_TOKENS if getattr(spec, "page_size", 1) == 1 else MAX_CHUNK_PAGES
 
 
 def chunk_pages_expr(spec, chunk_pages: int) -> str:
     """The launch-time expression for the item size: the fixed value, or for -1 the size that
     spreads the table over the machine's compute units (each request boundary adds an item)."""
     if chunk_pages > 0:
-        return str(min(chunk_pages, MAX_CHUNK_PAGES))
+        return str(min(chunk_pages, max_chunk_pages(spec)))
     from ...core.target import current_target
 
     cus = current_target().arch.compute_units
+    if getattr(spec, "page_size", 1) == 1:       # whole 32-token steps
+        return f"max(32, min({MAX_CHUNK_TOKENS}, ceildiv(ceildiv({spec.index_dim}, max(1, {cus} - {spec.batch_dim})), 32) * 32))"
     return (f"max(1, min({MAX_CHUNK_PAGES}, ceildiv({spec.index_dim}, "
             f"max(1, {cus} - {spec.batch_dim}))))")
 
@@ -450,9 +457,9 @@ def build_split_decode(spec, dense: DenseAttention, split: int, comb: CombineTil
     # split-major partials: one request's splits sit one stride apart
     # (python/cleave/dynamic/paging/tensor_maps.py:41-69)
     if dense.chunk_pages:
-        if dense.chunk_pages < -1 or dense.chunk_pages > MAX_CHUNK_PAGES or dense.query_rows > 16 \
+        if dense.chunk_pages < -1 or dense.chunk_pages > max_chunk_pages(spec) or dense.query_rows > 16 \
                 or spec.num_kv_heads > 16:
-            raise UnsupportedTiling(f"chunked items need chunk_pages in 1..{MAX_CHUNK_PAGES} (or -1), one 16-row "
+            raise UnsupportedTiling(f"chunked items need chunk_pages in 1..{max_chunk_pages(spec)} (or -1), one 16-row "
                                     "query tile and at most 16 kv heads")
         # one partial per work item: a new item at every chunk_pages table entries and every request
         items = f"ceildiv({spec.index_dim}, chunk_pages) + {b}"

@@ -110,7 +110,10 @@ def schedule_paged(graphs, spec, config, *, split_graphs=(), filter_before_topk=
                 # pages of many tokens: work items of a few pages each (one wave per kv head, the waves in step),
                 # sized at launch so that one item lands on each compute unit -- requests of unlike lengths then
                 # cost items in proportion, where a fixed split gives every request the same number of parts
-                if getattr(spec, "page_size", 1) >= 16 and single.dense.query_rows <= 16 and factor == max(factors):
+                # (a token table has them too, of up to 2048 tokens.  us, bf16, 32 / 8 heads, the better of single kernel and fixed
+                # split / these: 64 requests, 68237 tokens 66 / 41.6, 40 of up to 4000 91 / 66, 23 of 2682 40 / 28.8, 18 of 1056 16.2 / 14.9;
+                # behind the fixed split for few requests, 3 of 2882 10.1 / 11.4, and the single kernel for short ones, 63 of 50 8.1 / 10.5)
+                if (getattr(spec, "page_size", 1) == 1 or spec.page_size >= 16) and single.dense.query_rows <= 16 and factor == max(factors):
                     forms.append(dataclasses.replace(single.dense, chunk_pages=-1, lockstep=True, waves=spec.num_kv_heads,
                                                      n_threads=spec.num_kv_heads * 64))
             for d in forms:
