@@ -1,6 +1,6 @@
 // ---- MFMA matmul in two wave groups that alternate between memory and matrix work ----------------
 //
-// C[M, N] = A[M, K] * B[K, N] on 256 x 256, 128 x 256 or 256 x 128 tiles, eight waves (two per SIMD), K in
+// C[M, N] = A[M, K] * B[K, N] on 256 x 256, 192 x 256, 128 x 256 or 256 x 128 tiles, eight waves (two per SIMD), K in
 // steps of 64, tiles global -> LDS directly.  The lock-step kernel (gemm_dma.hip) lets all eight waves
 // load, read and multiply at the same time: after every barrier both waves of a SIMD stand in their tile
 // loads and operand reads with the matrix unit idle (2870 clocks a 256 x 256 step for 2048 of matrix work).
@@ -16,6 +16,9 @@
 //     2      A0 B1        B1                           A0
 //     3      A1 B1        A1                           B1
 //     4      A1 B0        B0 of the next step          A1
+//
+// 192 x 256 (GP_UNEVEN): A's halves are 128 and 64 rows, so phases 3 and 4 have half the matrix ops; a product of one round of
+// either tile takes 0.87 of the time of 256 x 256 ones (2300 x 5120 x 2048 39.0 us against 45.5, 5900 x 2048 x 1536 32.4 against 37.1).
 //
 // The smaller tiles have half the matrix ops, so a phase takes both B halves:
 //
@@ -37,8 +40,10 @@
 //   CL_BM, CL_BN, CL_WM x CL_WN = 8 waves; CL_TRANS_A / CL_TRANS_B, CL_BATCH_A/B, CL_SPLITS, CL_TAIL (256 x 256
 //   only), CL_SWIGLU (B half 1 = the gate weight's columns) as in gemm_dma.hip.
 
-#define GP_QUADS (CL_BM == 256 && CL_BN == 256)
-static_assert(GD_WAVES == 8 && CL_BM % 128 == 0 && CL_BN % 128 == 0, "the phased matmul: eight waves, halves of whole 64-row pieces");
+#define GP_UNEVEN (CL_BM == 192)                       // A's halves are 128 and 64 rows
+#define GP_QUADS ((CL_BM == 256 || GP_UNEVEN) && CL_BN == 256)
+static_assert(GD_WAVES == 8 && (CL_BM % 128 == 0 || GP_UNEVEN) && CL_BN % 128 == 0, "the phased matmul: eight waves, halves of whole 64-row pieces");
+static_assert(!GP_UNEVEN || (GP_QUADS && CL_WM == 2 && !CL_TRANS_A && !CL_TAIL), "192 rows: four phases, row-major A, whole tiles");
 static_assert(CL_N % 8 == 0, "rows of C leave as 16-byte pieces");
 #if CL_NORM || CL_ROWSUM
 #error "the phased matmul has no fused norm and no row-sum walk"
@@ -102,12 +107,13 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
 
   // BM = 256, or 128 for a half tile of the last round
   auto body = [&](auto bm_tag, const int m0) {
-  constexpr int BM = decltype(bm_tag)::value, HM = BM / 2;
-  constexpr int TMH = HM / CL_WM / 16;                 // row fragments per wave and half
-  GdOperand<HM, CL_TRANS_A != 0> opa0, opa1;
+  constexpr int BM = decltype(bm_tag)::value, HM = GP_UNEVEN ? 128 : BM / 2, HM1 = BM - HM;   // rows of A's halves
+  constexpr int TMH = HM / CL_WM / 16, TMH1 = HM1 / CL_WM / 16;   // row fragments per wave and half
+  GdOperand<HM, CL_TRANS_A != 0> opa0;
+  GdOperand<HM1, CL_TRANS_A != 0> opa1;
   GdOperand<GP_HN, CL_TRANS_B == 0> opb0, opb1;
-  constexpr int la = decltype(opa0)::PER, lb = decltype(opb0)::PER;      // loads per wave and half
-  static_assert(decltype(opa0)::UNITS % GD_WAVES == 0 && decltype(opb0)::UNITS % GD_WAVES == 0, "every wave loads the same");
+  constexpr int la = decltype(opa0)::PER, la1 = decltype(opa1)::PER, lb = decltype(opb0)::PER;      // loads per wave and half
+  static_assert(decltype(opa0)::UNITS % GD_WAVES == 0 && decltype(opa1)::UNITS % GD_WAVES == 0 && decltype(opb0)::UNITS % GD_WAVES == 0, "every wave loads the same");
 #if CL_TRANS_A
   opa0.init(m0, CL_M, CL_M, 0, 0);
   opa1.init(m0, CL_M, CL_M, 0, HM);
@@ -142,19 +148,22 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
   // else is a constant -----------------------------------------------------------------------------
   const int am = wm * (HM / CL_WM), bn = wn * (GP_HN / CL_WN);
   constexpr int NA = CL_TRANS_A ? TMH : 2, NB = CL_TRANS_B ? 2 : GP_TNH;
-  int a_at[NA], b_at[NB];
+  int a_at[NA], a1_at[NA], b_at[NB];                   // (a1_at: the lower half's, where it differs)
   const int lds0 = (int)GD_LDS_BYTE(gp_lds);
 #if CL_TRANS_A
   const int a_f = gd_swz_kmaj<HM>(8 * g + (c >> 2));
   const int a_off = (8 * g + (c >> 2)) * HM + 8 * (((am / 8) ^ a_f) + ((c & 3) >> 1)) + 4 * (c & 1);
 #pragma unroll
   for (int i = 0; i < NA; ++i) a_at[i] = lds0 + 4 * GP_SLOT * 2 + (a_off ^ (i << 4)) * 2;
-#define GP_AFRAG(slot, i, s) gp_read_kmaj<HM>(a_at[i], slot, s)
+#define GP_AFRAG(half, slot, i, s) gp_read_kmaj<HM>(a_at[i], slot, s)
 #else
   const int a_off = (am + c) * 64 + ((g ^ gd_swz_kmin(am + c)) << 3);
 #pragma unroll
-  for (int i = 0; i < NA; ++i) a_at[i] = lds0 + 4 * GP_SLOT * 2 + (a_off ^ (i * 32)) * 2;
-#define GP_AFRAG(slot, i, s) gp_read_kmin(a_at[s], slot, i)
+  for (int i = 0; i < NA; ++i) {
+    a_at[i] = lds0 + 4 * GP_SLOT * 2 + (a_off ^ (i * 32)) * 2;
+    a1_at[i] = a_at[i] - wm * ((HM - HM1) / CL_WM) * 128;
+  }
+#define GP_AFRAG(half, slot, i, s) gp_read_kmin(GP_UNEVEN && (half) ? a1_at[s] : a_at[s], slot, i)
 #endif
 #if CL_TRANS_B
   const int b_off = (bn + c) * 64 + ((g ^ gd_swz_kmin(bn + c)) << 3);
@@ -174,6 +183,10 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
   auto keep_addresses = [&]() {
 #pragma unroll
     for (int i = 0; i < NA; ++i) asm volatile("" : "+v"(a_at[i]));
+#if GP_UNEVEN
+#pragma unroll
+    for (int i = 0; i < NA; ++i) asm volatile("" : "+v"(a1_at[i]));
+#endif
 #pragma unroll
     for (int i = 0; i < NB; ++i) asm volatile("" : "+v"(b_at[i]));
   };
@@ -191,7 +204,7 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
 
 #define GP_READ_A(stage, item)                                                                      \
   _Pragma("unroll") for (int s = 0; s < 2; ++s)                                                     \
-  _Pragma("unroll") for (int i = 0; i < TMH; ++i) fa[s][i] = GP_AFRAG((stage) * 2 + ((item) & 1), i, s);
+  _Pragma("unroll") for (int i = 0; i < ((item) & 1 ? TMH1 : TMH); ++i) fa[s][i] = GP_AFRAG((item) & 1, (stage) * 2 + ((item) & 1), i, s);
 #define GP_READ_B(f, stage, item)                                                                   \
   _Pragma("unroll") for (int s = 0; s < 2; ++s)                                                     \
   _Pragma("unroll") for (int j = 0; j < GP_TNH; ++j) f[s][j] = GP_BFRAG((stage) * 2 + ((item) & 1), j, s);
@@ -210,7 +223,7 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
   gp_barrier();                                                                                     \
   __builtin_amdgcn_s_setprio(1);                                                                    \
   _Pragma("unroll") for (int s = 0; s < 2; ++s)                                                     \
-  _Pragma("unroll") for (int i = 0; i < TMH; ++i)                                                   \
+  _Pragma("unroll") for (int i = 0; i < (ha ? TMH1 : TMH); ++i)                                     \
   _Pragma("unroll") for (int j = 0; j < GP_TNH; ++j)                                                \
     acc[ha][i][hb][j] = mfma16(f[s][j], fa[s][i], acc[ha][i][hb][j]);                               \
   __builtin_amdgcn_s_setprio(0);                                                                    \
@@ -225,13 +238,14 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
 #define GP_NEXT(S, q) GP_READ_B(q, 1 - (S), GP_B0)
 #define GP_STEP(S, p, q, NEXT_STEP, LATER_, LATER)                                                  \
   GP_STEP_(S, p, q, LATER(opb0, pb0, S, GP_B0), LATER(opa0, pa, S, GP_A0), LATER(opb1, pb1, S, GP_B1), LATER(opa1, pa, S, GP_A1), \
-           3 * (la + lb), 3 * (la + lb), 3 * (la + lb), 3 * (la + lb), GP_NEXT(S, q))               \
+           la + 2 * la1 + 3 * lb, 2 * la + la1 + 3 * lb, 2 * la + la1 + 3 * lb, la + 2 * la1 + 3 * lb, GP_NEXT(S, q)) \
   pa += a_step; pb0 += b_step; pb1 += b_step;
   // The last two steps ask for nothing more: the waits count down what is still on its way.
 #define GP_STEP_LAST2(S, p, q)                                                                      \
-  GP_STEP_(S, p, q, GP_NONE, GP_NONE, GP_NONE, GP_NONE, 3 * la + 2 * lb, 2 * la + 2 * lb, 2 * la + lb, la + lb, GP_NEXT(S, q))
+  GP_STEP_(S, p, q, GP_NONE, GP_NONE, GP_NONE, GP_NONE, la + 2 * la1 + 2 * lb, la + la1 + 2 * lb, la + la1 + lb, la1 + lb, \
+           GP_NEXT(S, q))
 #define GP_STEP_LAST(S, p, q)                                                                       \
-  GP_STEP_(S, p, q, GP_NONE, GP_NONE, GP_NONE, GP_NONE, la, 0, 0, 0, GP_NONE)
+  GP_STEP_(S, p, q, GP_NONE, GP_NONE, GP_NONE, GP_NONE, la1, 0, 0, 0, GP_NONE)
 
 #define GP_END(S, p, q) GP_STEP_LAST2(S, p, q) GP_STEP_LAST(1 - (S), q, p)
 
@@ -240,7 +254,7 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
   pa += a_step; pb0 += b_step; pb1 += b_step;
   GP_ASK(0, GP_LOAD)
   if constexpr (GD_LEFT && KT == 2) { GP_ASK(1, GP_LOAD_LEFT) } else { GP_ASK(1, GP_LOAD) }
-  constexpr int ahead = 3 * (la + lb);                 // loads still out when a phase's operands have landed
+  constexpr int ahead = la + 2 * la1 + 3 * lb;                         // loads still out when a phase's operands have landed
 #else
   // One phase: the memory part (operand reads, loads, the wait for both the reads and what the next
   // phase reads), and behind a barrier the matrix part: A half h times both B halves.
@@ -329,13 +343,13 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
   int tid = threadIdx.x;
   asm volatile("" : "+v"(tid));
   const int ec = tid & 15, eg = (tid >> 4) & 3;
-  const int erow = (tid >> 6) / CL_WN * (HM / CL_WM) + ec, ecol = (tid >> 6) % CL_WN * (GP_HN / CL_WN);
-  // ---- epilogue: acc[h][i][v][j][r] = C[m0 + h HM + am + 16 i + c][n0 + HN v + bn + 16 j + 4 g + r]
+  const int ewm = (tid >> 6) / CL_WN, ecol = (tid >> 6) % CL_WN * (GP_HN / CL_WN);
+  // ---- epilogue: acc[h][i][v][j][r] = C[m0 + h HM + (the wave's first row of that half) + 16 i + c][n0 + HN v + bn + 16 j + 4 g + r]
 #pragma unroll
   for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int i = 0; i < TMH; ++i) {
-      const int m = m0 + h * HM + erow + 16 * i;
+    for (int i = 0; i < (h ? TMH1 : TMH); ++i) {
+      const int m = m0 + h * HM + ewm * ((h ? HM1 : HM) / CL_WM) + ec + 16 * i;
 #if CL_SPLITS > 1
 #pragma unroll
       for (int v = 0; v < 2; ++v)

@@ -50,7 +50,7 @@
 #define CL_ASM_MFMA (GD_TM * GD_TN * 4 > 128)   // wave tiles whose accumulators fill a register half
 #endif
 static_assert(CL_BK == 64, "K steps are 64 wide (128-byte K-minor rows)");
-static_assert((GD_TM & (GD_TM - 1)) == 0 && (GD_TN & (GD_TN - 1)) == 0, "wave tiles are powers of two");
+static_assert(((GD_TM & (GD_TM - 1)) == 0 || (CL_BM == 192 && CL_BN == 256 && CL_WM == 2 && CL_WN == 4)) && (GD_TN & (GD_TN - 1)) == 0, "wave tiles are powers of two");
 static_assert(CL_BM % 16 == 0 && CL_BN % 16 == 0, "tiles are multiples of 16");
 
 // The contraction is dealt out to CL_SPLITS ranges of CL_K_RANGE, walked in GD_KT 64-wide steps each; the last step of a

@@ -121,9 +121,10 @@ def phased_matmul(family, problem, splits, tile) -> bool:
     and matrix-op knobs are the lock-step kernel's.  us, lock-step / phased: 8192^3 bf16 (N, K) weight 806 / 701,
     4096 x 14336 x 4096 f16 393 / 352 (with the last half round split), SwiGLU of that size 752 / 676, 3000 x 5000 x 2048
     56 / 52; 128 x 256 tiles (three stages lock-step) 2048 x 4096 x 4096 60.1 / 56.3, 724 x 6272 x 640 13.3 / 10.7; at the
-    small end 2999 x 1000 x 192 9.8 / 8.2."""
+    small end 2999 x 1000 x 192 9.8 / 8.2.  192 x 256 tiles (A's halves of 128 and 64 rows) exist here only, for row-major A."""
     bm, bn, wm, wn = (int(tile[k]) for k in ("BM", "BN", "WM", "WN"))
-    sizes = (bm, bn) == (256, 256) or ((bm, bn) in ((128, 256), (256, 128)) and not int(tile.get("TAIL", 0)))
+    sizes = ((bm, bn) == (256, 256) or ((bm, bn) in ((128, 256), (256, 128)) and not int(tile.get("TAIL", 0)))
+             or ((bm, bn, wm) == (192, 256, 2) and not problem["trans_A"] and not int(tile.get("TAIL", 0))))
     return (sizes and wm * wn == 8 and bn // 2 // wn % 32 == 0 and bm // 2 // wm % 16 == 0 and family in ("matmul", "swiglu")
             and problem["K"] // splits > 64 and problem["N"] % 8 == 0 and int(tile.get("STAGES", 2)) == 2
             and not {"ASM_LOADS", "ASM_MFMA", "SPREAD_LOADS"} & set(tile))
@@ -149,15 +150,22 @@ def gemm_dma_candidates(low, role, factor, arch: Arch, twin_of=None):
     batch = max(p["batch_A"], p["batch_B"])
     out = []
     shapes = (16, 32, 64, 128, 256)
-    for bm, bn, (wm, wn) in itertools.product(
-            shapes, shapes, ((1, 1), (1, 2), (2, 1), (2, 2), (1, 4), (4, 1), (2, 4), (4, 2))):
+    grids = ((1, 1), (1, 2), (2, 1), (2, 2), (1, 4), (4, 1), (2, 4), (4, 2))
+    # 192 x 256 tiles, of the two-group kernel only: a round of them takes 0.87 of one of 256 x 256 ones, so they are proposed where that
+    # many rounds (one workgroup per compute unit) are less.  us, 256 x 256 / these: 3479 x 3264 x 1984 45.8 / 41.6, 2300 x 5120 x 2048 45.5 /
+    # 39.0, 1536 x 8000 x 4096 84.4 / 72.4 (one round each); where they cost one round more 3000 x 5000 x 2048 52.7 / 72.4.
+    uneven = (192, 256, (2, 4))
+    rounds = {bm: _ceil(_ceil(M, bm) * _ceil(N, 256) * batch, arch.compute_units) for bm in (192, 256)}
+    fits = (not post_norm and twin_of != "matmul_rowsum" and splits == 1 and 0.87 * rounds[192] < rounds[256]
+            and phased_matmul("matmul", p, 1, dict(BM=192, BN=256, WM=2, WN=4)))
+    for bm, bn, (wm, wn) in itertools.chain(itertools.product(shapes, shapes, grids), (uneven,) if fits else ()):
         if bm % (16 * wm) or bn % (16 * wn):
             continue
         if bm > max(16, 2 * M) or bn > max(16, 2 * N):
             continue
         threads = wm * wn * 64
         tm, tn = bm // wm // 16, bn // wn // 16
-        if tm & (tm - 1) or tn & (tn - 1) or tm * tn * 4 > 128:
+        if (tm & (tm - 1) and bm != 192) or tn & (tn - 1) or tm * tn * 4 > 128:
             continue
         if post_norm and low.dtype == "bfloat16" and tm * tn * 4 > 64 and wm > wn:
             continue      # bf16 squares go through float conversions: beside a 128-register, 4-row-fragment tile they spill
@@ -206,7 +214,7 @@ def gemm_dma_candidates(low, role, factor, arch: Arch, twin_of=None):
         # workgroups each (row-major A, one workgroup per compute unit, unsplit, unbatched).
         tail = blocks % arch.compute_units
         if (blocks > arch.compute_units and 0 < tail <= arch.compute_units // 2 and per_cu == 1 and splits == 1
-                and batch == 1 and not p["trans_A"] and tm >= 2 and M % bm == 0):
+                and batch == 1 and not p["trans_A"] and tm >= 2 and M % bm == 0 and bm != 192):
             out.append(TileDict("gemm_dma", role, dict(tiling, TAIL=tail), output_tile=[bm, bn], rstep_map={"k": 64},
                                 n_threads=threads, split_factor=factor, score=(passes - 0.45) * pass_clk,
                                 lds_bytes=lds, est_vgprs=vgprs))

@@ -134,3 +134,22 @@ def test_swiglu(m, n, k):
     _check(C.swiglu, cl.f16, dict(M=m, N=n, K=k), tile=TILES["256x128_4x2"], SWIGLU=1)
     _check(C.swiglu, cl.f16, dict(M=m, N=n, K=k), SWIGLU=1)
     _check(C.swiglu, cl.bf16, dict(M=m, N=n, K=k), tile=TILES["256x256_4x2"], SWIGLU=1)
+
+
+@pytest.mark.parametrize("m,n,k", [(192, 256, 128), (193, 264, 192), (320, 72, 256), (130, 520, 136), (700, 392, 200), (385, 264, 328), (64, 256, 448)])
+def test_tiles_whose_halves_are_128_and_64_rows(m, n, k):
+    """Two to seven steps, a partly filled last one, edges within either half and whole halves past the edge; batches, ranges and SwiGLU."""
+    tiling = dict(BM=192, BN=256, BK=64, WM=2, WN=4)
+    for fn, dtype, shapes, knobs in ((C.matmul, cl.f16, {}, {}), (C.matmul_nt, cl.bf16, {}, {}), (C.batched_matmul, cl.bf16, dict(BX=4, BW=2), {}),
+                                     *([(C.matmul, cl.f16, {}, dict(KS=2))] if k >= 256 else []), *([(C.swiglu, cl.f16, {}, dict(SWIGLU=1))] if k % 64 == 0 else [])):
+        shapes = dict(shapes, M=m, N=n, K=k) if fn is not C.swiglu else dict(M=m, N=-(-n // 128) * 128, K=k)
+        prog = fn.trace(dtype, **shapes)
+        x, *weights = prog.random_inputs(seed=7)
+        args = [x] + [(w.float() / k ** 0.5).to(w.dtype) for w in weights]
+        print(f"case {prog.name} {dtype} {shapes} {knobs}", flush=True)
+        kernel = kernel_for(prog, template="gemm_dma" if k % 64 == 0 else "gemm", tiling=dict(tiling, **knobs, **({} if k % 64 == 0 else dict(DMA=1))))
+        assert "#define GP_UNEVEN" in kernel.get_kernel_source()
+        got = kernel(*args)
+        torch.cuda.synchronize()
+        want = program_oracle.evaluate(prog, [t.cpu() for t in args])[0]
+        np.testing.assert_allclose(got.float().cpu().numpy().reshape(want.shape), want, rtol=1e-2, atol=1e-2)
