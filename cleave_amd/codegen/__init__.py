@@ -90,10 +90,12 @@ class _Unit:
         self.define(macro, ", ".join(parts))
         return [p.name for p in params] + list(dyn_dims)
 
-    def launch(self, entry, grid, block, lds, args, optional=False):
-        """``optional``: left out where its grid is empty (any other empty grid means that the call has nothing to do)."""
+    def launch(self, entry, grid, block, lds, args, optional=False, shared_grid=None):
+        """``optional``: left out where its grid is empty (any other empty grid means that the call has nothing to do).
+        ``shared_grid``: its grid in calls whose scratch is an array that other calls on the GPU use as well."""
         self.launches.append({"entry": entry, "grid": [str(g) for g in grid], "block": [int(block), 1, 1],
-                              "lds": int(lds), "args": list(args), **({"optional": True} if optional else {})})
+                              "lds": int(lds), "args": list(args), **({"optional": True} if optional else {}),
+                              **({"shared_grid": [str(g) for g in shared_grid]} if shared_grid else {})})
 
 
 class HipCodeGen:
@@ -866,9 +868,11 @@ class HipCodeGen:
         walk = unit.signature("CL_STAY_PARAMS", "CL_STAY_NAME", ENTRY + "_stay",
                               [q for q in params if q.role in ("input", "scalar")] + [tickets] + [q for q in params if q.role == "output"], dyn, dyn_c)
         unit.templates += ["mla_decode_duo.hip", "mla_prefill_duo.hip"]
-        unit.launch(ENTRY, (f"{items} * (1 - {stay})", groups, 1), 512, 0, self._partial_args, optional=True)
-        unit.launch(ENTRY + "_tickets", (stay, 1, 1), 64, 0, zero, optional=True)
-        unit.launch(ENTRY + "_stay", (f"{units} * {stay}", 1, 1), 512, 0, walk, optional=True)
+        # (calls that share their scratch with others keep to one workgroup an item, which needs none: two calls that overlap would
+        # draw from one counter)
+        unit.launch(ENTRY, (f"{items} * (1 - {stay})", groups, 1), 512, 0, self._partial_args, optional=True, shared_grid=(items, groups, 1))
+        unit.launch(ENTRY + "_tickets", (stay, 1, 1), 64, 0, zero, optional=True, shared_grid=(0, 1, 1))
+        unit.launch(ENTRY + "_stay", (f"{units} * {stay}", 1, 1), 512, 0, walk, optional=True, shared_grid=(0, 1, 1))
 
 
 def aligned_inputs(source: str, params) -> frozenset:

@@ -275,7 +275,7 @@ class CompiledKernel:
         into its fixed scratch array."""
         keep, descs = [], []
         for l in self.manifest["launches"]:
-            grid = [eval_extent(g, dims) for g in l["grid"]]
+            grid = [eval_extent(g, dims) for g in (l["grid"] if fixed is None else l.get("shared_grid", l["grid"]))]
             if min(grid) < 1 and l.get("optional"):
                 continue           # a launch that this call has no use for
             values = []
@@ -337,10 +337,12 @@ class CompiledKernel:
 
     def fixed_scratch_layout(self, dims) -> tuple:
         """``({scratch parameter: byte offset}, bytes)``: the kernel's scratch buffers laid out
-        one after the other at multiples of 256 bytes (two names of one buffer share an offset)."""
+        one after the other at multiples of 256 bytes (two names of one buffer share an offset).  Buffers that only
+        launches left out of calls with shared scratch use are not among them."""
         offsets, owners, end = {}, {}, 0
+        used = {name for l in self.manifest["launches"] if l.get("shared_grid", l["grid"])[0] != "0" for name in l["args"]}
         for p in self.params:
-            if p.role != "scratch":
+            if p.role != "scratch" or p.name not in used:
                 continue
             owner = p.alias or p.name
             if owner not in owners:

@@ -91,3 +91,17 @@ def test_one_of_the_two_forms_is_launched(heads):
     assert grids(1, 1) == [8, 0, 0] and grids(0, 0) == [0, 0, 0]
     scratch = next(p for p in manifest["params"] if p["role"] == "scratch")
     assert [eval_extent(scratch["shape"][0], dict(total_q=t, batch=8)) for t in (64, 8192)] == [0, 64]
+
+
+@pytest.mark.gpu
+def test_calls_that_share_their_scratch_need_none():
+    """Overlapping calls through the fixed array would draw items from one counter: they run one workgroup an item."""
+    args = [a.cuda() if isinstance(a, torch.Tensor) else a for a in inputs(*LARGE["mixed"], 16, 512, "bfloat16", 0.05)]
+    loaded = _load_main_kernel_from_code(source(16, 512, "bfloat16", 0))
+    want = _compile(loaded, loaded.manifest["out_idx"])(*args)
+    caller = _compile(loaded, None)
+    assert caller.fixed_scratch_layout(dict(total_q=1 << 20, batch=44)) == ({}, 0)
+    got = [torch.full_like(t, float("nan")) for t in want]
+    caller.call_fixed_scratch(*args, *got)
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
