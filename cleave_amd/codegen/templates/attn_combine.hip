@@ -10,6 +10,15 @@
 #ifndef CL_COMBINE_GROUPS
 #define CL_COMBINE_GROUPS 1
 #endif
+#if CL_EMIT_COMBINE
+template <int V> struct CbTag { static constexpr int value = V; };
+// Adds a partial of weight f to a row's sums, or, of a slot past the last partial, nothing.  (Weight 0 is not nothing: a partial may hold
+// infinite values.)
+CL_DEVICE void cb_add(bool there, float f, float pl, f32x4 po, float& l, f32x4& o) {
+  l += (there ? pl : 0.f) * f;
+  o += (there ? po : (f32x4){0.f, 0.f, 0.f, 0.f}) * f;
+}
+#endif
 #if CL_EMIT_COMBINE && CL_COMBINE_GROUPS > 1
 // Where CL_COMBINE_GROUPS groups of threads share the partials of a row's CB_COLS columns (thread t: group t / CB_THREADS, columns
 // 4 (t % CB_THREADS) .. + 3): each adds its own up against the largest of their reference points, and the first group adds the
@@ -53,7 +62,7 @@ CL_DEVICE void cb_finish(float m, float l, f32x4 o, elem_t* out, float* lse) {
 // Combine of chunked items: request b owns items b + p0/C .. b + (p1-1)/C (p0, p1 its page-table range); partials are (item,
 // query head[, d]).  A group takes every CL_COMBINE_GROUPS-th item, CB_EACH of them at a time, every load of a round issued before
 // the first use (the trip count is a run-time value: left alone, each item's loads wait for the previous item's); the running
-// maximum is carried along and the sums rescaled when a round raises it; slots past the end repeat the last item with weight zero.
+// maximum is carried along and the sums rescaled when a round raises it; slots past the end read the last item again and leave it out.
 // What bounds it: round trips to memory, of which a request of up to CB_EACH * CL_COMBINE_GROUPS items costs one: one thread walking all
 // items of its columns, eight at a time, was most of a call of few long requests.  us, one thread / groups, f16, 32 / 8 heads, pages of 64: one
 // request of 12705 keys (199 items) 34.2 / 16.7, 2 of up to 3644 17.6 / 12.6, 6 of 4345 20.9 / 15.4, 19 of 1787 17.8 / 15.8, 12 of 9000
@@ -72,12 +81,13 @@ CL_COMBINE_NAME(CL_COMBINE_PARAMS) {
   const int count = p1 > p0 ? (p1 - 1) / chunk_pages - p0 / chunk_pages + 1 : 0;
   float m = CL_NEG_BIG, l = 0.f;
   f32x4 o = (f32x4){0.f, 0.f, 0.f, 0.f};
-  for (int s = group; s < count; s += CB_EACH * CL_COMBINE_GROUPS) {
+  // one round; `whole`: all its items are there
+  auto round = [&](auto whole, const int s) __attribute__((always_inline)) {
     float pm[CB_EACH], pl[CB_EACH];
     f32x4 po[CB_EACH];
 #pragma unroll
     for (int u = 0; u < CB_EACH; ++u) {
-      const int it = s + u * CL_COMBINE_GROUPS < count ? s + u * CL_COMBINE_GROUPS : count - 1;
+      const int it = decltype(whole)::value || s + u * CL_COMBINE_GROUPS < count ? s + u * CL_COMBINE_GROUPS : count - 1;
       const i64 prow = (i64)(first + it) * CL_Q_HEADS + qh;
       pm[u] = CL_CARG_PM[prow];
       pl[u] = CL_CARG_PL[prow];
@@ -91,12 +101,14 @@ CL_COMBINE_NAME(CL_COMBINE_PARAMS) {
     l *= keep;
     o *= keep;
 #pragma unroll
-    for (int u = 0; u < CB_EACH; ++u) {
-      const float f = s + u * CL_COMBINE_GROUPS < count ? fast_exp2(pm[u] - m) : 0.f;
-      l += pl[u] * f;
-      o += po[u] * f;
-    }
-  }
+    for (int u = 0; u < CB_EACH; ++u)
+      cb_add(decltype(whole)::value || s + u * CL_COMBINE_GROUPS < count, fast_exp2(pm[u] - m), pl[u], po[u], l, o);
+  };
+  // (the groups of a wave go on to the last round together)
+  constexpr int per_wave = 64 / CB_THREADS;
+  int s = group;
+  for (; s - group % per_wave + per_wave - 1 + (CB_EACH - 1) * CL_COMBINE_GROUPS < count; s += CB_EACH * CL_COMBINE_GROUPS) round(CbTag<1>(), s);
+  if (s < count) round(CbTag<0>(), s);
 #if CL_EMIT_LSE
   cb_finish(m, l, o, CL_CARG_OUT + row * CL_VDIM + d, d == 0 ? CL_CARG_LSE + row : nullptr);
 #else
@@ -160,22 +172,19 @@ CL_COMBINE_NAME(CL_COMBINE_PARAMS) {
 #pragma unroll
   for (int u = 0; u < CB_EACH; ++u) {
     const int s = group + u * CL_COMBINE_GROUPS;
-    const i64 prow = (i64)(s < CL_SPLITS ? s : CL_SPLITS - 1) * CL_TOTAL_ROWS + row;      // (past the last: it again, with weight 0)
+    const i64 prow = (i64)(s < CL_SPLITS ? s : CL_SPLITS - 1) * CL_TOTAL_ROWS + row;      // (past the last: it again, left out below)
     pm[u] = CL_CARG_PM[prow];
     pl[u] = CL_CARG_PL[prow];
     po[u] = *reinterpret_cast<const f32x4*>(CL_CARG_PO + prow * CL_VDIM + d);
   }
-  float m = pm[0];
+  float m = CL_NEG_BIG;
 #pragma unroll
-  for (int u = 1; u < CB_EACH; ++u) m = fmaxf(m, pm[u]);
+  for (int u = 0; u < CB_EACH; ++u) m = fmaxf(m, pm[u]);
   float l = 0.f;
   f32x4 o = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int u = 0; u < CB_EACH; ++u) {
-    const float f = group + u * CL_COMBINE_GROUPS < CL_SPLITS ? fast_exp2(pm[u] - m) : 0.f;
-    l += pl[u] * f;
-    o += po[u] * f;
-  }
+  for (int u = 0; u < CB_EACH; ++u)
+    cb_add((u + 1) * CL_COMBINE_GROUPS <= CL_SPLITS || group + u * CL_COMBINE_GROUPS < CL_SPLITS, fast_exp2(pm[u] - m), pl[u], po[u], l, o);
 #if CL_EMIT_LSE
   cb_finish(m, l, o, CL_CARG_OUT + row * CL_VDIM + d, d == 0 ? CL_CARG_LSE + row : nullptr);
 #else
