@@ -488,13 +488,17 @@ class HipCodeGen:
         params[at:at] = scratch
         return dataclasses.replace(plan, role="fused", operands=operands, split_factor=keys)
 
-    def _launch_chunk_combine(self, unit, rows, vdim):
-        """The launch that merges the partials of chunked items: groups of threads share the items of a row."""
+    def _launch_chunk_combine(self, unit, rows, vdim, items):
+        """The launch that merges the partials of chunked items: groups of threads share the items of a row where one thread per four
+        columns would be fewer workgroups than there are ``items`` (the kernel makes the same choice)."""
         from ..schedule.policy import COMBINE_GROUPS
 
         groups = next(n for n in COMBINE_GROUPS if vdim * n % 1024 == 0)
         unit.define("CL_COMBINE_GROUPS", groups)
-        unit.launch(self._combine_args[0], (f"{rows} * {vdim * groups // 1024}", 1, 1), 256, 0, self._combine_args[1])
+        plain = f"ceildiv({rows} * {vdim // 4}, 256)"
+        grouped = f"min(max({items} - {plain}, 0), 1)"
+        unit.launch(self._combine_args[0], (f"{plain} + ({rows} * {vdim * groups // 1024} - {plain}) * {grouped}", 1, 1), 256, 0,
+                    self._combine_args[1])
 
     def _launch_combine(self, unit, rows, vdim, splits, po_elem=False, plain=None):
         """The launch that merges the f32 (or, ``po_elem``, element-type) partials of ``splits`` key ranges.
@@ -574,7 +578,7 @@ class HipCodeGen:
         if combine:
             plain = f"ceildiv({grid_rows} * {p['vdim'] // 4}, 256)"
             if chunk_pages:
-                self._launch_chunk_combine(unit, grid_rows, p["vdim"])
+                self._launch_chunk_combine(unit, grid_rows, p["vdim"], f"ceildiv({p['dim_names']['n_idx']}, chunk_pages) + {batch_name}")
             elif paged:
                 unit.launch(self._combine_args[0], (plain, 1, 1), 256, 0, self._combine_args[1])
             else:
@@ -841,7 +845,7 @@ class HipCodeGen:
                 items = f"ceildiv({p['dim_names']['total_q']}, {tok}) + batch"
             unit.launch(ENTRY, (items, p["heads"] // 16, 1), 64 * max(tok, ksplit), 0, self._partial_args)
         if combine:
-            self._launch_chunk_combine(unit, f"({batch_name} * {p['heads']})", p["ckv"])
+            self._launch_chunk_combine(unit, f"({batch_name} * {p['heads']})", p["ckv"], items)
 
 
     def _mla_prefill_duo(self, unit, plan, params):

@@ -8,7 +8,8 @@ import pytest
 import torch
 
 from cleave_amd import examples as C
-from cleave_amd.dynamic.paging import DenseAttention, PagingSpec, build_split_decode, CombineTiling
+from cleave_amd.codegen import HipCodeGen, parse_manifest
+from cleave_amd.dynamic.paging import PAGED_DECODE_SLAB, DenseAttention, PagingSpec, build_split_decode, CombineTiling
 from cleave_amd.dynamic.paging.apply import MAX_CHUNK_TOKENS, UnsupportedTiling, chunk_pages_expr, max_chunk_pages
 from cleave_amd.runtime.compile import eval_extent
 from tests.test_gpu_paged import check, paged_kernel, run
@@ -79,3 +80,30 @@ def test_item_sizes():
     dense = DenseAttention(16, 32, 128, 512, "float16", "float16", waves=8, chunk_pages=MAX_CHUNK_TOKENS + 1, lockstep=True)
     with pytest.raises(UnsupportedTiling, match="chunk_pages in 1..2048"):
         build_split_decode(spec, dense, 8, CombineTiling(split=8))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("page", [1, 16])
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_one_thread_for_the_items_of_many_rows(page, d):
+    """Six items a round: 6, 7, 12, 13 and 19 items among short requests, and an empty one."""
+    unit = 32
+    lens = [6 * unit, 7 * unit, 1, 12 * unit - 5, 0, 13 * unit, 19 * unit] + [1 + i % 9 for i in range(200)]
+    args = token_table(lens, 3200, d=d) if page == 1 else C.paged_workload(lens, page_size=page, num_pages=400, d=d)
+    assert -(-args[4].numel() // (32 // page)) + len(lens) <= len(lens) * 32 * d // 1024       # (as many items as workgroups, or fewer)
+    check(args, lens, page, d=d, split=8, waves=8, chunk_pages=32 // page, lockstep=True)
+
+
+@pytest.mark.parametrize("page,d", [(1, 128), (64, 64), (64, 256)])
+def test_who_adds_the_items_up(page, d):
+    """Groups of threads where one thread per four columns would be fewer workgroups than there are items."""
+    spec = PagingSpec(num_qo_heads=32, num_kv_heads=8, kind="paged_decode" if page == 1 else PAGED_DECODE_SLAB, page_size=page)
+    dense = DenseAttention(16, 32, d, 512, "float16", "float16", waves=8, chunk_pages=32, lockstep=True)
+    launches = parse_manifest(HipCodeGen().gen(build_split_decode(spec, dense, 8, CombineTiling(split=8, cols=min(128, d)))))["launches"]
+
+    def grid(batch, table):
+        return eval_extent(launches[1]["grid"][0], {spec.batch_dim: batch, spec.index_dim: table, "chunk_pages": 32})
+
+    one = 10 * 32 * d // 1024                               # ten requests, one thread per four columns
+    assert grid(10, 32 * (one - 10)) == one and grid(10, 32 * (one - 10) + 1) == 10 * 32 * max(1, d // 128)
+    assert grid(0, 64) == 0

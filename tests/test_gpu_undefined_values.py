@@ -47,10 +47,10 @@ def test_an_infinite_value_of_a_key_range(keys, ranges, d, where):
 
 @pytest.mark.parametrize("page,requests", [(1, 3), (64, 3), (1, 90), (64, 90)])
 def test_an_infinite_value_of_an_item(page, requests):
-    """Requests of one to nine items (one whole round of a thread group and less), the value in the first, a middle and the last of them;
-    few requests, whose items are added up by groups of threads, and many, where one thread takes a row's."""
+    """In the first, a middle and the last item of requests; few requests of five to nine items, which are added up by groups of threads,
+    and many of one to five, where one thread takes a row's."""
     unit = 32 if page == 1 else 64
-    lens = [unit * (1 + i % 9) for i in range(requests - 1)] + [5 * unit]
+    lens = [unit * (9 - 2 * i if requests == 3 else 1 + i % 3) for i in range(requests - 1)] + [5 * unit]
     places = {0: 3, requests // 2: lens[requests // 2] // 2, requests - 1: 5 * unit - 9}
     args = token_table(lens, sum(lens) + 8) if page == 1 else C.paged_workload(lens, page_size=64, num_pages=sum(lens) // 64 + 2)
     indptr, table = args[3].tolist(), args[4].tolist()
