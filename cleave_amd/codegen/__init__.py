@@ -854,12 +854,21 @@ class HipCodeGen:
 
         The line lies at three rounds of one workgroup per compute unit.  us, one workgroup an item / that stay, 16 heads: 1380 items
         of 24 requests 95.1 / 86.3, 2336 of 32 149.9 / 137.8, 1136 of 16 68.3 / 65.0; 568 of 8 33.8 / 34.9, 520 of 32 (up to 160 keys)
-        25.7 / 25.8, 464 of 12 24.1 / 26.7: there the clearing launch (2 us) and the last round's uneven ends outweigh what overlaps."""
+        25.7 / 25.8, 464 of 12 24.1 / 26.7: there the clearing launch and the last round's uneven ends outweigh what overlaps.
+        Rows so narrow that a compute unit holds two workgroups never stay: their items overlap without, and workgroups that stay are
+        one a unit.  128 latent features, 816 items 15.2 / 21.0, 1368 of 24 requests 35.0 / 49.5, 2440 of 32 59.4 / 84.2; 256 (one a unit)
+        59.6 / 61.5 and 103.8 / 105.2 on one card, 62.0 / 60.5 and 104.7 / 102.2 on another, 384 74.5 / 74.5 and 127.9 / 124.1."""
+        from ..schedule.policy import mla_duo_lds_bytes
+
         p = plan.problem
         dyn = tuple(plan.dyn_dims) + tuple(name for name, _ in plan.extra["derived_dims"])
         groups, units = p["heads"] // 16, current_target().arch.compute_units // 8 * 8
         # (the item axis is padded to a multiple of 8: the kernels deal runs of items out to the XCDs)
         items = f"ceildiv(ceildiv({p['dim_names']['total_q']}, 4) + batch, 8) * 8"
+        if 2 * mla_duo_lds_bytes(p["ckv"], p["kpe"], prefill=True) <= current_target().arch.lds_bytes and "FEW" not in plan.tiling:
+            unit.templates += ["mla_decode_duo.hip"]
+            unit.launch(ENTRY, (items, groups, 1), 512, 0, self._partial_args)
+            return
         few = int(plan.tiling.get("FEW", 3 * units)) // groups
         stay = f"min(max({items} - {few}, 0), 1)"
         tickets = ParamSpec("Tickets", "int32", (f"64 * {stay}",), "scratch")

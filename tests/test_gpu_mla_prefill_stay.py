@@ -93,6 +93,15 @@ def test_one_of_the_two_forms_is_launched(heads):
     assert [eval_extent(scratch["shape"][0], dict(total_q=t, batch=8)) for t in (64, 8192)] == [0, 64]
 
 
+@pytest.mark.parametrize("ckv,launches", [(128, 1), (256, 3), (384, 3), (512, 3)])
+def test_rows_of_which_a_unit_holds_two_workgroups_run_one_an_item(ckv, launches):
+    manifest = parse_manifest(source(16, ckv, "bfloat16"))
+    assert len(manifest["launches"]) == launches and any(p["role"] == "scratch" for p in manifest["params"]) == (launches > 1)
+    if launches == 1:
+        assert not manifest["launches"][0].get("optional")
+        assert eval_extent(manifest["launches"][0]["grid"][0], dict(total_q=40000, batch=8)) == 10008
+
+
 @pytest.mark.gpu
 def test_calls_that_share_their_scratch_need_none():
     """Overlapping calls through the fixed array would draw items from one counter: they run one workgroup an item."""
