@@ -112,7 +112,8 @@ def schedule_paged(graphs, spec, config, *, split_graphs=(), filter_before_topk=
                 # cost items in proportion, where a fixed split gives every request the same number of parts
                 # (a token table has them too, of up to 2048 tokens.  us, bf16, 32 / 8 heads, the better of single kernel and fixed
                 # split / these: 64 requests, 68237 tokens 66 / 41.6, 40 of up to 4000 91 / 66, 23 of 2682 40 / 28.8, 18 of 1056 16.2 / 14.9;
-                # behind the fixed split for few requests, 3 of 2882 10.1 / 11.4, and the single kernel for short ones, 63 of 50 8.1 / 10.5)
+                # behind the fixed split for four requests and fewer, 3 of 2882 11.5 / 12.9, which keep it by the calibrated rule, and the single
+                # kernel for short ones, 63 of 50 8.1 / 10.5)
                 if (getattr(spec, "page_size", 1) == 1 or spec.page_size >= 16) and single.dense.query_rows <= 16 and factor == max(factors):
                     forms.append(dataclasses.replace(single.dense, chunk_pages=-1, lockstep=True, waves=spec.num_kv_heads,
                                                      n_threads=spec.num_kv_heads * 64))
@@ -219,16 +220,21 @@ def few_requests(spec, compute_units: int) -> int:
     return compute_units // (4 * per_request) + 1
 
 
-def calibrate_dispatch(pair, solo, factory, spec) -> dict:
+def calibrate_dispatch(pair, solo, factory, spec, fixed=None) -> dict:
     """When should a call run the split pair rather than the single kernel?
 
     Both are timed on every workload.  A workload is described by the kv tiles of its longest request
     (``indptr`` units x page size / kv tile, rounded up), and the rule is "split from ``min_tiles`` tiles on".
     What a split is worth also depends on whether the single kernel's workgroups fill the chip: for batches of
-    fewer than ``few_requests`` requests (workgroups for less than a quarter of the compute units; 18 requests of
-    up to 1056 tokens, 144 workgroups, still run 16 us unsplit and 22 split) the threshold is ``lone_tiles``,
+    fewer than ``few_requests`` requests (workgroups for less than a quarter of the compute units) the threshold is ``lone_tiles``,
     calibrated on each workload's longest request alone.  (With one threshold, taken from batches of 64 requests,
-    three requests of up to 2882 tokens ran the single kernel in 26 us where the pair takes 11.)"""
+    three requests of up to 2882 tokens ran the single kernel in 26 us where the pair takes 11.)
+
+    ``fixed``: the pair that gives every request the same number of parts, where ``pair`` cuts the table into items.  Batches so small
+    that its parts are no more workgroups than compute units run it for requests of ``from_tiles`` tiles on and below ``until_tiles``
+    a request (three at most): an item's ids pass through LDS and its partials are found through the row pointers, which costs such a
+    call more than the even cut saves.  us, fixed / items, bf16, 32 / 8 heads: 1 x 500 tokens 6.4 / 8.2, 1 x 3000 10.1 / 9.8, 1 x 9000 18.5 / 14.5,
+    2 x 3000 10.4 / 11.0, 2 x 9000 19.8 / 18.3, 3 x 3000 11.5 / 13.1, 4 x 6000 21.3 / 22.0, 4 x 9000 33.1 / 32.7; 5 x 500 9.8 / 8.8, 5 x 3000 19.5 / 16.6."""
     import dataclasses
 
     from ..core.target import current_target
@@ -252,11 +258,17 @@ def calibrate_dispatch(pair, solo, factory, spec) -> dict:
 
     benchmark_over_workloads([pair, solo], observed, ramp_seconds=0.2)
     min_tiles = split_threshold(longest, pair.latency_us, solo.latency_us)
-    few = few_requests(spec, current_target().arch.compute_units)
-    lone_pair, lone_solo = dataclasses.replace(pair, latency_us={}), dataclasses.replace(solo, latency_us={})
-    benchmark_over_workloads([lone_pair, lone_solo], alone, ramp_seconds=0.0)
+    units = current_target().arch.compute_units
+    few = few_requests(spec, units)
+    lone_pair, lone_solo, lone_fixed = (c and dataclasses.replace(c, latency_us={}) for c in (pair, solo, fixed))
+    benchmark_over_workloads([c for c in (lone_pair, lone_solo, lone_fixed) if c], alone, ramp_seconds=0.0)
     lone_tiles = split_threshold(longest, lone_pair.latency_us, lone_solo.latency_us)
     keys = [k for k in longest if k in pair.latency_us and k in solo.latency_us]
+
+    few_parts = {}
+    if fixed and units >= fixed.split * int(spec.num_kv_heads):
+        few_parts = {"requests": units // (fixed.split * int(spec.num_kv_heads)),
+                     "until_tiles": split_threshold(longest, lone_pair.latency_us, lone_fixed.latency_us), "label": fixed.label}
 
     def splits(key):
         return longest[key] >= (lone_tiles if requests[key] < few else min_tiles)
@@ -271,7 +283,7 @@ def calibrate_dispatch(pair, solo, factory, spec) -> dict:
         "n_workloads": len(keys), "split_runs": sum(map(splits, keys)),
         "geomean_us": {"hybrid": geomean(list(per_workload.values())), "split": geomean([pair.latency_us[k] for k in keys]),
                        "single": geomean([solo.latency_us[k] for k in keys])},
-        "per_workload_us": per_workload,
+        "per_workload_us": per_workload, **({"fixed": few_parts} if few_parts else {}),
     }
 
 
@@ -476,13 +488,21 @@ class PagedKernel(Kernel):
     def dispatch_role(self, longest: int, requests: int | None = None) -> str:
         """``"split"`` or ``"single"`` for a batch of ``requests`` requests whose longest spans ``longest``
         page-table units, by the calibrated rule (kv tiles of the longest request against ``min_tiles``, or
-        ``lone_tiles`` where the requests are too few to fill the chip)."""
+        ``lone_tiles`` where the requests are too few to fill the chip); ``"fixed"`` where the split pair cuts the table into
+        items and a pair of equal parts was kept beside it for batches as small as this one."""
         rule, sources = self.dispatch, self.dispatch_sources
         if not rule or "split" not in sources or "single" not in sources:
             raise CleaveError(f"{self.name}: no split / single calibration was made (or saved) for this operator")
         few = requests is not None and requests < rule.get("few_requests", 0)
         # (tiles of the longest request, rounded up, against a whole number of them)
-        return "split" if int(longest) * rule["page_size"] > (rule["lone_tiles" if few else "min_tiles"] - 1) * rule["kv_tile"] else "single"
+        tokens, kv_tile = int(longest) * rule["page_size"], rule["kv_tile"]
+        if tokens <= (rule["lone_tiles" if few else "min_tiles"] - 1) * kv_tile:
+            return "single"
+        if requests is not None and "fixed" in sources and "fixed" in rule:
+            parts = rule["fixed"]
+            if requests <= parts["requests"] and tokens <= (parts["until_tiles"] * min(requests, max(1, parts["requests"] - 1)) - 1) * kv_tile:
+                return "fixed"
+        return "split"
 
     def token_role(self, tokens: int):
         """``"few"`` or ``"many"`` for a call with ``tokens`` packed query tokens, by the rule
@@ -618,7 +638,7 @@ def compile_dynamic(fn, *, dtype=None, preset="default", superopt=None, schedule
     value)`` is called after each stage."""
     from ..dynamic.paging import SPLIT_KINDS
     from ..frontend.paged import trace_paged
-    from ..runtime.autotune import WorkloadCandidate, benchmark_over_workloads, compile_and_validate_over_workloads
+    from ..runtime.autotune import WorkloadCandidate, benchmark_over_workloads, compile_and_validate_over_workloads, pick_best, rank
 
     others.pop("cache_kernels", None)
     if others:
@@ -673,9 +693,13 @@ def compile_dynamic(fn, *, dtype=None, preset="default", superopt=None, schedule
     both = {}
     if dispatch and pair is not None and single is not None:
         with search.stage("dispatch"):
-            report.dispatch = calibrate_dispatch(pair, single, factory, spec)
+            # (pages of many tokens go by the pair and the single kernel alone: an item of them has its ids in registers)
+            equal = [c for c in report.timed if c.eligible and c.split and not getattr(c.tiling, "chunk_pages", 0)]
+            items = getattr(pair.tiling, "chunk_pages", 0) and getattr(spec, "page_size", 1) == 1 and hasattr(spec, "num_kv_heads")
+            fixed = pick_best(rank(equal)) if items and equal else None
+            report.dispatch = calibrate_dispatch(pair, single, factory, spec, fixed)
         report.timings["dispatch"] = search.seconds["dispatch"]
-        both = {"split": pair.source, "single": single.source}
+        both = {"split": pair.source, "single": single.source, **({"fixed": fixed.source} if "fixed" in report.dispatch else {})}
     elif dispatch and attention.is_prefill:
         from ..runtime.autotune import param_index
 
