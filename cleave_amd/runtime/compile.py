@@ -269,15 +269,23 @@ class CompiledKernel:
             bound[p.name] = bound[owner]
         return outs
 
+    def _grids(self, dims, shared=False) -> dict:
+        """Position in the manifest -> grid of the launches a call of these extents makes: all but the optional ones whose grid is
+        empty.  ``shared``: of a call through the library's scratch array."""
+        grids = {}
+        for i, l in enumerate(self.manifest["launches"]):
+            grid = [eval_extent(g, dims) for g in (l.get("shared_grid", l["grid"]) if shared else l["grid"])]
+            if min(grid) >= 1 or not l.get("optional"):
+                grids[i] = grid
+        return grids
+
     def _descs(self, bound, dims, fixed=None, refs=None):
         """Launch descriptors.  ``fixed``: ``{scratch parameter: byte offset}``; those arguments are
         left null here and listed in ``refs`` as (launch, argument, offset) for the library to point
         into its fixed scratch array."""
         keep, descs = [], []
-        for l in self.manifest["launches"]:
-            grid = [eval_extent(g, dims) for g in (l["grid"] if fixed is None else l.get("shared_grid", l["grid"]))]
-            if min(grid) < 1 and l.get("optional"):
-                continue           # a launch that this call has no use for
+        for i, grid in self._grids(dims, shared=fixed is not None).items():
+            l = self.manifest["launches"][i]
             values = []
             for name in l["args"]:
                 if name in dims and name not in bound:
@@ -376,11 +384,21 @@ class CompiledKernel:
                 shim.launch_seq_fixed_scratch(descs, torch.cuda.current_stream(device).cuda_stream, refs, nbytes, clear)
         del keep
 
+    def _chosen(self, dims, only) -> list:
+        """Where, among the launches a call of these extents makes, those at the positions ``only`` of the manifest stand."""
+        launches, made = self.manifest["launches"], list(self._grids(dims))
+        wanted = [range(len(launches))[i] for i in only]
+        absent = [launches[i]["entry"] for i in wanted if i not in made]
+        if absent:
+            raise ValueError(f"a call of these extents leaves out {', '.join(absent)}")
+        return [made.index(i) for i in wanted]
+
     def time(self, *args, warmup: int = 4, iters: int = 100, rotate=None, only=None, graph_batch: int = 0) -> float:
         """Milliseconds per call measured with HIP events inside the native library.  ``rotate``:
         further argument tuples (same signature) cycled through call by call, so a working set
-        larger than the 256 MB last-level cache keeps every call reading HBM.  ``only``: indices
-        of the launches to time (e.g. ``[0]`` for the partial kernel of a fused pair alone).
+        larger than the 256 MB last-level cache keeps every call reading HBM.  ``only``: positions in the manifest
+        of the launches to time (e.g. ``[0]`` for the partial kernel of a fused pair alone); one that a call of these
+        extents leaves out is an error.
         ``graph_batch`` > 0: time replays of a HIP graph holding that many calls (the reference's
         way of timing) instead of an eager launch loop."""
         import torch
@@ -401,7 +419,8 @@ class CompiledKernel:
             if not descs:
                 raise ValueError("cannot time an empty launch")
             if only is not None:
-                descs, keep = [descs[i] for i in only], [keep[i] for i in only]
+                at = self._chosen(dims, only)
+                descs, keep = [descs[i] for i in at], [keep[i] for i in at]
             all_descs.append(descs)
             all_keep.append(keep)
         with torch.cuda.device(device):

@@ -114,3 +114,29 @@ def test_calls_that_share_their_scratch_need_none():
     caller.call_fixed_scratch(*args, *got)
     torch.cuda.synchronize()
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_launches_are_named_by_their_place_in_the_manifest():
+    """Also where a call leaves one out ahead of them."""
+    loaded = _load_main_kernel_from_code(source(16, 512, "bfloat16"))
+    kernel = _compile(loaded, None)
+    few, many = dict(total_q=64, batch=2), dict(total_q=8192, batch=2)
+    assert list(kernel._grids(few)) == [0] and list(kernel._grids(many)) == [1, 2] and list(kernel._grids(many, shared=True)) == [0]
+    assert kernel._chosen(few, [0]) == [0] and kernel._chosen(many, [2]) == kernel._chosen(many, [-1]) == [1] and kernel._chosen(many, [2, 1]) == [1, 0]
+    for dims, only in ((many, [0]), (few, [2]), (few, [0, 1])):
+        with pytest.raises(ValueError, match="leaves out main_kernel"):
+            kernel._chosen(dims, only)
+    with pytest.raises(IndexError):
+        kernel._chosen(many, [3])
+
+
+@pytest.mark.gpu
+def test_the_launch_that_was_asked_for_is_timed():
+    args = [a.cuda() if isinstance(a, torch.Tensor) else a for a in inputs([700] * 6, [900] * 6, 16, 512, "bfloat16", 0.05)]
+    loaded = _load_main_kernel_from_code(source(16, 512, "bfloat16"))
+    timed = _compile(loaded, loaded.manifest["out_idx"])
+    print("mla prefill stay: one launch timed", flush=True)
+    stay, clear = (timed.time(*args, warmup=4, iters=20, only=[i]) for i in (2, 1))
+    assert stay > 4 * clear                                  # (well over 50 us, and a few)
+    with pytest.raises(ValueError, match="leaves out main_kernel$"):
+        timed.time(*args, only=[0])
