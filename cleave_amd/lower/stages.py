@@ -43,7 +43,8 @@ def mla_po_elem(heads: int) -> bool:
 def partial_buffers(low: Lowered, factor: int) -> list:
     """``[(name, shape, dtype)]`` of what a split partial writes and its combine reads, split-major
     like the reference's ``(split, batch, heads[, D])`` layout
-    (``python/cleave/dynamic/paging/tensor_maps.py:41-69``); f32 except the MLA value partials of 64 heads or more."""
+    (``python/cleave/dynamic/paging/tensor_maps.py:41-69``); f32 except the MLA value partials of head counts that are
+    multiples of 64."""
     p = low.problem
     if low.family in ("matmul", "rmsnorm_matmul", "lora"):
         batch = max(p["batch_A"], p["batch_B"])

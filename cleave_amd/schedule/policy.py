@@ -23,6 +23,7 @@ import itertools
 import math
 
 from ..arch import Arch
+from ..lower.stages import mla_po_elem
 from .hint import TileDict
 
 ELEM_BYTES = {"float16": 2, "bfloat16": 2}
@@ -689,9 +690,9 @@ def mla_candidates(low, role, factor, arch: Arch):
         # a step's loads have (stages - 1) steps of matrix work to arrive in
         latency_clk = 4000.0 / (stages - 1)
         step_clk = max(step_clk, latency_clk)
-        # split partials go out and come back once (element type): 2 * splits * rows * ckv * 2 bytes
-        partial_clk = (4 * splits * p["batch"] * p["heads"] * p["ckv"]) / (arch.hbm_gbps * 1e3 * 0.6) * 2400 \
-            if splits > 1 else 0.0
+        # split partials go out and come back once
+        partial_bytes = 2 * splits * p["batch"] * p["heads"] * p["ckv"] * (2 if mla_po_elem(p["heads"]) else 4)
+        partial_clk = partial_bytes / (arch.hbm_gbps * 1e3 * 0.6) * 2400 if splits > 1 else 0.0
         score = passes * steps * step_clk * (1.0 + 0.3 * (1 - util)) + 8000 + partial_clk
         out.append(TileDict("mla_decode", role, dict(WAVES=waves, HG=hg, VSPLIT=vsplit, STAGES=stages),
                             output_tile=[heads_per_block, p["ckv"]], rstep_map={"kv": 32}, n_threads=waves * 64,
@@ -720,7 +721,7 @@ def mla_key_ranges(p, base, arch: Arch):
     in scratch, folded by a second launch.  As many ranges as give every compute unit the workgroups it holds, and one or half a
     workgroup each: requests x heads x keys, us, one range / ranges: 3 x 16 x 7233 345 / 15.5 (57; 30 with 16), 24 x 16 x 2869 156 / 24.1
     (18; 28.1 with 10, 39.4 with 5), 2 x 16 x 639 34 / 8.2 (20; 9.9 with 10), 6 x 128 x 7649 198 / 28.8 (20; 34.0 as the split form
-    at 8).  The split form, where a program asks for it, stays ahead for 64 heads and more on few keys, whose partials it halves
+    at 8).  The split form, where a program asks for it, stays ahead for multiples of 64 heads on few keys, whose partials it halves
     by keeping them in 16 bits: 4 x 64 x 1819 15.7 (8) against 17.7 (12)."""
     rows, steps = p["batch"] * p["heads"], _ceil(p["skv"], 32)
     blocks = p["batch"] * _ceil(p["heads"], base.output_tile[0])

@@ -54,3 +54,18 @@ def test_search_proposes_them_where_workgroups_are_few():
     assert ranges(B=2, H=16, SKV=32) == [] and ranges(B=32, H=16, SKV=40) == [2]
     assert combine_groups(48, 512, 57) == 8 and combine_groups(48, 64, 17) == 16
     assert combine_groups(48, 512, 16) == combine_groups(384, 512, 18) == combine_groups(48, 96, 57) == 1
+
+
+@pytest.mark.parametrize("heads,halved", [(16, False), (32, False), (64, True), (80, False), (128, True)])
+def test_the_cost_of_a_split_has_the_bytes_its_partials_are(heads, halved, monkeypatch):
+    from cleave_amd.lower.stages import partial_buffers
+    from cleave_amd.schedule import policy
+
+    graph = stage_graph(C.mla_decode.trace(cl.bf16, B=2, H=heads, D=512, PE=64, SKV=4096))
+    assert (partial_buffers(graph.lowered, 8)[2][2] == "bfloat16") == halved
+    partial = split_stages(graph, 8)[0]
+    cost = {c.key(): c.score for c in search_tiling(partial)}
+    monkeypatch.setattr(policy, "mla_po_elem", lambda heads: True)
+    for c in search_tiling(partial):
+        if "DUO" not in c.tiling:
+            assert (cost[c.key()] == c.score) == halved and cost[c.key()] >= c.score
