@@ -18,7 +18,7 @@
 //     4      A1 B0        B0 of the next step          A1
 //
 // 192 x 256 (GP_UNEVEN): A's halves are 128 and 64 rows, so phases 3 and 4 have half the matrix ops; a product of one round of
-// either tile takes 0.87 of the time of 256 x 256 ones (2300 x 5120 x 2048 39.0 us against 45.5, 5900 x 2048 x 1536 32.4 against 37.1).
+// either tile takes 0.9 of the time of 256 x 256 ones (f16, 2300 x 5120 x 2048 41.6 us against 46.1, 5900 x 2048 x 1536 33.7 against 37.6).
 //
 // The smaller tiles have half the matrix ops, so a phase takes both B halves:
 //

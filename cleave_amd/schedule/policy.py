@@ -152,12 +152,14 @@ def gemm_dma_candidates(low, role, factor, arch: Arch, twin_of=None):
     out = []
     shapes = (16, 32, 64, 128, 256)
     grids = ((1, 1), (1, 2), (2, 1), (2, 2), (1, 4), (4, 1), (2, 4), (4, 2))
-    # 192 x 256 tiles, of the two-group kernel only: a round of them takes 0.87 of one of 256 x 256 ones, so they are proposed where that
-    # many rounds (one workgroup per compute unit) are less.  us, 256 x 256 / these: 3479 x 3264 x 1984 45.8 / 41.6, 2300 x 5120 x 2048 45.5 /
-    # 39.0, 1536 x 8000 x 4096 84.4 / 72.4 (one round each); where they cost one round more 3000 x 5000 x 2048 52.7 / 72.4.
+    # 192 x 256 tiles, of the two-group kernel only: a round of them takes about 0.9 of one of 256 x 256 ones (0.78 to 0.93), so they are
+    # proposed where that many rounds (one workgroup per compute unit) are less.  us a call, f16, 256 x 256 / these: one round each 3479 x
+    # 3264 x 1984 44.3 / 40.9, 2300 x 5120 x 2048 46.1 / 41.6, 1536 x 8000 x 4096 83.4 / 77.8, 3916 x 3072 x 384 15.6 / 13.9, two each 2226 x
+    # 7296 x 544 35.2 / 29.0; where they cost one round more 3000 x 5000 x 2048 53.5 / 83.6.  Of 24 drawn products that are offered them
+    # they were the fastest of the eight tried in all, and none was fastest on the tiling they push out.
     uneven = (192, 256, (2, 4))
     rounds = {bm: _ceil(_ceil(M, bm) * _ceil(N, 256) * batch, arch.compute_units) for bm in (192, 256)}
-    fits = (not post_norm and twin_of != "matmul_rowsum" and splits == 1 and 0.87 * rounds[192] < rounds[256]
+    fits = (not post_norm and twin_of != "matmul_rowsum" and splits == 1 and 0.9 * rounds[192] < rounds[256]
             and phased_matmul("matmul", p, 1, dict(BM=192, BN=256, WM=2, WN=4)))
     for bm, bn, (wm, wn) in itertools.chain(itertools.product(shapes, shapes, grids), (uneven,) if fits else ()):
         if bm % (16 * wm) or bn % (16 * wn):
