@@ -69,3 +69,42 @@ def test_the_cost_of_a_split_has_the_bytes_its_partials_are(heads, halved, monke
     for c in search_tiling(partial):
         if "DUO" not in c.tiling:
             assert (cost[c.key()] == c.score) == halved and cost[c.key()] >= c.score
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,width,tiling", [(16, 128, dict(WAVES=1, STAGES=2)), (48, 256, dict(WAVES=1, STAGES=3)), (32, 64, dict(WAVES=2)), (64, 256, dict(DUO=1))],
+                         ids=lambda v: str(v) if isinstance(v, int) else "duo" if "DUO" in v else "w")
+@pytest.mark.parametrize("skv,ranges", [(65, 2), (640, 5), (1043, 17), (1043, 33)])
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+def test_ranges_of_other_widths(dtype, skv, ranges, heads, width, tiling):
+    """Latent rows of 64 to 256 features, whose combine has 8 or 16 thread groups above 16 ranges."""
+    prog = C.mla_decode.trace(getattr(cl, dtype), B=3, H=heads, D=width, PE=64, SKV=skv)
+    args = prog.random_inputs(seed=skv + heads, device="cpu")
+    print(f"mla ranges {dtype} h={heads} d={width} {tiling} {skv} / {ranges}", flush=True)
+    got = kernel_for(prog, template="mla_decode", tiling=dict(tiling, KEYS=ranges))(*[a.cuda() for a in args]).float().cpu().numpy()
+    want = program_oracle.evaluate(prog, args)[0]
+    # weights and result rounded once each, to 2^-9 (bf16) or 2^-12 (f16), of either sign
+    assert np.linalg.norm(got.reshape(want.shape) - want) / np.linalg.norm(want) < (2.0 ** -7 if dtype == "bf16" else 2.0 ** -10)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,batch", [(16, 3), (32, 2), (48, 1), (64, 2)])
+@pytest.mark.parametrize("split,skv", [(4, 640), (8, 1043), (8, 97)])
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+def test_the_split_form(dtype, split, skv, heads, batch):
+    """Partial and combine in one kernel's launches and as two kernels: f32 value partials, or (64 heads) element ones normalised per
+    split, which are rounded once more."""
+    prog = C.mla_decode.trace(getattr(cl, dtype), B=batch, H=heads, D=512, PE=64, SKV=skv)
+    args = prog.random_inputs(seed=heads, device="cpu")
+    print(f"mla split {dtype} h={heads} {split} x {skv}", flush=True)
+    cuda = [a.cuda() for a in args]
+    fused = kernel_for(prog, split=split)(*cuda)
+    partial, combine = (apply_tiling(search_tiling(g)[0]) for g in split_stages(stage_graph(prog), split))
+    first, second = (_load_main_kernel_from_code(HipCodeGen().gen(p)) for p in (partial, combine))
+    parts = _compile(first, first.manifest["out_idx"])(*cuda)
+    assert parts[2].dtype == (prog.dtype.torch if heads == 64 else torch.float32)
+    apart = _compile(second, second.manifest["out_idx"])(*parts)
+    want = program_oracle.evaluate(prog, args)[0]
+    for got in (fused, apart):
+        got = got.float().cpu().numpy().reshape(want.shape)
+        assert np.linalg.norm(got - want) / np.linalg.norm(want) < (2.0 ** -7 if dtype == "bf16" else 2.0 ** -10)
