@@ -854,7 +854,8 @@ class HipCodeGen:
 
         The line lies at three rounds of one workgroup per compute unit.  us, one workgroup an item / that stay, 16 heads: 1380 items
         of 24 requests 95.1 / 86.3, 2336 of 32 149.9 / 137.8, 1136 of 16 68.3 / 65.0; 568 of 8 33.8 / 34.9, 520 of 32 (up to 160 keys)
-        25.7 / 25.8, 464 of 12 24.1 / 26.7: there the clearing launch and the last round's uneven ends outweigh what overlaps.
+        25.7 / 25.8, 464 of 12 24.1 / 26.7: there the clearing launch (1.2 us by itself) and the last round's uneven
+        ends outweigh what overlaps.
         Rows so narrow that a compute unit holds two workgroups never stay: their items overlap without, and workgroups that stay are
         one a unit.  128 latent features, 816 items 15.2 / 21.0, 1368 of 24 requests 35.0 / 49.5, 2440 of 32 59.4 / 84.2; 256 (one a unit)
         59.6 / 61.5 and 103.8 / 105.2 on one card, 62.0 / 60.5 and 104.7 / 102.2 on another, 384 74.5 / 74.5 and 127.9 / 124.1."""
