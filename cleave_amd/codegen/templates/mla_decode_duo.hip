@@ -199,6 +199,70 @@ CL_DEVICE int md_clamp(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? h
 // every LDS access of this wave has completed, then the workgroup barrier
 CL_DEVICE void md_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
+// ---- parts of a step, of this kernel and of mla_prefill_duo.hip -----------------------------------
+// the value operand of feature block fb of an image; v_lo: the lane's place in the wave's first block
+CL_DEVICE void md_operand(const elem_t* tile, const int v_lo, const int fb, md_s16x4& lo, md_s16x4& hi) {
+  const elem_t* p = tile + (fb >> 2) * MD_PANEL + (v_lo ^ (((2 * fb) & 7) << 3));
+  lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((md_lds_s16x4*)(p));
+  hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((md_lds_s16x4*)(p + 16 * 64));
+}
+CL_DEVICE elem8 md_elem8(md_s16x4 lo, md_s16x4 hi) {
+  return __builtin_bit_cast(elem8, (md_s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+#if CL_PREFILL
+// Cold: a score wave raised a reference point at this step.  The half that stands against the lower point is multiplied here, by
+// itself, and the sums with it move to the higher point: its weights are 16 bits already, scaled they would be rounded a second
+// time.  Per head tile, as mostly one of the two has a raised head: 8987 tokens at a scale that raises a point on every sixth
+// step 160 us, both tiles together 163, weights rounded twice 157.
+CL_DEVICE void md_move_points(const elem_t* tile, const int v_lo, const f32x2 (&ref)[2], const elem8 ones, elem8 (&pf)[2], float (&m_acc)[2],
+                              f32x4 (&l_acc)[2], f32x4 (&acc)[2][MD_FBW]) {
+  elem8 p_low[2];
+  float alpha[2];
+  if (__builtin_amdgcn_ballot_w64(fminf(ref[0][0], ref[0][1]) > m_acc[0] || fminf(ref[1][0], ref[1][1]) > m_acc[1])) {
+    // (both halves raised theirs: the sums move to the lower one first)
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const float low = fminf(ref[t][0], ref[t][1]), a = fast_exp2(m_acc[t] - low);
+      m_acc[t] = low;
+#pragma unroll
+      for (int fb = 0; fb < MD_FBW; ++fb) acc[t][fb] *= a;
+      l_acc[t] *= a;
+    }
+  }
+  bool raised[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const float m_new = fmaxf(ref[t][0], ref[t][1]);          // never below m_acc
+    alpha[t] = fast_exp2(m_acc[t] - m_new);
+    raised[t] = __builtin_amdgcn_ballot_w64(ref[t][0] != m_acc[t] || ref[t][1] != m_acc[t]) != 0;
+    m_acc[t] = m_new;
+    p_low[t] = md_halves(pf[t], ref[t][0] < ref[t][1], ref[t][1] < ref[t][0]);
+    pf[t] = md_halves(pf[t], ref[t][0] >= ref[t][1], ref[t][1] >= ref[t][0]);
+    l_acc[t] = mfma16(ones, p_low[t], l_acc[t]) * alpha[t];
+  }
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    if (!raised[t]) continue;
+#pragma unroll
+    for (int fb0 = 0; fb0 < MD_FBW; fb0 += MD_COLD) {
+      __builtin_amdgcn_sched_barrier(0);
+      elem8 a[MD_COLD];
+#pragma unroll
+      for (int q = 0; q < MD_COLD; ++q) {
+        md_s16x4 lo, hi;
+        md_operand(tile, v_lo, fb0 + q, lo, hi);
+        a[q] = md_elem8(lo, hi);
+      }
+#pragma unroll
+      for (int q = 0; q < MD_COLD; ++q) acc[t][fb0 + q] = mfma16(a[q], p_low[t], acc[t][fb0 + q]);
+#pragma unroll
+      for (int q = 0; q < MD_COLD; ++q) acc[t][fb0 + q] *= alpha[t];
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+}
+#endif
+
 #if !CL_PREFILL
 // value wave `lw` (0..3): its loads of one step, panel P onwards -- token rows 8 lw + lane / 8 of
 // every panel, the chunk that belongs in slot lane % 8
@@ -617,11 +681,6 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
   md_s16x4 pre_lo[MD_PRE], pre_hi[MD_PRE];
 #pragma unroll
   for (int fb = 0; fb < MD_PRE; ++fb) pre_lo[fb] = pre_hi[fb] = (md_s16x4){0, 0, 0, 0};
-  auto operand = [&](const elem_t* tile, int fb, md_s16x4& lo, md_s16x4& hi) __attribute__((always_inline)) {
-    const elem_t* p = tile + (fb >> 2) * MD_PANEL + (v_lo ^ (((2 * fb) & 7) << 3));
-    lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((md_lds_s16x4*)(p));
-    hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((md_lds_s16x4*)(p + 16 * 64));
-  };
   for (int it = 0; it <= n_own; ++it) {
     // image `it` must have landed before the barrier lets the score waves read it: at most the
     // loads of image it + 1 may be outstanding (none are issued for an empty split)
@@ -646,7 +705,7 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
       }
 #endif
 #pragma unroll
-      for (int fb = 0; fb < MD_PRE; ++fb) operand(next_tile, fb, pre_lo[fb], pre_hi[fb]);
+      for (int fb = 0; fb < MD_PRE; ++fb) md_operand(next_tile, v_lo, fb, pre_lo[fb], pre_hi[fb]);
       continue;
     }
     const elem_t* tile = md_tiles + ((it - 1) % MD_STAGES) * MD_TILE;
@@ -662,56 +721,8 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
     }
 #if CL_PREFILL
     if (__builtin_amdgcn_ballot_w64(ref[0][0] != m_acc[0] || ref[0][1] != m_acc[0] || ref[1][0] != m_acc[1] ||
-                                    ref[1][1] != m_acc[1])) {
-      // cold: a score wave raised a reference point at this step.  The half that stands against the lower point is multiplied
-      // here, by itself, and the sums with it move to the higher point: its weights are 16 bits already, scaled they would
-      // be rounded a second time.  Per head tile, as mostly one of the two has a raised head: 8987 tokens at a scale that
-      // raises a point on every sixth step 160 us, both tiles together 163, weights rounded twice 157.
-      elem8 p_low[2];
-      float alpha[2];
-      if (__builtin_amdgcn_ballot_w64(fminf(ref[0][0], ref[0][1]) > m_acc[0] || fminf(ref[1][0], ref[1][1]) > m_acc[1])) {
-        // (both halves raised theirs: the sums move to the lower one first)
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          const float low = fminf(ref[t][0], ref[t][1]), a = fast_exp2(m_acc[t] - low);
-          m_acc[t] = low;
-#pragma unroll
-          for (int fb = 0; fb < MD_FBW; ++fb) acc[t][fb] *= a;
-          l_acc[t] *= a;
-        }
-      }
-      bool raised[2];
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const float m_new = fmaxf(ref[t][0], ref[t][1]);          // never below m_acc
-        alpha[t] = fast_exp2(m_acc[t] - m_new);
-        raised[t] = __builtin_amdgcn_ballot_w64(ref[t][0] != m_acc[t] || ref[t][1] != m_acc[t]) != 0;
-        m_acc[t] = m_new;
-        p_low[t] = md_halves(pf[t], ref[t][0] < ref[t][1], ref[t][1] < ref[t][0]);
-        pf[t] = md_halves(pf[t], ref[t][0] >= ref[t][1], ref[t][1] >= ref[t][0]);
-        l_acc[t] = mfma16(ones, p_low[t], l_acc[t]) * alpha[t];
-      }
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        if (!raised[t]) continue;
-#pragma unroll
-        for (int fb0 = 0; fb0 < MD_FBW; fb0 += MD_COLD) {
-          __builtin_amdgcn_sched_barrier(0);
-          elem8 a[MD_COLD];
-#pragma unroll
-          for (int q = 0; q < MD_COLD; ++q) {
-            md_s16x4 lo, hi;
-            operand(tile, fb0 + q, lo, hi);
-            a[q] = __builtin_bit_cast(elem8, (md_s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-          }
-#pragma unroll
-          for (int q = 0; q < MD_COLD; ++q) acc[t][fb0 + q] = mfma16(a[q], p_low[t], acc[t][fb0 + q]);
-#pragma unroll
-          for (int q = 0; q < MD_COLD; ++q) acc[t][fb0 + q] *= alpha[t];
-        }
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
+                                    ref[1][1] != m_acc[1]))
+      md_move_points(tile, v_lo, ref, ones, pf, m_acc, l_acc, acc);
 #else
     if (__builtin_amdgcn_ballot_w64(ref[0][0] != m_acc[0] || ref[0][1] != m_acc[0] || ref[1][0] != m_acc[1] ||
                                     ref[1][1] != m_acc[1])) {
@@ -749,14 +760,14 @@ CL_PARTIAL_NAME(CL_PARTIAL_PARAMS) {
 #pragma unroll
     for (int fb = 0; fb < MD_FBW; ++fb) {
       md_s16x4 lo = pre_lo[fb % MD_PRE], hi = pre_hi[fb % MD_PRE];
-      const elem8 a = __builtin_bit_cast(elem8, (md_s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+      const elem8 a = md_elem8(lo, hi);
 #pragma unroll
       for (int t = 0; t < 2; ++t) acc[t][fb] = mfma16(a, pf[t], acc[t][fb]);
       // the operand MD_PRE blocks on: of this image, or (the last MD_PRE) of the next one
       if (fb + MD_PRE < MD_FBW)
-        operand(tile, fb + MD_PRE, pre_lo[fb % MD_PRE], pre_hi[fb % MD_PRE]);
+        md_operand(tile, v_lo, fb + MD_PRE, pre_lo[fb % MD_PRE], pre_hi[fb % MD_PRE]);
       else
-        operand(next_tile, fb + MD_PRE - MD_FBW, pre_lo[fb % MD_PRE], pre_hi[fb % MD_PRE]);
+        md_operand(next_tile, v_lo, fb + MD_PRE - MD_FBW, pre_lo[fb % MD_PRE], pre_hi[fb % MD_PRE]);
 #pragma unroll
       for (int pn = CL_S_PANELS; pn < MD_PANELS; ++pn)
         if (((pn - CL_S_PANELS) * MD_FBW) / MD_V_UNITS == fb) {

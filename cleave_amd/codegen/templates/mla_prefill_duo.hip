@@ -1,10 +1,10 @@
 // ---- paged causal MLA prefill with score waves and value waves, workgroups that stay -----------------------
 //
-// The operator, images, LDS layouts and division of labour of mla_decode_duo.hip (read that first) over ragged query rows: the 64 rows
-// of an item are four consecutive query tokens of one request (a new item at every multiple of four packed tokens and at
-// every request boundary) x 16 heads, so a 16-row tile is one token and its causal limit is uniform over a wave; key rows are looked
-// up in the token table.  Where one token half raises its reference point, the other's weights are not scaled and rounded again:
-// their product is taken by itself and moved (cold).  The score waves sum the unrounded weights for the lse.
+// The operator, images, LDS arrays and division of labour of mla_decode_duo.hip (which stands ahead of this one: read it first) over
+// ragged query rows: the 64 rows of an item are four consecutive query tokens of one request (a new item at every multiple of four
+// packed tokens and at every request boundary) x 16 heads, so a 16-row tile is one token and its causal limit is uniform over a wave;
+// key rows are looked up in the token table.  Where one token half raises its reference point, the other's weights are not scaled and
+// rounded again: their product is taken by itself and moved (cold).  The score waves sum the unrounded weights for the lse.
 //
 // A compute unit holds one workgroup (four images fill its LDS), so whatever an item does before its first and after its last step
 // used to stand still: of 15.7 us an item of 8.4 steps (24 requests of up to 350 tokens, stamps in the kernel) 0.5 went to finding its
@@ -28,81 +28,29 @@
 // Addresses that follow from the lane alone are hidden from the optimiser where they are worked out once an item: hoisted out of
 // the walk they took the registers that the key fragments of a step are read ahead into (1.07 -> 1.41 us a step).
 //
+// The scores, weights and value product of a step are written out in both kernels: as functions that both call, the 512-wide form
+// of this one spilled, and its other forms compiled to other schedules.
+//
 //   CL_HEADS (multiple of 16)  CL_CKV (multiple of 128)  CL_KPE (odd multiple of 64)
 //   run-time: total_q, num_pages, n_idx, batch; scalar sm_scale (any sign)
 
 #if CL_EMIT_STAY
-#define MS_STEP 32
-#define MS_D (CL_CKV + CL_KPE)
-#define MS_PANEL (MS_STEP * 64)
-#define MS_PANELS (MS_D / 64)                    // also the 1 KiB loads of a value wave per image
-#define MS_LAT_PANELS (CL_CKV / 64)
-#define MS_TILE (MS_PANELS * MS_PANEL)           // elements of one image: 32 key rows, or 32 query rows
-#define MS_STAGES 4
-#define MS_KJ (MS_D / 32)
-#define MS_FBW (CL_CKV / 32)                     // feature blocks one value wave accumulates
-#define MS_TOKENS 4                              // query tokens of an item, 16 heads each
 #define MS_GROUPS (CL_HEADS / 16)
-#define MS_RESCALE_STEP 8.0f
-#define MS_QCHUNKS (MS_D / 8)                    // 16-byte chunks of one query row (latent + rope)
-#define MS_REF_FLOOR (-1.0e20f)                  // lowest reference point: a token half with every token masked stands here
-#define MS_COLD (MS_FBW % 8 == 0 ? 8 : 4)        // feature blocks read together where a reference point was raised
-#define MS_STORES MS_FBW                         // stores of a value wave per full item: two tiles of FBW / 2
-#ifndef CL_LDS_AHEAD
-#define CL_LDS_AHEAD 8
-#endif
-static_assert(CL_HEADS % 16 == 0 && CL_CKV % 128 == 0 && CL_KPE % 128 == 64, "16 heads a tile, halved latent panels, an odd number of panels");
-static_assert(MS_QCHUNKS % 16 == 8, "the query rows in LDS: a row's parity moves it by eight 16-byte bank groups");
-static_assert(MS_PANELS + 1 + MS_STORES < 64 && MS_FBW % 4 == 0, "load counter range; an item's stores leave in quarters");
+#define MS_STORES MD_FBW                         // stores of a value wave per full item: two tiles of FBW / 2
+static_assert(CL_KPE % 128 == 64, "an odd number of panels");
+static_assert(MD_PANELS + 1 + MS_STORES < 64 && MD_FBW % 4 == 0, "load counter range; an item's stores leave in quarters");
 
-__shared__ __attribute__((aligned(1024))) elem_t ms_tiles[MS_STAGES * MS_TILE];
-// [image parity][head set][head tile][token half][lane]: the lane's four weights of each token half
-__shared__ __attribute__((aligned(16))) u32x2 ms_weights[2][2][2][2][64];
-// [image parity][head set][head tile][head][token half]: the reference point those weights stand against
-__shared__ __attribute__((aligned(8))) float ms_ref[2][2][2][16][2];
-// [value wave][image % 4][lane]: the table entry of the key row this lane fetches
-__shared__ __attribute__((aligned(256))) int ms_ids[4][MS_STAGES][64];
-// [head set][tile][head][token half]: the reference point and the sum of the unrounded weights a score wave ends with
-__shared__ __attribute__((aligned(8))) f32x2 ms_sums[2][2][16][2];
 __shared__ __attribute__((aligned(16))) int ms_items[2][8];     // [item parity]: what MsItem holds
 
-typedef short ms_s16x4 __attribute__((ext_vector_type(4)));
-typedef short ms_s16x8 __attribute__((ext_vector_type(8)));
-typedef __attribute__((address_space(3))) ms_s16x4 ms_lds_s16x4;
-
-CL_DEVICE int ms_swz(int token) { return token & 6; }
-CL_DEVICE int ms_clamp(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
-// x with bits 0 and 3 trading places
-CL_DEVICE int ms_trade03(int x) { return (x & ~9) | ((x & 1) << 3) | ((x >> 3) & 1); }
 // rows (16 lanes) 1 and 3 of a0 and a1 trade places with rows 0 and 2 of b0 and b1
 CL_DEVICE void ms_swap_rows16(unsigned& a0, unsigned& a1, unsigned& b0, unsigned& b1) {
   asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %2\n\tv_permlane16_swap_b32 %1, %3\n\ts_nop 0" : "+v"(a0), "+v"(a1), "+v"(b0), "+v"(b1));
-}
-// 16 and 4 bytes per lane, global -> LDS; not counted by the compiler, the issuing wave waits itself.  (No compiler-level memory
-// barrier: what they write no wave reads before the next workgroup barrier, so LDS reads may be scheduled across them.)
-CL_DEVICE void ms_dma16(const void* gptr, unsigned lds_byte) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
-               :: "v"(gptr), "s"(__builtin_amdgcn_readfirstlane(lds_byte)) : "m0");
-}
-CL_DEVICE void ms_dma4(const void* gptr, unsigned lds_byte) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off"
-               :: "v"(gptr), "s"(__builtin_amdgcn_readfirstlane(lds_byte)) : "memory", "m0");
 }
 // 16 bytes per lane, counted with the loads (in the order they are written here).  (The wait state: the registers of a wide store
 // may be written again only behind it.)
 CL_DEVICE void ms_store16(void* gptr, u32x4 v) {
   asm volatile("global_store_dwordx4 %0, %1, off\n\ts_nop 1" :: "v"(gptr), "v"(v) : "memory");
 }
-// a lane's eight weights with the token halves that are not wanted set to zero.  (Hidden from the optimiser: seeing a
-// selection it copied the whole value product for weights taken as they are, and spilled the second set of accumulators.)
-CL_DEVICE elem8 ms_halves(elem8 p, bool want_lo, bool want_hi) {
-  const u32x4 w = __builtin_bit_cast(u32x4, p);
-  u32x4 y = {want_lo ? w[0] : 0u, want_lo ? w[1] : 0u, want_hi ? w[2] : 0u, want_hi ? w[3] : 0u};
-  asm volatile("" : "+v"(y));
-  return as_elem8(y);
-}
-// every LDS access of this wave has completed, then the workgroup barrier
-CL_DEVICE void ms_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 // waits until at most n of the wave's loads and stores are out
 #define MS_WAITCNT(n) __builtin_amdgcn_s_waitcnt(0x0F70 | ((n) & 15) | (((n) >> 4) << 14))
 
@@ -131,7 +79,7 @@ CL_STAY_NAME(CL_STAY_PARAMS) {
   // (value) (w / 2) % 2.  Wave w runs on SIMD w % 4: one score wave and one value wave on every SIMD.
   const bool scores = wave < 4;
   const int set = wave & 1, half = (wave >> 1) & 1;
-  const unsigned tiles_byte = (unsigned)(size_t)(__attribute__((address_space(3))) elem_t*)ms_tiles;
+  const unsigned tiles_byte = (unsigned)(size_t)(__attribute__((address_space(3))) elem_t*)md_tiles;
   const int grid = (int)gridDim.x;
 
   // ---- items (score wave 0) --------------------------------------------------------------------
@@ -139,10 +87,10 @@ CL_STAY_NAME(CL_STAY_PARAMS) {
   // more keys, and what starts last should be short.  First round: runs of four neighbouring items go to one XCD (launch index
   // % 8; the grid is a multiple of eight): they read the same keys, which every XCD that works on a request fetches into its own
   // L2.  After it, tickets in order.
-  const int axis = (((total_q + MS_TOKENS - 1) / MS_TOKENS + batch + 7) / 8) * 8, total = axis * MS_GROUPS;
+  const int axis = (((total_q + MD_TOKENS - 1) / MD_TOKENS + batch + 7) / 8) * 8, total = axis * MS_GROUPS;
   const int ptr_q = cl_clamp_ptr(CL_ARG_QINDPTR[lane < batch ? lane : batch], total_q);     // fewer than 64 requests: one a lane
   const int ptr_k = cl_clamp_ptr(CL_ARG_INDPTR[lane < batch ? lane : batch], n_idx);
-  const int first_chunk = lane < batch ? lane + ptr_q / MS_TOKENS : 0x7fffffff;
+  const int first_chunk = lane < batch ? lane + ptr_q / MD_TOKENS : 0x7fffffff;
   auto find_item = [&](int order) __attribute__((always_inline)) {
     MsItem it = {0, 0, 0, 0, 0, 0, 0, 0};
     int index = total - 1 - order;
@@ -159,16 +107,16 @@ CL_STAY_NAME(CL_STAY_PARAMS) {
       found.s0 = __builtin_amdgcn_readlane(ptr_k, found.req);
       found.s1 = __builtin_amdgcn_readlane(ptr_k, found.req + 1);
     } else {
-      found = cl_find_request(CL_ARG_QINDPTR, batch, total_q, MS_TOKENS, 1, index, lane, CL_ARG_INDPTR, n_idx);
+      found = cl_find_request(CL_ARG_QINDPTR, batch, total_q, MD_TOKENS, 1, index, lane, CL_ARG_INDPTR, n_idx);
     }
     const int chunk = index - found.req;
-    it.t_lo = found.p0 > chunk * MS_TOKENS ? found.p0 : chunk * MS_TOKENS;
-    it.t_hi = found.p1 < (chunk + 1) * MS_TOKENS ? found.p1 : (chunk + 1) * MS_TOKENS;
+    it.t_lo = found.p0 > chunk * MD_TOKENS ? found.p0 : chunk * MD_TOKENS;
+    it.t_hi = found.p1 < (chunk + 1) * MD_TOKENS ? found.p1 : (chunk + 1) * MD_TOKENS;
     it.lo = found.s0;
     it.kv_len = found.s1 > found.s0 ? found.s1 - found.s0 : 0;
     it.first_seen = it.kv_len - (found.p1 - found.p0) + (it.t_lo - found.p0) + 1;
-    it.hi = it.lo + ms_clamp(it.first_seen + (it.t_hi - 1 - it.t_lo), 0, it.kv_len);
-    it.n = it.t_hi > it.t_lo ? (it.hi - it.lo + MS_STEP - 1) / MS_STEP : 0;
+    it.hi = it.lo + md_clamp(it.first_seen + (it.t_hi - 1 - it.t_lo), 0, it.kv_len);
+    it.n = it.t_hi > it.t_lo ? (it.hi - it.lo + MD_STEP - 1) / MD_STEP : 0;
     return ms_uniform(it);
   };
   auto draw = [&]() __attribute__((always_inline)) {
@@ -215,46 +163,46 @@ CL_STAY_NAME(CL_STAY_PARAMS) {
       write_nothing(cur);
       publish(draw(), 0);
     }
-    ms_barrier();
+    md_barrier();
     cur = ms_item(0);
     if (cur.n == 0) return;
-    ms_barrier();                                   // (read by everybody before it is written again)
+    md_barrier();                                   // (read by everybody before it is written again)
   }
   // this wave's share of the loads: 8-row group `loader` of every image
   const int loader = 2 * (wave & 1) + half;
-  // Query rows 32 part .. + 31 of an item (rows past its tokens repeat the last one): row n / MS_QCHUNKS holds the row whose number
-  // is that with bits 0 and 3 traded, and slot n % MS_QCHUNKS of it the 16-byte chunk whose low three bits are the slot's
+  // Query rows 32 part .. + 31 of an item (rows past its tokens repeat the last one): row n / MD_QCHUNKS holds the row whose number
+  // is that with bits 0 and 3 traded, and slot n % MD_QCHUNKS of it the 16-byte chunk whose low three bits are the slot's
   // XOR head % 8: a fragment read has the sixteen heads of a tile side by side, spread over all banks.
   auto query_piece = [&](const MsItem& it, int part, int j, int at) __attribute__((always_inline)) {
     const int n = 64 * j + at;
-    const int row = 32 * part + 8 * loader + n / MS_QCHUNKS, pos = n % MS_QCHUNKS;
-    const int h = ms_trade03(row);
+    const int row = 32 * part + 8 * loader + n / MD_QCHUNKS, pos = n % MD_QCHUNKS;
+    const int h = md_trade03(row);
     const int q = (pos & ~7) | ((pos ^ h) & 7);
     const int token = it.t_lo + (h >> 4) < it.t_hi ? it.t_lo + (h >> 4) : it.t_hi - 1;
     const i64 qrow = (i64)token * CL_HEADS + it.head0 + (h & 15);
     return reinterpret_cast<const char*>(q < CL_CKV / 8 ? CL_ARG_Q + qrow * CL_CKV + 8 * q : CL_ARG_QPE + qrow * CL_KPE + 8 * (q - CL_CKV / 8));
   };
-  const unsigned query_dst = tiles_byte + (unsigned)(loader * (MS_PANELS * 1024));
+  const unsigned query_dst = tiles_byte + (unsigned)(loader * (MD_PANELS * 1024));
 
   if (scores) {
     // =========================================================================== score wave
     // Q fragments (B operand): lane (c, g) holds q[row c of tile t][32 j + 8 g .. + 8]
-    elem8 qf[2][MS_KJ];
+    elem8 qf[2][MD_KJ];
     float m_run[2] = {CL_NEG_BIG, CL_NEG_BIG};      // reference point of head c of each tile (log2 domain), uniform over g
     float l_exact[2] = {0.f, 0.f};                  // this lane's share of the sum of the unrounded weights
     const float scale_log2e = sm_scale * 1.4426950408889634f;
-    const int a_lo = (16 * half + c) * 64 + ((g ^ ms_swz(c)) << 3);
+    const int a_lo = (16 * half + c) * 64 + ((g ^ md_swz(c)) << 3);
     auto read_queries = [&](int image) __attribute__((always_inline)) {
       int at = lane;
       asm volatile("" : "+v"(at));                  // (its addresses are worked out again for every item: kept, they take the registers
       const int col = at & 15, grp = at >> 4;       // that the key fragments of a step are read ahead into)
-      const elem_t* rows = ms_tiles + (image % MS_STAGES) * MS_TILE;
+      const elem_t* rows = md_tiles + (image % MD_STAGES) * MD_TILE;
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int j = 0; j < MS_KJ; ++j) {
-          const int row = 16 * t + ms_trade03(col), q = 4 * j + grp;
-          qf[t][j] = *reinterpret_cast<const elem8*>(rows + (row * MS_QCHUNKS + ((q & ~7) | ((q ^ col) & 7))) * 8);
+        for (int j = 0; j < MD_KJ; ++j) {
+          const int row = 16 * t + md_trade03(col), q = 4 * j + grp;
+          qf[t][j] = *reinterpret_cast<const elem8*>(rows + (row * MD_QCHUNKS + ((q & ~7) | ((q ^ col) & 7))) * 8);
         }
     };
     // what this wave ends an item with, ahead of the barrier that ends it
@@ -263,7 +211,7 @@ CL_STAY_NAME(CL_STAY_PARAMS) {
       for (int t = 0; t < 2; ++t) {
         l_exact[t] += lane_xor(l_exact[t], lane, 16);
         l_exact[t] += lane_xor(l_exact[t], lane, 32);
-        if (g == 0) ms_sums[set][t][c][half] = (f32x2){m_run[t], l_exact[t]};
+        if (g == 0) md_sums[set][t][c][half] = (f32x2){m_run[t], l_exact[t]};
       }
     };
     // the lse rows of an item, behind that barrier
@@ -274,7 +222,7 @@ CL_STAY_NAME(CL_STAY_PARAMS) {
         for (int t = 0; t < 2; ++t) {
           const int token = it.t_lo + 2 * set + t;
           if (token >= it.t_hi) continue;
-          const f32x2 a = ms_sums[set][t][c][0], b = ms_sums[set][t][c][1];
+          const f32x2 a = md_sums[set][t][c][0], b = md_sums[set][t][c][1];
           const float m_both = fmaxf(a[0], b[0]);
           const float l_both = a[1] * fast_exp2(a[0] - m_both) + b[1] * fast_exp2(b[0] - m_both);
           CL_ARG_LSE[(i64)token * CL_HEADS + it.head0 + c] = l_both > 0.f ? m_both + fast_log2(l_both) : CL_NEG_INF;
@@ -285,7 +233,7 @@ CL_STAY_NAME(CL_STAY_PARAMS) {
     };
     // (the first item's first image comes through these waves)
 #pragma unroll
-    for (int j = 0; j < MS_PANELS; ++j) ms_dma16(query_piece(cur, 0, j, lane), query_dst + 1024 * j);
+    for (int j = 0; j < MD_PANELS; ++j) md_dma16_loose(query_piece(cur, 0, j, lane), query_dst + 1024 * j);
     MS_WAITCNT(0);
     MsItem last = cur;
     int ticket = 0;
@@ -299,19 +247,19 @@ CL_STAY_NAME(CL_STAY_PARAMS) {
         }
       };
       if (k > 0) leave_sums();
-      ms_barrier();                                 // image Q 0 has landed
+      md_barrier();                                 // image Q 0 has landed
       if (set == 0) read_queries(image);
       look_ahead(0);
       if (k > 0) write_lse(last);
       ++image;
-      ms_barrier();                                 // image Q 1 has landed
+      md_barrier();                                 // image Q 1 has landed
       if (set == 1) read_queries(image);
       look_ahead(1);
       ++image;
       int n_tok[2];                                 // keys the token of each tile sees
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
-        n_tok[t] = cur.t_lo + 2 * set + t < cur.t_hi ? ms_clamp(cur.first_seen + 2 * set + t, 0, cur.kv_len) : 0;
+        n_tok[t] = cur.t_lo + 2 * set + t < cur.t_hi ? md_clamp(cur.first_seen + 2 * set + t, 0, cur.kv_len) : 0;
         m_run[t] = CL_NEG_BIG;
         l_exact[t] = 0.f;
       }
@@ -319,14 +267,14 @@ CL_STAY_NAME(CL_STAY_PARAMS) {
       int it = 0;
       for (int stop = cur.n > 4 ? cur.n - 5 : cur.n > 2 ? cur.n - 3 : cur.n;;) {
       for (; it < stop; ++it, ++image) {
-        ms_barrier();                               // this key image has landed (the value waves waited for it)
-        const elem_t* tile = ms_tiles + (image % MS_STAGES) * MS_TILE;
+        md_barrier();                               // this key image has landed (the value waves waited for it)
+        const elem_t* tile = md_tiles + (image % MD_STAGES) * MD_TILE;
         const int par = image & 1;
         // the points the other token half used one step ago: asked for first, so that the answer is
         // there when the matrix ops are done
         float other[2];
 #pragma unroll
-        for (int t = 0; t < 2; ++t) other[t] = ms_ref[par ^ 1][set][t][c][half ^ 1];
+        for (int t = 0; t < 2; ++t) other[t] = md_ref[par ^ 1][set][t][c][half ^ 1];
         __builtin_amdgcn_sched_barrier(0);
         // scores^T: rows = tokens 16 half + (0..15), columns = heads of tile t; even and odd
         // 32-feature slices in accumulators of their own
@@ -334,14 +282,14 @@ CL_STAY_NAME(CL_STAY_PARAMS) {
 #pragma unroll
         for (int t = 0; t < 2; ++t) sp[t][0] = sp[t][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int j = 0; j < MS_KJ; ++j) {
-          const elem8 a = *reinterpret_cast<const elem8*>(tile + (j >> 1) * MS_PANEL + (a_lo ^ ((4 * (j & 1)) << 3)));
+        for (int j = 0; j < MD_KJ; ++j) {
+          const elem8 a = *reinterpret_cast<const elem8*>(tile + (j >> 1) * MD_PANEL + (a_lo ^ ((4 * (j & 1)) << 3)));
 #pragma unroll
           for (int t = 0; t < 2; ++t) sp[t][j & 1] = mfma16(a, qf[t][j], sp[t][j & 1]);
         }
         __builtin_amdgcn_sched_group_barrier(0x100, CL_LDS_AHEAD, 0);
 #pragma unroll
-        for (int n = 0; n < MS_KJ - CL_LDS_AHEAD; ++n) {
+        for (int n = 0; n < MD_KJ - CL_LDS_AHEAD; ++n) {
           __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
           __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         }
@@ -351,8 +299,8 @@ CL_STAY_NAME(CL_STAY_PARAMS) {
         for (int t = 0; t < 2; ++t) st[t] = (sp[t][0] + sp[t][1]) * scale_log2e;
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-          if ((it + 1) * MS_STEP > n_tok[t]) {      // keys past the token's limit: weight exp2(-huge) = 0
-            const int t0 = it * MS_STEP + 16 * half + 4 * g;
+          if ((it + 1) * MD_STEP > n_tok[t]) {      // keys past the token's limit: weight exp2(-huge) = 0
+            const int t0 = it * MD_STEP + 16 * half + 4 * g;
 #pragma unroll
             for (int r = 0; r < 4; ++r)
               if (t0 + r >= n_tok[t]) st[t][r] = CL_NEG_BIG;
@@ -365,7 +313,7 @@ CL_STAY_NAME(CL_STAY_PARAMS) {
           mx[t] = fmaxf(fmaxf(st[t][0], st[t][1]), fmaxf(st[t][2], st[t][3]));
           m_run[t] = it > 0 ? fmaxf(m_run[t], other[t]) : m_run[t];      // adopted where higher
         }
-        if (it == 0 || __builtin_amdgcn_ballot_w64(mx[0] > m_run[0] + MS_RESCALE_STEP || mx[1] > m_run[1] + MS_RESCALE_STEP)) {
+        if (it == 0 || __builtin_amdgcn_ballot_w64(mx[0] > m_run[0] + MD_RESCALE_STEP || mx[1] > m_run[1] + MD_RESCALE_STEP)) {
           // cold after the first step: each head's largest score of this step over all four lane groups
 #pragma unroll
           for (int t = 0; t < 2; ++t) {
@@ -373,17 +321,17 @@ CL_STAY_NAME(CL_STAY_PARAMS) {
             v = fmaxf(v, lane_xor(v, lane, 16));
             v = fmaxf(v, lane_xor(v, lane, 32));
             if (it == 0)
-              m_run[t] = fmaxf(v, MS_REF_FLOOR);    // nothing behind it yet: the step's own maximum
-            else if (v > m_run[t] + MS_RESCALE_STEP)
+              m_run[t] = fmaxf(v, MD_REF_FLOOR);    // nothing behind it yet: the step's own maximum
+            else if (v > m_run[t] + MD_RESCALE_STEP)
               m_run[t] = v;
-            if (it == 0 && g == 0) ms_ref[par ^ 1][set][t][c][half] = m_run[t];
+            if (it == 0 && g == 0) md_ref[par ^ 1][set][t][c][half] = m_run[t];
           }
           if (it == 0) {
             // both token halves start from the larger of their maxima: no weight of the first step is scaled (and
             // rounded) a second time.  (This slot is written again behind the next iteration's barrier.)
-            ms_barrier();
+            md_barrier();
 #pragma unroll
-            for (int t = 0; t < 2; ++t) m_run[t] = fmaxf(m_run[t], ms_ref[par ^ 1][set][t][c][half ^ 1]);
+            for (int t = 0; t < 2; ++t) m_run[t] = fmaxf(m_run[t], md_ref[par ^ 1][set][t][c][half ^ 1]);
           }
         }
         if (__builtin_amdgcn_ballot_w64(m_run[0] != m_before[0] || m_run[1] != m_before[1])) {
@@ -399,8 +347,8 @@ CL_STAY_NAME(CL_STAY_PARAMS) {
             l_exact[t] += p;
             pf[r] = to_elem(p);
           }
-          ms_weights[par][set][t][half][lane] = __builtin_bit_cast(u32x2, pf);
-          if (g == 0) ms_ref[par][set][t][c][half] = m_run[t];
+          md_weights[par][set][t][half][lane] = __builtin_bit_cast(u32x2, pf);
+          if (g == 0) md_ref[par][set][t][c][half] = m_run[t];
         }
       }
       if (it == cur.n) break;
@@ -413,7 +361,7 @@ CL_STAY_NAME(CL_STAY_PARAMS) {
       cur = next;
     }
     leave_sums();
-    ms_barrier();                                   // (the value waves take the last step's product)
+    md_barrier();                                   // (the value waves take the last step's product)
     write_lse(last);
     return;
   }
@@ -423,49 +371,49 @@ CL_STAY_NAME(CL_STAY_PARAMS) {
   // (positions past the item's end repeat the last one; ids are clamped into the pool) travel through LDS on the same load
   // counter as the rows: those of image i + 4 are asked for ahead of the rows of image i + 2.
   const int row_in_step = 8 * loader + (lane >> 3);
-  const int row_chunk = (lane & 7) ^ ms_swz(row_in_step);
-  const unsigned ids_byte = (unsigned)(size_t)(__attribute__((address_space(3))) int*)&ms_ids[loader][0][0];
+  const int row_chunk = (lane & 7) ^ md_swz(row_in_step);
+  const unsigned ids_byte = (unsigned)(size_t)(__attribute__((address_space(3))) int*)&md_ids[loader][0][0];
   auto ask_ids = [&](const MsItem& it, int step, int image) __attribute__((always_inline)) {
-    const int pos = it.lo + step * MS_STEP + row_in_step;
-    ms_dma4(CL_ARG_INDICES + (pos < it.hi - 1 ? pos : it.hi - 1), ids_byte + (unsigned)((image % MS_STAGES) * 256));
+    const int pos = it.lo + step * MD_STEP + row_in_step;
+    md_dma4(CL_ARG_INDICES + (pos < it.hi - 1 ? pos : it.hi - 1), ids_byte + (unsigned)((image % MD_STAGES) * 256));
   };
   // where the loads of an image come from, and the LDS bytes of the first of them and from one to the next
-  const char* src[MS_PANELS];
+  const char* src[MD_PANELS];
   unsigned dst, pitch;
   auto key_rows = [&](int image) __attribute__((always_inline)) {
-    const int id = ms_clamp(ms_ids[loader][image % MS_STAGES][lane], 0, num_pages - 1);
+    const int id = md_clamp(md_ids[loader][image % MD_STAGES][lane], 0, num_pages - 1);
     const char* lat = reinterpret_cast<const char*>(CL_ARG_KV) + ((i64)id * CL_CKV + 8 * row_chunk) * 2;
     const char* pe = reinterpret_cast<const char*>(CL_ARG_KPE) + ((i64)id * CL_KPE + 8 * row_chunk) * 2;
 #pragma unroll
-    for (int p = 0; p < MS_PANELS; ++p) src[p] = p < MS_LAT_PANELS ? lat + 128 * p : pe + 128 * (p - MS_LAT_PANELS);
-    dst = tiles_byte + (unsigned)((image % MS_STAGES) * MS_TILE * 2 + loader * 1024);
-    pitch = MS_PANEL * 2;
+    for (int p = 0; p < MD_PANELS; ++p) src[p] = p < MD_LAT_PANELS ? lat + 128 * p : pe + 128 * (p - MD_LAT_PANELS);
+    dst = tiles_byte + (unsigned)((image % MD_STAGES) * MD_TILE * 2 + loader * 1024);
+    pitch = MD_PANEL * 2;
   };
   auto query_rows = [&](const MsItem& it, int part, int image) __attribute__((always_inline)) {
     int at = lane;
     asm volatile("" : "+v"(at));                   // (what follows from it is kept from leaving the loop: 27 registers for its whole length)
 #pragma unroll
-    for (int j = 0; j < MS_PANELS; ++j) src[j] = query_piece(it, part, j, at);
-    dst = query_dst + (unsigned)((image % MS_STAGES) * MS_TILE * 2);
+    for (int j = 0; j < MD_PANELS; ++j) src[j] = query_piece(it, part, j, at);
+    dst = query_dst + (unsigned)((image % MD_STAGES) * MD_TILE * 2);
     pitch = 1024;
   };
   auto load_all = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int p = 0; p < MS_PANELS; ++p) ms_dma16(src[p], dst + p * pitch);
+    for (int p = 0; p < MD_PANELS; ++p) md_dma16_loose(src[p], dst + p * pitch);
   };
-  f32x4 acc[2][MS_FBW];                             // acc[t][fb][r] = O[head 16 t + c][16 (FBW half + fb) + 4 g + r]
+  f32x4 acc[2][MD_FBW];                             // acc[t][fb][r] = O[head 16 t + c][16 (FBW half + fb) + 4 g + r]
   elem8 ones;
 #pragma unroll
   for (int i = 0; i < 8; ++i) ones[i] = to_elem(1.0f);
   f32x4 l_acc[2];                                   // every component: sum of the weights of head c (both feature halves keep it)
   float m_acc[2];                                   // the reference point accumulators and sums stand against
   const int vtok = 4 * g + (c >> 2);
-  const int v_lo = half * (MS_FBW / 4) * MS_PANEL + vtok * 64 + (((((c & 3) >> 1)) ^ ms_swz(vtok)) << 3) + 4 * (c & 1);
+  const int v_lo = half * (MD_FBW / 4) * MD_PANEL + vtok * 64 + (((((c & 3) >> 1)) ^ md_swz(vtok)) << 3) + 4 * (c & 1);
   auto clear = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
 #pragma unroll
-      for (int fb = 0; fb < MS_FBW; ++fb) acc[t][fb] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      for (int fb = 0; fb < MD_FBW; ++fb) acc[t][fb] = (f32x4){0.f, 0.f, 0.f, 0.f};
       l_acc[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
       m_acc[t] = CL_NEG_BIG;
     }
@@ -474,22 +422,17 @@ CL_STAY_NAME(CL_STAY_PARAMS) {
   // the value operands of the first MS_PRE feature blocks of the next image: read at the end of an
   // iteration, they are on their way while the waves meet at the barrier
   constexpr int MS_PRE = CL_LDS_AHEAD / 2;
-  static_assert(MS_PRE >= 1 && MS_FBW % MS_PRE == 0, "the read-ahead operands are a ring the feature blocks walk whole turns of");
-  ms_s16x4 pre_lo[MS_PRE], pre_hi[MS_PRE];
+  static_assert(MS_PRE >= 1 && MD_FBW % MS_PRE == 0, "the read-ahead operands are a ring the feature blocks walk whole turns of");
+  md_s16x4 pre_lo[MS_PRE], pre_hi[MS_PRE];
 #pragma unroll
-  for (int fb = 0; fb < MS_PRE; ++fb) pre_lo[fb] = pre_hi[fb] = (ms_s16x4){0, 0, 0, 0};
-  auto operand = [&](const elem_t* tile, int fb, ms_s16x4& lo, ms_s16x4& hi) __attribute__((always_inline)) {
-    const elem_t* p = tile + (fb >> 2) * MS_PANEL + (v_lo ^ (((2 * fb) & 7) << 3));
-    lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ms_lds_s16x4*)(p));
-    hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ms_lds_s16x4*)(p + 16 * 64));
-  };
+  for (int fb = 0; fb < MS_PRE; ++fb) pre_lo[fb] = pre_hi[fb] = (md_s16x4){0, 0, 0, 0};
   // An item's rows: a lane holds features 16 fb + 4 g .. + 3 of its head for every block fb of the wave's half.  Lanes g and g ^ 1
   // trade halves of a pair of blocks (one row swap per register), so that each stores 16 contiguous bytes.
   auto store_rows = [&](const MsItem& it, int t, int from, int to) __attribute__((always_inline)) {
     const int token = it.t_lo + 2 * set + t;
     if (token >= it.t_hi) return;
     const float inv = 1.0f / fmaxf(l_acc[t][0], 1.0e-30f);
-    elem_t* row = CL_ARG_OUT + ((i64)token * CL_HEADS + it.head0 + c) * CL_CKV + 16 * MS_FBW * half + 16 * (g & 1) + 4 * (g & 2);
+    elem_t* row = CL_ARG_OUT + ((i64)token * CL_HEADS + it.head0 + c) * CL_CKV + 16 * MD_FBW * half + 16 * (g & 1) + 4 * (g & 2);
 #pragma unroll
     for (int fp = from; fp < to; ++fp) {
       elem4 y0, y1;
@@ -509,7 +452,7 @@ CL_STAY_NAME(CL_STAY_PARAMS) {
   ask_ids(cur, 1, 3);
   query_rows(cur, 1, 1);                            // (image 0 comes through the score waves)
   load_all();
-  MS_WAITCNT(MS_PANELS);                            // (the entries)
+  MS_WAITCNT(MD_PANELS);                            // (the entries)
   key_rows(2);
   load_all();
   MsItem next = cur, last = cur;
@@ -523,12 +466,12 @@ CL_STAY_NAME(CL_STAY_PARAMS) {
   // its stores; the entries that this iteration reads are ahead of it.  (The stores of an item of fewer tokens are fewer:
   // they are waited for.)
   auto arrive = [&](int r) __attribute__((always_inline)) {
-    if (late == 0) MS_WAITCNT(MS_PANELS + 1);
-    else if (late == 1) MS_WAITCNT(MS_PANELS + 1 + MS_STORES * 3 / 4);
-    else if (late == 2) MS_WAITCNT(MS_PANELS + 1 + MS_STORES);
-    else MS_WAITCNT(MS_PANELS + 1 + MS_STORES / 4);
+    if (late == 0) MS_WAITCNT(MD_PANELS + 1);
+    else if (late == 1) MS_WAITCNT(MD_PANELS + 1 + MS_STORES * 3 / 4);
+    else if (late == 2) MS_WAITCNT(MD_PANELS + 1 + MS_STORES);
+    else MS_WAITCNT(MD_PANELS + 1 + MS_STORES / 4);
     late = late > 0 ? late - 1 : 0;
-    ms_barrier();
+    md_barrier();
     if (r == cur.n) next = ms_item(parity ^ 1);
     const bool more = r >= cur.n && next.n > 0;
     if (more) ask_ids(next, r - cur.n, image + 4);
@@ -536,118 +479,70 @@ CL_STAY_NAME(CL_STAY_PARAMS) {
     if (more && r < cur.n + 2) query_rows(next, r - cur.n, image + 2);
     else key_rows(image + 2);                       // (behind the last item: rows nobody reads)
   };
-  ms_barrier();
+  md_barrier();
   ask_ids(cur, 2, 4);                               // (image 2 is on its way)
   for (;;) {
     ++image;
     arrive(1);
     load_all();
     if (begun) {
-      store_rows(last, 0, 0, MS_FBW / 4);
-      late = last.t_hi - last.t_lo == MS_TOKENS ? 3 : 0;
+      store_rows(last, 0, 0, MD_FBW / 4);
+      late = last.t_hi - last.t_lo == MD_TOKENS ? 3 : 0;
     }
     ++image;
     arrive(2);
     load_all();
     if (begun) {
-      store_rows(last, 0, MS_FBW / 4, MS_FBW / 2);
-      store_rows(last, 1, 0, MS_FBW / 4);
+      store_rows(last, 0, MD_FBW / 4, MD_FBW / 2);
+      store_rows(last, 1, 0, MD_FBW / 4);
     }
-    ms_barrier();                                   // (the score waves exchange their first maxima: the points of step 0)
-    if (begun) store_rows(last, 1, MS_FBW / 4, MS_FBW / 2);
+    md_barrier();                                   // (the score waves exchange their first maxima: the points of step 0)
+    if (begun) store_rows(last, 1, MD_FBW / 4, MD_FBW / 2);
     clear();
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-      const f32x2 start = *reinterpret_cast<const f32x2*>(&ms_ref[(image & 1) ^ 1][set][t][c][0]);
+      const f32x2 start = *reinterpret_cast<const f32x2*>(&md_ref[(image & 1) ^ 1][set][t][c][0]);
       m_acc[t] = fmaxf(start[0], start[1]);
     }
 #pragma unroll
-    for (int fb = 0; fb < MS_PRE; ++fb) operand(ms_tiles + (image % MS_STAGES) * MS_TILE, fb, pre_lo[fb], pre_hi[fb]);
+    for (int fb = 0; fb < MS_PRE; ++fb) md_operand(md_tiles + (image % MD_STAGES) * MD_TILE, v_lo, fb, pre_lo[fb], pre_hi[fb]);
     for (int r = 3; r <= cur.n + 2; ++r) {
       ++image;
       arrive(r);
-      const elem_t* next_tile = ms_tiles + (image % MS_STAGES) * MS_TILE;      // image `image`: there from here on
-      const elem_t* tile = ms_tiles + ((image - 1) % MS_STAGES) * MS_TILE;
+      const elem_t* next_tile = md_tiles + (image % MD_STAGES) * MD_TILE;      // image `image`: there from here on
+      const elem_t* tile = md_tiles + ((image - 1) % MD_STAGES) * MD_TILE;
       elem8 pf[2];
       f32x2 ref[2];
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         {
-          const u32x2 lo2 = ms_weights[(image - 1) & 1][set][t][0][lane], hi2 = ms_weights[(image - 1) & 1][set][t][1][lane];
+          const u32x2 lo2 = md_weights[(image - 1) & 1][set][t][0][lane], hi2 = md_weights[(image - 1) & 1][set][t][1][lane];
           pf[t] = as_elem8((u32x4){lo2[0], lo2[1], hi2[0], hi2[1]});
         }
-        ref[t] = *reinterpret_cast<const f32x2*>(&ms_ref[(image - 1) & 1][set][t][c][0]);
+        ref[t] = *reinterpret_cast<const f32x2*>(&md_ref[(image - 1) & 1][set][t][c][0]);
       }
       if (__builtin_amdgcn_ballot_w64(ref[0][0] != m_acc[0] || ref[0][1] != m_acc[0] || ref[1][0] != m_acc[1] ||
-                                      ref[1][1] != m_acc[1])) {
-        // cold: a score wave raised a reference point at this step.  The half that stands against the lower point is multiplied
-        // here, by itself, and the sums with it move to the higher point: its weights are 16 bits already, scaled they would
-        // be rounded a second time.  Per head tile, as mostly one of the two has a raised head: 8987 tokens at a scale that
-        // raises a point on every sixth step 160 us, both tiles together 163, weights rounded twice 157.
-        elem8 p_low[2];
-        float alpha[2];
-        if (__builtin_amdgcn_ballot_w64(fminf(ref[0][0], ref[0][1]) > m_acc[0] || fminf(ref[1][0], ref[1][1]) > m_acc[1])) {
-          // (both halves raised theirs: the sums move to the lower one first)
-#pragma unroll
-          for (int t = 0; t < 2; ++t) {
-            const float low = fminf(ref[t][0], ref[t][1]), a = fast_exp2(m_acc[t] - low);
-            m_acc[t] = low;
-#pragma unroll
-            for (int fb = 0; fb < MS_FBW; ++fb) acc[t][fb] *= a;
-            l_acc[t] *= a;
-          }
-        }
-        bool raised[2];
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          const float m_new = fmaxf(ref[t][0], ref[t][1]);          // never below m_acc
-          alpha[t] = fast_exp2(m_acc[t] - m_new);
-          raised[t] = __builtin_amdgcn_ballot_w64(ref[t][0] != m_acc[t] || ref[t][1] != m_acc[t]) != 0;
-          m_acc[t] = m_new;
-          p_low[t] = ms_halves(pf[t], ref[t][0] < ref[t][1], ref[t][1] < ref[t][0]);
-          pf[t] = ms_halves(pf[t], ref[t][0] >= ref[t][1], ref[t][1] >= ref[t][0]);
-          l_acc[t] = mfma16(ones, p_low[t], l_acc[t]) * alpha[t];
-        }
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          if (!raised[t]) continue;
-#pragma unroll
-          for (int fb0 = 0; fb0 < MS_FBW; fb0 += MS_COLD) {
-            __builtin_amdgcn_sched_barrier(0);
-            elem8 a[MS_COLD];
-#pragma unroll
-            for (int q = 0; q < MS_COLD; ++q) {
-              ms_s16x4 lo, hi;
-              operand(tile, fb0 + q, lo, hi);
-              a[q] = __builtin_bit_cast(elem8, (ms_s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-            }
-#pragma unroll
-            for (int q = 0; q < MS_COLD; ++q) acc[t][fb0 + q] = mfma16(a[q], p_low[t], acc[t][fb0 + q]);
-#pragma unroll
-            for (int q = 0; q < MS_COLD; ++q) acc[t][fb0 + q] *= alpha[t];
-          }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
+                                      ref[1][1] != m_acc[1]))
+        md_move_points(tile, v_lo, ref, ones, pf, m_acc, l_acc, acc);
       // out^T block fb: rows = features 16 fb + (0..15), slots = tokens 4 g + (0..3), 16 + 4 g + (0..3); the loads between the
-      // matrix ops, panel p after feature block p * MS_FBW / MS_PANELS
+      // matrix ops, panel p after feature block p * MD_FBW / MD_PANELS
 #pragma unroll
-      for (int fb = 0; fb < MS_FBW; ++fb) {
-        ms_s16x4 lo = pre_lo[fb % MS_PRE], hi = pre_hi[fb % MS_PRE];
-        const elem8 a = __builtin_bit_cast(elem8, (ms_s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+      for (int fb = 0; fb < MD_FBW; ++fb) {
+        md_s16x4 lo = pre_lo[fb % MS_PRE], hi = pre_hi[fb % MS_PRE];
+        const elem8 a = md_elem8(lo, hi);
 #pragma unroll
         for (int t = 0; t < 2; ++t) acc[t][fb] = mfma16(a, pf[t], acc[t][fb]);
         // the operand MS_PRE blocks on: of this image, or (the last MS_PRE) of the next one
-        if (fb + MS_PRE < MS_FBW)
-          operand(tile, fb + MS_PRE, pre_lo[fb % MS_PRE], pre_hi[fb % MS_PRE]);
+        if (fb + MS_PRE < MD_FBW)
+          md_operand(tile, v_lo, fb + MS_PRE, pre_lo[fb % MS_PRE], pre_hi[fb % MS_PRE]);
         else
-          operand(next_tile, fb + MS_PRE - MS_FBW, pre_lo[fb % MS_PRE], pre_hi[fb % MS_PRE]);
+          md_operand(next_tile, v_lo, fb + MS_PRE - MD_FBW, pre_lo[fb % MS_PRE], pre_hi[fb % MS_PRE]);
 #pragma unroll
-        for (int p = 0; p < MS_PANELS; ++p)
-          if ((p * MS_FBW) / MS_PANELS == fb) ms_dma16(src[p], dst + p * pitch);
+        for (int p = 0; p < MD_PANELS; ++p)
+          if ((p * MD_FBW) / MD_PANELS == fb) md_dma16_loose(src[p], dst + p * pitch);
       }
 #pragma unroll
-      for (int n = 0; n < MS_FBW; ++n) {
+      for (int n = 0; n < MD_FBW; ++n) {
         __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
         __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
       }
@@ -660,8 +555,8 @@ CL_STAY_NAME(CL_STAY_PARAMS) {
     if (next.n == 0) break;
     cur = next;
   }
-  store_rows(last, 0, 0, MS_FBW / 2);
-  store_rows(last, 1, 0, MS_FBW / 2);
+  store_rows(last, 0, 0, MD_FBW / 2);
+  store_rows(last, 1, 0, MD_FBW / 2);
   MS_WAITCNT(0);                                    // no load may still be on its way into LDS when the workgroup ends
 }
 #endif  // CL_EMIT_STAY
